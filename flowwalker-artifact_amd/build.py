@@ -28,7 +28,7 @@ HIP_FLAGS = [
     "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
 ]
 
-KERNEL_SOURCES = ["fw_walk_kernel.hip", "fw_ref_walk.hip", "fw_sampler_baselines.hip", "fw_api.hip", "fw_gen.hip", "fw_csr_io.hip"]
+KERNEL_SOURCES = ["fw_walk_kernel.hip", "fw_table_walk.hip", "fw_ref_walk.hip", "fw_sampler_baselines.hip", "fw_api.hip", "fw_gen.hip", "fw_csr_io.hip"]
 HOST_TOOLS = {"flowwalker": ["flowwalker_main.cpp"], "fw_gen": ["fw_gen_main.cpp"], "fw_convert": ["fw_convert_main.cpp"],
               "fw_sampler_bench": ["fw_sampler_bench_main.cpp"]}
 
@@ -52,7 +52,7 @@ def build_library():
         src, obj = pair
         _run([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, src), "-o", obj])
 
-    with ThreadPoolExecutor(max_workers=4) as ex:
+    with ThreadPoolExecutor(max_workers=6) as ex:
         list(ex.map(compile_one, zip(KERNEL_SOURCES, objs)))
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs)
     return LIB

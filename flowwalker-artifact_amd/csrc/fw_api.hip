@@ -326,6 +326,8 @@ extern "C" int fw_graph_destroy(fw_graph* g) {
   }
   release_park_cache(g);
   release_batch_cache(g);
+  g->tables.reset();
+  if (g->call_result) (void)hipHostFree(g->call_result);
   for (hipEvent_t e : g->call_ev) if (e) (void)hipEventDestroy(e);
   void* index_ptrs[4] = {g->hub_index, g->hub_info, g->call_scratch, g->adj_hub};
   for (void* p : index_ptrs) {
@@ -351,6 +353,9 @@ extern "C" int fw_graph_create_placed(int32_t V, uint64_t E, const uint32_t* h_x
   if (!g) { fw_set_error("out of host memory"); return FW_ERR_NOMEM; }
   g->V = V;
   g->E = E;
+  double squares = 0.0;
+  for (int32_t v = 0; v < V; ++v) squares += (double)(h_xadj[v + 1] - h_xadj[v]) * (double)(h_xadj[v + 1] - h_xadj[v]);
+  g->mean_list = squares / (double)E;
   g->owns = 1;
   g->host_edges = placement == FW_GRAPH_HOST_PINNED;
   auto fail = [&](int code) { fw_graph_destroy(g); return code; };
@@ -389,6 +394,7 @@ extern "C" int fw_graph_adopt_device(int32_t V, uint64_t E, uint32_t* d_xadj, in
   g->V = V; g->E = E;
   g->xadj = d_xadj; g->adjncy = d_adjncy; g->weight = d_weight; g->label = d_label;
   g->owns = take_ownership ? 1 : 0;
+  g->borrowed = 1;
   if (hipGetDevice(&g->device) != hipSuccess) { (void)hipGetLastError(); }
   *out = g;
   return FW_OK;
@@ -1172,6 +1178,7 @@ struct BatchCache {
   int32_t* d_starts = nullptr;
   int32_t* d_paths = nullptr;
   Scratch* d_scr = nullptr;
+  unsigned long long* d_stripes = nullptr;  // counters of walks on list tables
   size_t starts_cap = 0, paths_cap = 0, scr_cap = 0;  // elements
   ParkBuffers pbs[2];
   hipStream_t streams[2] = {nullptr, nullptr};
@@ -1185,8 +1192,10 @@ struct BatchCache {
     if (d_starts) (void)hipFree(d_starts);
     if (d_paths) (void)hipFree(d_paths);
     if (d_scr) (void)hipFree(d_scr);
+    if (d_stripes) (void)hipFree(d_stripes);
     d_starts = d_paths = nullptr;
     d_scr = nullptr;
+    d_stripes = nullptr;
     starts_cap = paths_cap = scr_cap = 0;
     for (ParkBuffers& pb : pbs) pb.release();
     for (hipStream_t& s : streams) {
@@ -1567,6 +1576,203 @@ static TrafficModel traffic_model(const fw_walk_params* p, int32_t n, bool parke
 }
 
 
+// The same for a walk on list tables: a step reads its vertex's record, a row and a lane of the list's table; path entries leave in
+// lines.  made: the tables were made in this call.
+static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params* p, int32_t n, bool made, uint64_t steps) {
+  TrafficModel m;
+  m.scattered_reads = 3 * steps + (uint64_t)n;
+  if (p->app == FW_APP_NODE2VEC) m.scattered_reads += 4 * steps;  // the searches in N(prev)
+  m.scattered_writes = steps / 16u + 2u * (uint64_t)n;            // whole lines, the row's first and last entries
+  m.record_bytes = 4 * (uint64_t)n + 4 * (uint64_t)n * (uint64_t)p->max_depth;
+  if (made) {
+    m.list_bytes = 8 * g->E;
+    m.record_bytes += 9 * g->E + 24 * (uint64_t)g->V;
+  }
+  return m;
+}
+
+// ---- list tables: when, and making them ---------------------------------------------------------------------
+//
+// A walk on list tables reads three or four blocks of memory per step, whatever the lists' lengths; without them a step
+// reads its list.  Making them reads and writes about 17 bytes per edge and allocates, so they are made once the calls on a
+// graph have spent without them (measured) or are about to spend (estimated) what they cost: a serving loop of small calls gets
+// them after a call or two and never pays more than about twice what it would have.
+// Estimates in milliseconds: lists stream at 6.5 TB/s, a step of a walk that finds the chip idle takes 2 us; the tables are
+// made at 4 TB/s (17 bytes per edge: 5.8 ms on 521 M edges, 0.24 ms of allocations and launches on a small graph), with
+// half as much again asked for before they are.
+constexpr double kStreamBytesPerMs = 6.5e9;
+constexpr double kStepLatencyMs = 0.002;
+constexpr double kMakeBytesPerMs = 4.0e9;
+constexpr double kMakeFixedMs = 0.25;
+constexpr double kMakeMargin = 1.5;
+
+__global__ void fw_square_sum_kernel(const uint32_t* __restrict__ xadj, int32_t V, double* sum) {
+  const int stride = gridDim.x * blockDim.x;
+  double s = 0.0;
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < V; v += stride) {
+    const double d = (double)(xadj[v + 1] - xadj[v]);
+    s += d * d;
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) s += __shfl_xor(s, d);
+  if ((threadIdx.x & 63u) == 0u && s != 0.0) atomicAdd(sum, s);
+}
+
+// The graph's launch record: Scratch and the counters of a table walk, allocated once.
+static int call_scratch(fw_graph* g) {
+  if (!g->call_scratch) FW_HIP(hipMalloc(&g->call_scratch, sizeof(Scratch) + FW_TABLE_COUNTER_BYTES));
+  return FW_OK;
+}
+
+static int mean_list_length(fw_graph* g, double* out) {
+  if (g->mean_list < 0.0) {
+    int rc = call_scratch(g);
+    if (rc != FW_OK) return rc;
+    double* const d_sum = static_cast<double*>(g->call_scratch);
+    double sum = 0.0;
+    FW_HIP(hipMemset(d_sum, 0, sizeof(double)));
+    hipLaunchKernelGGL(fw_square_sum_kernel, dim3(256), dim3(256), 0, 0, g->xadj, g->V, d_sum);
+    FW_HIP(hipMemcpy(&sum, d_sum, sizeof(double), hipMemcpyDeviceToHost));
+    g->mean_list = sum / (double)g->E;
+  }
+  *out = g->mean_list;
+  return FW_OK;
+}
+
+// Room for the tables of `g`: positions of the regions, work lists, memory.  FW_ERR_NOMEM when there is no room for them.
+static int plan_tables(const fw_graph* g, fw_tables* t, uint32_t** d_base_out, hipStream_t stream) {
+  const size_t nv = (size_t)g->V + 1u;
+  const size_t item_cap = (size_t)(g->E / 500u) + 64u, long_cap = (size_t)(g->E / 1000u) + 64u;  // a list of several groups has over 1020 entries
+  uint32_t* d_blocks = nullptr;
+  uint32_t* d_ctrs = nullptr;
+  void* tmp = nullptr;
+  size_t tmp_bytes = 0;
+  auto alloc = [](void** p, size_t bytes) -> int {
+    if (hipMalloc(p, bytes ? bytes : 16) == hipSuccess) return FW_OK;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return FW_ERR_NOMEM;
+  };
+  uint32_t h[3] = {0u, 0u, 0u};
+  auto plan = [&]() -> int {
+    int rc;
+    FW_HIP(rocprim::exclusive_scan(nullptr, tmp_bytes, d_blocks, d_blocks, 0u, nv, rocprim::plus<uint32_t>(), stream));
+    if ((rc = alloc(reinterpret_cast<void**>(&d_blocks), nv * 4u)) || (rc = alloc(reinterpret_cast<void**>(&d_ctrs), 64)) ||
+        (rc = alloc(&tmp, tmp_bytes)) || (rc = alloc(reinterpret_cast<void**>(&t->longs), long_cap * 4u)) ||
+        (rc = alloc(reinterpret_cast<void**>(&t->items), item_cap * sizeof(uint2))) ||
+        (rc = alloc(reinterpret_cast<void**>(&t->flag), 64)) || (rc = alloc(reinterpret_cast<void**>(&t->vrec), (size_t)g->V * sizeof(uint4))))
+      return rc;
+    FW_HIP(hipMemsetAsync(d_ctrs, 0, 64, stream));
+    if ((rc = fw_table_plan(g, t->hub_threshold, d_blocks, t->longs, t->items, d_ctrs, stream)) != FW_OK) return rc;
+    FW_HIP(rocprim::exclusive_scan(tmp, tmp_bytes, d_blocks, d_blocks, 0u, nv, rocprim::plus<uint32_t>(), stream));
+    FW_HIP(hipMemcpyAsync(&h[0], d_ctrs, 8, hipMemcpyDeviceToHost, stream));
+    FW_HIP(hipMemcpyAsync(&h[2], d_blocks + g->V, 4, hipMemcpyDeviceToHost, stream));
+    FW_HIP(hipStreamSynchronize(stream));
+    t->n_longs = h[0];
+    t->n_items = h[1];
+    if (h[0] > long_cap || h[1] > item_cap) { fw_set_error("internal: %u long lists, %u groups", h[0], h[1]); return FW_ERR_INVALID; }
+    return alloc(reinterpret_cast<void**>(&t->data), (size_t)h[2] * 128u + 128u);
+  };
+  const int rc = plan();
+  if (d_ctrs) (void)hipFree(d_ctrs);
+  if (tmp) (void)hipFree(tmp);
+  if (rc != FW_OK) {
+    if (d_blocks) (void)hipFree(d_blocks);
+    return rc;
+  }
+  t->bytes = (size_t)h[2] * 128u + (size_t)g->V * sizeof(uint4);
+  *d_base_out = d_blocks;
+  return FW_OK;
+}
+
+// The tables a call over n queries walks on, or none (*out stays empty).  Called with the graph's busy flag held.  ev_start is
+// recorded before the making, ev0 and ev1 around it when its time is asked for; *launches: kernels it took.
+static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipStream_t stream, std::shared_ptr<fw_tables>* out,
+                           int* launches, hipEvent_t ev_start, hipEvent_t ev0, hipEvent_t ev1) {
+  *launches = 0;
+  // an explicit parking degree asks for the parking pipeline, a negative one for walkers that stream their lists
+  if (p->park_threshold != 0 || p->app == FW_APP_METAPATH || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) ||
+      g->host_edges || g->no_tables || (p->wg_threads != 256 && p->wg_threads != 512 && p->wg_threads != 1024) ||
+      (p->app == FW_APP_NODE2VEC && p->max_depth > FW_REC_LEN_MASK))
+    return FW_OK;
+  const uint32_t nw_shift = p->wg_threads == 256 ? 2u : (p->wg_threads == 512 ? 3u : 4u);
+  std::shared_ptr<fw_tables> t;
+  {
+    std::lock_guard<std::mutex> guard(g->tables_lock);
+    t = g->tables;
+  }
+  if (t && (t->hub_threshold != p->hub_threshold || t->nw_shift != nw_shift)) t.reset();
+  if (t && !g->borrowed && p->time_kernels == 0) {  // (a call that wants the split of its time makes them anew)
+    *out = t;
+    return FW_OK;
+  }
+  if (!t || g->borrowed) {
+    double steps = (double)(p->max_depth - 1);
+    if (p->app == FW_APP_PPR && p->tp > 0.0f && 1.0 / (double)p->tp < steps) steps = 1.0 / (double)p->tp;
+    double ms = steps * kStepLatencyMs;
+    if (steps * (double)n >= 1.0e6) {  // (a smaller first call costs little more than asking: 0.04 ms)
+      double mean = 0.0;
+      const int rc = mean_list_length(g, &mean);
+      if (rc != FW_OK) return rc;
+      const double stream_ms = steps * (double)n * mean * 4.0 / kStreamBytesPerMs;
+      if (ms < stream_ms) ms = stream_ms;
+    }
+    if (g->streamed_ms + ms < kMakeMargin * (17.0 * (double)g->E / kMakeBytesPerMs + kMakeFixedMs)) return FW_OK;
+  }
+  uint32_t* d_base = nullptr;
+  if (!t) {
+    {
+      std::lock_guard<std::mutex> guard(g->tables_lock);
+      g->tables.reset();  // another granularity: one set per graph
+    }
+    t = std::make_shared<fw_tables>();
+    t->hub_threshold = p->hub_threshold;
+    t->nw_shift = nw_shift;
+    const int rc = plan_tables(g, t.get(), &d_base, stream);
+    if (rc == FW_ERR_NOMEM) {
+      g->no_tables = 1;
+      return FW_OK;
+    }
+    if (rc != FW_OK) return rc;
+  }
+  uint32_t bad = 0u;
+  auto make = [&]() -> int {
+    if (ev_start) FW_HIP(hipEventRecord(ev_start, stream));
+    if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev0, stream));
+    FW_HIP(hipMemsetAsync(t->flag, 0, sizeof(uint32_t), stream));
+    const int rc = fw_table_make(g, t.get(), d_base, stream, launches);
+    if (rc != FW_OK) return rc;
+    if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
+    FW_HIP(hipMemcpyAsync(&bad, t->flag, sizeof(bad), hipMemcpyDeviceToHost, stream));
+    FW_HIP(hipStreamSynchronize(stream));
+    return FW_OK;
+  };
+  const int rc = make();
+  if (d_base) (void)hipFree(d_base);
+  if (rc != FW_OK) return rc;
+  if (bad != 0u) {  // the streaming kernels define what happens then
+    if (!g->borrowed) g->no_tables = 1;
+    *launches = 0;
+    return FW_OK;
+  }
+  {
+    std::lock_guard<std::mutex> guard(g->tables_lock);
+    g->tables = t;
+  }
+  *out = t;
+  return FW_OK;
+}
+
+static fw_table_args table_args(const fw_tables& t, unsigned long long* d_counters) {
+  fw_table_args tb;
+  tb.vrec = t.vrec;
+  tb.data = t.data;
+  tb.nw_shift = t.nw_shift;
+  tb.chunk = tb.lanes = 0u;
+  tb.counters = d_counters;
+  return tb;
+}
+
 // One walk call at a time per graph: the parking index, the parking lists and the launch record are cached in the
 // graph, so a second call that started while one is running would rebuild or overwrite them under it.
 struct BusyGuard {
@@ -1597,25 +1803,12 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
   const double t0 = now_ms();
 
   const int32_t park_threshold = resolve_park_threshold(g, p, n);
-  ParkBuffers* pb = nullptr;
-  bool use_pb = false;
-  if (park_threshold != INT_MAX) {
-    rc = ensure_hub_index(const_cast<fw_graph*>(g), park_threshold);
-    if (rc != FW_OK) return rc;
-    // buckets = parked-on vertices x labels must stay a 30-bit count (bucket ids travel in 32-bit record fields)
-    use_pb = g->n_hubs > 0 &&
-             (int64_t)g->n_hubs * (p->app == FW_APP_METAPATH ? p->schema_len : 1) <= ((int64_t)1 << 30);
-  }
-  if (use_pb) {
-    const int labels = p->app == FW_APP_METAPATH ? p->schema_len : 1;
-    pb = cached_park_buffers(const_cast<fw_graph*>(g), (size_t)n, g->n_hubs * labels, two_pass_rows(g, labels));
-    use_pb = pb != nullptr;  // no room for the parking lists: walk without parking (same results, one launch)
-  }
-  // the launch record and the two timing events are the graph's, made once
+  // the launch record and the timing events are the graph's, made once
   fw_graph* mg = const_cast<fw_graph*>(g);
-  if (!mg->call_scratch) FW_HIP(hipMalloc(&mg->call_scratch, sizeof(Scratch)));
-  for (hipEvent_t& e : mg->call_ev) if (!e) FW_HIP(hipEventCreate(&e));
+  if ((rc = call_scratch(mg)) != FW_OK) return rc;
+  for (int i = 0; i < (p->time_kernels != 0 ? 4 : 2); ++i) if (!mg->call_ev[i]) FW_HIP(hipEventCreate(&mg->call_ev[i]));
   Scratch* const d_scr = static_cast<Scratch*>(mg->call_scratch);
+  unsigned long long* const d_counters = reinterpret_cast<unsigned long long*>(d_scr + 1);  // of a table walk
   const hipEvent_t ev0 = mg->call_ev[0], ev1 = mg->call_ev[1];
   auto cleanup = [&]() {};
 #define FW_TRY(call)                                                 \
@@ -1623,9 +1816,6 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
     int rc_ = fw_check_hip((call), #call, __FILE__, __LINE__);       \
     if (rc_ != FW_OK) { cleanup(); return rc_; }                     \
   } while (0)
-  FW_TRY(hipMemsetAsync(d_scr, 0, sizeof(Scratch), stream));
-  // -1 fill of the path matrix: src/walk.cu:398, :536
-  FW_TRY(hipMemsetAsync(d_paths, 0xFF, (size_t)n * (size_t)p->max_depth * sizeof(int32_t), stream));
 
   fw_kargs a;
   fill_kargs(&a, g, p);
@@ -1636,15 +1826,57 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
   a.counters = d_scr->counters;
   int grid_used = 0, launches = 0;
   KernelTimes times;
-  FW_TRY(hipEventRecord(ev0, stream));
-  rc = run_walk_launches(g, p, a, park_threshold, use_pb ? pb : nullptr, stream, &grid_used, &launches, &times);
-  if (rc != FW_OK) { cleanup(); return rc; }
+  std::shared_ptr<fw_tables> tables;
+  rc = tables_for_call(mg, p, n, stream, &tables, &launches, ev0, mg->call_ev[2], mg->call_ev[3]);
+  if (rc != FW_OK) return rc;
+  if (tables) {
+    a.park_threshold = park_threshold;
+    if (launches == 0) FW_TRY(hipEventRecord(ev0, stream));  // (tables made in this call: recorded before that)
+    if (!mg->call_result) FW_TRY(hipHostMalloc(reinterpret_cast<void**>(&mg->call_result), 64, hipHostMallocDefault));
+    if ((rc = fw_table_begin(d_counters, stream)) != FW_OK) return rc;
+    rc = fw_launch_table_walk(a, table_args(*tables, d_counters), p->app, p->grid, stream, &grid_used);
+    if (rc != FW_OK) return rc;
+    if ((rc = fw_table_end(d_counters, mg->call_result, stream)) != FW_OK) return rc;
+    launches += 3;
+  } else {
+    FW_TRY(hipMemsetAsync(d_scr, 0, sizeof(Scratch), stream));
+    // -1 fill of the path matrix: src/walk.cu:398, :536
+    FW_TRY(hipMemsetAsync(d_paths, 0xFF, (size_t)n * (size_t)p->max_depth * sizeof(int32_t), stream));
+    ParkBuffers* pb = nullptr;
+    bool use_pb = false;
+    if (park_threshold != INT_MAX) {
+      rc = ensure_hub_index(mg, park_threshold);
+      if (rc != FW_OK) return rc;
+      // buckets = parked-on vertices x labels must stay a 30-bit count (bucket ids travel in 32-bit record fields)
+      use_pb = g->n_hubs > 0 &&
+               (int64_t)g->n_hubs * (p->app == FW_APP_METAPATH ? p->schema_len : 1) <= ((int64_t)1 << 30);
+    }
+    if (use_pb) {
+      const int labels = p->app == FW_APP_METAPATH ? p->schema_len : 1;
+      pb = cached_park_buffers(mg, (size_t)n, g->n_hubs * labels, two_pass_rows(g, labels));
+      use_pb = pb != nullptr;  // no room for the parking lists: walk without parking (same results, one launch)
+    }
+    FW_TRY(hipEventRecord(ev0, stream));
+    rc = run_walk_launches(g, p, a, park_threshold, use_pb ? pb : nullptr, stream, &grid_used, &launches, &times);
+    if (rc != FW_OK) { cleanup(); return rc; }
+  }
   FW_TRY(hipEventRecord(ev1, stream));
   FW_TRY(hipStreamSynchronize(stream));
   float ms = 0.0f;
   FW_TRY(hipEventElapsedTime(&ms, ev0, ev1));
   Scratch h;
-  FW_TRY(hipMemcpy(&h, d_scr, sizeof(h), hipMemcpyDeviceToHost));
+  if (!tables) FW_TRY(hipMemcpy(&h, d_scr, sizeof(h), hipMemcpyDeviceToHost));
+  if (tables) {
+    memcpy(h.counters, mg->call_result, sizeof(h.counters));
+    if (p->time_kernels != 0) {  // the split: the making of the tables, and the walk
+      float make_ms = 0.0f;
+      FW_TRY(hipEventElapsedTime(&make_ms, mg->call_ev[2], mg->call_ev[3]));
+      times.hub_ms = make_ms;
+      times.walk_ms = (double)ms - (double)make_ms;  // exact: both are floats
+    }
+  } else if (p->park_threshold == 0) {
+    mg->streamed_ms += (double)ms;
+  }
   cleanup();
   if (stats) {
     stats->kernel_ms = ms;
@@ -1657,8 +1889,9 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
     stats->hub_kernel_ms = times.hub_ms;
     stats->hub_steps = h.counters[2];
     stats->hub_sampled_edges = h.counters[3];
-    const TrafficModel tm = traffic_model(p, n, launches > 1, park_threshold, g->adj_hub != nullptr, h.counters[0],
-                                          h.counters[1], h.counters[2], times);
+    const TrafficModel tm = tables ? table_traffic_model(g, p, n, launches > 3, stats->steps)
+                                   : traffic_model(p, n, launches > 1, park_threshold, g->adj_hub != nullptr, h.counters[0],
+                                                   h.counters[1], h.counters[2], times);
     stats->requested_bytes = tm.total();
     stats->list_bytes = tm.list_bytes;
     stats->scattered_reads = tm.scattered_reads;
@@ -1833,8 +2066,19 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
   const int nbuf = sync || nbatch == 1 ? 1 : 2;  // buffers in flight
 
   const int32_t park_threshold = resolve_park_threshold(g, p, (int32_t)bs);
+  for (hipEvent_t& e : mg->call_ev) if (!e) FW_HIP(hipEventCreate(&e));
+  std::shared_ptr<fw_tables> tables;
+  int make_launches = 0;
+  rc = tables_for_call(mg, p, n, nullptr, &tables, &make_launches, mg->call_ev[0], mg->call_ev[2], mg->call_ev[3]);
+  if (rc != FW_OK) return rc;
+  float make_ms = 0.0f;
+  if (make_launches != 0) {
+    FW_HIP(hipEventRecord(mg->call_ev[1], nullptr));
+    FW_HIP(hipEventSynchronize(mg->call_ev[1]));
+    FW_HIP(hipEventElapsedTime(&make_ms, mg->call_ev[0], mg->call_ev[1]));
+  }
   bool use_pb = false;
-  if (park_threshold != INT_MAX) {
+  if (!tables && park_threshold != INT_MAX) {
     rc = ensure_hub_index(mg, park_threshold);
     if (rc != FW_OK) return rc;
     // buckets = parked-on vertices x labels must stay a 30-bit count (bucket ids travel in 32-bit record fields)
@@ -1879,7 +2123,12 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     FW_TRY(hipMalloc(reinterpret_cast<void**>(&bc->d_scr), sizeof(Scratch) * (size_t)nbatch));
     bc->scr_cap = (size_t)nbatch;
   }
-  FW_TRY(hipMemset(bc->d_scr, 0, sizeof(Scratch) * (size_t)nbatch));
+  if (!tables) FW_TRY(hipMemset(bc->d_scr, 0, sizeof(Scratch) * (size_t)nbatch));
+  if (tables) {  // the batches share one set of counters
+    if (!bc->d_stripes) FW_TRY(hipMalloc(reinterpret_cast<void**>(&bc->d_stripes), FW_TABLE_COUNTER_BYTES));
+    if (!mg->call_result) FW_TRY(hipHostMalloc(reinterpret_cast<void**>(&mg->call_result), 64, hipHostMallocDefault));
+    if ((rc = fw_table_begin(bc->d_stripes, nullptr)) != FW_OK) { cleanup(); return rc; }
+  }
   for (int i = 0; i < nbuf; ++i) if (!bc->streams[i]) FW_TRY(hipStreamCreate(&bc->streams[i]));
   while (bc->events.size() < (size_t)nbatch * 2) {
     hipEvent_t e = nullptr;
@@ -1897,7 +2146,7 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
   fill_kargs(&a, g, p);
   int grid_used = 0;
   KernelTimes times;
-  const double t0 = now_ms();
+  const double t0 = now_ms() - (double)make_ms;
   for (int b = 0; b < nbatch; ++b) {
     const int s = b % nbuf;
     const size_t first = (size_t)b * bs;
@@ -1905,7 +2154,7 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     int32_t* ds = d_starts + (size_t)s * bs;
     int32_t* dp = d_paths + (size_t)s * bs * md;
     FW_TRY(hipMemcpyAsync(ds, h_starts + first, (size_t)cnt * sizeof(int32_t), hipMemcpyHostToDevice, streams[s]));
-    FW_TRY(hipMemsetAsync(dp, 0xFF, (size_t)cnt * md * sizeof(int32_t), streams[s]));
+    if (!tables) FW_TRY(hipMemsetAsync(dp, 0xFF, (size_t)cnt * md * sizeof(int32_t), streams[s]));
     a.starts = ds;
     a.paths = dp;
     a.n = cnt;
@@ -1914,14 +2163,24 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     a.counters = d_scr[b].counters;
     FW_TRY(hipEventRecord(events[2 * b], streams[s]));
     int launches = 0;
-    rc = run_walk_launches(g, p, a, park_threshold, use_pb ? &pbs[s] : nullptr, streams[s], &grid_used, &launches,
-                           &times);
+    if (tables) {
+      a.park_threshold = park_threshold;
+      rc = fw_launch_table_walk(a, table_args(*tables, bc->d_stripes), p->app, p->grid, streams[s], &grid_used);
+    } else {
+      rc = run_walk_launches(g, p, a, park_threshold, use_pb ? &pbs[s] : nullptr, streams[s], &grid_used, &launches,
+                             &times);
+    }
     if (rc != FW_OK) { cleanup(); return rc; }
     FW_TRY(hipEventRecord(events[2 * b + 1], streams[s]));
     FW_TRY(hipMemcpyAsync(h_paths + first * md, dp, (size_t)cnt * md * sizeof(int32_t), hipMemcpyDeviceToHost, streams[s]));
     if (sync) FW_TRY(hipStreamSynchronize(streams[s]));
   }
-  for (int i = 0; i < nbuf; ++i) FW_TRY(hipStreamSynchronize(streams[i]));
+  if (tables) {  // the sums of the counters come last on the null stream, which waits for the two batch streams
+    if ((rc = fw_table_end(bc->d_stripes, mg->call_result, nullptr)) != FW_OK) { cleanup(); return rc; }
+    FW_TRY(hipStreamSynchronize(nullptr));
+  } else {
+    for (int i = 0; i < nbuf; ++i) FW_TRY(hipStreamSynchronize(streams[i]));
+  }
   const double total = now_ms() - t0;
 
   double kernel_ms = 0.0;
@@ -1931,7 +2190,17 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     kernel_ms += ms;
   }
   std::vector<Scratch> h((size_t)nbatch);
-  FW_TRY(hipMemcpy(h.data(), d_scr, sizeof(Scratch) * (size_t)nbatch, hipMemcpyDeviceToHost));
+  if (tables) {
+    memcpy(h[0].counters, mg->call_result, sizeof(h[0].counters));
+    if (p->time_kernels != 0) {
+      times.hub_ms = make_ms;
+      times.walk_ms = kernel_ms;
+    }
+    kernel_ms += make_ms;
+  } else {
+    FW_TRY(hipMemcpy(h.data(), d_scr, sizeof(Scratch) * (size_t)nbatch, hipMemcpyDeviceToHost));
+    if (p->park_threshold == 0) mg->streamed_ms += kernel_ms;
+  }
   if (stats) {
     stats->kernel_ms = kernel_ms;
     stats->total_ms = total;
@@ -1947,11 +2216,12 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     }
     stats->launches = nbatch;
     stats->grid = grid_used;
-    stats->walk_kernel_ms = stats->hub_steps == 0 ? kernel_ms : times.walk_ms;  // the split: with time_kernels only
+    stats->walk_kernel_ms = stats->hub_steps == 0 && make_launches == 0 ? kernel_ms : times.walk_ms;  // the split: with time_kernels only
     stats->hub_kernel_ms = times.hub_ms;
-    const TrafficModel tm = traffic_model(p, n, times.sorted_records != 0, park_threshold, g->adj_hub != nullptr,
-                                          stats->steps - stats->hub_steps,
-                                          stats->sampled_edges - stats->hub_sampled_edges, stats->hub_steps, times);
+    const TrafficModel tm = tables ? table_traffic_model(g, p, n, make_launches != 0, stats->steps)
+                                   : traffic_model(p, n, times.sorted_records != 0, park_threshold, g->adj_hub != nullptr,
+                                                   stats->steps - stats->hub_steps,
+                                                   stats->sampled_edges - stats->hub_sampled_edges, stats->hub_steps, times);
     stats->requested_bytes = tm.total();
     stats->list_bytes = tm.list_bytes;
     stats->scattered_reads = tm.scattered_reads;

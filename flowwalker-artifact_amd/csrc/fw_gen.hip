@@ -198,5 +198,6 @@ extern "C" int fw_gen_rmat(const fw_rmat_params* rp, fw_graph** out) {
   if (rc != FW_OK) return rc;
   xadj.release(); adjncy.release(); weight.release(); label.release();
   (*out)->sorted = 1;
+  (*out)->borrowed = 0;  // nobody outside the library knows these arrays
   return FW_OK;
 }

@@ -5,6 +5,8 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <memory>
+#include <mutex>
 
 #include "flowwalker.h"
 
@@ -16,6 +18,24 @@ struct fw_hub_info {
   uint32_t row;  // two-pass steps: first row of this list's groups (times the labels per hub), FW_NO_ROWS: none
 };
 constexpr uint32_t FW_NO_ROWS = 0xFFFFFFFFu;
+
+// List tables (fw_table_walk.hip): the walker-independent part of every sampling step on a graph.  Not changed once made, and
+// held by reference count: a call that walks on a set keeps it alive while another call replaces it in the graph.
+struct fw_tables {
+  uint4* vrec = nullptr;          // [V] {region in 128-byte blocks, degree, total, CSR offset}
+  unsigned char* data = nullptr;  // the regions
+  uint32_t* longs = nullptr;      // vertices whose lists have more than one group
+  uint2* items = nullptr;         // {vertex, group} for every group of those
+  uint32_t* flag = nullptr;       // set by the make kernels when a bias or a total is not a finite, non-negative number
+  uint32_t n_longs = 0, n_items = 0;
+  int32_t hub_threshold = 0;      // which long lists are cut into sequences, and how many of them (as a power of two):
+  uint32_t nw_shift = 0;          // part of the sampler's definition
+  size_t bytes = 0;
+  ~fw_tables() {
+    void* ptrs[5] = {vrec, data, longs, items, flag};
+    for (void* p : ptrs) if (p) (void)hipFree(p);
+  }
+};
 
 // Device CSR mirror (include/gpu_graph.cuh:28-36 in the reference).  Edge arrays are allocated with
 // FW_EDGE_PAD extra elements so that aligned 16-byte loads of the last quartet stay in bounds.
@@ -44,7 +64,15 @@ struct fw_graph {
   void* park_cache = nullptr;         // the parking lists of the last fw_walk_device call, kept for the next one
   void* batch_cache = nullptr;        // the device buffers of the last fw_walk_batch call, kept for the next one
   void* call_scratch = nullptr;       // launch record (dispenser word + counters) of fw_walk_device, allocated once
-  hipEvent_t call_ev[2] = {nullptr, nullptr};  // and its two timing events
+  unsigned long long* call_result = nullptr;  // pinned: the sums of a table walk's counters
+  hipEvent_t call_ev[4] = {};         // and its timing events: the call, the making of the list tables
+  int borrowed = 0;                   // the arrays came through fw_graph_adopt_device: their owner may change the biases
+                                      // between calls, so list tables are made anew in every call that walks on them
+  double mean_list = -1.0;            // sum of squared degrees / E: the list length a step meets, on average; lazily computed
+  double streamed_ms = 0.0;           // device time of the walk calls that had no list tables and might have had them
+  int no_tables = 0;                  // biases or totals the tables cannot hold, or no room for them: do not try again
+  std::mutex tables_lock;
+  std::shared_ptr<fw_tables> tables;
   std::atomic<int> busy{0};           // a walk call is running on this graph (the caches above are per graph)
 };
 
@@ -162,6 +190,20 @@ struct fw_hub_args {
   int32_t* lastpos;
 };
 
+// Workload counters of a table walk: FW_TABLE_STRIPES lines of {steps, source degrees, the same two for vertices above
+// the parking degree}, added up by the host.
+constexpr uint32_t FW_TABLE_STRIPES = 64;
+constexpr size_t FW_TABLE_COUNTER_BYTES = FW_TABLE_STRIPES * 64u;
+
+struct fw_table_args {
+  const uint4* vrec;
+  const unsigned char* data;
+  uint32_t nw_shift;
+  uint32_t chunk;                // queries of a wave (set by the launch)
+  uint32_t lanes;                // lanes of a wave that walk (set by the launch)
+  unsigned long long* counters;  // [FW_TABLE_STRIPES * 8]
+};
+
 #ifdef __HIPCC__
 // counter[key] += 1 for every lane with pred; returns the value the lane's own increment found (its rank among the
 // increments of that counter).  When several lanes of the wave share the first active lane's key (then the first
@@ -229,3 +271,13 @@ int fw_launch_hub_quad(const fw_kargs& a, const fw_hub_args& h, int app, uint32_
 // Launches the scan kernel of the two-pass steps (it finds its task count in h.nstasks on the device).
 // tasks_hint: about how many scan tasks to expect, to size the grid (0 = no idea: a full resident set).
 int fw_launch_hub_scan(const fw_kargs& a, const fw_hub_args& h, int app, uint32_t tasks_hint, hipStream_t stream);
+
+// List tables.  plan: region sizes into d_blocks[0 .. V], work lists and their sizes (d_ctrs[0]: long lists, [1]: items);
+// make: fills the tables (d_base: region positions, NULL when vrec has them); walk: every query from start to end, between
+// begin (counters to zero) and end (their sums to pinned host memory).
+int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
+                  hipStream_t stream);
+int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches);
+int fw_launch_table_walk(const fw_kargs& a, const fw_table_args& tb, int app, int grid, hipStream_t stream, int* grid_used);
+int fw_table_begin(unsigned long long* d_counters, hipStream_t stream);
+int fw_table_end(const unsigned long long* d_counters, unsigned long long* h_out, hipStream_t stream);

@@ -1,0 +1,806 @@
+// List tables and the walk over them.
+//
+// A sampling step of fw_walk_kernel.hip reads a whole neighbour list, and everything it computes from it -- the scan of a
+// group of 1024 biases, the group totals, their running sums -- is the same for every walker that ever stands there; a
+// walker contributes two uniforms per accepted group.  When the walkers of a call would read the lists many times over,
+// the walker-independent part is made once (one pass over the edges: 8 bytes read and 8 written per edge) and a step
+// becomes a few look-ups, so one lane walks one walker from its start to its end: no task table, no parking, no sorting.
+// The sampler's definition (fw_walk_kernel.hip) is untouched: the tables hold the very sums, prefixes and totals the streaming
+// kernels compute, in their order of additions, and the walk takes the same draws, so every walker gets the same vertex.
+//
+// Reference behaviour: as fw_walk_kernel.hip (include/walker.cuh:1307-1580, include/sampler.cuh:46-200).
+//
+// Layout.  vrec[v] = {region, degree, total, CSR offset}: `region` in blocks of 128 bytes (the memory's request size) into
+// `data`, `total` = the list's total as the step's sampler adds it up.  A region, in units of 32 bytes:
+//   list of one group (at most 256 aligned quartets):  row M, then the entries
+//   longer list:  header (sums), then per group {row M (8 units), entries}
+//   row M: for every lane of the group (a lane holds J quartets, J = 1 .. 4) the running maximum of the positive lanes' prefixes;
+//     from the last positive lane on +inf.  "First lane whose prefix exceeds the target, else the last positive lane" is then
+//     "first entry above the target".
+//   entries: lane after lane, 4 J pairs {key, neighbour}; key = the lane's running sum up to the element, for an element
+//     without bias the key before it, from the lane's last positive element on +inf: the element is the first key
+//     above the target.  A lane of a full group is 16 pairs = one block, so the pick and the neighbour come in one request.
+//   sums: per group {running sum of the group's sequence, group total}, sequence after sequence; with more than one
+//     sequence (workgroup granularity) 16 floats in front: the inclusive scan of the sequences' totals, as keys like the above.
+// All keys of a row or a lane never decrease, so any search finds the same entry; weights are close to evenly spread
+// over a list, so the searches start from the proportional guess and mostly end there.
+
+#include <hip/hip_runtime.h>
+
+#include "fw_internal.h"
+#include "fw_step_device.h"
+
+namespace {
+
+constexpr uint32_t kGq = 64u * kGroupQuartets;  // quartets of a full group
+constexpr uint32_t kGroupUnits = 8u + kGq;      // units of a group in a list of several: row M and the entries of 64 lanes
+constexpr float kInf = __builtin_inff();
+
+typedef float f4_at4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f4_at8 __attribute__((ext_vector_type(4), aligned(8)));
+typedef uint32_t u4_at8 __attribute__((ext_vector_type(4), aligned(8)));
+
+__device__ __forceinline__ uint32_t list_quartets(uint32_t off, uint32_t deg) { return ((off & 3u) + deg + 3u) >> 2; }
+
+// units of a long list's header: the sequences' keys (workgroup granularity only) and 8 bytes per group, whole blocks
+__device__ __forceinline__ uint32_t header_units(uint32_t ngroups, bool wg) {
+  return ((wg ? 2u : 0u) + ((ngroups + 3u) >> 2) + 3u) & ~3u;
+}
+
+// first entry of sequence `s` among a list's sums
+__device__ __forceinline__ uint32_t seq_start(uint32_t ngroups, uint32_t s, uint32_t nw_shift) {
+  const uint32_t per = ngroups >> nw_shift, rest = ngroups & ((1u << nw_shift) - 1u);
+  return s * per + (s < rest ? s : rest);
+}
+
+__device__ __forceinline__ uint32_t region_blocks(uint32_t off, uint32_t deg, bool wg) {
+  if (deg == 0u) return 0u;
+  const uint32_t nq = list_quartets(off, deg);
+  uint32_t units;
+  if (nq <= kGq) {
+    const uint32_t nl = nq < 64u ? nq : 64u;
+    units = ((nl + 7u) >> 3) + nl * ((nq + 63u) >> 6);
+  } else {
+    const uint32_t ngroups = (nq + kGq - 1u) / kGq;
+    const uint32_t last = nq - (ngroups - 1u) * kGq;
+    const uint32_t nl = last < 64u ? last : 64u;
+    units = header_units(ngroups, wg) + kGroupUnits * (ngroups - 1u) + 8u + nl * ((last + 63u) >> 6);
+  }
+  return (units + 3u) >> 2;
+}
+
+// ---- making the tables --------------------------------------------------------------------------------
+
+// Region sizes (scanned into positions afterwards) and the work lists of the lists longer than a group: `longs` their
+// vertices, `items` {vertex, group} for every group of them.  ctrs: [0] long lists, [1] items.  Every workgroup counts its
+// range of vertices first, so that it takes its places in the work lists with one update each.
+__global__ __launch_bounds__(1024) void fw_table_plan_kernel(const uint32_t* __restrict__ xadj, int32_t V, int32_t hub_threshold,
+                                                             uint32_t* __restrict__ blocks, uint32_t* longs, uint2* items,
+                                                             uint32_t* ctrs) {
+  __shared__ uint32_t s_n[2], s_at[2];
+  if (threadIdx.x < 2u) s_n[threadIdx.x] = 0u;
+  __syncthreads();
+  const uint32_t per = ((uint32_t)V + gridDim.x - 1u) / gridDim.x;
+  const uint32_t v0 = blockIdx.x * per;
+  const uint32_t v1 = v0 + per < (uint32_t)V ? v0 + per : (uint32_t)V;
+  uint32_t n_long = 0u, n_items = 0u;
+  for (uint32_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) {
+    const uint32_t off = xadj[v], deg = xadj[v + 1] - off;
+    blocks[v] = region_blocks(off, deg, (int32_t)deg > hub_threshold);
+    const uint32_t nq = list_quartets(off, deg);
+    if (nq > kGq) {
+      ++n_long;
+      n_items += (nq + kGq - 1u) / kGq;
+    }
+  }
+  if (n_long != 0u) {
+    atomicAdd(&s_n[0], n_long);
+    atomicAdd(&s_n[1], n_items);
+  }
+  __syncthreads();
+  if (threadIdx.x < 2u) s_at[threadIdx.x] = s_n[threadIdx.x] != 0u ? atomicAdd(&ctrs[threadIdx.x], s_n[threadIdx.x]) : 0u;
+  if (blockIdx.x == 0u && threadIdx.x == 0u) blocks[V] = 0u;
+  __syncthreads();
+  if (s_n[0] == 0u) return;
+  for (uint32_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) {
+    const uint32_t off = xadj[v], deg = xadj[v + 1] - off;
+    const uint32_t nq = list_quartets(off, deg);
+    if (nq > kGq) {
+      const uint32_t ngroups = (nq + kGq - 1u) / kGq;
+      longs[atomicAdd(&s_at[0], 1u)] = v;
+      const uint32_t at = atomicAdd(&s_at[1], ngroups);
+      for (uint32_t g = 0; g < ngroups; ++g) items[at + g] = make_uint2(v, g);
+    }
+  }
+}
+
+// The 4 kJ biases and neighbours of lane `lane` in the group of `nqg` quartets that starts at quartet kb of a list (an entry outside the
+// list has no bias).  Sets `bad` when a bias is negative or not a number.
+template <int kJ>
+__device__ __forceinline__ void load_lane(const float* __restrict__ weight, const int32_t* __restrict__ adjncy, uint32_t off,
+                                          uint32_t deg, uint32_t kb, uint32_t nqg, uint32_t lane, float (&x)[4 * kJ],
+                                          int32_t (&nb)[4 * kJ], bool& bad) {
+  const uint32_t a0 = off & ~3u;
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) {
+    const uint32_t k = lane + 64u * (uint32_t)j;
+    float4 w = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    int4 n = make_int4(-1, -1, -1, -1);
+    const uint32_t base = a0 + 4u * (kb + k);
+    if (k < nqg) {
+      w = *reinterpret_cast<const float4*>(weight + base);
+      n = *reinterpret_cast<const int4*>(adjncy + base);
+    }
+    const uint32_t li = base - off;  // wraps below 0 for the head quartet
+    const uint32_t lim = k < nqg ? deg : 0u;
+    x[4 * j + 0] = li < lim ? w.x : 0.0f;
+    x[4 * j + 1] = li + 1u < lim ? w.y : 0.0f;
+    x[4 * j + 2] = li + 2u < lim ? w.z : 0.0f;
+    x[4 * j + 3] = li + 3u < lim ? w.w : 0.0f;
+    nb[4 * j + 0] = li < lim ? n.x : -1;
+    nb[4 * j + 1] = li + 1u < lim ? n.y : -1;
+    nb[4 * j + 2] = li + 2u < lim ? n.z : -1;
+    nb[4 * j + 3] = li + 3u < lim ? n.w : -1;
+  }
+#pragma unroll
+  for (int i = 0; i < 4 * kJ; ++i) bad = bad || !(x[i] >= 0.0f);
+}
+
+// The lane's pairs: e0 = its prefix before its own elements.  The first 4 J of the 4 kJ elements are stored.
+template <int kJ>
+__device__ __forceinline__ void store_lane(uint2* out, uint32_t J, float e0, const float (&x)[4 * kJ], const int32_t (&nb)[4 * kJ]) {
+  uint32_t pm = 0u;
+#pragma unroll
+  for (int i = 0; i < 4 * kJ; ++i) pm |= (x[i] > 0.0f ? 1u : 0u) << i;
+  const int last = 31 - __builtin_clz(pm | 1u);
+  float e = e0, key = 0.0f;
+  uint4* o = reinterpret_cast<uint4*>(out);
+#pragma unroll
+  for (int i = 0; i < 4 * kJ; i += 2) {
+    uint32_t k[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      e = e + x[i + b];
+      key = x[i + b] > 0.0f ? e : key;
+      k[b] = __float_as_uint(pm != 0u && i + b >= last ? kInf : key);
+    }
+    if ((uint32_t)i < 4u * J) o[i >> 1] = make_uint4(k[0], (uint32_t)nb[i], k[1], (uint32_t)nb[i + 1]);
+  }
+}
+
+// One list of at most kSeg quartets per segment of kSeg lanes (one or two DPP rows, or the wave); off, deg, region are the
+// segment's.  Returns the list's total in every lane of the segment.  The scan network is the packed step's.
+template <int kSeg>
+__device__ __forceinline__ float table_segment(const float* __restrict__ weight, const int32_t* __restrict__ adjncy, uint32_t off,
+                                               uint32_t deg, unsigned char* region, int lane, bool& bad) {
+  const uint32_t c = (uint32_t)lane & (uint32_t)(kSeg - 1);
+  const uint32_t nq = deg != 0u ? list_quartets(off, deg) : 0u;
+  float x[4];
+  int32_t nb[4];
+  load_lane<1>(weight, adjncy, off, deg, 0u, nq, c, x, nb, bad);
+  float q = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q = q + x[i];
+  float I = row_scan(q);
+  if (kSeg >= 32) I = dpp_add_bcast15(I);
+  if (kSeg == 64) I = dpp_add_bcast31(I);
+  const bool pos = q > 0.0f;
+  float M = pos ? I : 0.0f;
+  M = dpp_max<0x111, 0xF>(M);
+  M = dpp_max<0x112, 0xF>(M);
+  M = dpp_max<0x114, 0xF>(M);
+  M = dpp_max<0x118, 0xF>(M);
+  if (kSeg >= 32) M = dpp_max<0x142, 0xA>(M);
+  if (kSeg == 64) M = dpp_max<0x143, 0xC>(M);
+  const float T = bperm_f((lane | (kSeg - 1)) << 2, I);
+  const uint64_t mpos = __ballot(pos) >> (lane & ~(kSeg - 1));
+  const uint64_t mine = kSeg == 64 ? mpos : (mpos & ((1ull << (kSeg & 63)) - 1ull));
+  const uint32_t lastpos = 63u - (uint32_t)__builtin_clzll(mine | 1ull);
+  const uint32_t mu = (nq + 7u) >> 3;
+  if (c < 8u * mu) reinterpret_cast<float*>(region)[c] = c >= lastpos ? kInf : M;
+  if (c < nq) store_lane<1>(reinterpret_cast<uint2*>(region + 32u * (mu + c)), 1u, I - q, x, nb);
+  return T;
+}
+
+// One group of more than 64 quartets or of a long list, by a whole wave.  Returns its total.
+__device__ __forceinline__ float table_group(const float* __restrict__ weight, const int32_t* __restrict__ adjncy, uint32_t off,
+                                             uint32_t deg, uint32_t kb, uint32_t nqg, unsigned char* row, uint32_t row_units,
+                                             int lane, bool& bad) {
+  constexpr int kEl = 4 * kGroupQuartets;
+  float x[kEl];
+  int32_t nb[kEl];
+  load_lane<kGroupQuartets>(weight, adjncy, off, deg, kb, nqg, (uint32_t)lane, x, nb, bad);
+  float q = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kEl; ++i) q = q + x[i];
+  const float I = wave_scan(q);
+  const bool pos = q > 0.0f;
+  const float M = wave_prefix_max(pos ? I : 0.0f);
+  const uint32_t lastpos = 63u - (uint32_t)__builtin_clzll(__ballot(pos) | 1ull);
+  const uint32_t nl = nqg < 64u ? nqg : 64u, J = (nqg + 63u) >> 6;
+  reinterpret_cast<float*>(row)[lane] = (uint32_t)lane >= lastpos ? kInf : M;
+  if ((uint32_t)lane < nl)
+    store_lane<kGroupQuartets>(reinterpret_cast<uint2*>(row + 32u * (row_units + (uint32_t)lane * J)), J, I - q, x, nb);
+  return readlane_f(I, 63);
+}
+
+// Lists of one group: a wave takes 64 consecutive vertices; lists of at most 16 (32) quartets four (two) at a time, the others
+// one after the other.  vrec of the wave's vertices is stored together at the end (long lists get their total from
+// fw_table_sums_kernel).  base: region positions, or NULL: the ones vrec holds already.
+// Bound: memory (8 bytes read and about 9 written per edge; one pass).
+__global__ __launch_bounds__(256) void fw_table_lists_kernel(const uint32_t* __restrict__ xadj, const int32_t* __restrict__ adjncy,
+                                                             const float* __restrict__ weight, int32_t V,
+                                                             const uint32_t* base, uint4* vrec, unsigned char* data,
+                                                             uint32_t* flag) {
+  __shared__ float s_total[4][64];
+  const int lane = lane_id();
+  const int wave = (int)(threadIdx.x >> 6);
+  const uint64_t chunks = ((uint64_t)(uint32_t)V + 63u) >> 6;
+  bool bad = false;
+  for (uint64_t ch = (uint64_t)blockIdx.x * 4u + (uint64_t)wave; ch < chunks; ch += (uint64_t)gridDim.x * 4u) {
+    const uint32_t v = (uint32_t)(ch * 64u) + (uint32_t)lane;
+    const bool have = v < (uint32_t)V;
+    uint32_t off = 0u, deg = 0u, reg = 0u;
+    if (have) {
+      off = xadj[v];
+      deg = xadj[v + 1] - off;
+      reg = base != nullptr ? base[v] : vrec[v].x;
+    }
+    const uint32_t nq = deg != 0u ? list_quartets(off, deg) : 0u;
+    s_total[wave][lane] = 0.0f;
+    uint64_t m = __ballot(nq != 0u && nq <= 16u);
+    while (m != 0ull) {
+      int src = -1;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int l = m != 0ull ? __builtin_ctzll(m) : -1;
+        m &= m - 1ull;
+        src = (lane >> 4) == r ? l : src;
+      }
+      const int from = src < 0 ? 0 : src;
+      const uint32_t o = __shfl(off, from), df = __shfl(deg, from), g = __shfl(reg, from);  // every lane takes part
+      const uint32_t d = src < 0 ? 0u : df;
+      const float T = table_segment<16>(weight, adjncy, o, d, data + (uint64_t)g * 128u, lane, bad);
+      if (src >= 0 && (lane & 15) == 0) s_total[wave][src] = T;
+    }
+    m = __ballot(nq > 16u && nq <= 32u);
+    while (m != 0ull) {
+      int src = -1;
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        const int l = m != 0ull ? __builtin_ctzll(m) : -1;
+        m &= m - 1ull;
+        src = (lane >> 5) == r ? l : src;
+      }
+      const int from = src < 0 ? 0 : src;
+      const uint32_t o = __shfl(off, from), df = __shfl(deg, from), g = __shfl(reg, from);  // every lane takes part
+      const uint32_t d = src < 0 ? 0u : df;
+      const float T = table_segment<32>(weight, adjncy, o, d, data + (uint64_t)g * 128u, lane, bad);
+      if (src >= 0 && (lane & 31) == 0) s_total[wave][src] = T;
+    }
+    for (m = __ballot(nq > 32u && nq <= 64u); m != 0ull; m &= m - 1ull) {
+      const int l = __builtin_ctzll(m);
+      const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)off, l), d = (uint32_t)__builtin_amdgcn_readlane((int)deg, l);
+      const uint32_t g = (uint32_t)__builtin_amdgcn_readlane((int)reg, l);
+      const float T = table_segment<64>(weight, adjncy, o, d, data + (uint64_t)g * 128u, lane, bad);
+      if (lane == 0) s_total[wave][l] = T;
+    }
+    for (m = __ballot(nq > 64u && nq <= kGq); m != 0ull; m &= m - 1ull) {
+      const int l = __builtin_ctzll(m);
+      const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)off, l), d = (uint32_t)__builtin_amdgcn_readlane((int)deg, l);
+      const uint32_t g = (uint32_t)__builtin_amdgcn_readlane((int)reg, l);
+      const float T = table_group(weight, adjncy, o, d, 0u, list_quartets(o, d), data + (uint64_t)g * 128u, 8u, lane, bad);
+      if (lane == 0) s_total[wave][l] = T;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const float total = s_total[wave][lane];
+    bad = bad || !(total < kInf);
+    if (have) vrec[v] = make_uint4(reg, deg, __float_as_uint(total), off);
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (__ballot(bad) != 0ull && lane == 0) *flag = 1u;
+}
+
+// The groups of the long lists, one wave per group.  Group totals go to the list's sums.
+__global__ __launch_bounds__(256) void fw_table_groups_kernel(const uint4* __restrict__ vrec, const int32_t* __restrict__ adjncy,
+                                                              const float* __restrict__ weight, const uint2* __restrict__ items,
+                                                              uint32_t n_items, int32_t hub_threshold, uint32_t nw_shift,
+                                                              unsigned char* data, uint32_t* flag) {
+  const int lane = lane_id();
+  bool bad = false;
+  for (uint32_t it = blockIdx.x * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); it < n_items;
+       it += gridDim.x * 4u) {
+    const uint2 item = items[it];
+    const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int)item.x), g = (uint32_t)__builtin_amdgcn_readfirstlane((int)item.y);
+    const uint4 rec = vrec[v];
+    const uint32_t off = (uint32_t)__builtin_amdgcn_readfirstlane((int)rec.w), deg = (uint32_t)__builtin_amdgcn_readfirstlane((int)rec.y);
+    unsigned char* const region = data + (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)rec.x) * 128u;
+    const uint32_t nq = list_quartets(off, deg);
+    const uint32_t ngroups = (nq + kGq - 1u) / kGq;
+    const bool wg = (int32_t)deg > hub_threshold;
+    const uint32_t left = nq - g * kGq;
+    unsigned char* const row = region + (uint64_t)32u * (header_units(ngroups, wg) + kGroupUnits * g);
+    const float T = table_group(weight, adjncy, off, deg, g * kGq, left < kGq ? left : kGq, row, 8u, lane, bad);
+    float2* const sums = reinterpret_cast<float2*>(region + (wg ? 64u : 0u));
+    const uint32_t at = wg ? seq_start(ngroups, g & ((1u << nw_shift) - 1u), nw_shift) + (g >> nw_shift) : g;
+    if (lane == 0) sums[at].y = T;
+  }
+  if (__ballot(bad) != 0ull && lane == 0) *flag = 1u;
+}
+
+// The running sums of the long lists, one wave per list: at wave granularity one sequence (64 totals at a time, added up
+// in order), at workgroup granularity one sequence per lane and the scan of their totals.
+__global__ __launch_bounds__(256) void fw_table_sums_kernel(uint4* __restrict__ vrec, const uint32_t* __restrict__ longs, uint32_t n_longs,
+                                                            int32_t hub_threshold, uint32_t nw_shift, unsigned char* data, uint32_t* flag) {
+  const int lane = lane_id();
+  bool bad = false;
+  for (uint32_t it = blockIdx.x * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); it < n_longs;
+       it += gridDim.x * 4u) {
+    const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int)longs[it]);
+    const uint4 rec = vrec[v];
+    const uint32_t ngroups = (list_quartets(rec.w, rec.y) + kGq - 1u) / kGq;
+    unsigned char* const region = data + (uint64_t)rec.x * 128u;
+    float total;
+    if ((int32_t)rec.y > hub_threshold) {
+      float2* const sums = reinterpret_cast<float2*>(region + 64u);
+      const uint32_t nw = 1u << nw_shift;
+      float S = 0.0f;
+      if ((uint32_t)lane < nw) {
+        const uint32_t b = seq_start(ngroups, (uint32_t)lane, nw_shift), e = seq_start(ngroups, (uint32_t)lane + 1u, nw_shift);
+        for (uint32_t i = b; i < e; ++i) {
+          S = S + sums[i].y;
+          sums[i].x = S;
+        }
+      }
+      const float J = row_scan(S);
+      total = readlane_f(J, (int)nw - 1);
+      const uint64_t mpos = __ballot(S > 0.0f);
+      const uint32_t lastpos = 63u - (uint32_t)__builtin_clzll(mpos | 1ull);
+      const float key = wave_prefix_max(S > 0.0f ? J : 0.0f);
+      if (lane < 16) reinterpret_cast<float*>(region)[lane] = (uint32_t)lane >= lastpos ? kInf : key;
+    } else {
+      float2* const sums = reinterpret_cast<float2*>(region);
+      float S = 0.0f;
+      for (uint32_t g0 = 0; g0 < ngroups; g0 += 64u) {
+        const uint32_t g = g0 + (uint32_t)lane;
+        const float T = g < ngroups ? sums[g].y : 0.0f;
+        float mine = 0.0f;
+#pragma unroll 8
+        for (int l = 0; l < 64; ++l) {
+          S = S + readlane_f(T, l);  // + 0 past the end changes nothing
+          mine = lane == l ? S : mine;
+        }
+        if (g < ngroups) sums[g].x = mine;
+      }
+      total = S;
+    }
+    bad = bad || !(total < kInf);
+    if (lane == 0) vrec[v].z = __float_as_uint(total);
+  }
+  if (__ballot(bad) != 0ull && lane == 0) *flag = 1u;
+}
+
+// ---- the walk -----------------------------------------------------------------------------------------
+
+// First entry above t of the n entries of a row (they never decrease, the last one is above t; rows are padded to 8
+// entries), from a guess.  Four entries per look; when the guess was off twice the rest is halved.
+__device__ __forceinline__ uint32_t row_search(const float* row, uint32_t n, uint32_t guess, float t, float& below) {
+  uint32_t lo = 0u, hi = n - 1u;
+  const uint32_t wmax = n > 4u ? n - 4u : 0u;
+  uint32_t w = guess > 1u ? guess - 1u : 0u;
+  below = 0.0f;
+  for (;;) {
+    w = w < wmax ? w : wmax;
+    const f4_at4 m = *reinterpret_cast<const f4_at4*>(row + w);
+    const uint32_t cnt = (m.x <= t ? 1u : 0u) + (m.y <= t ? 1u : 0u) + (m.z <= t ? 1u : 0u) + (m.w <= t ? 1u : 0u);
+    if (cnt == 0u) {
+      if (w <= lo) return w;
+      hi = w;
+      w = hi - lo > 12u ? (lo + hi) >> 1 : (hi > lo + 3u ? hi - 3u : lo);
+    } else if (cnt == 4u) {
+      below = m.w;
+      lo = w + 4u;
+      if (lo >= hi) return hi;
+      w = hi - lo > 12u ? (lo + hi) >> 1 : lo;
+    } else {
+      below = cnt == 1u ? m.x : (cnt == 2u ? m.y : m.z);
+      return w + cnt;
+    }
+  }
+}
+
+// The neighbour of the first pair whose key is above t (n = 4 J pairs of one lane, keys as above).
+__device__ __forceinline__ int32_t pair_search(const uint2* pairs, uint32_t n, uint32_t guess, float t) {
+  uint32_t lo = 0u, hi = n - 1u;
+  const uint32_t wmax = n - 4u;
+  uint32_t w = guess > 1u ? guess - 1u : 0u;
+  for (;;) {
+    w = w < wmax ? w : wmax;
+    const u4_at8 a = *reinterpret_cast<const u4_at8*>(pairs + w);
+    const u4_at8 b = *reinterpret_cast<const u4_at8*>(pairs + w + 2u);
+    const bool b0 = __uint_as_float(a.x) <= t, b1 = __uint_as_float(a.z) <= t;
+    const bool b2 = __uint_as_float(b.x) <= t, b3 = __uint_as_float(b.z) <= t;
+    if (!b0) {
+      if (w <= lo) return (int32_t)a.y;
+      hi = w;
+      w = hi > lo + 3u ? hi - 3u : lo;
+    } else if (b3) {
+      lo = w + 4u;
+      if (lo > hi) return (int32_t)b.w;
+      w = lo;
+    } else {
+      return (int32_t)(b2 ? b.w : (b1 ? b.y : a.w));
+    }
+  }
+}
+
+// The reservoir over the groups of one sequence (L sums): the group it ends with and the target inside it.  The test of the
+// streaming kernels, S_k u > S_j, is monotone in k, so the next accepted group is searched for, from where the sums
+// would reach S_j / u if they grew evenly.
+__device__ __forceinline__ void sums_reservoir(const fw_kargs& a, const float2* sums, const uint32_t L, const float S_last,
+                                               LaneDraw& dq, const uint32_t walker, const uint32_t step, const uint32_t stream,
+                                               uint32_t& k_out, float& t_out) {
+  uint32_t k = 0u;
+  float2 e = sums[0];
+  while (!(e.x > 0.0f) && k + 1u < L) e = sums[++k];
+  float Sj = e.x, T = e.y;
+  float tu = next_uniform_lane(dq, a, walker, step, stream);
+  float u = next_uniform_lane(dq, a, walker, step, stream);
+  const float rate = (float)L * __builtin_amdgcn_rcpf(S_last);
+  while (k + 1u < L && S_last * u > Sj) {
+    uint32_t lo = k, hi = L - 1u;
+    const float want = Sj * __builtin_amdgcn_rcpf(u);
+    uint32_t i = k + 1u + (uint32_t)fmaxf((want - Sj) * rate, 0.0f);
+    float S_new, T_new;
+    for (int tries = 0;; ++tries) {
+      i = i < hi ? (i > lo ? i : lo + 1u) : hi;
+      const f4_at8 p = *reinterpret_cast<const f4_at8*>(sums + i - 1u);
+      S_new = p.z;
+      T_new = p.w;
+      if (p.x * u > Sj && i - 1u > lo) {
+        hi = i - 1u;
+      } else if (p.z * u > Sj || i == hi) {
+        break;
+      } else {
+        lo = i;
+      }
+      i = tries < 2 ? (uint32_t)((int32_t)i + 1 + (int32_t)((want - p.z) * rate)) : lo + ((hi - lo + 1u) >> 1);
+    }
+    k = i;
+    Sj = S_new;
+    T = T_new;
+    tu = next_uniform_lane(dq, a, walker, step, stream);
+    u = next_uniform_lane(dq, a, walker, step, stream);
+  }
+  k_out = k;
+  t_out = tu * T;
+}
+
+// One proposal of the step's sampler for a list with a positive total: the selected neighbour.  d: block 0 of the step's stream 0.
+__device__ __forceinline__ int32_t table_pick(const fw_kargs& a, const fw_table_args& tb, const uint4 rec, const uint4 d,
+                                              const uint32_t walker, const uint32_t step, const uint32_t sbase) {
+  const float total = __uint_as_float(rec.z);
+  const uint32_t nq = list_quartets(rec.w, rec.y);
+  const unsigned char* row = tb.data + (uint64_t)rec.x * 128u;
+  uint32_t nqg = nq, row_units = 8u;
+  float T = total, t;
+  if (nq <= kGq) {
+    if (nq < 64u) row_units = (nq + 7u) >> 3;
+    t = u24(d.x) * total;
+  } else {
+    const uint32_t ngroups = (nq + kGq - 1u) / kGq;
+    const bool wg = (int32_t)rec.y > a.hub_threshold;
+    const float2* sums = reinterpret_cast<const float2*>(row);
+    uint32_t L = ngroups, seq = 0u;
+    float S_last = total;
+    LaneDraw dq;
+    if (wg) {  // which sequence, then the reservoir over it with draws of its own stream
+      const float target = u24(philox4x32_10(walker, step, kStreamWave | sbase, 0u, a.seed_lo, a.seed_hi).x) * total;
+      const float4* keys = reinterpret_cast<const float4*>(row);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 k4 = keys[i];
+        seq += (k4.x <= target ? 1u : 0u) + (k4.y <= target ? 1u : 0u) + (k4.z <= target ? 1u : 0u) + (k4.w <= target ? 1u : 0u);
+      }
+      const uint32_t b = seq_start(ngroups, seq, tb.nw_shift);
+      L = seq_start(ngroups, seq + 1u, tb.nw_shift) - b;
+      sums = reinterpret_cast<const float2*>(row + 64u) + b;
+      S_last = sums[L - 1u].x;
+    } else {
+      dq.q0 = d.x; dq.q1 = d.y; dq.q2 = d.z; dq.q3 = d.w;
+      dq.avail = 4u;
+      dq.blk = 1u;
+    }
+    uint32_t k;
+    sums_reservoir(a, sums, L, S_last, dq, walker, step, seq | sbase, k, t);
+    const uint32_t g = wg ? seq + (k << tb.nw_shift) : k;
+    row += (uint64_t)32u * (header_units(ngroups, wg) + kGroupUnits * g);
+    nqg = nq - g * kGq < kGq ? nq - g * kGq : kGq;
+    T = total * (float)kGq / (float)nq;  // about a group's share (the guess below needs no more)
+    if (nqg < kGq) T = total * (float)nqg / (float)nq;
+  }
+  const uint32_t nl = nqg < 64u ? nqg : 64u;
+  const uint32_t J = (nqg + 63u) >> 6;
+  const float lanes_per_t = (float)nl * __builtin_amdgcn_rcpf(T);
+  float below;
+  const uint32_t l = row_search(reinterpret_cast<const float*>(row), nl, (uint32_t)(t * lanes_per_t), t, below);
+  const uint2* pairs = reinterpret_cast<const uint2*>(row + 32u * (row_units + l * J));
+  const uint32_t guess = J == 1u ? 0u : (uint32_t)fmaxf((t - below) * lanes_per_t * (float)(4u * J), 0.0f);
+  return pair_search(pairs, 4u * J, guess, t);
+}
+
+// One lane, one walker, from its start to its end; a lane whose walk is over takes the next query of its wave's range.
+// Path entries are collected in LDS (16 per walker, by their place in the path matrix modulo 16) and leave as whole 64-byte
+// lines; the entries of a row before its first and after its last whole line, and the -1 behind the walk, are stored by the
+// wave together, one row at a time.
+template <int kApp>
+__global__ __launch_bounds__(256, 4) void fw_table_walk(const fw_kargs a, const fw_table_args tb) {
+  __shared__ __align__(16) int32_t s_buf[4][64 * 16];
+  __shared__ unsigned long long s_acc[4];
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (threadIdx.x < 4u) s_acc[threadIdx.x] = 0ull;
+  __syncthreads();
+  int32_t* const buf = s_buf[wave];
+  const uint32_t my_buf = (uint32_t)lane * 16u;
+  const uint32_t swz = ((uint32_t)lane >> 2) & 3u;  // spreads the lanes' 16-byte pieces over the banks
+  auto slot_at = [&](uint32_t slot) { return my_buf + ((((slot >> 2) ^ swz) << 2) | (slot & 3u)); };
+  const uint32_t md = (uint32_t)a.max_depth;
+  const uint32_t align0 = (uint32_t)(reinterpret_cast<uintptr_t>(a.paths) >> 2) & 15u;
+
+  uint64_t next64 = ((uint64_t)blockIdx.x * 4u + (uint64_t)wave) * tb.chunk;
+  const uint32_t n = (uint32_t)a.n;
+  uint32_t cursor = next64 < n ? (uint32_t)next64 : n;
+  const uint32_t last = next64 + tb.chunk < n ? (uint32_t)(next64 + tb.chunk) : n;
+
+  bool active = false, fresh = false;
+  uint32_t q = 0u, len = 0u, s0 = 0u, fpos = 0u;
+  int32_t v = 0, prev = -1;
+  uint32_t prev_off = 0u, prev_deg = 0u, trial = 0u;
+  float w_ret = 0.0f;
+  uint4 rec = make_uint4(0u, 0u, 0u, 0u);
+  uint32_t n_steps = 0u, n_hub = 0u;
+  unsigned long long n_edges = 0ull, hub_edges = 0ull;
+
+  for (;;) {
+    bool ended = false;
+    bool partial = false;  // the row's first entries fill up a line that is not all its own
+    {
+      const bool want = !active && (uint32_t)lane < tb.lanes;
+      const uint64_t m = __ballot(want);
+      if (m != 0ull && cursor < last) {
+        const uint32_t qn = cursor + (uint32_t)__builtin_popcountll(m & ((1ull << lane) - 1ull));
+        if (want && qn < last) {
+          q = qn;
+          v = a.starts[qn];
+          len = 1u;
+          fpos = 0u;
+          s0 = (align0 + q * md) & 15u;
+          if (s0 == 15u) {
+            a.paths[(uint64_t)q * md] = v;
+            fpos = 1u;
+          } else {
+            buf[slot_at(s0)] = v;
+          }
+          prev = -1;
+          trial = 0u;
+          active = true;
+          fresh = true;
+          ended = !((uint32_t)v < (uint32_t)a.V && md > 1u);
+        }
+        const uint32_t took = (uint32_t)__builtin_popcountll(m);
+        cursor = last - cursor > took ? cursor + took : last;
+      }
+      if (__ballot(active) == 0ull) break;
+    }
+    const uint32_t walker = a.walker_base + q;
+    const uint32_t step = len - 1u;
+    const uint32_t sbase = kApp == FW_APP_NODE2VEC ? trial << 8 : 0u;
+    if (active && !ended && fresh) rec = tb.vrec[v];
+    const uint4 d = philox4x32_10(walker, step, sbase, 0u, a.seed_lo, a.seed_hi);
+    if (active && !ended) {
+      if (!(__uint_as_float(rec.z) > 0.0f)) {
+        ended = true;  // no neighbour with a positive bias (include/walker.cuh:1373-1374)
+      } else {
+        int32_t nv = table_pick(a, tb, rec, d, walker, step, sbase);
+        bool moved = true;
+        if (kApp == FW_APP_NODE2VEC && prev >= 0) {
+          if (a.n2v_extra > 0.0f && fresh) w_ret = return_weight(a.adjncy + rec.w, a.weight + rec.w, rec.y, prev);
+          const N2vTest t = n2v_test(a, nv, prev, walker, step, trial, __uint_as_float(rec.z), w_ret);
+          if (t.take_prev) {
+            nv = prev;
+          } else {
+            bool common = false;
+            if (!t.decided) common = sorted_contains(a.adjncy + prev_off, (int32_t)prev_deg, nv);
+            moved = n2v_finish(a, t, common);
+          }
+        }
+        fresh = moved;
+        if (moved) {
+          if ((int32_t)rec.y > a.park_threshold) {
+            n_hub += 1u;
+            hub_edges += rec.y;
+          } else {
+            n_steps += 1u;
+            n_edges += rec.y;
+          }
+          const uint32_t slot = (s0 + len) & 15u;
+          buf[slot_at(slot)] = nv;
+          if (kApp == FW_APP_NODE2VEC) {
+            prev = v;
+            prev_off = rec.w;
+            prev_deg = rec.y;
+            trial = 0u;
+          }
+          v = nv;
+          len += 1u;
+          ended = len >= md;
+          if (kApp == FW_APP_PPR && !ended) {  // include/app.cuh:88-94
+            const uint32_t bits = philox4x32_10(walker, step, kStreamStop, 0u, a.seed_lo, a.seed_hi).x;
+            ended = u24(bits) < a.tp;
+          }
+          if (slot == 15u) {
+            if (len >= 16u) {
+              const uint4* src = reinterpret_cast<const uint4*>(buf + my_buf);
+              uint4* dst = reinterpret_cast<uint4*>(a.paths + ((uint64_t)q * md + (uint64_t)(len - 16u)));
+#pragma unroll
+              for (uint32_t j = 0; j < 4u; ++j) dst[j] = src[j ^ swz];
+              fpos = len;
+            } else {
+              partial = true;
+            }
+          }
+        } else {
+          trial += 1u;
+        }
+      }
+    }
+    uint64_t ev = __ballot(active && (ended || partial));
+    if (ev != 0ull) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const uint32_t end = ended ? md : len;
+      for (; ev != 0ull; ev &= ev - 1ull) {
+        const int l = __builtin_ctzll(ev);
+        const uint32_t lq = (uint32_t)__builtin_amdgcn_readlane((int)q, l);
+        const uint32_t from = (uint32_t)__builtin_amdgcn_readlane((int)fpos, l);
+        const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)end, l);
+        const uint32_t have = (uint32_t)__builtin_amdgcn_readlane((int)len, l);
+        const uint32_t ls0 = (uint32_t)__builtin_amdgcn_readlane((int)s0, l);
+        int32_t* const row = a.paths + (uint64_t)lq * md;
+        for (uint32_t p = from + (uint32_t)lane; p < to; p += 64u) {
+          const uint32_t slot = (ls0 + p) & 15u;
+          const uint32_t at = (uint32_t)l * 16u + ((((slot >> 2) ^ (((uint32_t)l >> 2) & 3u)) << 2) | (slot & 3u));
+          row[p] = p < have ? buf[at] : -1;
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+      if (partial) fpos = len;
+      if (ended) active = false;
+    }
+  }
+  // workload counters: summed inside the workgroup, then one of 64 lines of counters (one line would be contended)
+  if (n_steps != 0u) {
+    atomicAdd(&s_acc[0], (unsigned long long)n_steps);
+    atomicAdd(&s_acc[1], n_edges);
+  }
+  if (n_hub != 0u) {
+    atomicAdd(&s_acc[2], (unsigned long long)n_hub);
+    atomicAdd(&s_acc[3], hub_edges);
+  }
+  __syncthreads();
+  if (threadIdx.x < 4u && s_acc[threadIdx.x] != 0ull)
+    atomicAdd(&tb.counters[(blockIdx.x & (FW_TABLE_STRIPES - 1u)) * 8u + threadIdx.x], s_acc[threadIdx.x]);
+}
+
+// Around the walk: the counters start at zero, and their sums go to the host (pinned memory: the call waits for the stream
+// anyway, and a copy of its own would cost a small call as much as its launch).
+__global__ void fw_table_begin_kernel(unsigned long long* counters) {
+  for (uint32_t i = threadIdx.x; i < FW_TABLE_STRIPES * 8u; i += blockDim.x) counters[i] = 0ull;
+}
+__global__ __launch_bounds__(64) void fw_table_end_kernel(const unsigned long long* __restrict__ counters, unsigned long long* out) {
+  unsigned long long c[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    c[k] = counters[threadIdx.x * 8u + (uint32_t)k];
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) c[k] += __shfl_xor(c[k], d);
+  }
+  if (threadIdx.x == 0u) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) out[k] = c[k];
+  }
+}
+
+template <int kApp>
+int launch_table_walk(const fw_kargs& a, fw_table_args tb, int grid, hipStream_t stream, int* grid_used) {
+  int dev = 0, cus = 0;
+  FW_HIP(hipGetDevice(&dev));
+  FW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  const uint32_t n = (uint32_t)a.n;
+  uint64_t waves;
+  if (grid > 0) {
+    waves = (uint64_t)grid * 4u;
+    tb.lanes = 64u;
+  } else {
+    // few queries are spread over the chip, down to one lane per wave: their walks are chains of dependent look-ups, and a
+    // wave waits for the slowest of its lanes
+    const uint32_t spread = (uint32_t)cus * 8u;
+    tb.lanes = n / spread < 64u ? n / spread + 1u : 64u;
+    if (tb.lanes > 64u) tb.lanes = 64u;
+    waves = ((uint64_t)n + tb.lanes - 1u) / tb.lanes;
+    // many: a wave takes query after query.  Waves come and go (sixteen times as many as fit at half occupancy), so that the
+    // chip stays full to the end; PPR's short walks, whose lanes rarely end together, want longer ranges (4 / 16 times:
+    // PPR on R-MAT 22 1.60 / 1.95 ms, DeepWalk there 12.6 / 10.4, on R-MAT 24 80.7 / 74.2)
+    const uint64_t most = (uint64_t)cus * 16u * (kApp == FW_APP_PPR ? 4u : 16u);
+    if (waves > most) waves = most;
+  }
+  uint64_t chunk = ((uint64_t)n + waves - 1u) / waves;
+  tb.chunk = (uint32_t)chunk;
+  const uint64_t need = ((uint64_t)n + chunk - 1u) / chunk;
+  const unsigned blocks = (unsigned)((need + 3u) / 4u);
+  hipLaunchKernelGGL((fw_table_walk<kApp>), dim3(blocks), dim3(256), 0, stream, a, tb);
+  FW_HIP(hipGetLastError());
+  if (grid_used) *grid_used = (int)blocks;
+  return FW_OK;
+}
+
+}  // namespace
+
+int fw_launch_table_walk(const fw_kargs& a, const fw_table_args& tb, int app, int grid, hipStream_t stream, int* grid_used) {
+  switch (app) {
+    case FW_APP_DEEPWALK: return launch_table_walk<FW_APP_DEEPWALK>(a, tb, grid, stream, grid_used);
+    case FW_APP_PPR: return launch_table_walk<FW_APP_PPR>(a, tb, grid, stream, grid_used);
+    case FW_APP_NODE2VEC: return launch_table_walk<FW_APP_NODE2VEC>(a, tb, grid, stream, grid_used);
+    default:
+      fw_set_error("no list tables for app %d", app);
+      return FW_ERR_INVALID;
+  }
+}
+
+int fw_table_begin(unsigned long long* d_counters, hipStream_t stream) {
+  hipLaunchKernelGGL(fw_table_begin_kernel, dim3(1), dim3(512), 0, stream, d_counters);
+  FW_HIP(hipGetLastError());
+  return FW_OK;
+}
+
+int fw_table_end(const unsigned long long* d_counters, unsigned long long* h_out, hipStream_t stream) {
+  static_assert(FW_TABLE_STRIPES == 64u, "one lane per line of counters");
+  hipLaunchKernelGGL(fw_table_end_kernel, dim3(1), dim3(64), 0, stream, d_counters, h_out);
+  FW_HIP(hipGetLastError());
+  return FW_OK;
+}
+
+int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
+                  hipStream_t stream) {
+  hipLaunchKernelGGL(fw_table_plan_kernel, dim3(1024), dim3(1024), 0, stream, g->xadj, g->V, hub_threshold, d_blocks, d_longs,
+                     d_items, d_ctrs);
+  FW_HIP(hipGetLastError());
+  return FW_OK;
+}
+
+int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches) {
+  int cus = 0;
+  FW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
+  auto grid_for = [&](uint64_t waves) {
+    const uint64_t blocks = (waves + 3u) / 4u, most = (uint64_t)cus * 64u;
+    return (unsigned)(blocks < most ? (blocks ? blocks : 1u) : most);
+  };
+  hipLaunchKernelGGL(fw_table_lists_kernel, dim3(grid_for(((uint64_t)g->V + 63u) / 64u)), dim3(256), 0, stream, g->xadj, g->adjncy,
+                     g->weight, g->V, d_base, t->vrec, t->data, t->flag);
+  FW_HIP(hipGetLastError());
+  *launches += 1;
+  if (t->n_longs != 0u) {
+    hipLaunchKernelGGL(fw_table_groups_kernel, dim3(grid_for(t->n_items)), dim3(256), 0, stream, t->vrec, g->adjncy, g->weight,
+                       t->items, t->n_items, t->hub_threshold, t->nw_shift, t->data, t->flag);
+    FW_HIP(hipGetLastError());
+    hipLaunchKernelGGL(fw_table_sums_kernel, dim3(grid_for(t->n_longs)), dim3(256), 0, stream, t->vrec, t->longs, t->n_longs,
+                       t->hub_threshold, t->nw_shift, t->data, t->flag);
+    FW_HIP(hipGetLastError());
+    *launches += 2;
+  }
+  return FW_OK;
+}

@@ -88,9 +88,12 @@ typedef struct {
   int32_t grid;          /* workgroups to launch; 0 = library default (src/walk.cu:84-92 analogue) */
   int32_t park_threshold; /* hub parking, an execution strategy that never changes results: walkers that arrive on a
                             vertex of larger degree wait there and are served 64 at a time by one shared scan of its
-                            list (by a workgroup above hub_threshold, by one wave below).  0 = library default (on
-                            for batches >= 65536 queries), < 0 = off, > 0 = degree.  node2vec: the shared scan
-                            proposes, each walker accepts with its own adjacency test (max_depth <= 65535). */
+                            list (by a workgroup above hub_threshold, by one wave below).  > 0 = degree, < 0 = off (a
+                            walker reads its lists itself).  0 = library default: where the walks would read the lists
+                            several times over, one scan of every list is shared by all walkers of all calls (list
+                            tables, kept with the graph; DeepWalk, PPR and node2vec on graphs in device memory), else
+                            parking for batches >= 65536 queries.  node2vec: the shared scan proposes, each walker
+                            accepts with its own adjacency test (max_depth <= 65535). */
   /* node2vec is sampled in two stages: a neighbour is proposed with probability w / sum w and accepted with
    * probability f / F, f = 1 (common neighbour of the previous vertex) or 1/q, F = max(1, 1/q); a rejected walker
    * proposes again.  The return edge (f = 1/p) is accepted with probability (1/p) / F when that is at most 1; when 1/p
@@ -115,13 +118,16 @@ typedef struct {
   double total_ms;        /* wall time of the call, transfers included (src/walk.cu:388,459,465) */
   uint64_t steps;         /* "Total sampled vertex" */
   uint64_t sampled_edges; /* "Total sampled edge": sum over steps of deg(source) */
-  int32_t launches;       /* fw_walk_batch: batches; fw_walk_device: walk + hub-batch kernel launches */
+  int32_t launches;       /* fw_walk_batch: batches; fw_walk_device: walk + hub-batch kernel launches (a walk on list
+                             tables: begin, walk, end, and the launches that made the tables when it made them) */
   int32_t grid;           /* workgroups per launch actually used */
   /* per-kernel breakdown of kernel_ms / steps / sampled_edges (hub parking splits a pass over two kernels) */
   double walk_kernel_ms;      /* sum over fw_walk_zprs launches (with fw_walk_params.time_kernels, else 0) */
   double hub_kernel_ms;       /* sum over the hub launches of every round: fw_hub_scan, fw_hub_batch, fw_hub_quad
-                                 (with fw_walk_params.time_kernels, else 0) */
-  uint64_t hub_steps;         /* steps taken in the hub launches (included in steps) */
+                                 (with fw_walk_params.time_kernels, else 0); a walk on list tables: the making of the
+                                 tables, which a call with time_kernels does anew */
+  uint64_t hub_steps;         /* steps taken in the hub launches (included in steps); a walk on list tables: steps
+                                 from vertices above the parking degree of the batch */
   uint64_t hub_sampled_edges; /* their source degrees (included in sampled_edges) */
   /* What the call's kernels asked of the memory, MODELLED from the run's own counters (steps, records moved, list
    * quartets streamed): requested_bytes = list_bytes + 128 * scattered_reads + 32 * scattered_writes + record_bytes.
@@ -213,7 +219,8 @@ int fw_graph_create_placed(int32_t V, uint64_t E, const uint32_t* h_xadj, const 
                            const float* h_weight, const int32_t* h_label, int placement, fw_graph** out);
 
 /*
- * Adopts device arrays that already hold a CSR (e.g. produced by fw_gen_rmat).  The arrays must
+ * Adopts device arrays that already hold a CSR (e.g. produced by fw_gen_rmat).  The caller may change the biases
+ * between calls (what is derived from them is derived anew in every call).  The arrays must
  * stay valid until fw_graph_destroy and must be readable 12 bytes past their last element
  * (the kernels use aligned 16-byte loads).  take_ownership != 0: destroy frees them with hipFree.
  */
