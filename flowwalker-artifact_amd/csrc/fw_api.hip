@@ -1663,7 +1663,7 @@ static int plan_tables(const fw_graph* g, fw_tables* t, uint32_t** d_base_out, h
         (rc = alloc(reinterpret_cast<void**>(&t->flag), 64)) || (rc = alloc(reinterpret_cast<void**>(&t->vrec), (size_t)g->V * sizeof(uint4))))
       return rc;
     FW_HIP(hipMemsetAsync(d_ctrs, 0, 64, stream));
-    if ((rc = fw_table_plan(g, t->hub_threshold, d_blocks, t->longs, t->items, d_ctrs, stream)) != FW_OK) return rc;
+    if ((rc = fw_table_plan(g, t->hub_threshold, t->nw_shift, d_blocks, t->longs, t->items, d_ctrs, stream)) != FW_OK) return rc;
     FW_HIP(rocprim::exclusive_scan(tmp, tmp_bytes, d_blocks, d_blocks, 0u, nv, rocprim::plus<uint32_t>(), stream));
     FW_HIP(hipMemcpyAsync(&h[0], d_ctrs, 8, hipMemcpyDeviceToHost, stream));
     FW_HIP(hipMemcpyAsync(&h[2], d_blocks + g->V, 4, hipMemcpyDeviceToHost, stream));
@@ -1768,7 +1768,7 @@ static fw_table_args table_args(const fw_tables& t, unsigned long long* d_counte
   tb.vrec = t.vrec;
   tb.data = t.data;
   tb.nw_shift = t.nw_shift;
-  tb.chunk = tb.lanes = 0u;
+  tb.lanes = 0u;
   tb.counters = d_counters;
   return tb;
 }
@@ -1833,7 +1833,7 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
     a.park_threshold = park_threshold;
     if (launches == 0) FW_TRY(hipEventRecord(ev0, stream));  // (tables made in this call: recorded before that)
     if (!mg->call_result) FW_TRY(hipHostMalloc(reinterpret_cast<void**>(&mg->call_result), 64, hipHostMallocDefault));
-    if ((rc = fw_table_begin(d_counters, stream)) != FW_OK) return rc;
+    if ((rc = fw_table_begin(d_counters, &d_scr->dispenser, sizeof(Scratch) / 4u, stream)) != FW_OK) return rc;
     rc = fw_launch_table_walk(a, table_args(*tables, d_counters), p->app, p->grid, stream, &grid_used);
     if (rc != FW_OK) return rc;
     if ((rc = fw_table_end(d_counters, mg->call_result, stream)) != FW_OK) return rc;
@@ -2127,7 +2127,7 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
   if (tables) {  // the batches share one set of counters
     if (!bc->d_stripes) FW_TRY(hipMalloc(reinterpret_cast<void**>(&bc->d_stripes), FW_TABLE_COUNTER_BYTES));
     if (!mg->call_result) FW_TRY(hipHostMalloc(reinterpret_cast<void**>(&mg->call_result), 64, hipHostMallocDefault));
-    if ((rc = fw_table_begin(bc->d_stripes, nullptr)) != FW_OK) { cleanup(); return rc; }
+    if ((rc = fw_table_begin(bc->d_stripes, &bc->d_scr->dispenser, (uint32_t)(sizeof(Scratch) / 4u * (size_t)nbatch), nullptr)) != FW_OK) { cleanup(); return rc; }
   }
   for (int i = 0; i < nbuf; ++i) if (!bc->streams[i]) FW_TRY(hipStreamCreate(&bc->streams[i]));
   while (bc->events.size() < (size_t)nbatch * 2) {

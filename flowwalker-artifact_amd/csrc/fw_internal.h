@@ -199,8 +199,7 @@ struct fw_table_args {
   const uint4* vrec;
   const unsigned char* data;
   uint32_t nw_shift;
-  uint32_t chunk;                // queries of a wave (set by the launch)
-  uint32_t lanes;                // lanes of a wave that walk (set by the launch)
+  uint32_t lanes;                // lanes of a wave that walk, and the queries it takes at a time (set by the launch)
   unsigned long long* counters;  // [FW_TABLE_STRIPES * 8]
 };
 
@@ -274,10 +273,10 @@ int fw_launch_hub_scan(const fw_kargs& a, const fw_hub_args& h, int app, uint32_
 
 // List tables.  plan: region sizes into d_blocks[0 .. V], work lists and their sizes (d_ctrs[0]: long lists, [1]: items);
 // make: fills the tables (d_base: region positions, NULL when vrec has them); walk: every query from start to end, between
-// begin (counters to zero) and end (their sums to pinned host memory).
-int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
+// begin (counters and launch records to zero) and end (their sums to pinned host memory).
+int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t nw_shift, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
                   hipStream_t stream);
 int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches);
 int fw_launch_table_walk(const fw_kargs& a, const fw_table_args& tb, int app, int grid, hipStream_t stream, int* grid_used);
-int fw_table_begin(unsigned long long* d_counters, hipStream_t stream);
+int fw_table_begin(unsigned long long* d_counters, uint32_t* d_scratch, uint32_t words, hipStream_t stream);
 int fw_table_end(const unsigned long long* d_counters, unsigned long long* h_out, hipStream_t stream);

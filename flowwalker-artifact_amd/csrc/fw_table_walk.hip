@@ -20,8 +20,9 @@
 //   entries: lane after lane, 4 J pairs {key, neighbour}; key = the lane's running sum up to the element, for an element
 //     without bias the key before it, from the lane's last positive element on +inf: the element is the first key
 //     above the target.  A lane of a full group is 16 pairs = one block, so the pick and the neighbour come in one request.
-//   sums: per group {running sum of the group's sequence, group total}, sequence after sequence; with more than one
-//     sequence (workgroup granularity) 16 floats in front: the inclusive scan of the sequences' totals, as keys like the above.
+//   sums: blocks of 16 running sums of a sequence's groups and their 16 totals, every sequence from a block of its own, filled up
+//     with the last sum; with more than one sequence (workgroup granularity) a block in front: the inclusive scan of the
+//     sequences' totals, as keys like the above (16 floats).
 // All keys of a row or a lane never decrease, so any search finds the same entry; weights are close to evenly spread
 // over a list, so the searches start from the proportional guess and mostly end there.
 
@@ -35,25 +36,27 @@ namespace {
 constexpr uint32_t kGq = 64u * kGroupQuartets;  // quartets of a full group
 constexpr uint32_t kGroupUnits = 8u + kGq;      // units of a group in a list of several: row M and the entries of 64 lanes
 constexpr float kInf = __builtin_inff();
+// Waves per SIMD of the walk: 4, 5, 6 and 8 were measured (DeepWalk R-MAT 24 47.9 / 49.1 / 50.0 / 72.1 ms, the last one with
+// spilled registers; R-MAT 22 6.8 / 6.8 / 7.0 / 11.3): more walkers in flight only compete for the caches.
+constexpr int kWaves = 4;
 
 typedef float f4_at4 __attribute__((ext_vector_type(4), aligned(4)));
-typedef float f4_at8 __attribute__((ext_vector_type(4), aligned(8)));
-typedef uint32_t u4_at8 __attribute__((ext_vector_type(4), aligned(8)));
 
 __device__ __forceinline__ uint32_t list_quartets(uint32_t off, uint32_t deg) { return ((off & 3u) + deg + 3u) >> 2; }
 
-// units of a long list's header: the sequences' keys (workgroup granularity only) and 8 bytes per group, whole blocks
-__device__ __forceinline__ uint32_t header_units(uint32_t ngroups, bool wg) {
-  return ((wg ? 2u : 0u) + ((ngroups + 3u) >> 2) + 3u) & ~3u;
+// blocks of sums of one sequence of a list of `ngroups` groups (the longest sequence has ceil(ngroups / sequences))
+__device__ __forceinline__ uint32_t seq_blocks(uint32_t ngroups, bool wg, uint32_t nw_shift) {
+  const uint32_t most = wg ? (ngroups + (1u << nw_shift) - 1u) >> nw_shift : ngroups;
+  return (most + 15u) >> 4;
 }
 
-// first entry of sequence `s` among a list's sums
-__device__ __forceinline__ uint32_t seq_start(uint32_t ngroups, uint32_t s, uint32_t nw_shift) {
-  const uint32_t per = ngroups >> nw_shift, rest = ngroups & ((1u << nw_shift) - 1u);
-  return s * per + (s < rest ? s : rest);
+// units of a long list's header
+__device__ __forceinline__ uint32_t header_units(uint32_t ngroups, bool wg, uint32_t nw_shift) {
+  const uint32_t nb = seq_blocks(ngroups, wg, nw_shift);
+  return 4u * (wg ? 1u + (nb << nw_shift) : nb);
 }
 
-__device__ __forceinline__ uint32_t region_blocks(uint32_t off, uint32_t deg, bool wg) {
+__device__ __forceinline__ uint32_t region_blocks(uint32_t off, uint32_t deg, bool wg, uint32_t nw_shift) {
   if (deg == 0u) return 0u;
   const uint32_t nq = list_quartets(off, deg);
   uint32_t units;
@@ -64,7 +67,7 @@ __device__ __forceinline__ uint32_t region_blocks(uint32_t off, uint32_t deg, bo
     const uint32_t ngroups = (nq + kGq - 1u) / kGq;
     const uint32_t last = nq - (ngroups - 1u) * kGq;
     const uint32_t nl = last < 64u ? last : 64u;
-    units = header_units(ngroups, wg) + kGroupUnits * (ngroups - 1u) + 8u + nl * ((last + 63u) >> 6);
+    units = header_units(ngroups, wg, nw_shift) + kGroupUnits * (ngroups - 1u) + 8u + nl * ((last + 63u) >> 6);
   }
   return (units + 3u) >> 2;
 }
@@ -75,8 +78,8 @@ __device__ __forceinline__ uint32_t region_blocks(uint32_t off, uint32_t deg, bo
 // vertices, `items` {vertex, group} for every group of them.  ctrs: [0] long lists, [1] items.  Every workgroup counts its
 // range of vertices first, so that it takes its places in the work lists with one update each.
 __global__ __launch_bounds__(1024) void fw_table_plan_kernel(const uint32_t* __restrict__ xadj, int32_t V, int32_t hub_threshold,
-                                                             uint32_t* __restrict__ blocks, uint32_t* longs, uint2* items,
-                                                             uint32_t* ctrs) {
+                                                             uint32_t nw_shift, uint32_t* __restrict__ blocks, uint32_t* longs,
+                                                             uint2* items, uint32_t* ctrs) {
   __shared__ uint32_t s_n[2], s_at[2];
   if (threadIdx.x < 2u) s_n[threadIdx.x] = 0u;
   __syncthreads();
@@ -86,7 +89,7 @@ __global__ __launch_bounds__(1024) void fw_table_plan_kernel(const uint32_t* __r
   uint32_t n_long = 0u, n_items = 0u;
   for (uint32_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) {
     const uint32_t off = xadj[v], deg = xadj[v + 1] - off;
-    blocks[v] = region_blocks(off, deg, (int32_t)deg > hub_threshold);
+    blocks[v] = region_blocks(off, deg, (int32_t)deg > hub_threshold, nw_shift);
     const uint32_t nq = list_quartets(off, deg);
     if (nq > kGq) {
       ++n_long;
@@ -321,11 +324,11 @@ __global__ __launch_bounds__(256) void fw_table_groups_kernel(const uint4* __res
     const uint32_t ngroups = (nq + kGq - 1u) / kGq;
     const bool wg = (int32_t)deg > hub_threshold;
     const uint32_t left = nq - g * kGq;
-    unsigned char* const row = region + (uint64_t)32u * (header_units(ngroups, wg) + kGroupUnits * g);
+    unsigned char* const row = region + (uint64_t)32u * (header_units(ngroups, wg, nw_shift) + kGroupUnits * g);
     const float T = table_group(weight, adjncy, off, deg, g * kGq, left < kGq ? left : kGq, row, 8u, lane, bad);
-    float2* const sums = reinterpret_cast<float2*>(region + (wg ? 64u : 0u));
-    const uint32_t at = wg ? seq_start(ngroups, g & ((1u << nw_shift) - 1u), nw_shift) + (g >> nw_shift) : g;
-    if (lane == 0) sums[at].y = T;
+    const uint32_t k = wg ? g >> nw_shift : g;
+    const uint32_t block = wg ? 1u + (g & ((1u << nw_shift) - 1u)) * seq_blocks(ngroups, wg, nw_shift) + (k >> 4) : k >> 4;
+    if (lane == 0) reinterpret_cast<float*>(region)[32u * block + 16u + (k & 15u)] = T;
   }
   if (__ballot(bad) != 0ull && lane == 0) *flag = 1u;
 }
@@ -341,17 +344,20 @@ __global__ __launch_bounds__(256) void fw_table_sums_kernel(uint4* __restrict__ 
     const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int)longs[it]);
     const uint4 rec = vrec[v];
     const uint32_t ngroups = (list_quartets(rec.w, rec.y) + kGq - 1u) / kGq;
-    unsigned char* const region = data + (uint64_t)rec.x * 128u;
+    float* const region = reinterpret_cast<float*>(data + (uint64_t)rec.x * 128u);
+    const bool wg = (int32_t)rec.y > hub_threshold;
+    const uint32_t nb = seq_blocks(ngroups, wg, nw_shift);
     float total;
-    if ((int32_t)rec.y > hub_threshold) {
-      float2* const sums = reinterpret_cast<float2*>(region + 64u);
+    if (wg) {
       const uint32_t nw = 1u << nw_shift;
       float S = 0.0f;
       if ((uint32_t)lane < nw) {
-        const uint32_t b = seq_start(ngroups, (uint32_t)lane, nw_shift), e = seq_start(ngroups, (uint32_t)lane + 1u, nw_shift);
-        for (uint32_t i = b; i < e; ++i) {
-          S = S + sums[i].y;
-          sums[i].x = S;
+        float* const sums = region + 32u + 32u * nb * (uint32_t)lane;
+        const uint32_t L = (ngroups >> nw_shift) + ((uint32_t)lane < (ngroups & (nw - 1u)) ? 1u : 0u);
+        for (uint32_t k = 0; k < 16u * nb; ++k) {
+          float* const at = sums + 32u * (k >> 4) + (k & 15u);
+          if (k < L) S = S + at[16];
+          at[0] = S;
         }
       }
       const float J = row_scan(S);
@@ -359,20 +365,20 @@ __global__ __launch_bounds__(256) void fw_table_sums_kernel(uint4* __restrict__ 
       const uint64_t mpos = __ballot(S > 0.0f);
       const uint32_t lastpos = 63u - (uint32_t)__builtin_clzll(mpos | 1ull);
       const float key = wave_prefix_max(S > 0.0f ? J : 0.0f);
-      if (lane < 16) reinterpret_cast<float*>(region)[lane] = (uint32_t)lane >= lastpos ? kInf : key;
+      if (lane < 16) region[lane] = (uint32_t)lane >= lastpos ? kInf : key;
     } else {
-      float2* const sums = reinterpret_cast<float2*>(region);
       float S = 0.0f;
-      for (uint32_t g0 = 0; g0 < ngroups; g0 += 64u) {
+      for (uint32_t g0 = 0; g0 < 16u * nb; g0 += 64u) {
         const uint32_t g = g0 + (uint32_t)lane;
-        const float T = g < ngroups ? sums[g].y : 0.0f;
+        float* const at = region + 32u * (g >> 4) + (g & 15u);
+        const float T = g < ngroups ? at[16] : 0.0f;
         float mine = 0.0f;
 #pragma unroll 8
         for (int l = 0; l < 64; ++l) {
           S = S + readlane_f(T, l);  // + 0 past the end changes nothing
           mine = lane == l ? S : mine;
         }
-        if (g < ngroups) sums[g].x = mine;
+        if (g < 16u * nb) at[0] = mine;
       }
       total = S;
     }
@@ -385,97 +391,127 @@ __global__ __launch_bounds__(256) void fw_table_sums_kernel(uint4* __restrict__ 
 // ---- the walk -----------------------------------------------------------------------------------------
 
 // First entry above t of the n entries of a row (they never decrease, the last one is above t; rows are padded to 8
-// entries), from a guess.  Four entries per look; when the guess was off twice the rest is halved.
+// entries with +inf), from a guess.  Eight entries per look, so that nearly every walker of a wave finds its entry with the first; when
+// the guess was off twice the rest is halved.  below: the entry before, 0 for the first.
 __device__ __forceinline__ uint32_t row_search(const float* row, uint32_t n, uint32_t guess, float t, float& below) {
+  const uint32_t wmax = ((n + 7u) & ~7u) - 8u;
   uint32_t lo = 0u, hi = n - 1u;
-  const uint32_t wmax = n > 4u ? n - 4u : 0u;
-  uint32_t w = guess > 1u ? guess - 1u : 0u;
+  uint32_t w = guess > 3u ? guess - 3u : 0u;
   below = 0.0f;
-  for (;;) {
+  for (int looks = 0;; ++looks) {
     w = w < wmax ? w : wmax;
-    const f4_at4 m = *reinterpret_cast<const f4_at4*>(row + w);
-    const uint32_t cnt = (m.x <= t ? 1u : 0u) + (m.y <= t ? 1u : 0u) + (m.z <= t ? 1u : 0u) + (m.w <= t ? 1u : 0u);
+    const f4_at4 m0 = *reinterpret_cast<const f4_at4*>(row + w);
+    const f4_at4 m1 = *reinterpret_cast<const f4_at4*>(row + w + 4u);
+    uint32_t cnt = 0u;
+    float at = 0.0f;  // the largest entry that is not above t
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float m = i < 4 ? m0[i & 3] : m1[i & 3];
+      const bool le = m <= t;
+      cnt += le ? 1u : 0u;
+      at = le ? m : at;
+    }
     if (cnt == 0u) {
       if (w <= lo) return w;
       hi = w;
-      w = hi - lo > 12u ? (lo + hi) >> 1 : (hi > lo + 3u ? hi - 3u : lo);
-    } else if (cnt == 4u) {
-      below = m.w;
-      lo = w + 4u;
-      if (lo >= hi) return hi;
-      w = hi - lo > 12u ? (lo + hi) >> 1 : lo;
+      w = looks == 0 || hi - lo <= 16u ? (hi > lo + 7u ? hi - 7u : lo) : (lo + hi) >> 1;
     } else {
-      below = cnt == 1u ? m.x : (cnt == 2u ? m.y : m.z);
-      return w + cnt;
+      below = at;
+      if (cnt < 8u) return w + cnt;
+      lo = w + 8u;
+      if (lo >= hi) return hi;
+      w = looks == 0 || hi - lo <= 16u ? lo : (lo + hi) >> 1;
     }
   }
 }
 
-// The neighbour of the first pair whose key is above t (n = 4 J pairs of one lane, keys as above).
+// The neighbour of the first pair whose key is above t (n = 4 J pairs of one lane, keys as above), kW pairs per look.
+template <uint32_t kW>
 __device__ __forceinline__ int32_t pair_search(const uint2* pairs, uint32_t n, uint32_t guess, float t) {
-  uint32_t lo = 0u, hi = n - 1u;
-  const uint32_t wmax = n - 4u;
-  uint32_t w = guess > 1u ? guess - 1u : 0u;
+  const uint32_t wmax = n - kW;
+  uint32_t lo = 0u;
+  uint32_t w = guess > kW / 2u - 1u ? (guess - (kW / 2u - 1u)) & ~1u : 0u;
   for (;;) {
     w = w < wmax ? w : wmax;
-    const u4_at8 a = *reinterpret_cast<const u4_at8*>(pairs + w);
-    const u4_at8 b = *reinterpret_cast<const u4_at8*>(pairs + w + 2u);
-    const bool b0 = __uint_as_float(a.x) <= t, b1 = __uint_as_float(a.z) <= t;
-    const bool b2 = __uint_as_float(b.x) <= t, b3 = __uint_as_float(b.z) <= t;
-    if (!b0) {
-      if (w <= lo) return (int32_t)a.y;
-      hi = w;
-      w = hi > lo + 3u ? hi - 3u : lo;
-    } else if (b3) {
-      lo = w + 4u;
-      if (lo > hi) return (int32_t)b.w;
-      w = lo;
-    } else {
-      return (int32_t)(b2 ? b.w : (b1 ? b.y : a.w));
+    uint4 p[kW / 2u];
+#pragma unroll
+    for (uint32_t i = 0; i < kW / 2u; ++i) p[i] = *reinterpret_cast<const uint4*>(pairs + w + 2u * i);
+    const bool first = !(__uint_as_float(p[0].x) <= t);
+    if (first && w > lo) {  // (lo: nothing before it is above t)
+      w = w > lo + kW - 1u ? (w - (kW - 2u)) & ~1u : lo & ~1u;
+      continue;
     }
+    uint32_t nb = p[kW / 2u - 1u].w;
+    const bool all = __uint_as_float(p[kW / 2u - 1u].z) <= t;
+#pragma unroll
+    for (int i = (int)kW - 2; i >= 0; --i) {
+      const uint32_t key = (i & 1) ? p[i >> 1].z : p[i >> 1].x, v = (i & 1) ? p[i >> 1].w : p[i >> 1].y;
+      nb = __uint_as_float(key) <= t ? nb : v;
+    }
+    lo = w + kW;
+    if (!all || lo >= n) return (int32_t)nb;
+    w = lo;
   }
 }
 
-// The reservoir over the groups of one sequence (L sums): the group it ends with and the target inside it.  The test of the
-// streaming kernels, S_k u > S_j, is monotone in k, so the next accepted group is searched for, from where the sums
-// would reach S_j / u if they grew evenly.
-__device__ __forceinline__ void sums_reservoir(const fw_kargs& a, const float2* sums, const uint32_t L, const float S_last,
-                                               LaneDraw& dq, const uint32_t walker, const uint32_t step, const uint32_t stream,
-                                               uint32_t& k_out, float& t_out) {
-  uint32_t k = 0u;
-  float2 e = sums[0];
-  while (!(e.x > 0.0f) && k + 1u < L) e = sums[++k];
-  float Sj = e.x, T = e.y;
-  float tu = next_uniform_lane(dq, a, walker, step, stream);
-  float u = next_uniform_lane(dq, a, walker, step, stream);
-  const float rate = (float)L * __builtin_amdgcn_rcpf(S_last);
-  while (k + 1u < L && S_last * u > Sj) {
-    uint32_t lo = k, hi = L - 1u;
-    const float want = Sj * __builtin_amdgcn_rcpf(u);
-    uint32_t i = k + 1u + (uint32_t)fmaxf((want - Sj) * rate, 0.0f);
-    float S_new, T_new;
-    for (int tries = 0;; ++tries) {
-      i = i < hi ? (i > lo ? i : lo + 1u) : hi;
-      const f4_at8 p = *reinterpret_cast<const f4_at8*>(sums + i - 1u);
-      S_new = p.z;
-      T_new = p.w;
-      if (p.x * u > Sj && i - 1u > lo) {
-        hi = i - 1u;
-      } else if (p.z * u > Sj || i == hi) {
-        break;
-      } else {
-        lo = i;
+__device__ __forceinline__ void load16(const float* p, float (&s)[16]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 x = reinterpret_cast<const float4*>(p)[i];
+    s[4 * i] = x.x; s[4 * i + 1] = x.y; s[4 * i + 2] = x.z; s[4 * i + 3] = x.w;
+  }
+}
+
+// The reservoir over the groups of one sequence (nb blocks of sums): the group it ends with, its uniform and where its total is.  The
+// test of the streaming kernels, S_k u > S_j, is monotone in k, so the next accepted group is the first of the 16 sums in
+// registers that passes it; only when none does is another block looked for, from where the sums would reach S_j / u if
+// they grew evenly.  (One look at memory per accepted group made every wave wait for the longest such chain of its 64 walkers.)
+__device__ __forceinline__ const float* sums_reservoir(const fw_kargs& a, const float* sums, const uint32_t nb, LaneDraw& dq,
+                                                       const uint32_t walker, const uint32_t step, const uint32_t stream,
+                                                       uint32_t& k_out, float& tu_out) {
+  float s[16];
+  load16(sums, s);
+  float S_last = s[15];
+  if (nb > 1u) S_last = sums[32u * (nb - 1u) + 15u];
+  float Sj = 0.0f, u = 1.0f, tu = 0.0f;  // the first group that has a total is always accepted
+  uint32_t b = 0u, k = 0u;
+  while (S_last * u > Sj) {
+    if (!(s[15] * u > Sj)) {
+      uint32_t lo = b, hi = nb - 1u;  // block lo has none, block hi has one
+      const float per = (float)nb * __builtin_amdgcn_rcpf(S_last);
+      const float want = Sj * __builtin_amdgcn_rcpf(u) * per;
+      uint32_t i = want < (float)nb ? (uint32_t)want : hi;
+      for (int tries = 0;; ++tries) {
+        i = i < hi ? (i > lo ? i : lo + 1u) : hi;
+        load16(sums + 32u * i, s);
+        const float before = sums[32u * i - 17u];  // the last sum of the block before
+        if (before * u > Sj && i - 1u > lo) {
+          hi = i - 1u;
+        } else if (s[15] * u > Sj || i == hi) {
+          break;
+        } else {
+          lo = i;
+        }
+        i = tries < 2 ? (hi == i - 1u ? hi : i + 1u) : lo + ((hi - lo + 1u) >> 1);
       }
-      i = tries < 2 ? (uint32_t)((int32_t)i + 1 + (int32_t)((want - p.z) * rate)) : lo + ((hi - lo + 1u) >> 1);
+      b = i;
     }
-    k = i;
+    uint32_t cnt = 0u;
+    float S_new = kInf;
+#pragma unroll
+    for (int i = 15; i >= 0; --i) {
+      const bool hit = s[i] * u > Sj;
+      cnt += hit ? 0u : 1u;
+      S_new = hit ? s[i] : S_new;
+    }
+    k = 16u * b + cnt;
     Sj = S_new;
-    T = T_new;
     tu = next_uniform_lane(dq, a, walker, step, stream);
     u = next_uniform_lane(dq, a, walker, step, stream);
   }
   k_out = k;
-  t_out = tu * T;
+  tu_out = tu;
+  return sums + 32u * (k >> 4) + 16u + (k & 15u);
 }
 
 // One proposal of the step's sampler for a list with a positive total: the selected neighbour.  d: block 0 of the step's stream 0.
@@ -485,50 +521,43 @@ __device__ __forceinline__ int32_t table_pick(const fw_kargs& a, const fw_table_
   const uint32_t nq = list_quartets(rec.w, rec.y);
   const unsigned char* row = tb.data + (uint64_t)rec.x * 128u;
   uint32_t nqg = nq, row_units = 8u;
-  float T = total, t;
+  float T = total, tu = u24(d.x);
   if (nq <= kGq) {
     if (nq < 64u) row_units = (nq + 7u) >> 3;
-    t = u24(d.x) * total;
   } else {
     const uint32_t ngroups = (nq + kGq - 1u) / kGq;
     const bool wg = (int32_t)rec.y > a.hub_threshold;
-    const float2* sums = reinterpret_cast<const float2*>(row);
-    uint32_t L = ngroups, seq = 0u;
-    float S_last = total;
+    const uint32_t nb = seq_blocks(ngroups, wg, tb.nw_shift);
+    const float* sums = reinterpret_cast<const float*>(row);
+    uint32_t seq = 0u;
     LaneDraw dq;
     if (wg) {  // which sequence, then the reservoir over it with draws of its own stream
       const float target = u24(philox4x32_10(walker, step, kStreamWave | sbase, 0u, a.seed_lo, a.seed_hi).x) * total;
-      const float4* keys = reinterpret_cast<const float4*>(row);
+      float keys[16];
+      load16(sums, keys);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float4 k4 = keys[i];
-        seq += (k4.x <= target ? 1u : 0u) + (k4.y <= target ? 1u : 0u) + (k4.z <= target ? 1u : 0u) + (k4.w <= target ? 1u : 0u);
-      }
-      const uint32_t b = seq_start(ngroups, seq, tb.nw_shift);
-      L = seq_start(ngroups, seq + 1u, tb.nw_shift) - b;
-      sums = reinterpret_cast<const float2*>(row + 64u) + b;
-      S_last = sums[L - 1u].x;
+      for (int i = 0; i < 16; ++i) seq += keys[i] <= target ? 1u : 0u;
+      sums += 32u + 32u * nb * seq;
     } else {
       dq.q0 = d.x; dq.q1 = d.y; dq.q2 = d.z; dq.q3 = d.w;
       dq.avail = 4u;
       dq.blk = 1u;
     }
     uint32_t k;
-    sums_reservoir(a, sums, L, S_last, dq, walker, step, seq | sbase, k, t);
+    T = *sums_reservoir(a, sums, nb, dq, walker, step, seq | sbase, k, tu);
     const uint32_t g = wg ? seq + (k << tb.nw_shift) : k;
-    row += (uint64_t)32u * (header_units(ngroups, wg) + kGroupUnits * g);
+    row += (uint64_t)32u * (header_units(ngroups, wg, tb.nw_shift) + kGroupUnits * g);
     nqg = nq - g * kGq < kGq ? nq - g * kGq : kGq;
-    T = total * (float)kGq / (float)nq;  // about a group's share (the guess below needs no more)
-    if (nqg < kGq) T = total * (float)nqg / (float)nq;
   }
+  const float t = tu * T;
   const uint32_t nl = nqg < 64u ? nqg : 64u;
   const uint32_t J = (nqg + 63u) >> 6;
-  const float lanes_per_t = (float)nl * __builtin_amdgcn_rcpf(T);
   float below;
-  const uint32_t l = row_search(reinterpret_cast<const float*>(row), nl, (uint32_t)(t * lanes_per_t), t, below);
+  const uint32_t l = row_search(reinterpret_cast<const float*>(row), nl, (uint32_t)(tu * (float)nl), t, below);
   const uint2* pairs = reinterpret_cast<const uint2*>(row + 32u * (row_units + l * J));
-  const uint32_t guess = J == 1u ? 0u : (uint32_t)fmaxf((t - below) * lanes_per_t * (float)(4u * J), 0.0f);
-  return pair_search(pairs, 4u * J, guess, t);
+  if (J == 1u) return pair_search<4>(pairs, 4u, 0u, t);
+  const float guess = (t - below) * (float)(4u * J * nl) * __builtin_amdgcn_rcpf(T);
+  return pair_search<8>(pairs, 4u * J, guess > 0.0f ? (guess < 15.0f ? (uint32_t)guess : 15u) : 0u, t);
 }
 
 // One lane, one walker, from its start to its end; a lane whose walk is over takes the next query of its wave's range.
@@ -536,7 +565,7 @@ __device__ __forceinline__ int32_t table_pick(const fw_kargs& a, const fw_table_
 // lines; the entries of a row before its first and after its last whole line, and the -1 behind the walk, are stored by the
 // wave together, one row at a time.
 template <int kApp>
-__global__ __launch_bounds__(256, 4) void fw_table_walk(const fw_kargs a, const fw_table_args tb) {
+__global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, const fw_table_args tb) {
   __shared__ __align__(16) int32_t s_buf[4][64 * 16];
   __shared__ unsigned long long s_acc[4];
   const int lane = lane_id();
@@ -550,10 +579,11 @@ __global__ __launch_bounds__(256, 4) void fw_table_walk(const fw_kargs a, const 
   const uint32_t md = (uint32_t)a.max_depth;
   const uint32_t align0 = (uint32_t)(reinterpret_cast<uintptr_t>(a.paths) >> 2) & 15u;
 
-  uint64_t next64 = ((uint64_t)blockIdx.x * 4u + (uint64_t)wave) * tb.chunk;
   const uint32_t n = (uint32_t)a.n;
-  uint32_t cursor = next64 < n ? (uint32_t)next64 : n;
-  const uint32_t last = next64 + tb.chunk < n ? (uint32_t)(next64 + tb.chunk) : n;
+  const uint64_t first = ((uint64_t)blockIdx.x * 4u + (uint64_t)wave) * tb.lanes;  // the next ranges come from the dispenser
+  uint32_t cursor = first < n ? (uint32_t)first : n;
+  uint32_t last = n - cursor > tb.lanes ? cursor + tb.lanes : n;
+  bool more = (uint64_t)gridDim.x * 4u * tb.lanes < n;
 
   bool active = false, fresh = false;
   uint32_t q = 0u, len = 0u, s0 = 0u, fpos = 0u;
@@ -570,6 +600,16 @@ __global__ __launch_bounds__(256, 4) void fw_table_walk(const fw_kargs a, const 
     {
       const bool want = !active && (uint32_t)lane < tb.lanes;
       const uint64_t m = __ballot(want);
+      if (m != 0ull && cursor == last && more) {
+        uint32_t at = 0u;
+        if (lane == 0) at = atomicAdd(a.dispenser, tb.lanes);
+        at = gridDim.x * 4u * tb.lanes + (uint32_t)__builtin_amdgcn_readfirstlane((int)at);  // (below 2^32: n is below 2^31)
+        more = at < n;
+        if (more) {
+          cursor = at;
+          last = n - at > tb.lanes ? at + tb.lanes : n;
+        }
+      }
       if (m != 0ull && cursor < last) {
         const uint32_t qn = cursor + (uint32_t)__builtin_popcountll(m & ((1ull << lane) - 1ull));
         if (want && qn < last) {
@@ -698,8 +738,9 @@ __global__ __launch_bounds__(256, 4) void fw_table_walk(const fw_kargs a, const 
 
 // Around the walk: the counters start at zero, and their sums go to the host (pinned memory: the call waits for the stream
 // anyway, and a copy of its own would cost a small call as much as its launch).
-__global__ void fw_table_begin_kernel(unsigned long long* counters) {
+__global__ void fw_table_begin_kernel(unsigned long long* counters, uint32_t* scratch, uint32_t words) {
   for (uint32_t i = threadIdx.x; i < FW_TABLE_STRIPES * 8u; i += blockDim.x) counters[i] = 0ull;
+  for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) scratch[i] = 0u;
 }
 __global__ __launch_bounds__(64) void fw_table_end_kernel(const unsigned long long* __restrict__ counters, unsigned long long* out) {
   unsigned long long c[4];
@@ -732,16 +773,14 @@ int launch_table_walk(const fw_kargs& a, fw_table_args tb, int grid, hipStream_t
     tb.lanes = n / spread < 64u ? n / spread + 1u : 64u;
     if (tb.lanes > 64u) tb.lanes = 64u;
     waves = ((uint64_t)n + tb.lanes - 1u) / tb.lanes;
-    // many: a wave takes query after query.  Waves come and go (sixteen times as many as fit at half occupancy), so that the
-    // chip stays full to the end; PPR's short walks, whose lanes rarely end together, want longer ranges (4 / 16 times:
-    // PPR on R-MAT 22 1.60 / 1.95 ms, DeepWalk there 12.6 / 10.4, on R-MAT 24 80.7 / 74.2)
-    const uint64_t most = (uint64_t)cus * 16u * (kApp == FW_APP_PPR ? 4u : 16u);
+    // many: as many waves as fit, and a wave takes as many queries as it has lanes from the dispenser whenever its own are
+    // used up, so that lanes are idle only at the very end (waves with a fixed share of the queries each idled for 30 % of
+    // their lanes' time, when the last of a share walked: DeepWalk R-MAT 24 76.6 -> 47.9 ms, R-MAT 22 9.86 -> 6.79, PPR
+    // there 1.62 -> 1.16)
+    const uint64_t most = (uint64_t)cus * 4u * kWaves;
     if (waves > most) waves = most;
   }
-  uint64_t chunk = ((uint64_t)n + waves - 1u) / waves;
-  tb.chunk = (uint32_t)chunk;
-  const uint64_t need = ((uint64_t)n + chunk - 1u) / chunk;
-  const unsigned blocks = (unsigned)((need + 3u) / 4u);
+  const unsigned blocks = (unsigned)((waves + 3u) / 4u);
   hipLaunchKernelGGL((fw_table_walk<kApp>), dim3(blocks), dim3(256), 0, stream, a, tb);
   FW_HIP(hipGetLastError());
   if (grid_used) *grid_used = (int)blocks;
@@ -761,8 +800,8 @@ int fw_launch_table_walk(const fw_kargs& a, const fw_table_args& tb, int app, in
   }
 }
 
-int fw_table_begin(unsigned long long* d_counters, hipStream_t stream) {
-  hipLaunchKernelGGL(fw_table_begin_kernel, dim3(1), dim3(512), 0, stream, d_counters);
+int fw_table_begin(unsigned long long* d_counters, uint32_t* d_scratch, uint32_t words, hipStream_t stream) {
+  hipLaunchKernelGGL(fw_table_begin_kernel, dim3(1), dim3(512), 0, stream, d_counters, d_scratch, words);
   FW_HIP(hipGetLastError());
   return FW_OK;
 }
@@ -774,10 +813,10 @@ int fw_table_end(const unsigned long long* d_counters, unsigned long long* h_out
   return FW_OK;
 }
 
-int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
+int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t nw_shift, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
                   hipStream_t stream) {
-  hipLaunchKernelGGL(fw_table_plan_kernel, dim3(1024), dim3(1024), 0, stream, g->xadj, g->V, hub_threshold, d_blocks, d_longs,
-                     d_items, d_ctrs);
+  hipLaunchKernelGGL(fw_table_plan_kernel, dim3(1024), dim3(1024), 0, stream, g->xadj, g->V, hub_threshold, nw_shift, d_blocks,
+                     d_longs, d_items, d_ctrs);
   FW_HIP(hipGetLastError());
   return FW_OK;
 }
