@@ -1685,6 +1685,31 @@ static int plan_tables(const fw_graph* g, fw_tables* t, uint32_t** d_base_out, h
   return FW_OK;
 }
 
+// Whether this call makes the hash sets of node2vec's adjacency tests (their memory is there then).  They are made once the calls' searches
+// have cost, or are about to cost, half as much again as making them: a search that finds the chip busy costs 0.05 ns (five
+// scattered reads at 51 G/s, half of the tests undecided; R-MAT 24: 41 ms of 709 M steps), one in a chain of a few walkers 4 us, and the sets take
+// 0.2 ms and 20 bytes per edge at 2.5 TB/s.
+static bool sets_for_call(const fw_graph* g, const fw_walk_params* p, fw_tables* t, double all_steps, double steps) {
+  const bool back = p->p < 1.0f && p->p < p->q;  // the return edge is a component of its own
+  if (p->app != FW_APP_NODE2VEC || (p->q == 1.0f && !back) || t->no_sets) return false;
+  const bool want_weights = back && t->set_weights == nullptr;
+  if (t->sets != nullptr && !want_weights) return p->time_kernels != 0 || (g->borrowed && back);
+  if (t->sets == nullptr) {
+    t->search_ms += all_steps * 0.05e-6 > steps * 0.004 ? all_steps * 0.05e-6 : steps * 0.004;
+    if (t->search_ms < kMakeMargin * (20.0 * (double)g->E / 2.5e9 + 0.2)) return false;
+  }
+  const size_t places = 16u * (size_t)(fw_set_first((uint32_t)g->E, (uint32_t)g->V) + 1u);
+  auto room = [&](void** at) {
+    if (hipMalloc(at, places * 4u) == hipSuccess) return;
+    (void)hipGetLastError();
+    *at = nullptr;
+    t->no_sets = 1;
+  };
+  if (t->sets == nullptr) room(reinterpret_cast<void**>(&t->sets));
+  if (t->sets != nullptr && want_weights) room(reinterpret_cast<void**>(&t->set_weights));
+  return t->sets != nullptr;  // (without their weights the return edge is searched for)
+}
+
 // The tables a call over n queries walks on, or none (*out stays empty).  Called with the graph's busy flag held.  ev_start is
 // recorded before the making, ev0 and ev1 around it when its time is asked for; *launches: kernels it took.
 static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipStream_t stream, std::shared_ptr<fw_tables>* out,
@@ -1702,12 +1727,9 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     t = g->tables;
   }
   if (t && (t->hub_threshold != p->hub_threshold || t->nw_shift != nw_shift)) t.reset();
-  if (t && !g->borrowed && p->time_kernels == 0) {  // (a call that wants the split of its time makes them anew)
-    *out = t;
-    return FW_OK;
-  }
+  const bool make_tables = !t || g->borrowed || p->time_kernels != 0;  // (a call that wants the split of its time makes them anew)
+  double steps = (double)(p->max_depth - 1);
   if (!t || g->borrowed) {
-    double steps = (double)(p->max_depth - 1);
     if (p->app == FW_APP_PPR && p->tp > 0.0f && 1.0 / (double)p->tp < steps) steps = 1.0 / (double)p->tp;
     double ms = steps * kStepLatencyMs;
     if (steps * (double)n >= 1.0e6) {  // (a smaller first call costs little more than asking: 0.04 ms)
@@ -1735,21 +1757,34 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     }
     if (rc != FW_OK) return rc;
   }
+  const bool make_sets = sets_for_call(g, p, t.get(), steps * (double)n, steps);
+  if (!make_tables && !make_sets) {
+    *out = t;
+    return FW_OK;
+  }
   uint32_t bad = 0u;
   auto make = [&]() -> int {
     if (ev_start) FW_HIP(hipEventRecord(ev_start, stream));
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev0, stream));
-    FW_HIP(hipMemsetAsync(t->flag, 0, sizeof(uint32_t), stream));
-    const int rc = fw_table_make(g, t.get(), d_base, stream, launches);
-    if (rc != FW_OK) return rc;
+    int rc = FW_OK;
+    if (make_tables) {
+      FW_HIP(hipMemsetAsync(t->flag, 0, sizeof(uint32_t), stream));
+      if ((rc = fw_table_make(g, t.get(), d_base, stream, launches)) != FW_OK) return rc;
+    }
+    if (make_sets && (rc = fw_sets_make(g, t.get(), stream, launches)) != FW_OK) return rc;
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
+    if (!make_tables) return FW_OK;
     FW_HIP(hipMemcpyAsync(&bad, t->flag, sizeof(bad), hipMemcpyDeviceToHost, stream));
     FW_HIP(hipStreamSynchronize(stream));
     return FW_OK;
   };
   const int rc = make();
   if (d_base) (void)hipFree(d_base);
-  if (rc != FW_OK) return rc;
+  if (rc != FW_OK) {  // nothing half made stays
+    std::lock_guard<std::mutex> guard(g->tables_lock);
+    g->tables.reset();
+    return rc;
+  }
   if (bad != 0u) {  // the streaming kernels define what happens then
     if (!g->borrowed) g->no_tables = 1;
     *launches = 0;
@@ -1767,6 +1802,8 @@ static fw_table_args table_args(const fw_tables& t, unsigned long long* d_counte
   fw_table_args tb;
   tb.vrec = t.vrec;
   tb.data = t.data;
+  tb.sets = t.sets;
+  tb.set_weights = t.set_weights;
   tb.nw_shift = t.nw_shift;
   tb.lanes = 0u;
   tb.counters = d_counters;

@@ -20,7 +20,7 @@ struct fw_hub_info {
 constexpr uint32_t FW_NO_ROWS = 0xFFFFFFFFu;
 
 // List tables (fw_table_walk.hip): the walker-independent part of every sampling step on a graph.  Not changed once made, and
-// held by reference count: a call that walks on a set keeps it alive while another call replaces it in the graph.
+// held by reference count: a call that walks on them keeps them alive while another call replaces them in the graph.
 struct fw_tables {
   uint4* vrec = nullptr;          // [V] {region in 128-byte blocks, degree, total, CSR offset}
   unsigned char* data = nullptr;  // the regions
@@ -31,8 +31,13 @@ struct fw_tables {
   int32_t hub_threshold = 0;      // which long lists are cut into sequences, and how many of them (as a power of two):
   uint32_t nw_shift = 0;          // part of the sampler's definition
   size_t bytes = 0;
+  // node2vec: the lists as hash sets (and the weights of their entries), made when its calls' work pays for them
+  int32_t* sets = nullptr;
+  float* set_weights = nullptr;
+  double search_ms = 0.0;         // what node2vec calls without sets spent on searches, estimated
+  int no_sets = 0;                // no room for them: do not try again
   ~fw_tables() {
-    void* ptrs[5] = {vrec, data, longs, items, flag};
+    void* ptrs[7] = {vrec, data, longs, items, flag, sets, set_weights};
     for (void* p : ptrs) if (p) (void)hipFree(p);
   }
 };
@@ -195,9 +200,16 @@ struct fw_hub_args {
 constexpr uint32_t FW_TABLE_STRIPES = 64;
 constexpr size_t FW_TABLE_COUNTER_BYTES = FW_TABLE_STRIPES * 64u;
 
+// Hash sets of the lists: buckets of 16 neighbours (64 bytes).  A list of d entries has d / 8 + 1 buckets, and its first one follows
+// from its place in the CSR, so that nothing has to be looked up to find it.
+__host__ __device__ inline uint64_t fw_set_first(uint32_t off, uint32_t v) { return (uint64_t)(off >> 3) + v; }
+__host__ __device__ inline uint32_t fw_set_buckets(uint32_t deg) { return (deg >> 3) + 1u; }
+
 struct fw_table_args {
   const uint4* vrec;
   const unsigned char* data;
+  const int32_t* sets;           // node2vec: NULL: search the lists
+  const float* set_weights;
   uint32_t nw_shift;
   uint32_t lanes;                // lanes of a wave that walk, and the queries it takes at a time (set by the launch)
   unsigned long long* counters;  // [FW_TABLE_STRIPES * 8]
@@ -272,11 +284,12 @@ int fw_launch_hub_quad(const fw_kargs& a, const fw_hub_args& h, int app, uint32_
 int fw_launch_hub_scan(const fw_kargs& a, const fw_hub_args& h, int app, uint32_t tasks_hint, hipStream_t stream);
 
 // List tables.  plan: region sizes into d_blocks[0 .. V], work lists and their sizes (d_ctrs[0]: long lists, [1]: items);
-// make: fills the tables (d_base: region positions, NULL when vrec has them); walk: every query from start to end, between
+// make: fills the tables (d_base: region positions, NULL when vrec has them); sets_make: fills sets and set_weights (if given); walk: every query from start to end, between
 // begin (counters and launch records to zero) and end (their sums to pinned host memory).
 int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t nw_shift, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
                   hipStream_t stream);
 int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches);
+int fw_sets_make(const fw_graph* g, const fw_tables* t, hipStream_t stream, int* launches);
 int fw_launch_table_walk(const fw_kargs& a, const fw_table_args& tb, int app, int grid, hipStream_t stream, int* grid_used);
 int fw_table_begin(unsigned long long* d_counters, uint32_t* d_scratch, uint32_t words, hipStream_t stream);
 int fw_table_end(const unsigned long long* d_counters, unsigned long long* h_out, hipStream_t stream);

@@ -388,6 +388,133 @@ __global__ __launch_bounds__(256) void fw_table_sums_kernel(uint4* __restrict__ 
   if (__ballot(bad) != 0ull && lane == 0) *flag = 1u;
 }
 
+// ---- hash sets (node2vec) -----------------------------------------------------------------------------
+//
+// node2vec asks whether the proposal is a neighbour of the previous vertex, and for a large 1/p what the entries that lead
+// back weigh.  A binary search answers with a chain of some ten dependent reads that scatter over the list (most of what a step
+// cost: R-MAT 24 spent 41 of 89 ms on it); a hash set answers with one read of 64 bytes.  Every list has a set of its own, half full on
+// average: one entry per distinct neighbour, in the bucket its hash names, -1 in free places.  A bucket more than 16
+// neighbours fall into (one in some hundred) says so, and its walkers search the list as before.
+
+constexpr int32_t kSetOverflow = (int32_t)0x80000000;  // in the last place of a bucket
+constexpr uint32_t kSetPart = 1040u;    // buckets a workgroup makes at a time, for every eight groups of a long list: the parts
+                                        // of a list of d > 1020 entries, ceil(groups / 8) of them, cover its d / 8 + 1 buckets
+constexpr uint32_t kSetSmall = 1024u / 8u + 1u;  // buckets of a list of one group
+
+__device__ __forceinline__ uint32_t set_bucket(int32_t neighbour, uint32_t buckets) {
+  uint32_t h = (uint32_t)neighbour * 0x9E3779B1u;  // Knuth's multiplicative hash, folded and repeated: R-MAT ids differ in few bits
+  h = (h ^ (h >> 15)) * 0x85EBCA77u;
+  return __umulhi(h, buckets);
+}
+
+// Entry i of a list into its bucket, if that is one of the `part` buckets from b0 on.  out_w: the weights' places of those buckets.
+__device__ __forceinline__ void set_insert(const int32_t* __restrict__ adj, const float* __restrict__ w, uint32_t deg, uint32_t i,
+                                           uint32_t buckets, uint32_t b0, uint32_t part, int32_t* s_slots, uint32_t* s_count,
+                                           float* out_w) {
+  const int32_t x = adj[i];
+  if (i != 0u && adj[i - 1u] == x) return;  // the lists ascend: equal neighbours lie together, the first stands for all
+  const uint32_t b = set_bucket(x, buckets) - b0;
+  if (b >= part) return;
+  const uint32_t at = atomicAdd(&s_count[b], 1u);
+  if (at >= 16u) return;
+  s_slots[16u * b + at] = x;
+  if (out_w != nullptr) {
+    float sum = 0.0f;
+    for (uint32_t j = i; j < deg && adj[j] == x; ++j) sum = sum + w[j];
+    out_w[16u * b + at] = sum;
+  }
+}
+
+// Lists of one group, one wave per list.  Bound: memory (4 bytes read and about 10 written per edge).
+__global__ __launch_bounds__(256) void fw_sets_small_kernel(const uint4* __restrict__ vrec, const int32_t* __restrict__ adjncy,
+                                                            const float* __restrict__ weight, int32_t V, int32_t* sets, float* set_weights) {
+  __shared__ __align__(16) int32_t s_slots[4][16u * kSetSmall];
+  __shared__ uint32_t s_count[4][kSetSmall];
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint64_t chunks = ((uint64_t)(uint32_t)V + 63u) >> 6;
+  for (uint64_t ch = (uint64_t)blockIdx.x * 4u + (uint64_t)wave; ch < chunks; ch += (uint64_t)gridDim.x * 4u) {
+    const uint32_t v0 = (uint32_t)(ch * 64u);
+    uint32_t off = 0u, deg = 0u;
+    if (v0 + (uint32_t)lane < (uint32_t)V) {
+      const uint4 rec = vrec[v0 + (uint32_t)lane];
+      off = rec.w;
+      deg = rec.y;
+    }
+    for (uint64_t m = __ballot(deg != 0u && list_quartets(off, deg) <= kGq); m != 0ull; m &= m - 1ull) {
+      const int l = __builtin_ctzll(m);
+      const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)off, l), d = (uint32_t)__builtin_amdgcn_readlane((int)deg, l);
+      const uint32_t nb = fw_set_buckets(d);
+      const uint64_t first = 16u * fw_set_first(o, v0 + (uint32_t)l);
+      int4* const slots = reinterpret_cast<int4*>(s_slots[wave]);
+      for (uint32_t i = (uint32_t)lane; i < 4u * nb; i += 64u) slots[i] = make_int4(-1, -1, -1, -1);
+      for (uint32_t i = (uint32_t)lane; i < nb; i += 64u) s_count[wave][i] = 0u;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      for (uint32_t i = (uint32_t)lane; i < d; i += 64u)
+        set_insert(adjncy + o, weight + o, d, i, nb, 0u, nb, s_slots[wave], s_count[wave], set_weights ? set_weights + first : nullptr);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      for (uint32_t i = (uint32_t)lane; i < 4u * nb; i += 64u) {
+        int4 x = slots[i];
+        if ((i & 3u) == 3u && s_count[wave][i >> 2] > 16u) x.w = kSetOverflow;
+        reinterpret_cast<int4*>(sets + first)[i] = x;
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+}
+
+// Long lists: one workgroup per eight groups of a list makes kSetPart buckets and reads the whole list for them (a list of
+// 100,000 entries is read 13 times, from the cache).
+__global__ __launch_bounds__(512) void fw_sets_long_kernel(const uint4* __restrict__ vrec, const int32_t* __restrict__ adjncy,
+                                                           const float* __restrict__ weight, const uint2* __restrict__ items,
+                                                           uint32_t n_items, int32_t* sets, float* set_weights) {
+  __shared__ __align__(16) int32_t s_slots[16u * kSetPart];
+  __shared__ uint32_t s_count[kSetPart];
+  for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
+    const uint2 item = items[it];
+    if ((item.y & 7u) != 0u) continue;
+    const uint4 rec = vrec[item.x];
+    const uint32_t nb = fw_set_buckets(rec.y);
+    const uint32_t b0 = (item.y >> 3) * kSetPart;
+    if (b0 >= nb) continue;
+    const uint32_t part = nb - b0 < kSetPart ? nb - b0 : kSetPart;
+    const uint64_t first = 16u * (fw_set_first(rec.w, item.x) + b0);
+    int4* const slots = reinterpret_cast<int4*>(s_slots);
+    for (uint32_t i = threadIdx.x; i < 4u * part; i += blockDim.x) slots[i] = make_int4(-1, -1, -1, -1);
+    for (uint32_t i = threadIdx.x; i < part; i += blockDim.x) s_count[i] = 0u;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < rec.y; i += blockDim.x)
+      set_insert(adjncy + rec.w, weight + rec.w, rec.y, i, nb, b0, part, s_slots, s_count, set_weights ? set_weights + first : nullptr);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < 4u * part; i += blockDim.x) {
+      int4 x = slots[i];
+      if ((i & 3u) == 3u && s_count[i >> 2] > 16u) x.w = kSetOverflow;
+      reinterpret_cast<int4*>(sets + first)[i] = x;
+    }
+    __syncthreads();
+  }
+}
+
+// The place of `target` in the set of vertex v's list: its index in the sets, -1 (not there) or -2 (its bucket overflowed).
+__device__ __forceinline__ int64_t set_find(const int32_t* __restrict__ sets, uint32_t v, uint32_t off, uint32_t deg, int32_t target) {
+  const uint64_t first = 16u * (fw_set_first(off, v) + set_bucket(target, fw_set_buckets(deg)));
+  int32_t at = -1;
+  int4 x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = reinterpret_cast<const int4*>(sets + first)[i];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    at = x[i].x == target ? 4 * i : at;
+    at = x[i].y == target ? 4 * i + 1 : at;
+    at = x[i].z == target ? 4 * i + 2 : at;
+    at = x[i].w == target ? 4 * i + 3 : at;
+  }
+  if (at >= 0) return (int64_t)first + at;
+  return x[3].w == kSetOverflow ? -2 : -1;
+}
+
 // ---- the walk -----------------------------------------------------------------------------------------
 
 // First entry above t of the n entries of a row (they never decrease, the last one is above t; rows are padded to 8
@@ -647,13 +774,21 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
         int32_t nv = table_pick(a, tb, rec, d, walker, step, sbase);
         bool moved = true;
         if (kApp == FW_APP_NODE2VEC && prev >= 0) {
-          if (a.n2v_extra > 0.0f && fresh) w_ret = return_weight(a.adjncy + rec.w, a.weight + rec.w, rec.y, prev);
+          if (a.n2v_extra > 0.0f && fresh) {
+            const int64_t at = tb.set_weights != nullptr ? set_find(tb.sets, (uint32_t)v, rec.w, rec.y, prev) : -2;
+            w_ret = at >= 0 ? tb.set_weights[at] : 0.0f;
+            if (at == -2) w_ret = return_weight(a.adjncy + rec.w, a.weight + rec.w, rec.y, prev);
+          }
           const N2vTest t = n2v_test(a, nv, prev, walker, step, trial, __uint_as_float(rec.z), w_ret);
           if (t.take_prev) {
             nv = prev;
           } else {
             bool common = false;
-            if (!t.decided) common = sorted_contains(a.adjncy + prev_off, (int32_t)prev_deg, nv);
+            if (!t.decided) {
+              const int64_t at = tb.sets != nullptr ? set_find(tb.sets, (uint32_t)prev, prev_off, prev_deg, nv) : -2;
+              common = at >= 0;
+              if (at == -2) common = sorted_contains(a.adjncy + prev_off, (int32_t)prev_deg, nv);
+            }
             moved = n2v_finish(a, t, common);
           }
         }
@@ -840,6 +975,23 @@ int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipSt
                        t->hub_threshold, t->nw_shift, t->data, t->flag);
     FW_HIP(hipGetLastError());
     *launches += 2;
+  }
+  return FW_OK;
+}
+
+int fw_sets_make(const fw_graph* g, const fw_tables* t, hipStream_t stream, int* launches) {
+  int cus = 0;
+  FW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
+  const uint64_t blocks = (((uint64_t)g->V + 63u) / 64u + 3u) / 4u, most = (uint64_t)cus * 64u;
+  hipLaunchKernelGGL(fw_sets_small_kernel, dim3((unsigned)(blocks < most ? blocks : most)), dim3(256), 0, stream, t->vrec, g->adjncy,
+                     g->weight, g->V, t->sets, t->set_weights);
+  FW_HIP(hipGetLastError());
+  *launches += 1;
+  if (t->n_items != 0u) {
+    hipLaunchKernelGGL(fw_sets_long_kernel, dim3(t->n_items < most ? t->n_items : (unsigned)most), dim3(512), 0, stream, t->vrec,
+                       g->adjncy, g->weight, t->items, t->n_items, t->sets, t->set_weights);
+    FW_HIP(hipGetLastError());
+    *launches += 1;
   }
   return FW_OK;
 }

@@ -2,8 +2,11 @@
 the tables' shapes (quartets, the lanes of a group, groups, sequences), biases that are zero, close to even and far from
 even, path rows of every alignment.  The tables are made when a call's walkers would read the edge array several times over,
 so the first call on a graph is a large one and later, smaller calls walk on what it made."""
+import ctypes as C
+
 import numpy as np
 import pytest
+import torch
 
 import fw_oracle_binding as _oracle
 
@@ -67,5 +70,59 @@ def test_walks_on_tables(gpu, kind, wg, thr):
                 assert st.launches >= 4  # the tables were made
             again, st2 = g.walk_batch(p, starts, batch_size=max(1, n // 3))
             assert (again == ref).all() and (st2.steps, st2.sampled_edges) == (steps, edges), (kw, n)
+    finally:
+        g.destroy()
+
+
+@pytest.mark.parametrize("kind", ["even", "uneven"])
+def test_node2vec_on_hash_sets(gpu, kind):
+    """The first call is long enough to pay for the sets (one walk of 100 steps counts as 0.4 ms of searches, 1.5 times 0.2 ms are asked
+    for); the lists hold equal neighbours, and the longest have buckets that more than 16 neighbours fall into."""
+    csr, at = _lists(kind)
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    rng = np.random.RandomState(7)
+    try:
+        warm = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21)
+        g.walk(warm, at[rng.randint(0, len(at), size=70000)].astype(np.int32))
+        for i, (p, q) in enumerate(((2.0, 0.5), (0.25, 4.0), (4.0, 0.25), (1.0, 1.0), (0.1, 1.0), (1.0, 3.0), (0.5, 0.25))):
+            par = gpu.default_params(app=gpu.APP_NODE2VEC, max_depth=101, p=p, q=q, seed=50 + i)
+            starts = at[rng.randint(0, len(at), size=400)].astype(np.int32)
+            ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(par), starts)
+            paths, st = g.walk(par, starts)
+            bad = np.nonzero((paths != ref).any(axis=1))[0]
+            assert len(bad) == 0, (p, q, bad[0], paths[bad[0]], ref[bad[0]])
+            assert (st.steps, st.sampled_edges) == (steps, edges)
+            assert st.launches == (5 if i < 2 else 3)  # the sets, then with the first return edge above the envelope their weights
+    finally:
+        g.destroy()
+
+
+def test_changed_biases_on_adopted_arrays(gpu):
+    """An adopted graph's owner may change the biases between calls: tables and the sets' weights are made anew."""
+    csr, at = _lists("even")
+    xadj, adj, w = csr
+    pad = lambda x: torch.from_numpy(np.concatenate([x, np.zeros(4, dtype=x.dtype)])).cuda()
+    dx, da, dw = pad(xadj.view(np.int32)), pad(adj), pad(w)
+    torch.cuda.synchronize()
+    h = C.c_void_p()
+    gpu.check(gpu.lib().fw_graph_adopt_device(V, len(adj), C.c_void_p(dx.data_ptr()), C.c_void_p(da.data_ptr()),
+                                              C.c_void_p(dw.data_ptr()), None, 0, C.byref(h)))
+    g = gpu.Graph(h)
+    rng = np.random.RandomState(8)
+    starts = at[rng.randint(0, len(at), size=70000)].astype(np.int32)
+    try:
+        for i in range(3):
+            if i:
+                w = np.roll(w, 17)
+                dw.copy_(pad(w))
+                torch.cuda.synchronize()
+            og = _oracle.Graph(xadj, adj, w)
+            for p, q in ((0.25, 4.0), (2.0, 0.5)):
+                par = gpu.default_params(app=gpu.APP_NODE2VEC, max_depth=21, p=p, q=q, seed=70 + i)
+                ref, _, _ = _oracle.walk(og, _oracle.from_walk_params(par), starts)
+                paths, st = g.walk(par, starts)
+                assert st.launches >= 6  # tables and sets, or tables made anew
+                assert (paths == ref).all()
     finally:
         g.destroy()
