@@ -327,6 +327,7 @@ extern "C" int fw_graph_destroy(fw_graph* g) {
   release_park_cache(g);
   release_batch_cache(g);
   g->tables.reset();
+  g->label_tables.reset();
   if (g->call_result) (void)hipHostFree(g->call_result);
   for (hipEvent_t e : g->call_ev) if (e) (void)hipEventDestroy(e);
   void* index_ptrs[4] = {g->hub_index, g->hub_info, g->call_scratch, g->adj_hub};
@@ -1660,10 +1661,11 @@ static int plan_tables(const fw_graph* g, fw_tables* t, uint32_t** d_base_out, h
     if ((rc = alloc(reinterpret_cast<void**>(&d_blocks), nv * 4u)) || (rc = alloc(reinterpret_cast<void**>(&d_ctrs), 64)) ||
         (rc = alloc(&tmp, tmp_bytes)) || (rc = alloc(reinterpret_cast<void**>(&t->longs), long_cap * 4u)) ||
         (rc = alloc(reinterpret_cast<void**>(&t->items), item_cap * sizeof(uint2))) ||
-        (rc = alloc(reinterpret_cast<void**>(&t->flag), 64)) || (rc = alloc(reinterpret_cast<void**>(&t->vrec), (size_t)g->V * sizeof(uint4))))
+        (rc = alloc(reinterpret_cast<void**>(&t->flag), 64)) || (rc = alloc(reinterpret_cast<void**>(&t->vrec), (size_t)g->V * sizeof(uint4) * (t->labels.n != 0 ? 2u : 1u))) ||
+        (t->labels.n != 0 && (rc = alloc(reinterpret_cast<void**>(&t->by_label), (size_t)g->E * 4u))))
       return rc;
     FW_HIP(hipMemsetAsync(d_ctrs, 0, 64, stream));
-    if ((rc = fw_table_plan(g, t->hub_threshold, t->nw_shift, d_blocks, t->longs, t->items, d_ctrs, stream)) != FW_OK) return rc;
+    if ((rc = fw_table_plan(g, t->hub_threshold, t->nw_shift, t->labels.n, d_blocks, t->longs, t->items, d_ctrs, stream)) != FW_OK) return rc;
     FW_HIP(rocprim::exclusive_scan(tmp, tmp_bytes, d_blocks, d_blocks, 0u, nv, rocprim::plus<uint32_t>(), stream));
     FW_HIP(hipMemcpyAsync(&h[0], d_ctrs, 8, hipMemcpyDeviceToHost, stream));
     FW_HIP(hipMemcpyAsync(&h[2], d_blocks + g->V, 4, hipMemcpyDeviceToHost, stream));
@@ -1710,13 +1712,103 @@ static bool sets_for_call(const fw_graph* g, const fw_walk_params* p, fw_tables*
   return t->sets != nullptr;  // (without their weights the return edge is searched for)
 }
 
+// MetaPath's tables, for the labels of the call's schema; otherwise as tables_for_call below.  Making them takes
+// 15 ps per edge (16 ms on R-MAT 26, 1.07 G edges).  A walk without them shares its lists through parking, which on R-MAT 26 took 7.1 ms
+// for 10^7 queries of 5 steps, most of which end before: 0.13 ns per step asked for; less where all lists together are short.  The first
+// one that parks makes the parking index as well (10 to 16 ps per edge), so a large first call is better off with the tables: 20 ms
+// on R-MAT 26 against 27.
+constexpr double kParkedStepMs = 0.13e-6;
+constexpr double kParkIndexEdgeMs = 10e-9;
+constexpr double kLabelMakeEdgeMs = 15e-9;
+
+static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipStream_t stream, std::shared_ptr<fw_tables>* out,
+                                 int* launches, hipEvent_t ev_start, hipEvent_t ev0, hipEvent_t ev1) {
+  if (p->park_threshold != 0 || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) || g->host_edges || g->no_label_tables ||
+      (p->wg_threads != 256 && p->wg_threads != 512 && p->wg_threads != 1024))
+    return FW_OK;
+  fw_label_set set;
+  for (int i = 0; i < p->schema_len; ++i) {
+    int at = 0;
+    while (at < set.n && set.label[at] != p->schema[i]) ++at;
+    if (at < set.n) continue;
+    if (set.n == FW_MAX_TABLE_LABELS) return FW_OK;
+    set.label[set.n++] = p->schema[i];
+  }
+  const uint32_t nw_shift = p->wg_threads == 256 ? 2u : (p->wg_threads == 512 ? 3u : 4u);
+  std::shared_ptr<fw_tables> t;
+  {
+    std::lock_guard<std::mutex> guard(g->tables_lock);
+    t = g->label_tables;
+  }
+  if (t && (t->hub_threshold != p->hub_threshold || t->nw_shift != nw_shift || t->labels.n != set.n ||
+            memcmp(t->labels.label, set.label, sizeof(set.label)) != 0))
+    t.reset();
+  if (t && !g->borrowed && p->time_kernels == 0) {
+    *out = t;
+    return FW_OK;
+  }
+  if (!t || g->borrowed) {
+    const double steps = (double)(p->max_depth - 1);
+    double ms = steps * kStepLatencyMs;
+    if (steps * (double)n >= 1.0e6) {
+      double mean = 0.0;
+      const int rc = mean_list_length(g, &mean);
+      if (rc != FW_OK) return rc;
+      const double stream_ms = steps * (double)n * mean * 4.0 / kStreamBytesPerMs, parked_ms = steps * (double)n * kParkedStepMs;
+      const double lists_ms = stream_ms < parked_ms ? stream_ms : parked_ms;
+      if (ms < lists_ms) ms = lists_ms;
+    }
+    const double make_ms = kLabelMakeEdgeMs * (double)g->E + kMakeFixedMs;
+    if (g->hub_index == nullptr && resolve_park_threshold(g, p, n) != INT_MAX) ms += kParkIndexEdgeMs * (double)g->E;
+    if ((g->borrowed ? 0.0 : g->label_ms) + ms < make_ms) return FW_OK;
+  }
+  uint32_t* d_base = nullptr;
+  if (!t) {
+    {
+      std::lock_guard<std::mutex> guard(g->tables_lock);
+      g->label_tables.reset();  // another schema or granularity: one set per graph
+    }
+    t = std::make_shared<fw_tables>();
+    t->hub_threshold = p->hub_threshold;
+    t->nw_shift = nw_shift;
+    t->labels = set;
+    const int rc = plan_tables(g, t.get(), &d_base, stream);
+    if (rc == FW_ERR_NOMEM) {
+      g->no_label_tables = 1;
+      return FW_OK;
+    }
+    if (rc != FW_OK) return rc;
+  }
+  auto make = [&]() -> int {
+    if (ev_start) FW_HIP(hipEventRecord(ev_start, stream));
+    if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev0, stream));
+    const int rc = fw_label_tables_make(g, t.get(), d_base, stream, launches);
+    if (rc != FW_OK) return rc;
+    if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
+    FW_HIP(hipStreamSynchronize(stream));  // (the batch entry walks on other streams; d_base is given back)
+    return FW_OK;
+  };
+  const int rc = make();
+  if (d_base) (void)hipFree(d_base);
+  std::lock_guard<std::mutex> guard(g->tables_lock);
+  if (rc != FW_OK) {
+    g->label_tables.reset();
+    return rc;
+  }
+  g->label_ms = 0.0;  // tables for another schema have to be earned again
+  g->label_tables = t;
+  *out = t;
+  return FW_OK;
+}
+
 // The tables a call over n queries walks on, or none (*out stays empty).  Called with the graph's busy flag held.  ev_start is
 // recorded before the making, ev0 and ev1 around it when its time is asked for; *launches: kernels it took.
 static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipStream_t stream, std::shared_ptr<fw_tables>* out,
                            int* launches, hipEvent_t ev_start, hipEvent_t ev0, hipEvent_t ev1) {
   *launches = 0;
   // an explicit parking degree asks for the parking pipeline, a negative one for walkers that stream their lists
-  if (p->park_threshold != 0 || p->app == FW_APP_METAPATH || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) ||
+  if (p->app == FW_APP_METAPATH) return label_tables_for_call(g, p, n, stream, out, launches, ev_start, ev0, ev1);
+  if (p->park_threshold != 0 || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) ||
       g->host_edges || g->no_tables || (p->wg_threads != 256 && p->wg_threads != 512 && p->wg_threads != 1024) ||
       (p->app == FW_APP_NODE2VEC && p->max_depth > FW_REC_LEN_MASK))
     return FW_OK;
@@ -1804,6 +1896,8 @@ static fw_table_args table_args(const fw_tables& t, unsigned long long* d_counte
   tb.data = t.data;
   tb.sets = t.sets;
   tb.set_weights = t.set_weights;
+  tb.by_label = t.by_label;
+  tb.labels = t.labels;
   tb.nw_shift = t.nw_shift;
   tb.lanes = 0u;
   tb.counters = d_counters;
@@ -1912,7 +2006,7 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
       times.walk_ms = (double)ms - (double)make_ms;  // exact: both are floats
     }
   } else if (p->park_threshold == 0) {
-    mg->streamed_ms += (double)ms;
+    (p->app == FW_APP_METAPATH ? mg->label_ms : mg->streamed_ms) += (double)ms;
   }
   cleanup();
   if (stats) {
@@ -2236,7 +2330,7 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     kernel_ms += make_ms;
   } else {
     FW_TRY(hipMemcpy(h.data(), d_scr, sizeof(Scratch) * (size_t)nbatch, hipMemcpyDeviceToHost));
-    if (p->park_threshold == 0) mg->streamed_ms += kernel_ms;
+    if (p->park_threshold == 0) (p->app == FW_APP_METAPATH ? mg->label_ms : mg->streamed_ms) += kernel_ms;
   }
   if (stats) {
     stats->kernel_ms = kernel_ms;

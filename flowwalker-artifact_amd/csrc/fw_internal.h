@@ -19,6 +19,13 @@ struct fw_hub_info {
 };
 constexpr uint32_t FW_NO_ROWS = 0xFFFFFFFFu;
 
+// The different labels of a MetaPath schema, in the order they first appear in it.
+constexpr int FW_MAX_TABLE_LABELS = 8;
+struct fw_label_set {
+  int32_t n = 0;
+  int32_t label[FW_MAX_TABLE_LABELS] = {};
+};
+
 // List tables (fw_table_walk.hip): the walker-independent part of every sampling step on a graph.  Not changed once made, and
 // held by reference count: a call that walks on them keeps them alive while another call replaces them in the graph.
 struct fw_tables {
@@ -36,8 +43,11 @@ struct fw_tables {
   float* set_weights = nullptr;
   double search_ms = 0.0;         // what node2vec calls without sets spent on searches, estimated
   int no_sets = 0;                // no room for them: do not try again
+  // MetaPath: the lists sorted by label inside every group of the sampler (fw_table_walk.hip); vrec then has two words per vertex
+  fw_label_set labels;
+  int32_t* by_label = nullptr;    // [E]
   ~fw_tables() {
-    void* ptrs[7] = {vrec, data, longs, items, flag, sets, set_weights};
+    void* ptrs[8] = {vrec, data, longs, items, flag, sets, set_weights, by_label};
     for (void* p : ptrs) if (p) (void)hipFree(p);
   }
 };
@@ -78,6 +88,9 @@ struct fw_graph {
   int no_tables = 0;                  // biases or totals the tables cannot hold, or no room for them: do not try again
   std::mutex tables_lock;
   std::shared_ptr<fw_tables> tables;
+  std::shared_ptr<fw_tables> label_tables;  // MetaPath's, for the labels of one schema
+  double label_ms = 0.0;              // device time of the MetaPath calls without them, since they were last made
+  int no_label_tables = 0;            // no room for them: do not try again
   std::atomic<int> busy{0};           // a walk call is running on this graph (the caches above are per graph)
 };
 
@@ -210,6 +223,8 @@ struct fw_table_args {
   const unsigned char* data;
   const int32_t* sets;           // node2vec: NULL: search the lists
   const float* set_weights;
+  const int32_t* by_label;       // MetaPath
+  fw_label_set labels;
   uint32_t nw_shift;
   uint32_t lanes;                // lanes of a wave that walk, and the queries it takes at a time (set by the launch)
   unsigned long long* counters;  // [FW_TABLE_STRIPES * 8]
@@ -284,11 +299,13 @@ int fw_launch_hub_quad(const fw_kargs& a, const fw_hub_args& h, int app, uint32_
 int fw_launch_hub_scan(const fw_kargs& a, const fw_hub_args& h, int app, uint32_t tasks_hint, hipStream_t stream);
 
 // List tables.  plan: region sizes into d_blocks[0 .. V], work lists and their sizes (d_ctrs[0]: long lists, [1]: items);
-// make: fills the tables (d_base: region positions, NULL when vrec has them); sets_make: fills sets and set_weights (if given); walk: every query from start to end, between
+// n_labels: 0, or the number of labels of MetaPath's tables;
+// make, label_tables_make: fill the tables (d_base: region positions, NULL when vrec has them); sets_make: fills sets and set_weights (if given); walk: every query from start to end, between
 // begin (counters and launch records to zero) and end (their sums to pinned host memory).
-int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t nw_shift, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
+int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t nw_shift, int n_labels, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
                   hipStream_t stream);
 int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches);
+int fw_label_tables_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches);
 int fw_sets_make(const fw_graph* g, const fw_tables* t, hipStream_t stream, int* launches);
 int fw_launch_table_walk(const fw_kargs& a, const fw_table_args& tb, int app, int grid, hipStream_t stream, int* grid_used);
 int fw_table_begin(unsigned long long* d_counters, uint32_t* d_scratch, uint32_t words, hipStream_t stream);

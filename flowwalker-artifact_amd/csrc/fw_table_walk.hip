@@ -28,6 +28,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "fw_internal.h"
 #include "fw_step_device.h"
 
@@ -72,14 +74,22 @@ __device__ __forceinline__ uint32_t region_blocks(uint32_t off, uint32_t deg, bo
   return (units + 3u) >> 2;
 }
 
+// blocks of a long list's region in MetaPath's tables: its totals, per label its sums, per group the ends of its labels
+__device__ __forceinline__ uint32_t label_region_blocks(uint32_t off, uint32_t deg, bool wg, uint32_t nw_shift, uint32_t n_labels) {
+  const uint32_t nq = list_quartets(off, deg);
+  if (nq <= kGq) return 0u;
+  const uint32_t ngroups = (nq + kGq - 1u) / kGq;
+  return 1u + n_labels * (header_units(ngroups, wg, nw_shift) >> 2) + ((ngroups + 7u) >> 3);
+}
+
 // ---- making the tables --------------------------------------------------------------------------------
 
 // Region sizes (scanned into positions afterwards) and the work lists of the lists longer than a group: `longs` their
 // vertices, `items` {vertex, group} for every group of them.  ctrs: [0] long lists, [1] items.  Every workgroup counts its
 // range of vertices first, so that it takes its places in the work lists with one update each.
 __global__ __launch_bounds__(1024) void fw_table_plan_kernel(const uint32_t* __restrict__ xadj, int32_t V, int32_t hub_threshold,
-                                                             uint32_t nw_shift, uint32_t* __restrict__ blocks, uint32_t* longs,
-                                                             uint2* items, uint32_t* ctrs) {
+                                                             uint32_t nw_shift, uint32_t n_labels, uint32_t* __restrict__ blocks,
+                                                             uint32_t* longs, uint2* items, uint32_t* ctrs) {
   __shared__ uint32_t s_n[2], s_at[2];
   if (threadIdx.x < 2u) s_n[threadIdx.x] = 0u;
   __syncthreads();
@@ -89,7 +99,8 @@ __global__ __launch_bounds__(1024) void fw_table_plan_kernel(const uint32_t* __r
   uint32_t n_long = 0u, n_items = 0u;
   for (uint32_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) {
     const uint32_t off = xadj[v], deg = xadj[v + 1] - off;
-    blocks[v] = region_blocks(off, deg, (int32_t)deg > hub_threshold, nw_shift);
+    const bool wg = (int32_t)deg > hub_threshold;
+    blocks[v] = n_labels != 0u ? label_region_blocks(off, deg, wg, nw_shift, n_labels) : region_blocks(off, deg, wg, nw_shift);
     const uint32_t nq = list_quartets(off, deg);
     if (nq > kGq) {
       ++n_long;
@@ -333,8 +344,49 @@ __global__ __launch_bounds__(256) void fw_table_groups_kernel(const uint4* __res
   if (__ballot(bad) != 0ull && lane == 0) *flag = 1u;
 }
 
-// The running sums of the long lists, one wave per list: at wave granularity one sequence (64 totals at a time, added up
-// in order), at workgroup granularity one sequence per lane and the scan of their totals.
+// The running sums of a list, from its groups' totals: at wave granularity one sequence (64 totals at a time, added up
+// in order), at workgroup granularity one sequence per lane and the scan of their totals.  Returns the list's total.
+__device__ __forceinline__ float list_sums(float* region, uint32_t ngroups, bool wg, uint32_t nw_shift, int lane) {
+  const uint32_t nb = seq_blocks(ngroups, wg, nw_shift);
+  float total;
+  if (wg) {
+    const uint32_t nw = 1u << nw_shift;
+    float S = 0.0f;
+    if ((uint32_t)lane < nw) {
+      float* const sums = region + 32u + 32u * nb * (uint32_t)lane;
+      const uint32_t L = (ngroups >> nw_shift) + ((uint32_t)lane < (ngroups & (nw - 1u)) ? 1u : 0u);
+      for (uint32_t k = 0; k < 16u * nb; ++k) {
+        float* const at = sums + 32u * (k >> 4) + (k & 15u);
+        if (k < L) S = S + at[16];
+        at[0] = S;
+      }
+    }
+    const float J = row_scan(S);
+    total = readlane_f(J, (int)nw - 1);
+    const uint64_t mpos = __ballot(S > 0.0f);
+    const uint32_t lastpos = 63u - (uint32_t)__builtin_clzll(mpos | 1ull);
+    const float key = wave_prefix_max(S > 0.0f ? J : 0.0f);
+    if (lane < 16) region[lane] = (uint32_t)lane >= lastpos ? kInf : key;
+  } else {
+    float S = 0.0f;
+    for (uint32_t g0 = 0; g0 < 16u * nb; g0 += 64u) {
+      const uint32_t g = g0 + (uint32_t)lane;
+      float* const at = region + 32u * (g >> 4) + (g & 15u);
+      const float T = g < ngroups ? at[16] : 0.0f;
+      float mine = 0.0f;
+#pragma unroll 8
+      for (int l = 0; l < 64; ++l) {
+        S = S + readlane_f(T, l);  // + 0 past the end changes nothing
+        mine = lane == l ? S : mine;
+      }
+      if (g < 16u * nb) at[0] = mine;
+    }
+    total = S;
+  }
+  return total;
+}
+
+// The long lists, one wave per list.
 __global__ __launch_bounds__(256) void fw_table_sums_kernel(uint4* __restrict__ vrec, const uint32_t* __restrict__ longs, uint32_t n_longs,
                                                             int32_t hub_threshold, uint32_t nw_shift, unsigned char* data, uint32_t* flag) {
   const int lane = lane_id();
@@ -346,42 +398,7 @@ __global__ __launch_bounds__(256) void fw_table_sums_kernel(uint4* __restrict__ 
     const uint32_t ngroups = (list_quartets(rec.w, rec.y) + kGq - 1u) / kGq;
     float* const region = reinterpret_cast<float*>(data + (uint64_t)rec.x * 128u);
     const bool wg = (int32_t)rec.y > hub_threshold;
-    const uint32_t nb = seq_blocks(ngroups, wg, nw_shift);
-    float total;
-    if (wg) {
-      const uint32_t nw = 1u << nw_shift;
-      float S = 0.0f;
-      if ((uint32_t)lane < nw) {
-        float* const sums = region + 32u + 32u * nb * (uint32_t)lane;
-        const uint32_t L = (ngroups >> nw_shift) + ((uint32_t)lane < (ngroups & (nw - 1u)) ? 1u : 0u);
-        for (uint32_t k = 0; k < 16u * nb; ++k) {
-          float* const at = sums + 32u * (k >> 4) + (k & 15u);
-          if (k < L) S = S + at[16];
-          at[0] = S;
-        }
-      }
-      const float J = row_scan(S);
-      total = readlane_f(J, (int)nw - 1);
-      const uint64_t mpos = __ballot(S > 0.0f);
-      const uint32_t lastpos = 63u - (uint32_t)__builtin_clzll(mpos | 1ull);
-      const float key = wave_prefix_max(S > 0.0f ? J : 0.0f);
-      if (lane < 16) region[lane] = (uint32_t)lane >= lastpos ? kInf : key;
-    } else {
-      float S = 0.0f;
-      for (uint32_t g0 = 0; g0 < 16u * nb; g0 += 64u) {
-        const uint32_t g = g0 + (uint32_t)lane;
-        float* const at = region + 32u * (g >> 4) + (g & 15u);
-        const float T = g < ngroups ? at[16] : 0.0f;
-        float mine = 0.0f;
-#pragma unroll 8
-        for (int l = 0; l < 64; ++l) {
-          S = S + readlane_f(T, l);  // + 0 past the end changes nothing
-          mine = lane == l ? S : mine;
-        }
-        if (g < 16u * nb) at[0] = mine;
-      }
-      total = S;
-    }
+    const float total = list_sums(region, ngroups, wg, nw_shift, lane);
     bad = bad || !(total < kInf);
     if (lane == 0) vrec[v].z = __float_as_uint(total);
   }
@@ -515,6 +532,222 @@ __device__ __forceinline__ int64_t set_find(const int32_t* __restrict__ sets, ui
   return x[3].w == kSetOverflow ? -2 : -1;
 }
 
+// ---- MetaPath: lists by label -----------------------------------------------------------------------------
+//
+// A bias is 1 where the edge has the step's label and 0 elsewhere, so every sum the sampler makes is a count, exact in
+// whichever order it is added up, and "the first element whose running sum is above t" is the element of rank floor(t)
+// among those of the label (the last one if t reaches the count).  So the neighbours of a group are stored sorted by label, in the order
+// the sampler's lanes hold them, at the group's own places of the edge array (4 bytes written per edge), and a step reads
+// its vertex's record and one neighbour: 10^7 walks of 5 steps on R-MAT 26 take 2.01 ms, 6.85 through parking.  vrec[2v] = {region, degree, 0, CSR offset}, vrec[2v + 1] = where each label's
+// neighbours end in a list of one group (8 x 16 bits).  A longer list has a region, in blocks of 128 bytes: the labels' totals (floats), per
+// label the sums of its groups as above, per group the ends of its labels.
+
+// The ends of up to 8 labels in a group of at most 1024 elements, two in a word.
+struct LabelCounts {
+  uint32_t w[FW_MAX_TABLE_LABELS / 2];
+};
+
+constexpr int kLabelWords = FW_MAX_TABLE_LABELS / 2;
+
+template <int kW = kLabelWords>
+__device__ __forceinline__ uint32_t label_field(const LabelCounts& c, uint32_t s) {
+  uint32_t x = c.w[0];
+#pragma unroll
+  for (uint32_t i = 1; i < (uint32_t)kW; ++i) x = (s >> 1) == i ? c.w[i] : x;
+  return (s & 1u) ? x >> 16 : x & 0xFFFFu;
+}
+
+template <int kW>
+__device__ __forceinline__ void label_count(LabelCounts& c, uint32_t s) {
+  const uint32_t add = 1u << ((s & 1u) * 16u);
+#pragma unroll
+  for (uint32_t i = 0; i < (uint32_t)kW; ++i) c.w[i] += (s >> 1) == i ? add : 0u;
+}
+
+// The value of the lane the DPP control names, 0 where there is none or the row is not in the mask.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ uint32_t dpp_or_0(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, kRows, 0xF, false);
+}
+
+// One group per segment of kSeg lanes (a quad, a DPP row or the wave), lane c holding the quartets c + 64 j as in load_lane: its neighbours by label into
+// by_label.  Returns the ends of the labels in every lane; totals: their counts.
+template <int kSeg, int kJ, int kW>
+__device__ __forceinline__ LabelCounts label_group(const int32_t* __restrict__ label, const int32_t* __restrict__ adjncy,
+                                                   const fw_label_set& set, uint32_t off, uint32_t deg, uint32_t kb, uint32_t nqg,
+                                                   int lane, int32_t* by_label, LabelCounts& totals) {
+  const uint32_t c = (uint32_t)lane & (uint32_t)(kSeg - 1);
+  const uint32_t a0 = off & ~3u;
+  uint64_t slots = 0u;  // four bits each
+  int32_t nb[4 * kJ];
+  LabelCounts mine = {}, at;
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) {
+    const uint32_t k = c + 64u * (uint32_t)j;
+    int4 l = make_int4(0, 0, 0, 0), n = make_int4(-1, -1, -1, -1);
+    const uint32_t base = a0 + 4u * (kb + k);
+    if (k < nqg) {
+      l = *reinterpret_cast<const int4*>(label + base);
+      n = *reinterpret_cast<const int4*>(adjncy + base);
+    }
+    const uint32_t lim = k < nqg ? deg : 0u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int32_t x = i == 0 ? l.x : i == 1 ? l.y : i == 2 ? l.z : l.w;
+      nb[4 * j + i] = i == 0 ? n.x : i == 1 ? n.y : i == 2 ? n.z : n.w;
+      uint32_t s = FW_MAX_TABLE_LABELS;  // none of the schema's, or not in the list (an index before it wraps)
+#pragma unroll
+      for (int m = 2 * kW - 1; m >= 0; --m) s = m < set.n && x == set.label[m] ? (uint32_t)m : s;
+      s = base + (uint32_t)i - off < lim ? s : (uint32_t)FW_MAX_TABLE_LABELS;
+      slots |= (uint64_t)s << (4 * (4 * j + i));
+      label_count<kW>(mine, s);  // (the slot of no label is in no word)
+    }
+  }
+  uint32_t before = 0u;
+  LabelCounts ends = {};
+  totals = LabelCounts{};
+#pragma unroll
+  for (int w = 0; w < kW; ++w) {
+    uint32_t x = mine.w[w], t;
+    if (kSeg == 4) {
+      const uint32_t y = dpp_or_0<0x111, 0xF>(x);
+      x += c >= 1u ? y : 0u;
+      const uint32_t z = dpp_or_0<0x112, 0xF>(x);
+      x += c >= 2u ? z : 0u;
+      t = dpp_or_0<0xFF, 0xF>(x);  // of the quad's last lane
+    } else {
+      x += dpp_or_0<0x111, 0xF>(x);
+      x += dpp_or_0<0x112, 0xF>(x);
+      x += dpp_or_0<0x114, 0xF>(x);
+      x += dpp_or_0<0x118, 0xF>(x);
+      if (kSeg == 64) x += dpp_or_0<0x142, 0xA>(x);
+      if (kSeg == 64) x += dpp_or_0<0x143, 0xC>(x);
+      t = kSeg == 64 ? (uint32_t)__builtin_amdgcn_readlane((int)x, 63) : (uint32_t)__shfl((int)x, kSeg - 1, kSeg);
+    }
+    totals.w[w] = t;
+    const uint32_t e0 = before + (t & 0xFFFFu), e1 = e0 + (t >> 16);
+    at.w[w] = (before | (e0 << 16)) + (x - mine.w[w]);
+    ends.w[w] = e0 | (e1 << 16);
+    before = e1;
+  }
+  const uint32_t first = kb == 0u ? off : a0 + 4u * kb;
+#pragma unroll
+  for (int i = 0; i < 4 * kJ; ++i) {
+    const uint32_t s = (uint32_t)(slots >> (4 * i)) & 15u;
+    if (s < (uint32_t)FW_MAX_TABLE_LABELS) by_label[first + label_field<kW>(at, s)] = nb[i];
+    label_count<kW>(at, s);
+  }
+  return ends;
+}
+
+__device__ __forceinline__ uint4 label_words(const LabelCounts& c) { return make_uint4(c.w[0], c.w[1], c.w[2], c.w[3]); }
+
+// The lists of the lanes with `mine`, 64 / kSeg at a time.
+template <int kSeg, int kW>
+__device__ __forceinline__ void label_segments(const int32_t* __restrict__ label, const int32_t* __restrict__ adjncy,
+                                               const fw_label_set& set, uint32_t off, uint32_t deg, bool mine, uint32_t v0, int lane,
+                                               uint4* vrec, int32_t* by_label) {
+  const uint64_t m = __ballot(mine);
+  const int n = __builtin_popcountll(m);
+  const uint64_t below = (1ull << lane) - 1ull;
+  // lane i: the i-th lane with a list (the others' numbers go behind them)
+  const int at = mine ? __builtin_popcountll(m & below) : n + __builtin_popcountll(~m & below);
+  const int order = __builtin_amdgcn_ds_permute(at << 2, lane);
+  for (int i0 = 0; i0 < n; i0 += 64 / kSeg) {
+    const int i = i0 + lane / kSeg;  // below 64: n is at most 64 and i0 a multiple of 64 / kSeg
+    const int src = __shfl(order, i);
+    const uint32_t o = __shfl(off, src), df = __shfl(deg, src);  // every lane takes part
+    const uint32_t d = i < n ? df : 0u;
+    LabelCounts totals;
+    const LabelCounts e = label_group<kSeg, 1, kW>(label, adjncy, set, o, d, 0u, d != 0u ? list_quartets(o, d) : 0u, lane, by_label, totals);
+    if (i < n && (lane & (kSeg - 1)) == 0) vrec[2u * (uint64_t)(v0 + (uint32_t)src) + 1u] = label_words(e);
+  }
+}
+
+// Lists of one group: a wave takes 64 consecutive vertices; lists of at most 4 (16) quartets sixteen (four) at a time, the others one
+// after the other.  kW: words of the labels' counts (two labels each).
+// Bound: instructions (12 bytes of traffic per edge and 32 per vertex would take 3 ms on R-MAT 26, 1.07 G edges, 67 M vertices;
+// measured 13.6 ms, 27.6 with sixteen lanes for the shortest lists, scans through LDS and 148 registers).
+template <int kW>
+__global__ __launch_bounds__(256, 7) void fw_label_lists_kernel(const uint32_t* __restrict__ xadj, const int32_t* __restrict__ adjncy,
+                                                             const int32_t* __restrict__ label, int32_t V, const fw_label_set set,
+                                                             const uint32_t* base, uint4* vrec, int32_t* by_label) {
+  const int lane = lane_id();
+  const uint64_t chunks = ((uint64_t)(uint32_t)V + 63u) >> 6;
+  for (uint64_t ch = (uint64_t)blockIdx.x * 4u + (uint64_t)(threadIdx.x >> 6); ch < chunks; ch += (uint64_t)gridDim.x * 4u) {
+    const uint32_t v0 = (uint32_t)(ch * 64u), v = v0 + (uint32_t)lane;
+    uint32_t off = 0u, deg = 0u;
+    if (v < (uint32_t)V) {
+      off = xadj[v];
+      deg = xadj[v + 1] - off;
+      const uint32_t reg = base != nullptr ? base[v] : vrec[2u * (uint64_t)v].x;
+      vrec[2u * (uint64_t)v] = make_uint4(reg, deg, 0u, off);
+    }
+    const uint32_t nq = deg != 0u ? list_quartets(off, deg) : 0u;
+    if (v < (uint32_t)V && (nq == 0u || nq > kGq)) vrec[2u * (uint64_t)v + 1u] = make_uint4(0u, 0u, 0u, 0u);
+    LabelCounts totals;
+    label_segments<4, kW>(label, adjncy, set, off, deg, nq != 0u && nq <= 4u, v0, lane, vrec, by_label);
+    label_segments<16, kW>(label, adjncy, set, off, deg, nq > 4u && nq <= 16u, v0, lane, vrec, by_label);
+    uint64_t m;
+    for (m = __ballot(nq > 16u && nq <= kGq); m != 0ull; m &= m - 1ull) {
+      const int l = __builtin_ctzll(m);
+      const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)off, l), d = (uint32_t)__builtin_amdgcn_readlane((int)deg, l);
+      const uint32_t n = list_quartets(o, d);
+      const LabelCounts e = n <= 64u ? label_group<64, 1, kW>(label, adjncy, set, o, d, 0u, n, lane, by_label, totals)
+                                     : label_group<64, kGroupQuartets, kW>(label, adjncy, set, o, d, 0u, n, lane, by_label, totals);
+      if (lane == 0) vrec[2u * (uint64_t)(v0 + (uint32_t)l) + 1u] = label_words(e);
+    }
+  }
+}
+
+// The groups of the long lists, one wave per group: their neighbours by label, ends and totals (1.8 ms on R-MAT 26).
+template <int kW>
+__global__ __launch_bounds__(256, 7) void fw_label_groups_kernel(const uint4* __restrict__ vrec, const int32_t* __restrict__ adjncy,
+                                                              const int32_t* __restrict__ label, const uint2* __restrict__ items,
+                                                              uint32_t n_items, const fw_label_set set, int32_t hub_threshold,
+                                                              uint32_t nw_shift, unsigned char* data, int32_t* by_label) {
+  const int lane = lane_id();
+  for (uint32_t it = blockIdx.x * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); it < n_items;
+       it += gridDim.x * 4u) {
+    const uint2 item = items[it];
+    const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int)item.x), g = (uint32_t)__builtin_amdgcn_readfirstlane((int)item.y);
+    const uint4 rec = vrec[2u * (uint64_t)v];
+    const uint32_t off = (uint32_t)__builtin_amdgcn_readfirstlane((int)rec.w), deg = (uint32_t)__builtin_amdgcn_readfirstlane((int)rec.y);
+    unsigned char* const region = data + (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)rec.x) * 128u;
+    const uint32_t nq = list_quartets(off, deg);
+    const uint32_t ngroups = (nq + kGq - 1u) / kGq;
+    const bool wg = (int32_t)deg > hub_threshold;
+    const uint32_t left = nq - g * kGq;
+    LabelCounts totals;
+    const LabelCounts e = label_group<64, kGroupQuartets, kW>(label, adjncy, set, off, deg, g * kGq, left < kGq ? left : kGq, lane, by_label, totals);
+    const uint32_t k = wg ? g >> nw_shift : g;
+    const uint32_t block = wg ? 1u + (g & ((1u << nw_shift) - 1u)) * seq_blocks(ngroups, wg, nw_shift) + (k >> 4) : k >> 4;
+    const uint32_t hb = header_units(ngroups, wg, nw_shift) >> 2;  // blocks of one label's sums
+    if (lane < set.n)
+      reinterpret_cast<float*>(region)[32u * (1u + (uint32_t)lane * hb + block) + 16u + (k & 15u)] = (float)label_field(totals, (uint32_t)lane);
+    if (lane == 0) reinterpret_cast<uint4*>(region + (uint64_t)128u * (1u + (uint32_t)set.n * hb))[g] = label_words(e);
+  }
+}
+
+// The running sums of the long lists, one wave per list and label.
+__global__ __launch_bounds__(256) void fw_label_sums_kernel(const uint4* __restrict__ vrec, const uint32_t* __restrict__ longs, uint32_t n_longs,
+                                                            const uint32_t n_labels, int32_t hub_threshold, uint32_t nw_shift,
+                                                            unsigned char* data) {
+  const int lane = lane_id();
+  const uint64_t n = (uint64_t)n_longs * n_labels;
+  for (uint64_t it = (uint64_t)blockIdx.x * 4u + (uint64_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); it < n;
+       it += (uint64_t)gridDim.x * 4u) {
+    const uint32_t s = (uint32_t)(it % n_labels);
+    const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int)longs[it / n_labels]);
+    const uint4 rec = vrec[2u * (uint64_t)v];
+    const uint32_t ngroups = (list_quartets(rec.w, rec.y) + kGq - 1u) / kGq;
+    const bool wg = (int32_t)rec.y > hub_threshold;
+    float* const region = reinterpret_cast<float*>(data + (uint64_t)rec.x * 128u);
+    const float total = list_sums(region + 32u * (1u + s * (header_units(ngroups, wg, nw_shift) >> 2)), ngroups, wg, nw_shift, lane);
+    if (lane == 0) region[s] = total;
+  }
+}
+
 // ---- the walk -----------------------------------------------------------------------------------------
 
 // First entry above t of the n entries of a row (they never decrease, the last one is above t; rows are padded to 8
@@ -641,6 +874,56 @@ __device__ __forceinline__ const float* sums_reservoir(const fw_kargs& a, const 
   return sums + 32u * (k >> 4) + 16u + (k & 15u);
 }
 
+// The sequence of groups a step at workgroup granularity goes to, by the scan of the sequences' totals.
+__device__ __forceinline__ uint32_t which_sequence(const fw_kargs& a, const float* scan, const float total, const uint32_t walker,
+                                                   const uint32_t step, const uint32_t sbase) {
+  const float target = u24(philox4x32_10(walker, step, kStreamWave | sbase, 0u, a.seed_lo, a.seed_hi).x) * total;
+  float keys[16];
+  load16(scan, keys);
+  uint32_t seq = 0u;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) seq += keys[i] <= target ? 1u : 0u;
+  return seq;
+}
+
+// MetaPath's step: the selected neighbour, or -1 when no edge has the label.  ends: vrec[2v + 1].
+__device__ __forceinline__ int32_t label_pick(const fw_kargs& a, const fw_table_args& tb, const uint4 rec, uint4 ends, const uint32_t s,
+                                              const uint4 d, const uint32_t walker, const uint32_t step) {
+  const uint32_t nq = list_quartets(rec.w, rec.y);
+  float tu = u24(d.x);
+  uint32_t first = rec.w;
+  if (nq > kGq) {
+    const unsigned char* region = tb.data + (uint64_t)rec.x * 128u;
+    const float total = reinterpret_cast<const float*>(region)[s];
+    if (!(total > 0.0f)) return -1;
+    const uint32_t ngroups = (nq + kGq - 1u) / kGq;
+    const bool wg = (int32_t)rec.y > a.hub_threshold;
+    const uint32_t nb = seq_blocks(ngroups, wg, tb.nw_shift);
+    const uint32_t hb = header_units(ngroups, wg, tb.nw_shift) >> 2;
+    const float* sums = reinterpret_cast<const float*>(region) + 32u * (1u + s * hb);
+    uint32_t seq = 0u;
+    LaneDraw dq;
+    dq.q0 = d.x; dq.q1 = d.y; dq.q2 = d.z; dq.q3 = d.w;
+    dq.avail = 4u;
+    dq.blk = 1u;
+    if (wg) {
+      seq = which_sequence(a, sums, total, walker, step, 0u);
+      sums += 32u + 32u * nb * seq;
+      dq = LaneDraw();
+    }
+    uint32_t k;
+    (void)sums_reservoir(a, sums, nb, dq, walker, step, seq, k, tu);
+    const uint32_t g = wg ? seq + (k << tb.nw_shift) : k;
+    if (g != 0u) first = (rec.w & ~3u) + 4u * kGq * g;
+    ends = reinterpret_cast<const uint4*>(region + (uint64_t)128u * (1u + (uint32_t)tb.labels.n * hb))[g];
+  }
+  const LabelCounts e = {{ends.x, ends.y, ends.z, ends.w}};
+  const uint32_t start = s != 0u ? label_field(e, s - 1u) : 0u, n = label_field(e, s) - start;
+  if (n == 0u) return -1;
+  const uint32_t r = (uint32_t)(tu * (float)n);
+  return tb.by_label[first + start + (r < n ? r : n - 1u)];
+}
+
 // One proposal of the step's sampler for a list with a positive total: the selected neighbour.  d: block 0 of the step's stream 0.
 __device__ __forceinline__ int32_t table_pick(const fw_kargs& a, const fw_table_args& tb, const uint4 rec, const uint4 d,
                                               const uint32_t walker, const uint32_t step, const uint32_t sbase) {
@@ -659,11 +942,7 @@ __device__ __forceinline__ int32_t table_pick(const fw_kargs& a, const fw_table_
     uint32_t seq = 0u;
     LaneDraw dq;
     if (wg) {  // which sequence, then the reservoir over it with draws of its own stream
-      const float target = u24(philox4x32_10(walker, step, kStreamWave | sbase, 0u, a.seed_lo, a.seed_hi).x) * total;
-      float keys[16];
-      load16(sums, keys);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) seq += keys[i] <= target ? 1u : 0u;
+      seq = which_sequence(a, sums, total, walker, step, sbase);
       sums += 32u + 32u * nb * seq;
     } else {
       dq.q0 = d.x; dq.q1 = d.y; dq.q2 = d.z; dq.q3 = d.w;
@@ -697,7 +976,13 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
   __shared__ unsigned long long s_acc[4];
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  __shared__ uint8_t s_slot[kApp == FW_APP_METAPATH ? FW_MAX_SCHEMA : 1];  // of every label of the schema, in the tables
   if (threadIdx.x < 4u) s_acc[threadIdx.x] = 0ull;
+  if (kApp == FW_APP_METAPATH && threadIdx.x < (uint32_t)a.schema_len) {
+    int slot = 0;
+    while (slot + 1 < tb.labels.n && tb.labels.label[slot] != a.schema[threadIdx.x]) ++slot;
+    s_slot[threadIdx.x] = (uint8_t)slot;
+  }
   __syncthreads();
   int32_t* const buf = s_buf[wave];
   const uint32_t my_buf = (uint32_t)lane * 16u;
@@ -765,13 +1050,29 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
     const uint32_t walker = a.walker_base + q;
     const uint32_t step = len - 1u;
     const uint32_t sbase = kApp == FW_APP_NODE2VEC ? trial << 8 : 0u;
-    if (active && !ended && fresh) rec = tb.vrec[v];
+    uint4 ends = make_uint4(0u, 0u, 0u, 0u);
+    if (active && !ended && fresh) {
+      if (kApp == FW_APP_METAPATH) {
+        rec = tb.vrec[2u * (uint64_t)(uint32_t)v];
+        ends = tb.vrec[2u * (uint64_t)(uint32_t)v + 1u];
+      } else {
+        rec = tb.vrec[v];
+      }
+    }
     const uint4 d = philox4x32_10(walker, step, sbase, 0u, a.seed_lo, a.seed_hi);
     if (active && !ended) {
-      if (!(__uint_as_float(rec.z) > 0.0f)) {
-        ended = true;  // no neighbour with a positive bias (include/walker.cuh:1373-1374)
+      int32_t nv = -1;
+      bool none;  // no neighbour with a positive bias (include/walker.cuh:1373-1374)
+      if (kApp == FW_APP_METAPATH) {
+        nv = label_pick(a, tb, rec, ends, s_slot[step % (uint32_t)a.schema_len], d, walker, step);
+        none = nv < 0;
       } else {
-        int32_t nv = table_pick(a, tb, rec, d, walker, step, sbase);
+        none = !(__uint_as_float(rec.z) > 0.0f);
+      }
+      if (none) {
+        ended = true;
+      } else {
+        if (kApp != FW_APP_METAPATH) nv = table_pick(a, tb, rec, d, walker, step, sbase);
         bool moved = true;
         if (kApp == FW_APP_NODE2VEC && prev >= 0) {
           if (a.n2v_extra > 0.0f && fresh) {
@@ -929,6 +1230,7 @@ int fw_launch_table_walk(const fw_kargs& a, const fw_table_args& tb, int app, in
     case FW_APP_DEEPWALK: return launch_table_walk<FW_APP_DEEPWALK>(a, tb, grid, stream, grid_used);
     case FW_APP_PPR: return launch_table_walk<FW_APP_PPR>(a, tb, grid, stream, grid_used);
     case FW_APP_NODE2VEC: return launch_table_walk<FW_APP_NODE2VEC>(a, tb, grid, stream, grid_used);
+    case FW_APP_METAPATH: return launch_table_walk<FW_APP_METAPATH>(a, tb, grid, stream, grid_used);
     default:
       fw_set_error("no list tables for app %d", app);
       return FW_ERR_INVALID;
@@ -948,9 +1250,9 @@ int fw_table_end(const unsigned long long* d_counters, unsigned long long* h_out
   return FW_OK;
 }
 
-int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t nw_shift, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
+int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t nw_shift, int n_labels, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
                   hipStream_t stream) {
-  hipLaunchKernelGGL(fw_table_plan_kernel, dim3(1024), dim3(1024), 0, stream, g->xadj, g->V, hub_threshold, nw_shift, d_blocks,
+  hipLaunchKernelGGL(fw_table_plan_kernel, dim3(1024), dim3(1024), 0, stream, g->xadj, g->V, hub_threshold, nw_shift, (uint32_t)n_labels, d_blocks,
                      d_longs, d_items, d_ctrs);
   FW_HIP(hipGetLastError());
   return FW_OK;
@@ -973,6 +1275,38 @@ int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipSt
     FW_HIP(hipGetLastError());
     hipLaunchKernelGGL(fw_table_sums_kernel, dim3(grid_for(t->n_longs)), dim3(256), 0, stream, t->vrec, t->longs, t->n_longs,
                        t->hub_threshold, t->nw_shift, t->data, t->flag);
+    FW_HIP(hipGetLastError());
+    *launches += 2;
+  }
+  return FW_OK;
+}
+
+int fw_label_tables_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches) {
+  int cus = 0;
+  FW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
+  auto grid_for = [&](uint64_t waves) {
+    const uint64_t blocks = (waves + 3u) / 4u, most = (uint64_t)cus * 64u;
+    return (unsigned)(blocks < most ? (blocks ? blocks : 1u) : most);
+  };
+  auto make = [&](auto words) -> int {
+    constexpr int kW = decltype(words)::value;
+    hipLaunchKernelGGL((fw_label_lists_kernel<kW>), dim3(grid_for(((uint64_t)g->V + 63u) / 64u)), dim3(256), 0, stream, g->xadj,
+                       g->adjncy, g->label, g->V, t->labels, d_base, t->vrec, t->by_label);
+    FW_HIP(hipGetLastError());
+    if (t->n_longs != 0u)
+      hipLaunchKernelGGL((fw_label_groups_kernel<kW>), dim3(grid_for(t->n_items)), dim3(256), 0, stream, t->vrec, g->adjncy,
+                         g->label, t->items, t->n_items, t->labels, t->hub_threshold, t->nw_shift, t->data, t->by_label);
+    FW_HIP(hipGetLastError());
+    return FW_OK;
+  };
+  const int n = t->labels.n;
+  const int rc = n <= 2 ? make(std::integral_constant<int, 1>()) : n <= 4 ? make(std::integral_constant<int, 2>())
+                 : n <= 6 ? make(std::integral_constant<int, 3>()) : make(std::integral_constant<int, 4>());
+  if (rc != FW_OK) return rc;
+  *launches += 1;
+  if (t->n_longs != 0u) {
+    hipLaunchKernelGGL(fw_label_sums_kernel, dim3(grid_for((uint64_t)t->n_longs * (uint64_t)t->labels.n)), dim3(256), 0, stream,
+                       t->vrec, t->longs, t->n_longs, (uint32_t)t->labels.n, t->hub_threshold, t->nw_shift, t->data);
     FW_HIP(hipGetLastError());
     *launches += 2;
   }

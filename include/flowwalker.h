@@ -91,7 +91,8 @@ typedef struct {
                             list (by a workgroup above hub_threshold, by one wave below).  > 0 = degree, < 0 = off (a
                             walker reads its lists itself).  0 = library default: where the walks would read the lists
                             several times over, one scan of every list is shared by all walkers of all calls (list
-                            tables, kept with the graph; DeepWalk, PPR and node2vec on graphs in device memory), else
+                            tables, kept with the graph, for MetaPath per schema of at most 8 different labels;
+                            graphs in device memory), else
                             parking for batches >= 65536 queries.  node2vec: the shared scan proposes, each walker
                             accepts with its own adjacency test (max_depth <= 65535). */
   /* node2vec is sampled in two stages: a neighbour is proposed with probability w / sum w and accepted with

@@ -126,3 +126,38 @@ def test_changed_biases_on_adopted_arrays(gpu):
                 assert (paths == ref).all()
     finally:
         g.destroy()
+
+
+@pytest.mark.parametrize("wg,thr", [(512, 16384), (256, 1024), (1024, 2000), (512, 1 << 30)])
+def test_metapath_on_label_tables(gpu, wg, thr):
+    """One label to as many as the tables hold, labels that no edge has, other values than 0 .. n; one more label than that
+    leaves the tables aside."""
+    (xadj, adj, _), at = _lists("even")
+    rng = np.random.RandomState(wg + 1)
+    values = np.array([7, -3, 0, 1 << 30, 5, 6, -(1 << 31), 11], dtype=np.int64)
+    lab = values[np.minimum((rng.exponential(2.0, size=len(adj))).astype(np.int64), 7)].astype(np.int32)
+    g = gpu.Graph.from_csr(xadj, adj, None, lab)
+    og = _oracle.Graph(xadj, adj, None, lab)
+    try:
+        cases = [([7, -3, 0], 70000, 10), ([7], 4001, 17), ([-3, 7, 7, 5], 70000, 33), ([-3, 7, 7, 5], 1, 81), ([-3, 7, 7, 5], 777, 2),
+                 ([7, -3, 0, 1 << 30, 5, 6, -(1 << 31), 11], 70000, 12), ([99, 7], 70000, 5), ([7, -3, 7, 99, 0], 70000, 9),
+                 (list(values) + [99], 70000, 20)]
+        for i, (schema, n, depth) in enumerate(cases):
+            p = gpu.default_params(app=gpu.APP_METAPATH, max_depth=depth, schema=schema, wg_threads=wg, hub_threshold=thr,
+                                   seed=300 + i, walker_base=i)
+            starts = np.where(rng.random_sample(n) < 0.8, at[rng.randint(0, len(at), size=n)], rng.randint(0, V, size=n)).astype(np.int32)
+            ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(p), starts)
+            launches = set()
+            for _ in range(20):  # the first calls with a schema may walk without tables
+                paths, st = g.walk(p, starts)
+                bad = np.nonzero((paths != ref).any(axis=1))[0]
+                assert len(bad) == 0, (schema, n, bad[0], paths[bad[0]], ref[bad[0]])
+                assert (st.steps, st.sampled_edges) == (steps, edges), (schema, n)
+                launches.add(st.launches)
+                if 6 in launches:
+                    break
+            assert (6 in launches) == (i not in (3, 4, 8)), (i, launches)  # made; there already (twice); too many labels
+            again, st2 = g.walk_batch(p, starts, batch_size=max(1, n // 3))
+            assert (again == ref).all() and (st2.steps, st2.sampled_edges) == (steps, edges), (schema, n)
+    finally:
+        g.destroy()
