@@ -161,3 +161,26 @@ def test_metapath_on_label_tables(gpu, wg, thr):
             assert (again == ref).all() and (st2.steps, st2.sampled_edges) == (steps, edges), (schema, n)
     finally:
         g.destroy()
+
+
+@pytest.mark.parametrize("grid,n,depth", [(1, 4097 + 64, 6), (1, 9001, 16), (2, 20000, 2), (3, 13001, 17)])
+def test_short_rows_of_many_queries(gpu, grid, n, depth):
+    """Rows of at most 16 entries: queries come 256 at a time while 1024 per workgroup are left, 64 at a time after that."""
+    csr, at = _lists("even")
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    rng = np.random.RandomState(n)
+    try:
+        warm = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21)
+        g.walk(warm, at[rng.randint(0, len(at), size=70000)].astype(np.int32))
+        for app in (gpu.APP_DEEPWALK, gpu.APP_PPR):
+            p = gpu.default_params(app=app, max_depth=depth, tp=0.3, seed=n, grid=grid)
+            starts = rng.randint(0, V, size=n).astype(np.int32)
+            ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(p), starts)
+            paths, st = g.walk(p, starts)
+            assert st.launches == 3
+            bad = np.nonzero((paths != ref).any(axis=1))[0]
+            assert len(bad) == 0, (app, bad[0], paths[bad[0]], ref[bad[0]])
+            assert (st.steps, st.sampled_edges) == (steps, edges)
+    finally:
+        g.destroy()
