@@ -50,8 +50,8 @@ CONFIG_OF = {"deepwalk_rmat22": "C2", "ppr_rmat22": "C3", "node2vec_rmat24_sym":
 # which is read at run time; the line says on which sources it was taken, and the JSON says whether those are the
 # sources of this run.
 PROFILE_OF = {
-    "deepwalk_rmat24_sym": "profiles/walk_pipeline_deepwalk_rmat24sym_pmc.txt",
-    "node2vec_rmat24_sym": "profiles/walk_pipeline_node2vec_rmat24sym_pmc.txt",
+    "deepwalk_rmat24_sym": "profiles/table_walk_pmc.txt",
+    "node2vec_rmat24_sym": "profiles/table_walk_pmc.txt",
 }
 
 

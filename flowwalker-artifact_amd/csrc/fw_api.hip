@@ -1579,10 +1579,10 @@ static TrafficModel traffic_model(const fw_walk_params* p, int32_t n, bool parke
 
 // The same for a walk on list tables: a step reads its vertex's record, a row and a lane of the list's table; path entries leave in
 // lines.  made: the tables were made in this call.
-static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params* p, int32_t n, bool made, uint64_t steps) {
+static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params* p, int32_t n, bool made, bool sets, uint64_t steps) {
   TrafficModel m;
   m.scattered_reads = 3 * steps + (uint64_t)n;
-  if (p->app == FW_APP_NODE2VEC) m.scattered_reads += 4 * steps;  // the searches in N(prev)
+  if (p->app == FW_APP_NODE2VEC) m.scattered_reads += (sets ? 1 : 4) * steps;  // the tests in N(prev): a hash set, or searches
   m.scattered_writes = steps / 16u + 2u * (uint64_t)n;            // whole lines, the row's first and last entries
   m.record_bytes = 4 * (uint64_t)n + 4 * (uint64_t)n * (uint64_t)p->max_depth;
   if (made) {
@@ -2020,7 +2020,7 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
     stats->hub_kernel_ms = times.hub_ms;
     stats->hub_steps = h.counters[2];
     stats->hub_sampled_edges = h.counters[3];
-    const TrafficModel tm = tables ? table_traffic_model(g, p, n, launches > 3, stats->steps)
+    const TrafficModel tm = tables ? table_traffic_model(g, p, n, launches > 3, tables->sets != nullptr, stats->steps)
                                    : traffic_model(p, n, launches > 1, park_threshold, g->adj_hub != nullptr, h.counters[0],
                                                    h.counters[1], h.counters[2], times);
     stats->requested_bytes = tm.total();
@@ -2349,7 +2349,7 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     stats->grid = grid_used;
     stats->walk_kernel_ms = stats->hub_steps == 0 && make_launches == 0 ? kernel_ms : times.walk_ms;  // the split: with time_kernels only
     stats->hub_kernel_ms = times.hub_ms;
-    const TrafficModel tm = tables ? table_traffic_model(g, p, n, make_launches != 0, stats->steps)
+    const TrafficModel tm = tables ? table_traffic_model(g, p, n, make_launches != 0, tables->sets != nullptr, stats->steps)
                                    : traffic_model(p, n, times.sorted_records != 0, park_threshold, g->adj_hub != nullptr,
                                                    stats->steps - stats->hub_steps,
                                                    stats->sampled_edges - stats->hub_sampled_edges, stats->hub_steps, times);
