@@ -1640,50 +1640,43 @@ static int mean_list_length(fw_graph* g, double* out) {
   return FW_OK;
 }
 
-// Room for the tables of `g`: positions of the regions, work lists, memory.  FW_ERR_NOMEM when there is no room for them.
-static int plan_tables(const fw_graph* g, fw_tables* t, uint32_t** d_base_out, hipStream_t stream) {
+// Room for the tables of `g`: positions of the regions, work lists, memory (what `t` holds already is used again).  FW_ERR_NOMEM when
+// there is no room for them.
+static int plan_tables(const fw_graph* g, fw_tables* t, hipStream_t stream) {
   const size_t nv = (size_t)g->V + 1u;
   const size_t item_cap = (size_t)(g->E / 500u) + 64u, long_cap = (size_t)(g->E / 1000u) + 64u;  // a list of several groups has over 1020 entries
-  uint32_t* d_blocks = nullptr;
-  uint32_t* d_ctrs = nullptr;
-  void* tmp = nullptr;
   size_t tmp_bytes = 0;
-  auto alloc = [](void** p, size_t bytes) -> int {
-    if (hipMalloc(p, bytes ? bytes : 16) == hipSuccess) return FW_OK;
+  auto room = [](auto** p, size_t bytes) -> int {
+    if (*p != nullptr || hipMalloc(reinterpret_cast<void**>(p), bytes ? bytes : 16) == hipSuccess) return FW_OK;
     (void)hipGetLastError();
     *p = nullptr;
     return FW_ERR_NOMEM;
   };
-  uint32_t h[3] = {0u, 0u, 0u};
-  auto plan = [&]() -> int {
-    int rc;
-    FW_HIP(rocprim::exclusive_scan(nullptr, tmp_bytes, d_blocks, d_blocks, 0u, nv, rocprim::plus<uint32_t>(), stream));
-    if ((rc = alloc(reinterpret_cast<void**>(&d_blocks), nv * 4u)) || (rc = alloc(reinterpret_cast<void**>(&d_ctrs), 64)) ||
-        (rc = alloc(&tmp, tmp_bytes)) || (rc = alloc(reinterpret_cast<void**>(&t->longs), long_cap * 4u)) ||
-        (rc = alloc(reinterpret_cast<void**>(&t->items), item_cap * sizeof(uint2))) ||
-        (rc = alloc(reinterpret_cast<void**>(&t->flag), 64)) || (rc = alloc(reinterpret_cast<void**>(&t->vrec), (size_t)g->V * sizeof(uint4) * (t->labels.n != 0 ? 2u : 1u))) ||
-        (t->labels.n != 0 && (rc = alloc(reinterpret_cast<void**>(&t->by_label), (size_t)g->E * 4u))))
-      return rc;
-    FW_HIP(hipMemsetAsync(d_ctrs, 0, 64, stream));
-    if ((rc = fw_table_plan(g, t->hub_threshold, t->nw_shift, t->labels.n, d_blocks, t->longs, t->items, d_ctrs, stream)) != FW_OK) return rc;
-    FW_HIP(rocprim::exclusive_scan(tmp, tmp_bytes, d_blocks, d_blocks, 0u, nv, rocprim::plus<uint32_t>(), stream));
-    FW_HIP(hipMemcpyAsync(&h[0], d_ctrs, 8, hipMemcpyDeviceToHost, stream));
-    FW_HIP(hipMemcpyAsync(&h[2], d_blocks + g->V, 4, hipMemcpyDeviceToHost, stream));
-    FW_HIP(hipStreamSynchronize(stream));
-    t->n_longs = h[0];
-    t->n_items = h[1];
-    if (h[0] > long_cap || h[1] > item_cap) { fw_set_error("internal: %u long lists, %u groups", h[0], h[1]); return FW_ERR_INVALID; }
-    return alloc(reinterpret_cast<void**>(&t->data), (size_t)h[2] * 128u + 128u);
-  };
-  const int rc = plan();
-  if (d_ctrs) (void)hipFree(d_ctrs);
-  if (tmp) (void)hipFree(tmp);
-  if (rc != FW_OK) {
-    if (d_blocks) (void)hipFree(d_blocks);
+  FW_HIP(rocprim::exclusive_scan(nullptr, tmp_bytes, t->blocks, t->blocks, 0u, nv, rocprim::plus<uint32_t>(), stream));
+  int rc;
+  if ((rc = room(&t->blocks, nv * 4u)) || (rc = room(&t->ctrs, 64)) || (rc = room(&t->scan_tmp, tmp_bytes)) ||
+      (rc = room(&t->longs, long_cap * 4u)) || (rc = room(&t->items, item_cap * sizeof(uint2))) || (rc = room(&t->flag, 64)) ||
+      (rc = room(&t->vrec, (size_t)g->V * sizeof(uint4) * (t->labels.n != 0 ? 2u : 1u))) ||
+      (t->labels.n != 0 && (rc = room(&t->by_label, (size_t)g->E * 4u))))
     return rc;
+  uint32_t h[3] = {0u, 0u, 0u};
+  FW_HIP(hipMemsetAsync(t->ctrs, 0, 64, stream));
+  if ((rc = fw_table_plan(g, t->hub_threshold, t->nw_shift, t->labels.n, t->blocks, t->longs, t->items, t->ctrs, stream)) != FW_OK) return rc;
+  FW_HIP(rocprim::exclusive_scan(t->scan_tmp, tmp_bytes, t->blocks, t->blocks, 0u, nv, rocprim::plus<uint32_t>(), stream));
+  FW_HIP(hipMemcpyAsync(&h[0], t->ctrs, 8, hipMemcpyDeviceToHost, stream));
+  FW_HIP(hipMemcpyAsync(&h[2], t->blocks + g->V, 4, hipMemcpyDeviceToHost, stream));
+  FW_HIP(hipStreamSynchronize(stream));
+  t->n_longs = h[0];
+  t->n_items = h[1];
+  if (h[0] > long_cap || h[1] > item_cap) { fw_set_error("internal: %u long lists, %u groups", h[0], h[1]); return FW_ERR_INVALID; }
+  const size_t bytes = (size_t)h[2] * 128u + 128u;
+  if (t->data_bytes < bytes) {
+    if (t->data) (void)hipFree(t->data);
+    t->data = nullptr;
+    t->data_bytes = 0;
+    if ((rc = room(&t->data, bytes)) != FW_OK) return rc;
+    t->data_bytes = bytes;
   }
-  t->bytes = (size_t)h[2] * 128u + (size_t)g->V * sizeof(uint4);
-  *d_base_out = d_blocks;
   return FW_OK;
 }
 
@@ -1694,10 +1687,11 @@ static int plan_tables(const fw_graph* g, fw_tables* t, uint32_t** d_base_out, h
 static bool sets_for_call(const fw_graph* g, const fw_walk_params* p, fw_tables* t, double all_steps, double steps) {
   const bool back = p->p < 1.0f && p->p < p->q;  // the return edge is a component of its own
   if (p->app != FW_APP_NODE2VEC || (p->q == 1.0f && !back) || t->no_sets) return false;
-  const bool want_weights = back && t->set_weights == nullptr;
-  if (t->sets != nullptr && !want_weights) return p->time_kernels != 0 || (g->borrowed && back);
-  if (t->sets == nullptr) {
-    t->search_ms += all_steps * 0.05e-6 > steps * 0.004 ? all_steps * 0.05e-6 : steps * 0.004;
+  const bool want_weights = back && !t->have_weights;
+  if (t->have_sets && !want_weights) return p->time_kernels != 0;
+  if (!t->have_sets) {
+    const double ms = all_steps * 0.05e-6 > steps * 0.004 ? all_steps * 0.05e-6 : steps * 0.004;
+    t->search_ms = (g->borrowed ? 0.0 : t->search_ms) + ms;  // (an adopted graph's sets last one call)
     if (t->search_ms < kMakeMargin * (20.0 * (double)g->E / 2.5e9 + 0.2)) return false;
   }
   const size_t places = 16u * (size_t)(fw_set_first((uint32_t)g->E, (uint32_t)g->V) + 1u);
@@ -1708,8 +1702,10 @@ static bool sets_for_call(const fw_graph* g, const fw_walk_params* p, fw_tables*
     t->no_sets = 1;
   };
   if (t->sets == nullptr) room(reinterpret_cast<void**>(&t->sets));
-  if (t->sets != nullptr && want_weights) room(reinterpret_cast<void**>(&t->set_weights));
-  return t->sets != nullptr;  // (without their weights the return edge is searched for)
+  if (t->sets != nullptr && t->set_weights == nullptr && want_weights) room(reinterpret_cast<void**>(&t->set_weights));
+  t->have_sets = t->sets != nullptr;
+  t->have_weights = t->have_sets && back && t->set_weights != nullptr;  // (without them the return edge is searched for)
+  return t->have_sets;
 }
 
 // MetaPath's tables, for the labels of the call's schema; otherwise as tables_for_call below.  Making them takes
@@ -1762,17 +1758,18 @@ static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n
     if (g->hub_index == nullptr && resolve_park_threshold(g, p, n) != INT_MAX) ms += kParkIndexEdgeMs * (double)g->E;
     if ((g->borrowed ? 0.0 : g->label_ms) + ms < make_ms) return FW_OK;
   }
-  uint32_t* d_base = nullptr;
-  if (!t) {
-    {
-      std::lock_guard<std::mutex> guard(g->tables_lock);
-      g->label_tables.reset();  // another schema or granularity: one set per graph
+  if (!t || g->borrowed) {
+    if (!t) {
+      {
+        std::lock_guard<std::mutex> guard(g->tables_lock);
+        g->label_tables.reset();  // another schema or granularity: one set per graph
+      }
+      t = std::make_shared<fw_tables>();
+      t->hub_threshold = p->hub_threshold;
+      t->nw_shift = nw_shift;
+      t->labels = set;
     }
-    t = std::make_shared<fw_tables>();
-    t->hub_threshold = p->hub_threshold;
-    t->nw_shift = nw_shift;
-    t->labels = set;
-    const int rc = plan_tables(g, t.get(), &d_base, stream);
+    const int rc = plan_tables(g, t.get(), stream);
     if (rc == FW_ERR_NOMEM) {
       g->no_label_tables = 1;
       return FW_OK;
@@ -1782,14 +1779,13 @@ static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n
   auto make = [&]() -> int {
     if (ev_start) FW_HIP(hipEventRecord(ev_start, stream));
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev0, stream));
-    const int rc = fw_label_tables_make(g, t.get(), d_base, stream, launches);
+    const int rc = fw_label_tables_make(g, t.get(), stream, launches);
     if (rc != FW_OK) return rc;
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
-    FW_HIP(hipStreamSynchronize(stream));  // (the batch entry walks on other streams; d_base is given back)
+    FW_HIP(hipStreamSynchronize(stream));  // (the batch entry walks on other streams)
     return FW_OK;
   };
   const int rc = make();
-  if (d_base) (void)hipFree(d_base);
   std::lock_guard<std::mutex> guard(g->tables_lock);
   if (rc != FW_OK) {
     g->label_tables.reset();
@@ -1808,6 +1804,10 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
   *launches = 0;
   // an explicit parking degree asks for the parking pipeline, a negative one for walkers that stream their lists
   if (p->app == FW_APP_METAPATH) return label_tables_for_call(g, p, n, stream, out, launches, ev_start, ev0, ev1);
+  if (g->skip_tables > 0) {
+    --g->skip_tables;
+    return FW_OK;
+  }
   if (p->park_threshold != 0 || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) ||
       g->host_edges || g->no_tables || (p->wg_threads != 256 && p->wg_threads != 512 && p->wg_threads != 1024) ||
       (p->app == FW_APP_NODE2VEC && p->max_depth > FW_REC_LEN_MASK))
@@ -1831,18 +1831,21 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
       const double stream_ms = steps * (double)n * mean * 4.0 / kStreamBytesPerMs;
       if (ms < stream_ms) ms = stream_ms;
     }
-    if (g->streamed_ms + ms < kMakeMargin * (17.0 * (double)g->E / kMakeBytesPerMs + kMakeFixedMs)) return FW_OK;
+    // (an adopted graph's tables last one call: only its own work can pay for them)
+    if ((g->borrowed ? 0.0 : g->streamed_ms) + ms < kMakeMargin * (17.0 * (double)g->E / kMakeBytesPerMs + kMakeFixedMs)) return FW_OK;
   }
-  uint32_t* d_base = nullptr;
-  if (!t) {
-    {
-      std::lock_guard<std::mutex> guard(g->tables_lock);
-      g->tables.reset();  // another granularity: one set per graph
+  if (!t || g->borrowed) {
+    if (!t) {
+      {
+        std::lock_guard<std::mutex> guard(g->tables_lock);
+        g->tables.reset();  // another granularity: one set per graph
+      }
+      t = std::make_shared<fw_tables>();
+      t->hub_threshold = p->hub_threshold;
+      t->nw_shift = nw_shift;
     }
-    t = std::make_shared<fw_tables>();
-    t->hub_threshold = p->hub_threshold;
-    t->nw_shift = nw_shift;
-    const int rc = plan_tables(g, t.get(), &d_base, stream);
+    t->have_sets = t->have_weights = false;
+    const int rc = plan_tables(g, t.get(), stream);
     if (rc == FW_ERR_NOMEM) {
       g->no_tables = 1;
       return FW_OK;
@@ -1861,7 +1864,7 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     int rc = FW_OK;
     if (make_tables) {
       FW_HIP(hipMemsetAsync(t->flag, 0, sizeof(uint32_t), stream));
-      if ((rc = fw_table_make(g, t.get(), d_base, stream, launches)) != FW_OK) return rc;
+      if ((rc = fw_table_make(g, t.get(), stream, launches)) != FW_OK) return rc;
     }
     if (make_sets && (rc = fw_sets_make(g, t.get(), stream, launches)) != FW_OK) return rc;
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
@@ -1871,14 +1874,17 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     return FW_OK;
   };
   const int rc = make();
-  if (d_base) (void)hipFree(d_base);
   if (rc != FW_OK) {  // nothing half made stays
     std::lock_guard<std::mutex> guard(g->tables_lock);
     g->tables.reset();
     return rc;
   }
   if (bad != 0u) {  // the streaming kernels define what happens then
-    if (!g->borrowed) g->no_tables = 1;
+    if (g->borrowed) {
+      g->skip_tables = 15;  // the owner may mend them: looked at again after a while
+    } else {
+      g->no_tables = 1;
+    }
     *launches = 0;
     return FW_OK;
   }
@@ -1894,8 +1900,8 @@ static fw_table_args table_args(const fw_tables& t, unsigned long long* d_counte
   fw_table_args tb;
   tb.vrec = t.vrec;
   tb.data = t.data;
-  tb.sets = t.sets;
-  tb.set_weights = t.set_weights;
+  tb.sets = t.have_sets ? t.sets : nullptr;
+  tb.set_weights = t.have_weights ? t.set_weights : nullptr;
   tb.by_label = t.by_label;
   tb.labels = t.labels;
   tb.nw_shift = t.nw_shift;
@@ -2020,7 +2026,7 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
     stats->hub_kernel_ms = times.hub_ms;
     stats->hub_steps = h.counters[2];
     stats->hub_sampled_edges = h.counters[3];
-    const TrafficModel tm = tables ? table_traffic_model(g, p, n, launches > 3, tables->sets != nullptr, stats->steps)
+    const TrafficModel tm = tables ? table_traffic_model(g, p, n, launches > 3, tables->have_sets, stats->steps)
                                    : traffic_model(p, n, launches > 1, park_threshold, g->adj_hub != nullptr, h.counters[0],
                                                    h.counters[1], h.counters[2], times);
     stats->requested_bytes = tm.total();
@@ -2349,7 +2355,7 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     stats->grid = grid_used;
     stats->walk_kernel_ms = stats->hub_steps == 0 && make_launches == 0 ? kernel_ms : times.walk_ms;  // the split: with time_kernels only
     stats->hub_kernel_ms = times.hub_ms;
-    const TrafficModel tm = tables ? table_traffic_model(g, p, n, make_launches != 0, tables->sets != nullptr, stats->steps)
+    const TrafficModel tm = tables ? table_traffic_model(g, p, n, make_launches != 0, tables->have_sets, stats->steps)
                                    : traffic_model(p, n, times.sorted_records != 0, park_threshold, g->adj_hub != nullptr,
                                                    stats->steps - stats->hub_steps,
                                                    stats->sampled_edges - stats->hub_sampled_edges, stats->hub_steps, times);

@@ -31,23 +31,27 @@ struct fw_label_set {
 struct fw_tables {
   uint4* vrec = nullptr;          // [V] {region in 128-byte blocks, degree, total, CSR offset}
   unsigned char* data = nullptr;  // the regions
+  size_t data_bytes = 0;          // room for them
   uint32_t* longs = nullptr;      // vertices whose lists have more than one group
   uint2* items = nullptr;         // {vertex, group} for every group of those
   uint32_t* flag = nullptr;       // set by the make kernels when a bias or a total is not a finite, non-negative number
   uint32_t n_longs = 0, n_items = 0;
   int32_t hub_threshold = 0;      // which long lists are cut into sequences, and how many of them (as a power of two):
   uint32_t nw_shift = 0;          // part of the sampler's definition
-  size_t bytes = 0;
+  uint32_t* blocks = nullptr;     // [V + 1] region sizes, then their positions
+  uint32_t* ctrs = nullptr;
+  void* scan_tmp = nullptr;
   // node2vec: the lists as hash sets (and the weights of their entries), made when its calls' work pays for them
   int32_t* sets = nullptr;
   float* set_weights = nullptr;
+  bool have_sets = false, have_weights = false;  // whether they hold the lists
   double search_ms = 0.0;         // what node2vec calls without sets spent on searches, estimated
   int no_sets = 0;                // no room for them: do not try again
   // MetaPath: the lists sorted by label inside every group of the sampler (fw_table_walk.hip); vrec then has two words per vertex
   fw_label_set labels;
   int32_t* by_label = nullptr;    // [E]
   ~fw_tables() {
-    void* ptrs[8] = {vrec, data, longs, items, flag, sets, set_weights, by_label};
+    void* ptrs[] = {vrec, data, longs, items, flag, blocks, ctrs, scan_tmp, sets, set_weights, by_label};
     for (void* p : ptrs) if (p) (void)hipFree(p);
   }
 };
@@ -81,8 +85,9 @@ struct fw_graph {
   void* call_scratch = nullptr;       // launch record (dispenser word + counters) of fw_walk_device, allocated once
   unsigned long long* call_result = nullptr;  // pinned: the sums of a table walk's counters
   hipEvent_t call_ev[4] = {};         // and its timing events: the call, the making of the list tables
-  int borrowed = 0;                   // the arrays came through fw_graph_adopt_device: their owner may change the biases
-                                      // between calls, so list tables are made anew in every call that walks on them
+  int borrowed = 0;                   // the arrays came through fw_graph_adopt_device: their owner may change them between
+                                      // calls, so list tables are planned and made anew in every call that walks on them
+  int skip_tables = 0;                // calls to come that do not try for tables: an adopted graph had biases they cannot hold
   double mean_list = -1.0;            // sum of squared degrees / E: the list length a step meets, on average; lazily computed
   double streamed_ms = 0.0;           // device time of the walk calls that had no list tables and might have had them
   int no_tables = 0;                  // biases or totals the tables cannot hold, or no room for them: do not try again
@@ -300,12 +305,12 @@ int fw_launch_hub_scan(const fw_kargs& a, const fw_hub_args& h, int app, uint32_
 
 // List tables.  plan: region sizes into d_blocks[0 .. V], work lists and their sizes (d_ctrs[0]: long lists, [1]: items);
 // n_labels: 0, or the number of labels of MetaPath's tables;
-// make, label_tables_make: fill the tables (d_base: region positions, NULL when vrec has them); sets_make: fills sets and set_weights (if given); walk: every query from start to end, between
+// make, label_tables_make: fill the tables (region positions: t->blocks); sets_make: fills sets and set_weights (if given); walk: every query from start to end, between
 // begin (counters and launch records to zero) and end (their sums to pinned host memory).
 int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t nw_shift, int n_labels, uint32_t* d_blocks, uint32_t* d_longs, uint2* d_items, uint32_t* d_ctrs,
                   hipStream_t stream);
-int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches);
-int fw_label_tables_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches);
+int fw_table_make(const fw_graph* g, fw_tables* t, hipStream_t stream, int* launches);
+int fw_label_tables_make(const fw_graph* g, fw_tables* t, hipStream_t stream, int* launches);
 int fw_sets_make(const fw_graph* g, const fw_tables* t, hipStream_t stream, int* launches);
 int fw_launch_table_walk(const fw_kargs& a, const fw_table_args& tb, int app, int grid, hipStream_t stream, int* grid_used);
 int fw_table_begin(unsigned long long* d_counters, uint32_t* d_scratch, uint32_t words, hipStream_t stream);

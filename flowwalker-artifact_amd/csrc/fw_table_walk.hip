@@ -240,11 +240,11 @@ __device__ __forceinline__ float table_group(const float* __restrict__ weight, c
 
 // Lists of one group: a wave takes 64 consecutive vertices; lists of at most 16 (32) quartets four (two) at a time, the others
 // one after the other.  vrec of the wave's vertices is stored together at the end (long lists get their total from
-// fw_table_sums_kernel).  base: region positions, or NULL: the ones vrec holds already.
+// fw_table_sums_kernel).  base: region positions.
 // Bound: memory (8 bytes read and about 9 written per edge; one pass).
 __global__ __launch_bounds__(256) void fw_table_lists_kernel(const uint32_t* __restrict__ xadj, const int32_t* __restrict__ adjncy,
                                                              const float* __restrict__ weight, int32_t V,
-                                                             const uint32_t* base, uint4* vrec, unsigned char* data,
+                                                             const uint32_t* __restrict__ base, uint4* vrec, unsigned char* data,
                                                              uint32_t* flag) {
   __shared__ float s_total[4][64];
   const int lane = lane_id();
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(256) void fw_table_lists_kernel(const uint32_t* __r
     if (have) {
       off = xadj[v];
       deg = xadj[v + 1] - off;
-      reg = base != nullptr ? base[v] : vrec[v].x;
+      reg = base[v];
     }
     const uint32_t nq = deg != 0u ? list_quartets(off, deg) : 0u;
     s_total[wave][lane] = 0.0f;
@@ -671,7 +671,7 @@ __device__ __forceinline__ void label_segments(const int32_t* __restrict__ label
 template <int kW>
 __global__ __launch_bounds__(256, 7) void fw_label_lists_kernel(const uint32_t* __restrict__ xadj, const int32_t* __restrict__ adjncy,
                                                              const int32_t* __restrict__ label, int32_t V, const fw_label_set set,
-                                                             const uint32_t* base, uint4* vrec, int32_t* by_label) {
+                                                             const uint32_t* __restrict__ base, uint4* vrec, int32_t* by_label) {
   const int lane = lane_id();
   const uint64_t chunks = ((uint64_t)(uint32_t)V + 63u) >> 6;
   for (uint64_t ch = (uint64_t)blockIdx.x * 4u + (uint64_t)(threadIdx.x >> 6); ch < chunks; ch += (uint64_t)gridDim.x * 4u) {
@@ -680,8 +680,7 @@ __global__ __launch_bounds__(256, 7) void fw_label_lists_kernel(const uint32_t* 
     if (v < (uint32_t)V) {
       off = xadj[v];
       deg = xadj[v + 1] - off;
-      const uint32_t reg = base != nullptr ? base[v] : vrec[2u * (uint64_t)v].x;
-      vrec[2u * (uint64_t)v] = make_uint4(reg, deg, 0u, off);
+      vrec[2u * (uint64_t)v] = make_uint4(base[v], deg, 0u, off);
     }
     const uint32_t nq = deg != 0u ? list_quartets(off, deg) : 0u;
     if (v < (uint32_t)V && (nq == 0u || nq > kGq)) vrec[2u * (uint64_t)v + 1u] = make_uint4(0u, 0u, 0u, 0u);
@@ -1271,7 +1270,7 @@ int fw_table_plan(const fw_graph* g, int32_t hub_threshold, uint32_t nw_shift, i
   return FW_OK;
 }
 
-int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches) {
+int fw_table_make(const fw_graph* g, fw_tables* t, hipStream_t stream, int* launches) {
   int cus = 0;
   FW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
   auto grid_for = [&](uint64_t waves) {
@@ -1279,7 +1278,7 @@ int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipSt
     return (unsigned)(blocks < most ? (blocks ? blocks : 1u) : most);
   };
   hipLaunchKernelGGL(fw_table_lists_kernel, dim3(grid_for(((uint64_t)g->V + 63u) / 64u)), dim3(256), 0, stream, g->xadj, g->adjncy,
-                     g->weight, g->V, d_base, t->vrec, t->data, t->flag);
+                     g->weight, g->V, t->blocks, t->vrec, t->data, t->flag);
   FW_HIP(hipGetLastError());
   *launches += 1;
   if (t->n_longs != 0u) {
@@ -1294,7 +1293,7 @@ int fw_table_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipSt
   return FW_OK;
 }
 
-int fw_label_tables_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base, hipStream_t stream, int* launches) {
+int fw_label_tables_make(const fw_graph* g, fw_tables* t, hipStream_t stream, int* launches) {
   int cus = 0;
   FW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
   auto grid_for = [&](uint64_t waves) {
@@ -1304,7 +1303,7 @@ int fw_label_tables_make(const fw_graph* g, fw_tables* t, const uint32_t* d_base
   auto make = [&](auto words) -> int {
     constexpr int kW = decltype(words)::value;
     hipLaunchKernelGGL((fw_label_lists_kernel<kW>), dim3(grid_for(((uint64_t)g->V + 63u) / 64u)), dim3(256), 0, stream, g->xadj,
-                       g->adjncy, g->label, g->V, t->labels, d_base, t->vrec, t->by_label);
+                       g->adjncy, g->label, g->V, t->labels, t->blocks, t->vrec, t->by_label);
     FW_HIP(hipGetLastError());
     if (t->n_longs != 0u)
       hipLaunchKernelGGL((fw_label_groups_kernel<kW>), dim3(grid_for(t->n_items)), dim3(256), 0, stream, t->vrec, g->adjncy,

@@ -221,7 +221,8 @@ int fw_graph_create_placed(int32_t V, uint64_t E, const uint32_t* h_xadj, const 
 
 /*
  * Adopts device arrays that already hold a CSR (e.g. produced by fw_gen_rmat).  The caller may change the biases
- * between calls (what is derived from them is derived anew in every call).  The arrays must
+ * between calls (list tables are derived anew in every call that walks on them, so only a call whose own work pays for
+ * them does).  The arrays must
  * stay valid until fw_graph_destroy and must be readable 12 bytes past their last element
  * (the kernels use aligned 16-byte loads).  take_ownership != 0: destroy frees them with hipFree.
  */

@@ -41,6 +41,19 @@ def _lists(kind):
     return (xadj, adj, w), at
 
 
+def _padded(x):
+    return torch.from_numpy(np.concatenate([x, np.zeros(4, dtype=x.dtype)])).cuda()
+
+
+def _adopt(gpu, xadj, adj, w):
+    """A graph over arrays that the caller keeps, and those arrays."""
+    arrays = _padded(xadj.view(np.int32)), _padded(adj), _padded(w)
+    torch.cuda.synchronize()
+    h = C.c_void_p()
+    gpu.check(gpu.lib().fw_graph_adopt_device(len(xadj) - 1, len(adj), *[C.c_void_p(x.data_ptr()) for x in arrays], None, 0, C.byref(h)))
+    return gpu.Graph(h), arrays
+
+
 @pytest.mark.parametrize("kind", ["even", "uneven"])
 @pytest.mark.parametrize("wg,thr", [(512, 16384), (256, 1024), (1024, 2000), (512, 1 << 30)])
 def test_walks_on_tables(gpu, kind, wg, thr):
@@ -102,20 +115,14 @@ def test_changed_biases_on_adopted_arrays(gpu):
     """An adopted graph's owner may change the biases between calls: tables and the sets' weights are made anew."""
     csr, at = _lists("even")
     xadj, adj, w = csr
-    pad = lambda x: torch.from_numpy(np.concatenate([x, np.zeros(4, dtype=x.dtype)])).cuda()
-    dx, da, dw = pad(xadj.view(np.int32)), pad(adj), pad(w)
-    torch.cuda.synchronize()
-    h = C.c_void_p()
-    gpu.check(gpu.lib().fw_graph_adopt_device(V, len(adj), C.c_void_p(dx.data_ptr()), C.c_void_p(da.data_ptr()),
-                                              C.c_void_p(dw.data_ptr()), None, 0, C.byref(h)))
-    g = gpu.Graph(h)
+    g, (_, _, dw) = _adopt(gpu, xadj, adj, w)
     rng = np.random.RandomState(8)
     starts = at[rng.randint(0, len(at), size=70000)].astype(np.int32)
     try:
         for i in range(3):
             if i:
                 w = np.roll(w, 17)
-                dw.copy_(pad(w))
+                dw.copy_(_padded(w))
                 torch.cuda.synchronize()
             og = _oracle.Graph(xadj, adj, w)
             for p, q in ((0.25, 4.0), (2.0, 0.5)):
@@ -124,6 +131,79 @@ def test_changed_biases_on_adopted_arrays(gpu):
                 paths, st = g.walk(par, starts)
                 assert st.launches >= 6  # tables and sets, or tables made anew
                 assert (paths == ref).all()
+    finally:
+        g.destroy()
+
+
+def test_small_calls_on_adopted_arrays(gpu):
+    """Tables of an adopted graph last one call, so what earlier calls took without them does not pay for them: a loop of small
+    calls streams its lists, however long it runs, also after a large call that made them."""
+    csr, at = _lists("even")
+    g, keep = _adopt(gpu, *csr)
+    rng = np.random.RandomState(12)
+    og = _oracle.Graph(*csr)
+    try:
+        for rounds in range(2):
+            for i in range(150):
+                par = gpu.default_params(app=gpu.APP_NODE2VEC if i % 3 == 0 else gpu.APP_DEEPWALK, max_depth=81, seed=i)
+                starts = at[rng.randint(0, len(at), size=100)].astype(np.int32)
+                paths, st = g.walk(par, starts)
+                assert st.launches == 1, (rounds, i)
+                if i % 50 == 0:
+                    assert (paths == _oracle.walk(og, _oracle.from_walk_params(par), starts)[0]).all()
+            par = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21, seed=5)
+            starts = at[rng.randint(0, len(at), size=60000)].astype(np.int32)  # too few to park
+            paths, st = g.walk(par, starts)
+            assert st.launches == 6
+            assert (paths == _oracle.walk(og, _oracle.from_walk_params(par), starts)[0]).all()
+    finally:
+        g.destroy()
+
+
+def test_changed_lists_on_adopted_arrays(gpu):
+    """Other lists in the same arrays, longer and shorter ones and other neighbours: the regions are planned anew and the sets too."""
+    (xadj, adj, w), at = _lists("even")
+    g, (dx, da, dw) = _adopt(gpu, xadj, adj, w)
+    rng = np.random.RandomState(13)
+    try:
+        for i in range(4):
+            if i:
+                deg = np.roll(np.diff(xadj.astype(np.int64)), 5 + i)[::-1]
+                xadj = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint32)
+                adj = rng.randint(0, V, size=len(adj)).astype(np.int32)
+                for v in range(V):
+                    adj[xadj[v]:xadj[v + 1]].sort()
+                for d, x in ((dx, xadj.view(np.int32)), (da, adj)):
+                    d.copy_(_padded(x))
+                torch.cuda.synchronize()
+            og = _oracle.Graph(xadj, adj, w)
+            starts = rng.randint(0, V, size=65000).astype(np.int32)  # too few to park
+            starts[::2] = np.argsort(-np.diff(xadj.astype(np.int64)))[:64][rng.randint(0, 64, size=32500)]
+            for app, p, q in ((gpu.APP_DEEPWALK, 1.0, 1.0), (gpu.APP_NODE2VEC, 0.25, 4.0), (gpu.APP_NODE2VEC, 2.0, 0.5)):
+                par = gpu.default_params(app=app, max_depth=31, p=p, q=q, seed=90 + i)
+                ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(par), starts)
+                paths, st = g.walk(par, starts)
+                assert st.launches >= 6, (i, app, p)
+                assert (paths == ref).all() and (st.steps, st.sampled_edges) == (steps, edges), (i, app, p)
+    finally:
+        g.destroy()
+
+
+def test_biases_that_tables_cannot_hold(gpu):
+    """A negative bias on an adopted graph (the upload of a host graph refuses it): the streaming kernels say what happens then, and
+    later calls do not make tables in vain."""
+    (xadj, adj, w), at = _lists("even")
+    w = w.copy()
+    w[np.random.RandomState(1).randint(0, len(w), size=50)] *= -1.0
+    g, keep = _adopt(gpu, xadj, adj, w)
+    starts = at[np.random.RandomState(2).randint(0, len(at), size=60000)].astype(np.int32)
+    try:
+        for i in range(3):
+            par = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21, seed=5)
+            paths, st = g.walk(par, starts)
+            par.park_threshold = -1
+            ref, _ = g.walk(par, starts)
+            assert (paths == ref).all() and st.launches == 1
     finally:
         g.destroy()
 
