@@ -1888,6 +1888,7 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     *launches = 0;
     return FW_OK;
   }
+  if (make_tables) g->streamed_ms = 0.0;  // tables for another granularity have to be earned again
   {
     std::lock_guard<std::mutex> guard(g->tables_lock);
     g->tables = t;

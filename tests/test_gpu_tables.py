@@ -160,6 +160,26 @@ def test_small_calls_on_adopted_arrays(gpu):
         g.destroy()
 
 
+def test_two_granularities_in_turn(gpu):
+    """One set of tables per graph: calls of two granularities in turn replace it only after lists have been streamed for as long as
+    making it takes, not in every call."""
+    csr, at = _lists("even")
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    rng = np.random.RandomState(14)
+    try:
+        made = 0
+        for i in range(60):
+            par = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=81, seed=i, hub_threshold=(16384, 2000)[i & 1])
+            starts = at[rng.randint(0, len(at), size=100)].astype(np.int32)
+            paths, st = g.walk(par, starts)
+            made += st.launches > 3
+            assert (paths == _oracle.walk(og, _oracle.from_walk_params(par), starts)[0]).all(), i
+        assert 1 <= made <= 15, made
+    finally:
+        g.destroy()
+
+
 def test_changed_lists_on_adopted_arrays(gpu):
     """Other lists in the same arrays, longer and shorter ones and other neighbours: the regions are planned anew and the sets too."""
     (xadj, adj, w), at = _lists("even")
