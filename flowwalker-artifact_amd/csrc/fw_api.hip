@@ -1680,7 +1680,8 @@ static int plan_tables(const fw_graph* g, fw_tables* t, hipStream_t stream) {
   return FW_OK;
 }
 
-// Whether this call makes the hash sets of node2vec's adjacency tests (their memory is there then).  They are made once the calls' searches
+// Whether this call makes the hash sets of node2vec's adjacency tests, and for the return edge their weights (the memory is there
+// then).  They are made once the calls' searches
 // have cost, or are about to cost, half as much again as making them: a search that finds the chip busy costs 0.05 ns (five
 // scattered reads at 51 G/s, half of the tests undecided; R-MAT 24: 41 ms of 709 M steps), one in a chain of a few walkers 4 us, and the sets take
 // 0.2 ms and 20 bytes per edge at 2.5 TB/s.
@@ -1703,9 +1704,7 @@ static bool sets_for_call(const fw_graph* g, const fw_walk_params* p, fw_tables*
   };
   if (t->sets == nullptr) room(reinterpret_cast<void**>(&t->sets));
   if (t->sets != nullptr && t->set_weights == nullptr && want_weights) room(reinterpret_cast<void**>(&t->set_weights));
-  t->have_sets = t->sets != nullptr;
-  t->have_weights = t->have_sets && back && t->set_weights != nullptr;  // (without them the return edge is searched for)
-  return t->have_sets;
+  return t->sets != nullptr;  // (without weights the return edge is searched for)
 }
 
 // MetaPath's tables, for the labels of the call's schema; otherwise as tables_for_call below.  Making them takes
@@ -1717,7 +1716,7 @@ constexpr double kParkedStepMs = 0.13e-6;
 constexpr double kParkIndexEdgeMs = 10e-9;
 constexpr double kLabelMakeEdgeMs = 15e-9;
 
-static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipStream_t stream, std::shared_ptr<fw_tables>* out,
+static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipStream_t stream, const fw_tables** out,
                                  int* launches, hipEvent_t ev_start, hipEvent_t ev0, hipEvent_t ev1) {
   if (p->park_threshold != 0 || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) || g->host_edges || g->no_label_tables ||
       (p->wg_threads != 256 && p->wg_threads != 512 && p->wg_threads != 1024))
@@ -1731,14 +1730,10 @@ static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n
     set.label[set.n++] = p->schema[i];
   }
   const uint32_t nw_shift = p->wg_threads == 256 ? 2u : (p->wg_threads == 512 ? 3u : 4u);
-  std::shared_ptr<fw_tables> t;
-  {
-    std::lock_guard<std::mutex> guard(g->tables_lock);
-    t = g->label_tables;
-  }
+  fw_tables* t = g->label_tables.get();
   if (t && (t->hub_threshold != p->hub_threshold || t->nw_shift != nw_shift || t->labels.n != set.n ||
             memcmp(t->labels.label, set.label, sizeof(set.label)) != 0))
-    t.reset();
+    t = nullptr;  // another schema or granularity: one set per graph
   if (t && !g->borrowed && p->time_kernels == 0) {
     *out = t;
     return FW_OK;
@@ -1760,16 +1755,15 @@ static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n
   }
   if (!t || g->borrowed) {
     if (!t) {
-      {
-        std::lock_guard<std::mutex> guard(g->tables_lock);
-        g->label_tables.reset();  // another schema or granularity: one set per graph
-      }
-      t = std::make_shared<fw_tables>();
+      g->label_tables.reset(new (std::nothrow) fw_tables);
+      t = g->label_tables.get();
+      if (!t) return FW_OK;
       t->hub_threshold = p->hub_threshold;
       t->nw_shift = nw_shift;
       t->labels = set;
     }
-    const int rc = plan_tables(g, t.get(), stream);
+    const int rc = plan_tables(g, t, stream);
+    if (rc != FW_OK) g->label_tables.reset();  // nothing half made stays
     if (rc == FW_ERR_NOMEM) {
       g->no_label_tables = 1;
       return FW_OK;
@@ -1779,28 +1773,27 @@ static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n
   auto make = [&]() -> int {
     if (ev_start) FW_HIP(hipEventRecord(ev_start, stream));
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev0, stream));
-    const int rc = fw_label_tables_make(g, t.get(), stream, launches);
+    const int rc = fw_label_tables_make(g, t, stream, launches);
     if (rc != FW_OK) return rc;
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
     FW_HIP(hipStreamSynchronize(stream));  // (the batch entry walks on other streams)
     return FW_OK;
   };
   const int rc = make();
-  std::lock_guard<std::mutex> guard(g->tables_lock);
   if (rc != FW_OK) {
     g->label_tables.reset();
     return rc;
   }
   g->label_ms = 0.0;  // tables for another schema have to be earned again
-  g->label_tables = t;
   *out = t;
   return FW_OK;
 }
 
-// The tables a call over n queries walks on, or none (*out stays empty).  Called with the graph's busy flag held.  ev_start is
+// The tables a call over n queries walks on, or none (*out is NULL).  Called with the graph's busy flag held.  ev_start is
 // recorded before the making, ev0 and ev1 around it when its time is asked for; *launches: kernels it took.
-static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipStream_t stream, std::shared_ptr<fw_tables>* out,
+static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipStream_t stream, const fw_tables** out,
                            int* launches, hipEvent_t ev_start, hipEvent_t ev0, hipEvent_t ev1) {
+  *out = nullptr;
   *launches = 0;
   // an explicit parking degree asks for the parking pipeline, a negative one for walkers that stream their lists
   if (p->app == FW_APP_METAPATH) return label_tables_for_call(g, p, n, stream, out, launches, ev_start, ev0, ev1);
@@ -1813,12 +1806,8 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
       (p->app == FW_APP_NODE2VEC && p->max_depth > FW_REC_LEN_MASK))
     return FW_OK;
   const uint32_t nw_shift = p->wg_threads == 256 ? 2u : (p->wg_threads == 512 ? 3u : 4u);
-  std::shared_ptr<fw_tables> t;
-  {
-    std::lock_guard<std::mutex> guard(g->tables_lock);
-    t = g->tables;
-  }
-  if (t && (t->hub_threshold != p->hub_threshold || t->nw_shift != nw_shift)) t.reset();
+  fw_tables* t = g->tables.get();
+  if (t && (t->hub_threshold != p->hub_threshold || t->nw_shift != nw_shift)) t = nullptr;  // another granularity: one set per graph
   const bool make_tables = !t || g->borrowed || p->time_kernels != 0;  // (a call that wants the split of its time makes them anew)
   double steps = (double)(p->max_depth - 1);
   if (!t || g->borrowed) {
@@ -1836,23 +1825,22 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
   }
   if (!t || g->borrowed) {
     if (!t) {
-      {
-        std::lock_guard<std::mutex> guard(g->tables_lock);
-        g->tables.reset();  // another granularity: one set per graph
-      }
-      t = std::make_shared<fw_tables>();
+      g->tables.reset(new (std::nothrow) fw_tables);
+      t = g->tables.get();
+      if (!t) return FW_OK;
       t->hub_threshold = p->hub_threshold;
       t->nw_shift = nw_shift;
     }
     t->have_sets = t->have_weights = false;
-    const int rc = plan_tables(g, t.get(), stream);
+    const int rc = plan_tables(g, t, stream);
+    if (rc != FW_OK) g->tables.reset();  // nothing half made stays
     if (rc == FW_ERR_NOMEM) {
       g->no_tables = 1;
       return FW_OK;
     }
     if (rc != FW_OK) return rc;
   }
-  const bool make_sets = sets_for_call(g, p, t.get(), steps * (double)n, steps);
+  const bool make_sets = sets_for_call(g, p, t, steps * (double)n, steps);
   if (!make_tables && !make_sets) {
     *out = t;
     return FW_OK;
@@ -1864,9 +1852,13 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     int rc = FW_OK;
     if (make_tables) {
       FW_HIP(hipMemsetAsync(t->flag, 0, sizeof(uint32_t), stream));
-      if ((rc = fw_table_make(g, t.get(), stream, launches)) != FW_OK) return rc;
+      if ((rc = fw_table_make(g, t, stream, launches)) != FW_OK) return rc;
     }
-    if (make_sets && (rc = fw_sets_make(g, t.get(), stream, launches)) != FW_OK) return rc;
+    if (make_sets) {
+      if ((rc = fw_sets_make(g, t, stream, launches)) != FW_OK) return rc;
+      t->have_sets = true;
+      t->have_weights = t->set_weights != nullptr;
+    }
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
     if (!make_tables) return FW_OK;
     FW_HIP(hipMemcpyAsync(&bad, t->flag, sizeof(bad), hipMemcpyDeviceToHost, stream));
@@ -1874,12 +1866,12 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     return FW_OK;
   };
   const int rc = make();
-  if (rc != FW_OK) {  // nothing half made stays
-    std::lock_guard<std::mutex> guard(g->tables_lock);
+  if (rc != FW_OK) {
     g->tables.reset();
     return rc;
   }
   if (bad != 0u) {  // the streaming kernels define what happens then
+    g->tables.reset();
     if (g->borrowed) {
       g->skip_tables = 15;  // the owner may mend them: looked at again after a while
     } else {
@@ -1889,10 +1881,6 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     return FW_OK;
   }
   if (make_tables) g->streamed_ms = 0.0;  // tables for another granularity have to be earned again
-  {
-    std::lock_guard<std::mutex> guard(g->tables_lock);
-    g->tables = t;
-  }
   *out = t;
   return FW_OK;
 }
@@ -1964,7 +1952,7 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
   a.counters = d_scr->counters;
   int grid_used = 0, launches = 0;
   KernelTimes times;
-  std::shared_ptr<fw_tables> tables;
+  const fw_tables* tables = nullptr;
   rc = tables_for_call(mg, p, n, stream, &tables, &launches, ev0, mg->call_ev[2], mg->call_ev[3]);
   if (rc != FW_OK) return rc;
   if (tables) {
@@ -2205,7 +2193,7 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
 
   const int32_t park_threshold = resolve_park_threshold(g, p, (int32_t)bs);
   for (hipEvent_t& e : mg->call_ev) if (!e) FW_HIP(hipEventCreate(&e));
-  std::shared_ptr<fw_tables> tables;
+  const fw_tables* tables = nullptr;
   int make_launches = 0;
   rc = tables_for_call(mg, p, n, nullptr, &tables, &make_launches, mg->call_ev[0], mg->call_ev[2], mg->call_ev[3]);
   if (rc != FW_OK) return rc;

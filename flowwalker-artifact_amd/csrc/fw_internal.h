@@ -6,7 +6,6 @@
 
 #include <atomic>
 #include <memory>
-#include <mutex>
 
 #include "flowwalker.h"
 
@@ -26,8 +25,8 @@ struct fw_label_set {
   int32_t label[FW_MAX_TABLE_LABELS] = {};
 };
 
-// List tables (fw_table_walk.hip): the walker-independent part of every sampling step on a graph.  Not changed once made, and
-// held by reference count: a call that walks on them keeps them alive while another call replaces them in the graph.
+// List tables (fw_table_walk.hip): the walker-independent part of every sampling step on a graph.  They belong to the graph, and only
+// a call that holds its busy flag makes, reads or drops them.
 struct fw_tables {
   uint4* vrec = nullptr;          // [V] {region in 128-byte blocks, degree, total, CSR offset}
   unsigned char* data = nullptr;  // the regions
@@ -91,9 +90,8 @@ struct fw_graph {
   double mean_list = -1.0;            // sum of squared degrees / E: the list length a step meets, on average; lazily computed
   double streamed_ms = 0.0;           // device time of the walk calls that had no list tables and might have had them
   int no_tables = 0;                  // biases or totals the tables cannot hold, or no room for them: do not try again
-  std::mutex tables_lock;
-  std::shared_ptr<fw_tables> tables;
-  std::shared_ptr<fw_tables> label_tables;  // MetaPath's, for the labels of one schema
+  std::unique_ptr<fw_tables> tables;
+  std::unique_ptr<fw_tables> label_tables;  // MetaPath's, for the labels of one schema
   double label_ms = 0.0;              // device time of the MetaPath calls without them, since they were last made
   int no_label_tables = 0;            // no room for them: do not try again
   std::atomic<int> busy{0};           // a walk call is running on this graph (the caches above are per graph)
