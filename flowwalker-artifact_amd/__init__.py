@@ -18,6 +18,7 @@ LIB_PATH = os.environ.get("FLOWWALKER_LIB") or os.path.join(_PKG, "lib", "libflo
 
 FW_MAX_SCHEMA = 64
 APP_DEEPWALK, APP_PPR, APP_NODE2VEC, APP_METAPATH = 0, 1, 2, 3
+ENGINE_NONE, ENGINE_STREAM, ENGINE_PARK, ENGINE_TABLES = 0, 1, 2, 3
 SAMPLER_ZPRS, SAMPLER_DPRS, SAMPLER_REF_ZPRS, SAMPLER_REF_DPRS, SAMPLER_REF_STATIC = 0, 1, 2, 3, 0x100
 SAMPLER_REF_RNG_LDS, SAMPLER_REF_RNG_GLOBAL = 0x200, 0x400
 FW_OK = 0
@@ -32,6 +33,7 @@ EXPORTED = [
     "fw_gen_rmat", "fw_csr_read_header", "fw_csr_load", "fw_csr_write", "fw_graph_load",
     "fw_graph_create_placed", "fw_graph_load_placed", "fw_walk_device_noalloc", "fw_csr_sort_neighbours",
     "fw_sampler_baseline_run", "fw_dev_random_access_rate",
+    "fw_graph_engine", "fw_graph_limit_tables",
 ]
 
 
@@ -120,6 +122,8 @@ def lib():
         L.fw_graph_destroy.argtypes = [C.c_void_p]
         L.fw_graph_info.argtypes = [C.c_void_p, C.POINTER(C.c_int32), C.POINTER(C.c_uint64), C.POINTER(C.c_int32),
                                     C.POINTER(C.c_int32)]
+        L.fw_graph_engine.argtypes = [C.c_void_p, C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_uint64)]
+        L.fw_graph_limit_tables.argtypes = [C.c_void_p, C.c_uint64]
         L.fw_graph_is_sorted.argtypes = [C.c_void_p, C.POINTER(C.c_int)]
         L.fw_graph_download.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
         L.fw_walk_device.argtypes = [C.c_void_p, C.POINTER(WalkParams), C.c_void_p, C.c_int32, C.c_void_p,
@@ -287,6 +291,16 @@ class Graph:
         md, mv = C.c_int32(), C.c_int32()
         check(lib().fw_graph_info(self.handle, None, None, C.byref(md), C.byref(mv)))
         return md.value, mv.value
+
+    def engine(self):
+        """(what the last walk call ran on: ENGINE_*, its launches that made tables, bytes that tables hold now)."""
+        e, made, held = C.c_int32(), C.c_int32(), C.c_uint64()
+        check(lib().fw_graph_engine(self.handle, C.byref(e), C.byref(made), C.byref(held)))
+        return e.value, made.value, held.value
+
+    def limit_tables(self, max_bytes):
+        """Most device memory that walk calls may keep with the graph as list tables; 0 for none."""
+        check(lib().fw_graph_limit_tables(self.handle, max_bytes))
 
     def is_sorted(self):
         s = C.c_int()

@@ -1640,18 +1640,50 @@ static int mean_list_length(fw_graph* g, double* out) {
   return FW_OK;
 }
 
+static uint64_t table_bytes(const fw_graph* g) {
+  return (g->tables ? g->tables->bytes : 0u) + (g->label_tables ? g->label_tables->bytes : 0u);
+}
+
+// Bytes that the graph's tables may take beyond what they hold: as far as its limit goes, and half of the memory that is free.
+static uint64_t table_room(const fw_graph* g) {
+  const uint64_t held = table_bytes(g);
+  size_t free_b = 0, total_b = 0;
+  if (held >= g->table_limit || hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0u;
+  }
+  const uint64_t left = g->table_limit - held;
+  return left < free_b / 2u ? left : free_b / 2u;
+}
+
+// Tables are an extra: after a call for which there was no room the next ones go without, and then it is looked at again.
+constexpr int kSkipTables = 15;
+
+// One array of the tables, when it is not there yet and `*left` has room for it.
+template <typename T>
+static int table_array(fw_tables* t, T** p, size_t bytes, uint64_t* left) {
+  if (*p != nullptr) return FW_OK;
+  if (bytes > *left) return FW_ERR_NOMEM;
+  if (hipMalloc(reinterpret_cast<void**>(p), bytes ? bytes : 16) != hipSuccess) {
+    (void)hipGetLastError();
+    *p = nullptr;
+    return FW_ERR_NOMEM;
+  }
+  *left -= bytes;
+  t->bytes += bytes;
+  return FW_OK;
+}
+
 // Room for the tables of `g`: positions of the regions, work lists, memory (what `t` holds already is used again).  FW_ERR_NOMEM when
 // there is no room for them.
 static int plan_tables(const fw_graph* g, fw_tables* t, hipStream_t stream) {
   const size_t nv = (size_t)g->V + 1u;
   const size_t item_cap = (size_t)(g->E / 500u) + 64u, long_cap = (size_t)(g->E / 1000u) + 64u;  // a list of several groups has over 1020 entries
   size_t tmp_bytes = 0;
-  auto room = [](auto** p, size_t bytes) -> int {
-    if (*p != nullptr || hipMalloc(reinterpret_cast<void**>(p), bytes ? bytes : 16) == hipSuccess) return FW_OK;
-    (void)hipGetLastError();
-    *p = nullptr;
-    return FW_ERR_NOMEM;
-  };
+  uint64_t left = table_room(g);
+  const uint64_t least = t->labels.n != 0 ? 4u * g->E + 32u * (uint64_t)g->V : 8u * g->E + 16u * (uint64_t)g->V;
+  if (left + t->bytes < least) return FW_ERR_NOMEM;  // nothing is allocated in vain
+  auto room = [&](auto** p, size_t bytes) { return table_array(t, p, bytes, &left); };
   FW_HIP(rocprim::exclusive_scan(nullptr, tmp_bytes, t->blocks, t->blocks, 0u, nv, rocprim::plus<uint32_t>(), stream));
   int rc;
   if ((rc = room(&t->blocks, nv * 4u)) || (rc = room(&t->ctrs, 64)) || (rc = room(&t->scan_tmp, tmp_bytes)) ||
@@ -1673,6 +1705,8 @@ static int plan_tables(const fw_graph* g, fw_tables* t, hipStream_t stream) {
   if (t->data_bytes < bytes) {
     if (t->data) (void)hipFree(t->data);
     t->data = nullptr;
+    t->bytes -= t->data_bytes;
+    left += t->data_bytes;
     t->data_bytes = 0;
     if ((rc = room(&t->data, bytes)) != FW_OK) return rc;
     t->data_bytes = bytes;
@@ -1687,7 +1721,7 @@ static int plan_tables(const fw_graph* g, fw_tables* t, hipStream_t stream) {
 // 0.2 ms and 20 bytes per edge at 2.5 TB/s.
 static bool sets_for_call(const fw_graph* g, const fw_walk_params* p, fw_tables* t, double all_steps, double steps) {
   const bool back = p->p < 1.0f && p->p < p->q;  // the return edge is a component of its own
-  if (p->app != FW_APP_NODE2VEC || (p->q == 1.0f && !back) || t->no_sets) return false;
+  if (p->app != FW_APP_NODE2VEC || (p->q == 1.0f && !back)) return false;
   const bool want_weights = back && !t->have_weights;
   if (t->have_sets && !want_weights) return p->time_kernels != 0;
   if (!t->have_sets) {
@@ -1695,15 +1729,16 @@ static bool sets_for_call(const fw_graph* g, const fw_walk_params* p, fw_tables*
     t->search_ms = (g->borrowed ? 0.0 : t->search_ms) + ms;  // (an adopted graph's sets last one call)
     if (t->search_ms < kMakeMargin * (20.0 * (double)g->E / 2.5e9 + 0.2)) return false;
   }
+  if (t->skip_sets > 0) {
+    --t->skip_sets;
+    return false;
+  }
   const size_t places = 16u * (size_t)(fw_set_first((uint32_t)g->E, (uint32_t)g->V) + 1u);
-  auto room = [&](void** at) {
-    if (hipMalloc(at, places * 4u) == hipSuccess) return;
-    (void)hipGetLastError();
-    *at = nullptr;
-    t->no_sets = 1;
-  };
-  if (t->sets == nullptr) room(reinterpret_cast<void**>(&t->sets));
-  if (t->sets != nullptr && t->set_weights == nullptr && want_weights) room(reinterpret_cast<void**>(&t->set_weights));
+  uint64_t left = table_room(g);
+  if (table_array(t, &t->sets, places * 4u, &left) != FW_OK || (want_weights && table_array(t, &t->set_weights, places * 4u, &left) != FW_OK)) {
+    t->skip_sets = kSkipTables;
+    if (t->have_sets) return false;
+  }
   return t->sets != nullptr;  // (without weights the return edge is searched for)
 }
 
@@ -1718,9 +1753,13 @@ constexpr double kLabelMakeEdgeMs = 15e-9;
 
 static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipStream_t stream, const fw_tables** out,
                                  int* launches, hipEvent_t ev_start, hipEvent_t ev0, hipEvent_t ev1) {
-  if (p->park_threshold != 0 || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) || g->host_edges || g->no_label_tables ||
+  if (p->park_threshold != 0 || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) || g->host_edges || g->table_limit == 0u ||
       (p->wg_threads != 256 && p->wg_threads != 512 && p->wg_threads != 1024))
     return FW_OK;
+  if (g->skip_label_tables > 0) {
+    --g->skip_label_tables;
+    return FW_OK;
+  }
   fw_label_set set;
   for (int i = 0; i < p->schema_len; ++i) {
     int at = 0;
@@ -1765,7 +1804,7 @@ static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n
     const int rc = plan_tables(g, t, stream);
     if (rc != FW_OK) g->label_tables.reset();  // nothing half made stays
     if (rc == FW_ERR_NOMEM) {
-      g->no_label_tables = 1;
+      g->skip_label_tables = kSkipTables;
       return FW_OK;
     }
     if (rc != FW_OK) return rc;
@@ -1797,14 +1836,14 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
   *launches = 0;
   // an explicit parking degree asks for the parking pipeline, a negative one for walkers that stream their lists
   if (p->app == FW_APP_METAPATH) return label_tables_for_call(g, p, n, stream, out, launches, ev_start, ev0, ev1);
+  if (p->park_threshold != 0 || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) ||
+      g->host_edges || g->no_tables || g->table_limit == 0u || (p->wg_threads != 256 && p->wg_threads != 512 && p->wg_threads != 1024) ||
+      (p->app == FW_APP_NODE2VEC && p->max_depth > FW_REC_LEN_MASK))
+    return FW_OK;
   if (g->skip_tables > 0) {
     --g->skip_tables;
     return FW_OK;
   }
-  if (p->park_threshold != 0 || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) ||
-      g->host_edges || g->no_tables || (p->wg_threads != 256 && p->wg_threads != 512 && p->wg_threads != 1024) ||
-      (p->app == FW_APP_NODE2VEC && p->max_depth > FW_REC_LEN_MASK))
-    return FW_OK;
   const uint32_t nw_shift = p->wg_threads == 256 ? 2u : (p->wg_threads == 512 ? 3u : 4u);
   fw_tables* t = g->tables.get();
   if (t && (t->hub_threshold != p->hub_threshold || t->nw_shift != nw_shift)) t = nullptr;  // another granularity: one set per graph
@@ -1835,7 +1874,7 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     const int rc = plan_tables(g, t, stream);
     if (rc != FW_OK) g->tables.reset();  // nothing half made stays
     if (rc == FW_ERR_NOMEM) {
-      g->no_tables = 1;
+      g->skip_tables = kSkipTables;
       return FW_OK;
     }
     if (rc != FW_OK) return rc;
@@ -1873,7 +1912,7 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
   if (bad != 0u) {  // the streaming kernels define what happens then
     g->tables.reset();
     if (g->borrowed) {
-      g->skip_tables = 15;  // the owner may mend them: looked at again after a while
+      g->skip_tables = kSkipTables;  // the owner may mend them: looked at again after a while
     } else {
       g->no_tables = 1;
     }
@@ -1913,6 +1952,30 @@ struct BusyGuard {
   bool ok() const { return held; }
   ~BusyGuard() { if (held) g->busy.store(0); }
 };
+
+extern "C" int fw_graph_engine(const fw_graph* g, int32_t* engine, int32_t* made, uint64_t* held) {
+  if (!g) { fw_set_error("fw_graph_engine: graph is NULL"); return FW_ERR_INVALID; }
+  BusyGuard busy(g);
+  if (!busy.ok()) return FW_ERR_INVALID;
+  if (engine) *engine = g->last_engine;
+  if (made) *made = g->last_made;
+  if (held) *held = table_bytes(g);
+  return FW_OK;
+}
+
+extern "C" int fw_graph_limit_tables(fw_graph* g, uint64_t max_bytes) {
+  if (!g) { fw_set_error("fw_graph_limit_tables: graph is NULL"); return FW_ERR_INVALID; }
+  BusyGuard busy(g);
+  if (!busy.ok()) return FW_ERR_INVALID;
+  g->table_limit = max_bytes;
+  if (table_bytes(g) > max_bytes) {
+    g->tables.reset();
+    g->label_tables.reset();
+  }
+  g->skip_tables = g->skip_label_tables = 0;
+  if (g->tables) g->tables->skip_sets = 0;
+  return FW_OK;
+}
 
 static double now_ms() {
   using clk = std::chrono::steady_clock;
@@ -1955,6 +2018,8 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
   const fw_tables* tables = nullptr;
   rc = tables_for_call(mg, p, n, stream, &tables, &launches, ev0, mg->call_ev[2], mg->call_ev[3]);
   if (rc != FW_OK) return rc;
+  mg->last_engine = tables ? FW_ENGINE_TABLES : FW_ENGINE_STREAM;
+  mg->last_made = launches;
   if (tables) {
     a.park_threshold = park_threshold;
     if (launches == 0) FW_TRY(hipEventRecord(ev0, stream));  // (tables made in this call: recorded before that)
@@ -1983,6 +2048,7 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
       use_pb = pb != nullptr;  // no room for the parking lists: walk without parking (same results, one launch)
     }
     FW_TRY(hipEventRecord(ev0, stream));
+    if (use_pb) mg->last_engine = FW_ENGINE_PARK;
     rc = run_walk_launches(g, p, a, park_threshold, use_pb ? pb : nullptr, stream, &grid_used, &launches, &times);
     if (rc != FW_OK) { cleanup(); return rc; }
   }
@@ -2261,6 +2327,8 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     FW_TRY(hipEventCreate(&e));
     bc->events.push_back(e);
   }
+  mg->last_engine = tables ? FW_ENGINE_TABLES : use_pb ? FW_ENGINE_PARK : FW_ENGINE_STREAM;
+  mg->last_made = make_launches;
   ParkBuffers* const pbs = bc->pbs;
   int32_t* const d_starts = bc->d_starts;
   int32_t* const d_paths = bc->d_paths;

@@ -45,10 +45,11 @@ struct fw_tables {
   float* set_weights = nullptr;
   bool have_sets = false, have_weights = false;  // whether they hold the lists
   double search_ms = 0.0;         // what node2vec calls without sets spent on searches, estimated
-  int no_sets = 0;                // no room for them: do not try again
+  int skip_sets = 0;              // calls to come that do not try for sets: there was no room for them
   // MetaPath: the lists sorted by label inside every group of the sampler (fw_table_walk.hip); vrec then has two words per vertex
   fw_label_set labels;
   int32_t* by_label = nullptr;    // [E]
+  size_t bytes = 0;               // of device memory, all of the above
   ~fw_tables() {
     void* ptrs[] = {vrec, data, longs, items, flag, blocks, ctrs, scan_tmp, sets, set_weights, by_label};
     for (void* p : ptrs) if (p) (void)hipFree(p);
@@ -86,14 +87,16 @@ struct fw_graph {
   hipEvent_t call_ev[4] = {};         // and its timing events: the call, the making of the list tables
   int borrowed = 0;                   // the arrays came through fw_graph_adopt_device: their owner may change them between
                                       // calls, so list tables are planned and made anew in every call that walks on them
-  int skip_tables = 0;                // calls to come that do not try for tables: an adopted graph had biases they cannot hold
+  int skip_tables = 0, skip_label_tables = 0;  // calls to come that do not try for tables: there was no room for them, or an adopted
+                                      // graph had biases they cannot hold
   double mean_list = -1.0;            // sum of squared degrees / E: the list length a step meets, on average; lazily computed
   double streamed_ms = 0.0;           // device time of the walk calls that had no list tables and might have had them
-  int no_tables = 0;                  // biases or totals the tables cannot hold, or no room for them: do not try again
+  int no_tables = 0;                  // biases or totals the tables cannot hold: do not try again
   std::unique_ptr<fw_tables> tables;
   std::unique_ptr<fw_tables> label_tables;  // MetaPath's, for the labels of one schema
   double label_ms = 0.0;              // device time of the MetaPath calls without them, since they were last made
-  int no_label_tables = 0;            // no room for them: do not try again
+  uint64_t table_limit = UINT64_MAX;  // bytes that all tables of the graph together may take (fw_graph_limit_tables)
+  int last_engine = FW_ENGINE_NONE, last_made = 0;  // fw_graph_engine
   std::atomic<int> busy{0};           // a walk call is running on this graph (the caches above are per graph)
 };
 

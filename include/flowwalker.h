@@ -148,6 +148,14 @@ typedef struct {
 
 typedef struct fw_graph fw_graph; /* device CSR mirror: include/gpu_graph.cuh:28-78 */
 
+/* What a walk call ran on.  The walks are the same whichever it was. */
+typedef enum {
+  FW_ENGINE_NONE = 0,   /* no call yet */
+  FW_ENGINE_STREAM = 1, /* one launch, walkers read their lists themselves */
+  FW_ENGINE_PARK = 2,   /* the parking pipeline */
+  FW_ENGINE_TABLES = 3  /* list tables */
+} fw_engine;
+
 /* ---- library ---------------------------------------------------------------------------------- */
 
 /* Thread-local text of the last error; replaces the print-and-exit of CUDA_RT_CALL (include/util.cuh:56-68). */
@@ -237,6 +245,19 @@ int fw_graph_info(const fw_graph* g, int32_t* V, uint64_t* E, int32_t* max_degre
 /* 1 when every neighbour list is ascending (equal neighbours allowed; needed by node2vec: include/gpu_graph.cuh:97-118; the walk
  * entry points return FW_ERR_INVALID for FW_APP_NODE2VEC on a graph where this is 0). */
 int fw_graph_is_sorted(const fw_graph* g, int* sorted);
+
+/*
+ * What the last fw_walk_device / fw_walk_batch on the graph ran on (fw_engine), how many launches of it made list tables or node2vec's
+ * sets, and the device memory that tables hold now.  Any output pointer may be NULL.
+ */
+int fw_graph_engine(const fw_graph* g, int32_t* engine, int32_t* made, uint64_t* table_bytes);
+/*
+ * Bounds the device memory that walk calls may keep with the graph as list tables (8 to 9 bytes per edge and 16 to 150 per vertex,
+ * node2vec's sets 8 per edge and 64 per vertex, twice that where 1/p > max(1, 1/q); by default as much as they need and is half
+ * free).  Gives back at once what is above the bound; 0: none are held or made, walks stream their lists or park.  The walks
+ * are the same either way.  FW_ERR_INVALID while a walk call is running on the graph.
+ */
+int fw_graph_limit_tables(fw_graph* g, uint64_t max_bytes);
 
 /* Copies the device CSR back (any output pointer may be NULL). */
 int fw_graph_download(const fw_graph* g, uint32_t* h_xadj, int32_t* h_adjncy, float* h_weight, int32_t* h_label);

@@ -101,7 +101,8 @@ def test_config4_rmat24_symmetrised(gpu):
         p = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=81, seed=1)
         print("deepwalk, %d queries" % g.V, flush=True)
         paths, st = g.walk(p, starts)
-        assert st.launches > 3 and st.hub_steps > 0                             # the default rule parks at this size
+        assert st.launches > 3 and st.hub_steps > 0
+        assert g.engine()[0] == gpu.ENGINE_TABLES                               # a call of this size pays for them by itself
         L = _check_paths(xadj, adj, paths, starts, st, 81, sample=50000)
         deg = np.diff(xadj.astype(np.int64))
         assert (L[deg > 0] == 81).all()                                         # undirected: no dead ends

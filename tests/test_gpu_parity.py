@@ -188,6 +188,7 @@ def test_default_parking_rule_and_its_tail(gpu, hub):
     starts = np.random.RandomState(8).randint(0, 12000, size=600000).astype(np.int32)  # ~50,000 of them park per round
     og = _oracle.Graph(xadj, adj, w, lab)
     g = gpu.Graph.from_csr(xadj, adj, w, lab)
+    g.limit_tables(0)
     try:
         for kw in (dict(app=gpu.APP_PPR, max_depth=61, tp=0.3), dict(app=gpu.APP_DEEPWALK, max_depth=9)):
             p = gpu.default_params(seed=21, **kw)
@@ -197,6 +198,7 @@ def test_default_parking_rule_and_its_tail(gpu, hub):
             assert (paths == ref).all()
             assert (st.steps, st.sampled_edges) == (steps, edges)
             assert st.launches >= 3 and 0 < st.hub_steps < st.steps
+            assert g.engine() == (gpu.ENGINE_PARK, 0, 0)
     finally:
         g.destroy()
 
@@ -449,11 +451,13 @@ def test_kernel_times_on_request(gpu):
     only (an event pair per launch costs the stream time); the walks and the counters are the same either way."""
     csr = _graphs.hub_graph(V=30000, hub_degrees=(20000, 8000), base_degree=8, seed=5)
     g = gpu.Graph.from_csr(*csr)
+    g.limit_tables(0)
     try:
         starts = np.random.RandomState(2).randint(0, 30000, size=200000).astype(np.int32)
         p = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21, seed=9)
         plain, st0 = g.walk(p, starts)
-        assert st0.launches > 1 and st0.hub_steps > 0                      # the parking pipeline ran
+        assert st0.launches > 1 and st0.hub_steps > 0
+        assert g.engine()[0] == gpu.ENGINE_PARK
         assert st0.kernel_ms > 0.0 and st0.walk_kernel_ms == 0.0 and st0.hub_kernel_ms == 0.0
         assert st0.requested_bytes > 0 and st0.scattered_writes > 0
         p.time_kernels = 1

@@ -79,6 +79,8 @@ def test_walks_on_tables(gpu, kind, wg, thr):
             bad = np.nonzero((paths != ref).any(axis=1))[0]
             assert len(bad) == 0, (kw, n, bad[0], paths[bad[0]], ref[bad[0]])
             assert (st.steps, st.sampled_edges) == (steps, edges), (kw, n)
+            assert g.engine()[0] == gpu.ENGINE_TABLES
+            assert (g.engine()[1] != 0) == (st.launches > 3)
             if i == 0:
                 assert st.launches >= 4  # the tables were made
             again, st2 = g.walk_batch(p, starts, batch_size=max(1, n // 3))
@@ -111,6 +113,50 @@ def test_node2vec_on_hash_sets(gpu, kind):
         g.destroy()
 
 
+def test_memory_of_tables(gpu):
+    """fw_graph_limit_tables: what is above the bound is given back at once and not taken again, tables without room for sets, sets without
+    room for their weights; the walks are the same."""
+    csr, at = _lists("even")
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    starts = at[np.random.RandomState(3).randint(0, len(at), size=70000)].astype(np.int32)
+    unlimited = (1 << 64) - 1
+
+    def walk(engine, n=70000, **kw):
+        par = gpu.default_params(max_depth=21, seed=6, **kw)
+        ref, _, _ = _oracle.walk(og, _oracle.from_walk_params(par), starts[:3000])
+        for _ in range(8 if kw["app"] == gpu.APP_NODE2VEC else 1):  # sets have to be earned by several calls
+            paths, _ = g.walk(par, starts[:n])
+            assert g.engine()[0] == engine
+            assert (paths[:3000] == ref[:n]).all()
+        return g.engine()[2]
+
+    back = dict(app=gpu.APP_NODE2VEC, p=0.25, q=4.0)
+    try:
+        assert g.engine() == (gpu.ENGINE_NONE, 0, 0)
+        held = walk(gpu.ENGINE_TABLES, app=gpu.APP_DEEPWALK)
+        assert held > 8 * g.E
+        g.limit_tables(held)
+        assert g.engine()[2] == held
+        assert walk(gpu.ENGINE_TABLES, **back) == held          # no room for sets: the lists are searched
+        g.limit_tables(held + 9 * g.E + 70 * V)
+        with_sets = walk(gpu.ENGINE_TABLES, **back)              # nor for their weights
+        assert held + 8 * g.E <= with_sets <= held + 9 * g.E + 70 * V
+        g.limit_tables(unlimited)
+        assert walk(gpu.ENGINE_TABLES, **back) > with_sets
+        g.limit_tables(held - 1)
+        assert g.engine()[2] == 0
+        for _ in range(20):
+            assert walk(gpu.ENGINE_PARK, app=gpu.APP_DEEPWALK) == 0
+        assert walk(gpu.ENGINE_STREAM, n=3000, app=gpu.APP_DEEPWALK) == 0
+        g.limit_tables(unlimited)
+        assert walk(gpu.ENGINE_TABLES, app=gpu.APP_DEEPWALK) == held
+        g.limit_tables(0)
+        assert walk(gpu.ENGINE_PARK, app=gpu.APP_DEEPWALK) == 0
+    finally:
+        g.destroy()
+
+
 def test_changed_biases_on_adopted_arrays(gpu):
     """An adopted graph's owner may change the biases between calls: tables and the sets' weights are made anew."""
     csr, at = _lists("even")
@@ -129,7 +175,7 @@ def test_changed_biases_on_adopted_arrays(gpu):
                 par = gpu.default_params(app=gpu.APP_NODE2VEC, max_depth=21, p=p, q=q, seed=70 + i)
                 ref, _, _ = _oracle.walk(og, _oracle.from_walk_params(par), starts)
                 paths, st = g.walk(par, starts)
-                assert st.launches >= 6  # tables and sets, or tables made anew
+                assert st.launches >= 6 and g.engine()[:2] == (gpu.ENGINE_TABLES, st.launches - 3)  # tables and sets, or tables made anew
                 assert (paths == ref).all()
     finally:
         g.destroy()
@@ -203,7 +249,7 @@ def test_changed_lists_on_adopted_arrays(gpu):
                 par = gpu.default_params(app=app, max_depth=31, p=p, q=q, seed=90 + i)
                 ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(par), starts)
                 paths, st = g.walk(par, starts)
-                assert st.launches >= 6, (i, app, p)
+                assert st.launches >= 6 and g.engine()[0] == gpu.ENGINE_TABLES, (i, app, p)
                 assert (paths == ref).all() and (st.steps, st.sampled_edges) == (steps, edges), (i, app, p)
     finally:
         g.destroy()
