@@ -1132,6 +1132,8 @@ struct ParkBuffers {
     buckets = ctrs = h_ctrs = nullptr;
     tasks = wtasks = qtasks = nullptr;
     tmp = nullptr;
+    cap = 0;
+    n_buckets = 0;
   }
 };
 

@@ -54,6 +54,42 @@ def _adopt(gpu, xadj, adj, w):
     return gpu.Graph(h), arrays
 
 
+def _fill_memory(gpu, leave):
+    """Takes device memory until at most `leave` bytes are free; returns the buffers."""
+    held = []
+    for chunk in (16 << 30, 1 << 30, 32 << 20):
+        while torch.cuda.mem_get_info()[0] > leave + chunk:
+            held.append(gpu.DeviceBuffer(chunk))
+    if torch.cuda.mem_get_info()[0] > leave:
+        held.append(gpu.DeviceBuffer(32 << 20))
+    return held
+
+
+def test_parking_lists_that_do_not_fit(gpu):
+    """fw_walk_batch without room for its parking lists (more than 180 MB) walks without parking, and so does the next call."""
+    g = gpu.Graph.rmat(20, 16, a=0.25, b=0.25, c=0.25, symmetrise=True, seed=3)  # (no list gets rows of its own)
+    n = 2500000
+    starts = np.random.RandomState(2).randint(0, g.V, size=n).astype(np.int32)
+    p = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=5, seed=4, park_threshold=16)
+    held = []
+    try:
+        ref, st = g.walk(p, starts)
+        assert g.engine()[0] == gpu.ENGINE_PARK
+        held = _fill_memory(gpu, 160 << 20)
+        for _ in range(2):
+            paths, st2 = g.walk_batch(p, starts, batch_size=n)
+            assert g.engine()[0] == gpu.ENGINE_STREAM
+            assert (paths == ref).all() and st2.steps == st.steps
+        while held:
+            held.pop().free()
+        paths, _ = g.walk_batch(p, starts, batch_size=n)
+        assert g.engine()[0] == gpu.ENGINE_PARK and (paths == ref).all()
+    finally:
+        for b in held:
+            b.free()
+        g.destroy()
+
+
 @pytest.mark.parametrize("kind", ["even", "uneven"])
 @pytest.mark.parametrize("wg,thr", [(512, 16384), (256, 1024), (1024, 2000), (512, 1 << 30)])
 def test_walks_on_tables(gpu, kind, wg, thr):
