@@ -1676,6 +1676,15 @@ static int table_array(fw_tables* t, T** p, size_t bytes, uint64_t* left) {
   return FW_OK;
 }
 
+// The memory of the graph's tables, for a call that cannot do without it.  False when they held none.
+static bool give_back_tables(fw_graph* g) {
+  if (table_bytes(g) == 0u) return false;
+  g->tables.reset();
+  g->label_tables.reset();
+  g->skip_tables = g->skip_label_tables = kSkipTables;
+  return true;
+}
+
 // Room for the tables of `g`: positions of the regions, work lists, memory (what `t` holds already is used again).  FW_ERR_NOMEM when
 // there is no room for them.
 static int plan_tables(const fw_graph* g, fw_tables* t, hipStream_t stream) {
@@ -2039,6 +2048,7 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
     bool use_pb = false;
     if (park_threshold != INT_MAX) {
       rc = ensure_hub_index(mg, park_threshold);
+      if (rc != FW_OK && give_back_tables(mg)) rc = ensure_hub_index(mg, park_threshold);
       if (rc != FW_OK) return rc;
       // buckets = parked-on vertices x labels must stay a 30-bit count (bucket ids travel in 32-bit record fields)
       use_pb = g->n_hubs > 0 &&
@@ -2047,6 +2057,7 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
     if (use_pb) {
       const int labels = p->app == FW_APP_METAPATH ? p->schema_len : 1;
       pb = cached_park_buffers(mg, (size_t)n, g->n_hubs * labels, two_pass_rows(g, labels));
+      if (!pb && give_back_tables(mg)) pb = cached_park_buffers(mg, (size_t)n, g->n_hubs * labels, two_pass_rows(g, labels));
       use_pb = pb != nullptr;  // no room for the parking lists: walk without parking (same results, one launch)
     }
     FW_TRY(hipEventRecord(ev0, stream));
@@ -2244,6 +2255,12 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     if (rc != FW_OK) return rc;
     free_b += bc->bytes();  // what the last call left with the graph is this call's to use
     batch_size = fw_autobatch_size(free_b, 512, p->max_depth, sync, (uint32_t)n);
+    if (batch_size == 0 && give_back_tables(mg)) {
+      rc = fw_device_mem_info(&free_b, &total_b);
+      if (rc != FW_OK) return rc;
+      free_b += bc->bytes();
+      batch_size = fw_autobatch_size(free_b, 512, p->max_depth, sync, (uint32_t)n);
+    }
     if (batch_size == 0) { fw_set_error("autobatch: not enough free device memory"); return FW_ERR_NOMEM; }
     if (resolve_park_threshold(g, p, (int32_t)batch_size) != INT_MAX) {
       // the reference's rule counts the path matrix only; the parking lists take about 72 bytes per query more
@@ -2258,6 +2275,38 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
   const size_t md = (size_t)p->max_depth;
   const int nbatch = (int)(((size_t)n + bs - 1) / bs);
   const int nbuf = sync || nbatch == 1 ? 1 : 2;  // buffers in flight
+
+  // The buffers stay with the graph (see BatchCache); a failed call gives them up.  What the call cannot do without comes first, and
+  // tables that earlier calls left give way to it; the tables and the parking lists get what is left.
+  auto cleanup = [&]() { release_batch_cache(mg); };
+  auto buffers = [&]() -> int {
+    if (bc->starts_cap < bs * (size_t)nbuf) {
+      if (bc->d_starts) (void)hipFree(bc->d_starts);
+      bc->d_starts = nullptr;
+      bc->starts_cap = 0;
+      FW_HIP(hipMalloc(reinterpret_cast<void**>(&bc->d_starts), bs * (size_t)nbuf * sizeof(int32_t)));
+      bc->starts_cap = bs * (size_t)nbuf;
+    }
+    if (bc->paths_cap < bs * (size_t)nbuf * md) {
+      if (bc->d_paths) (void)hipFree(bc->d_paths);
+      bc->d_paths = nullptr;
+      bc->paths_cap = 0;
+      FW_HIP(hipMalloc(reinterpret_cast<void**>(&bc->d_paths), bs * (size_t)nbuf * md * sizeof(int32_t)));
+      bc->paths_cap = bs * (size_t)nbuf * md;
+    }
+    if (bc->scr_cap < (size_t)nbatch) {
+      if (bc->d_scr) (void)hipFree(bc->d_scr);
+      bc->d_scr = nullptr;
+      bc->scr_cap = 0;
+      FW_HIP(hipMalloc(reinterpret_cast<void**>(&bc->d_scr), sizeof(Scratch) * (size_t)nbatch));
+      bc->scr_cap = (size_t)nbatch;
+    }
+    if (!bc->d_stripes) FW_HIP(hipMalloc(reinterpret_cast<void**>(&bc->d_stripes), FW_TABLE_COUNTER_BYTES));
+    return FW_OK;
+  };
+  rc = buffers();
+  if (rc != FW_OK && give_back_tables(mg)) rc = buffers();
+  if (rc != FW_OK) { cleanup(); return rc; }
 
   const int32_t park_threshold = resolve_park_threshold(g, p, (int32_t)bs);
   for (hipEvent_t& e : mg->call_ev) if (!e) FW_HIP(hipEventCreate(&e));
@@ -2274,26 +2323,11 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
   bool use_pb = false;
   if (!tables && park_threshold != INT_MAX) {
     rc = ensure_hub_index(mg, park_threshold);
+    if (rc != FW_OK && give_back_tables(mg)) rc = ensure_hub_index(mg, park_threshold);
     if (rc != FW_OK) return rc;
     // buckets = parked-on vertices x labels must stay a 30-bit count (bucket ids travel in 32-bit record fields)
     use_pb = g->n_hubs > 0 &&
              (int64_t)g->n_hubs * (p->app == FW_APP_METAPATH ? p->schema_len : 1) <= ((int64_t)1 << 30);
-  }
-  // The buffers stay with the graph (see BatchCache); a failed call gives them up.
-  auto cleanup = [&]() { release_batch_cache(mg); };
-  if (bc->starts_cap < bs * (size_t)nbuf) {
-    if (bc->d_starts) (void)hipFree(bc->d_starts);
-    bc->d_starts = nullptr;
-    bc->starts_cap = 0;
-    FW_TRY(hipMalloc(reinterpret_cast<void**>(&bc->d_starts), bs * (size_t)nbuf * sizeof(int32_t)));
-    bc->starts_cap = bs * (size_t)nbuf;
-  }
-  if (bc->paths_cap < bs * (size_t)nbuf * md) {
-    if (bc->d_paths) (void)hipFree(bc->d_paths);
-    bc->d_paths = nullptr;
-    bc->paths_cap = 0;
-    FW_TRY(hipMalloc(reinterpret_cast<void**>(&bc->d_paths), bs * (size_t)nbuf * md * sizeof(int32_t)));
-    bc->paths_cap = bs * (size_t)nbuf * md;
   }
   if (use_pb) {
     const int n_buckets = g->n_hubs * (p->app == FW_APP_METAPATH ? p->schema_len : 1);
@@ -2301,25 +2335,21 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     for (int i = 0; i < nbuf && use_pb; ++i) {
       ParkBuffers& pb = bc->pbs[i];
       if (pb.cap >= bs && pb.n_buckets == n_buckets && pb.rows_cap >= rows) continue;
-      pb.release();
-      if (pb.alloc(bs, n_buckets, rows) != FW_OK) {  // no room for the parking lists: walk without parking (same results)
-        bc->pbs[0].release();
+      auto lists = [&]() {
+        pb.release();
+        const int r = pb.alloc(bs, n_buckets, rows);
+        if (r != FW_OK) (void)hipGetLastError();
+        return r;
+      };
+      if (lists() != FW_OK && (!give_back_tables(mg) || lists() != FW_OK)) {  // no room for the parking lists: walk without
+        bc->pbs[0].release();                                                   // parking (same results)
         bc->pbs[1].release();
         use_pb = false;
-        (void)hipGetLastError();
       }
     }
   }
-  if (bc->scr_cap < (size_t)nbatch) {
-    if (bc->d_scr) (void)hipFree(bc->d_scr);
-    bc->d_scr = nullptr;
-    bc->scr_cap = 0;
-    FW_TRY(hipMalloc(reinterpret_cast<void**>(&bc->d_scr), sizeof(Scratch) * (size_t)nbatch));
-    bc->scr_cap = (size_t)nbatch;
-  }
   if (!tables) FW_TRY(hipMemset(bc->d_scr, 0, sizeof(Scratch) * (size_t)nbatch));
   if (tables) {  // the batches share one set of counters
-    if (!bc->d_stripes) FW_TRY(hipMalloc(reinterpret_cast<void**>(&bc->d_stripes), FW_TABLE_COUNTER_BYTES));
     if (!mg->call_result) FW_TRY(hipHostMalloc(reinterpret_cast<void**>(&mg->call_result), 64, hipHostMallocDefault));
     if ((rc = fw_table_begin(bc->d_stripes, &bc->d_scr->dispenser, (uint32_t)(sizeof(Scratch) / 4u * (size_t)nbatch), nullptr)) != FW_OK) { cleanup(); return rc; }
   }

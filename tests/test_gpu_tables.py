@@ -65,6 +65,46 @@ def _fill_memory(gpu, leave):
     return held
 
 
+def test_batches_come_before_tables(gpu):
+    """fw_walk_batch: tables give way to the path matrices of the call, those of earlier calls too, and to the parking lists of a later one."""
+    g = gpu.Graph.rmat(20, 16, a=0.25, b=0.25, c=0.25, symmetrise=True, seed=3)
+    n = 2500000
+    starts = np.random.RandomState(2).randint(0, g.V, size=n).astype(np.int32)
+    big = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=81, seed=4)  # 820 MB
+    held = []
+    try:
+        g.limit_tables(0)
+        ref, st = g.walk(big, starts)
+        g.limit_tables((1 << 64) - 1)
+        for tables in (False, True):  # whether the graph has some when the batch comes
+            if tables:
+                for _ in range(40):
+                    g.walk(big, starts[:70000])
+                assert g.engine()[0] == gpu.ENGINE_TABLES
+            assert (g.engine()[2] > 300 << 20) == tables
+            held = _fill_memory(gpu, 900 << 20 if not tables else 700 << 20)
+            paths, st2 = g.walk_batch(big, starts, batch_size=n)
+            assert g.engine()[0] == gpu.ENGINE_STREAM and g.engine()[2] == 0
+            assert (paths == ref).all() and st2.steps == st.steps
+            while held:
+                held.pop().free()
+            g.destroy()  # (with the batch's buffers)
+            g = gpu.Graph.rmat(20, 16, a=0.25, b=0.25, c=0.25, symmetrise=True, seed=3)
+        for _ in range(40):
+            g.walk(big, starts[:70000])
+        assert g.engine()[0] == gpu.ENGINE_TABLES
+        short = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=5, seed=4, park_threshold=16)
+        held = _fill_memory(gpu, 300 << 20)  # (the parking index takes some 20 MB and, where it fits, 270, the lists 200 and more)
+        paths, _ = g.walk_batch(short, starts, batch_size=n)
+        assert g.engine()[::2] == (gpu.ENGINE_PARK, 0)
+        short.park_threshold = -1
+        assert (paths == g.walk_batch(short, starts, batch_size=n)[0]).all()
+    finally:
+        for b in held:
+            b.free()
+        g.destroy()
+
+
 def test_parking_lists_that_do_not_fit(gpu):
     """fw_walk_batch without room for its parking lists (more than 180 MB) walks without parking, and so does the next call."""
     g = gpu.Graph.rmat(20, 16, a=0.25, b=0.25, c=0.25, symmetrise=True, seed=3)  # (no list gets rows of its own)
