@@ -1734,7 +1734,7 @@ static bool sets_for_call(const fw_graph* g, const fw_walk_params* p, fw_tables*
   const bool back = p->p < 1.0f && p->p < p->q;  // the return edge is a component of its own
   if (p->app != FW_APP_NODE2VEC || (p->q == 1.0f && !back)) return false;
   const bool want_weights = back && !t->have_weights;
-  if (t->have_sets && !want_weights) return p->time_kernels != 0;
+  if (t->have_sets && !want_weights) return false;
   if (!t->have_sets) {
     const double ms = all_steps * 0.05e-6 > steps * 0.004 ? all_steps * 0.05e-6 : steps * 0.004;
     t->search_ms = (g->borrowed ? 0.0 : t->search_ms) + ms;  // (an adopted graph's sets last one call)
@@ -1784,52 +1784,49 @@ static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n
   if (t && (t->hub_threshold != p->hub_threshold || t->nw_shift != nw_shift || t->labels.n != set.n ||
             memcmp(t->labels.label, set.label, sizeof(set.label)) != 0))
     t = nullptr;  // another schema or granularity: one set per graph
-  if (t && !g->borrowed && p->time_kernels == 0) {
+  if (t && !g->borrowed) {
     *out = t;
     return FW_OK;
   }
-  if (!t || g->borrowed) {
-    const double steps = (double)(p->max_depth - 1);
-    double ms = steps * kStepLatencyMs;
-    if (steps * (double)n >= 1.0e6) {
-      double mean = 0.0;
-      const int rc = mean_list_length(g, &mean);
-      if (rc != FW_OK) return rc;
-      const double stream_ms = steps * (double)n * mean * 4.0 / kStreamBytesPerMs, parked_ms = steps * (double)n * kParkedStepMs;
-      const double lists_ms = stream_ms < parked_ms ? stream_ms : parked_ms;
-      if (ms < lists_ms) ms = lists_ms;
-    }
-    const double make_ms = kLabelMakeEdgeMs * (double)g->E + kMakeFixedMs;
-    if (g->hub_index == nullptr && resolve_park_threshold(g, p, n) != INT_MAX) ms += kParkIndexEdgeMs * (double)g->E;
-    if ((g->borrowed ? 0.0 : g->label_ms) + ms < make_ms) return FW_OK;
-  }
-  if (!t || g->borrowed) {
-    if (!t) {
-      g->label_tables.reset(new (std::nothrow) fw_tables);
-      t = g->label_tables.get();
-      if (!t) return FW_OK;
-      t->hub_threshold = p->hub_threshold;
-      t->nw_shift = nw_shift;
-      t->labels = set;
-    }
-    const int rc = plan_tables(g, t, stream);
-    if (rc != FW_OK) g->label_tables.reset();  // nothing half made stays
-    if (rc == FW_ERR_NOMEM) {
-      g->skip_label_tables = kSkipTables;
-      return FW_OK;
-    }
+  int rc = FW_OK;
+  const double steps = (double)(p->max_depth - 1);
+  double ms = steps * kStepLatencyMs;
+  if (steps * (double)n >= 1.0e6) {
+    double mean = 0.0;
+    rc = mean_list_length(g, &mean);
     if (rc != FW_OK) return rc;
+    const double stream_ms = steps * (double)n * mean * 4.0 / kStreamBytesPerMs, parked_ms = steps * (double)n * kParkedStepMs;
+    const double lists_ms = stream_ms < parked_ms ? stream_ms : parked_ms;
+    if (ms < lists_ms) ms = lists_ms;
   }
+  const double make_ms = kLabelMakeEdgeMs * (double)g->E + kMakeFixedMs;
+  if (g->hub_index == nullptr && resolve_park_threshold(g, p, n) != INT_MAX) ms += kParkIndexEdgeMs * (double)g->E;
+  if ((g->borrowed ? 0.0 : g->label_ms) + ms < make_ms) return FW_OK;
+  if (!t) {
+    g->label_tables.reset(new (std::nothrow) fw_tables);
+    t = g->label_tables.get();
+    if (!t) return FW_OK;
+    t->hub_threshold = p->hub_threshold;
+    t->nw_shift = nw_shift;
+    t->labels = set;
+  }
+  rc = plan_tables(g, t, stream);
+  if (rc != FW_OK) g->label_tables.reset();  // nothing half made stays
+  if (rc == FW_ERR_NOMEM) {
+    g->skip_label_tables = kSkipTables;
+    return FW_OK;
+  }
+  if (rc != FW_OK) return rc;
   auto make = [&]() -> int {
     if (ev_start) FW_HIP(hipEventRecord(ev_start, stream));
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev0, stream));
-    const int rc = fw_label_tables_make(g, t, stream, launches);
-    if (rc != FW_OK) return rc;
+    const int made = fw_label_tables_make(g, t, stream, launches);
+    if (made != FW_OK) return made;
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
     FW_HIP(hipStreamSynchronize(stream));  // (the batch entry walks on other streams)
     return FW_OK;
   };
-  const int rc = make();
+  rc = make();
   if (rc != FW_OK) {
     g->label_tables.reset();
     return rc;
@@ -1858,9 +1855,9 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
   const uint32_t nw_shift = p->wg_threads == 256 ? 2u : (p->wg_threads == 512 ? 3u : 4u);
   fw_tables* t = g->tables.get();
   if (t && (t->hub_threshold != p->hub_threshold || t->nw_shift != nw_shift)) t = nullptr;  // another granularity: one set per graph
-  const bool make_tables = !t || g->borrowed || p->time_kernels != 0;  // (a call that wants the split of its time makes them anew)
+  const bool make_tables = !t || g->borrowed;
   double steps = (double)(p->max_depth - 1);
-  if (!t || g->borrowed) {
+  if (make_tables) {
     if (p->app == FW_APP_PPR && p->tp > 0.0f && 1.0 / (double)p->tp < steps) steps = 1.0 / (double)p->tp;
     double ms = steps * kStepLatencyMs;
     if (steps * (double)n >= 1.0e6) {  // (a smaller first call costs little more than asking: 0.04 ms)
@@ -1873,7 +1870,7 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     // (an adopted graph's tables last one call: only its own work can pay for them)
     if ((g->borrowed ? 0.0 : g->streamed_ms) + ms < kMakeMargin * (17.0 * (double)g->E / kMakeBytesPerMs + kMakeFixedMs)) return FW_OK;
   }
-  if (!t || g->borrowed) {
+  if (make_tables) {
     if (!t) {
       g->tables.reset(new (std::nothrow) fw_tables);
       t = g->tables.get();
@@ -2073,9 +2070,9 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
   if (!tables) FW_TRY(hipMemcpy(&h, d_scr, sizeof(h), hipMemcpyDeviceToHost));
   if (tables) {
     memcpy(h.counters, mg->call_result, sizeof(h.counters));
-    if (p->time_kernels != 0) {  // the split: the making of the tables, and the walk
+    if (p->time_kernels != 0) {  // the split: the making of the tables, where this call made some, and the walk
       float make_ms = 0.0f;
-      FW_TRY(hipEventElapsedTime(&make_ms, mg->call_ev[2], mg->call_ev[3]));
+      if (mg->last_made != 0) FW_TRY(hipEventElapsedTime(&make_ms, mg->call_ev[2], mg->call_ev[3]));
       times.hub_ms = make_ms;
       times.walk_ms = (double)ms - (double)make_ms;  // exact: both are floats
     }

@@ -125,8 +125,8 @@ typedef struct {
   /* per-kernel breakdown of kernel_ms / steps / sampled_edges (hub parking splits a pass over two kernels) */
   double walk_kernel_ms;      /* sum over fw_walk_zprs launches (with fw_walk_params.time_kernels, else 0) */
   double hub_kernel_ms;       /* sum over the hub launches of every round: fw_hub_scan, fw_hub_batch, fw_hub_quad
-                                 (with fw_walk_params.time_kernels, else 0); a walk on list tables: the making of the
-                                 tables, which a call with time_kernels does anew */
+                                 (with fw_walk_params.time_kernels, else 0); a walk on list tables: the making of
+                                 the tables, 0 in a call that found them made */
   uint64_t hub_steps;         /* steps taken in the hub launches (included in steps); a walk on list tables: steps
                                  from vertices above the parking degree of the batch */
   uint64_t hub_sampled_edges; /* their source degrees (included in sampled_edges) */

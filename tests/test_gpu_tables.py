@@ -233,6 +233,30 @@ def test_memory_of_tables(gpu):
         g.destroy()
 
 
+def test_kernel_times_leave_the_tables(gpu):
+    """A call that asks for the split of its time walks on the tables that are there, like any other: nothing is made anew."""
+    csr, at = _lists("even")
+    g = gpu.Graph.from_csr(*csr)
+    starts = at[np.random.RandomState(3).randint(0, len(at), size=70000)].astype(np.int32)
+    try:
+        for app in (gpu.APP_DEEPWALK, gpu.APP_NODE2VEC):
+            par = gpu.default_params(app=app, max_depth=21, seed=6, p=0.25, q=4.0)
+            for _ in range(8):  # sets have to be earned by several calls
+                plain, _ = g.walk(par, starts)
+            assert g.engine()[:2] == (gpu.ENGINE_TABLES, 0)
+            par.time_kernels = 1
+            paths, st = g.walk(par, starts)
+            assert g.engine()[:2] == (gpu.ENGINE_TABLES, 0) and st.launches == 3
+            assert st.hub_kernel_ms == 0.0 and st.walk_kernel_ms == st.kernel_ms > 0.0
+            assert (paths == plain).all()
+            paths, st = g.walk_batch(par, starts, batch_size=30000)
+            assert g.engine()[:2] == (gpu.ENGINE_TABLES, 0)
+            assert st.hub_kernel_ms == 0.0 and st.walk_kernel_ms == st.kernel_ms > 0.0
+            assert (paths == plain).all()
+    finally:
+        g.destroy()
+
+
 def test_changed_biases_on_adopted_arrays(gpu):
     """An adopted graph's owner may change the biases between calls: tables and the sets' weights are made anew."""
     csr, at = _lists("even")
