@@ -1597,17 +1597,35 @@ static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params*
 // ---- list tables: when, and making them ---------------------------------------------------------------------
 //
 // A walk on list tables reads three or four blocks of memory per step, whatever the lists' lengths; without them a step
-// reads its list.  Making them reads and writes about 17 bytes per edge and allocates, so they are made once the calls on a
-// graph have spent without them (measured) or are about to spend (estimated) what they cost: a serving loop of small calls gets
-// them after a call or two and never pays more than about twice what it would have.
-// Estimates in milliseconds: lists stream at 6.5 TB/s, a step of a walk that finds the chip idle takes 2 us; the tables are
-// made at 4 TB/s (17 bytes per edge: 5.8 ms on 521 M edges, 0.24 ms of allocations and launches on a small graph), with
-// half as much again asked for before they are.
+// reads its list, or shares it with the others that are parked there.  The tables are made once the calls on a graph have spent without
+// them (measured) or are about to spend (estimated) a quarter more than making them takes: a first call makes them only if it gains by
+// that itself, and a loop of small calls gets them after a few and never pays more than about twice what it would have.
+//
+// What a call takes without tables: lists stream at 6.5 TB/s; a step of a walk that finds the chip idle takes 2 us; a call that
+// parks takes 0.05 ms a round (one per step of its longest walks) and 0.1 ns per step asked for (R-MAT 14 to 26, 100,000 to 16.8 M
+// queries: 0.07 to 0.3; DeepWalk R-MAT 24 0.09, MetaPath R-MAT 26 0.14), and the first one makes the parking index, 17 ps
+// per edge (R-MAT 22 28, R-MAT 24 15.5, R-MAT 26 19).
 constexpr double kStreamBytesPerMs = 6.5e9;
 constexpr double kStepLatencyMs = 0.002;
-constexpr double kMakeBytesPerMs = 4.0e9;
-constexpr double kMakeFixedMs = 0.25;
-constexpr double kMakeMargin = 1.5;
+constexpr double kParkedRoundMs = 0.05;
+constexpr double kParkedStepMs = 0.1e-6;
+constexpr double kParkIndexEdgeMs = 17e-9;
+// What making tables takes: the bytes it moves at the rate the kernels reach, and 0.3 ms of launches, waits and small
+// allocations; arrays of megabytes are mapped by the driver, 0.4 ms more in all.  List tables hold about 8 bytes per edge, 64 per vertex (regions are
+// whole blocks of 128 bytes) and 20 of records and positions; measured against this estimate: R-MAT 24 symmetrised 7.4 ms (6.9),
+// R-MAT 23 with 134 M edges 2.65 (2.5), with 17 M edges 1.2 (1.2), R-MAT 17 with 2.1 M edges 0.72 (0.74), R-MAT 14 0.25 to 0.38 (0.3).
+// Label tables hold 4 bytes per edge and 36 per vertex: R-MAT 26 18.3 ms (16.5).
+constexpr double kListMakeBytesPerMs = 1.6e9;
+constexpr double kLabelMakeBytesPerMs = 0.97e9;
+constexpr double kMakeFixedMs = 0.3;
+constexpr double kMakeMapMs = 0.4;
+constexpr double kMakeMapBytes = 8.0e6;
+constexpr double kMakeMargin = 1.25;
+
+// Making something that moves `moved` bytes and allocates `held` of them.
+static double make_estimate_ms(double held, double moved, double bytes_per_ms) {
+  return kMakeFixedMs + (held > kMakeMapBytes ? kMakeMapMs : 0.0) + moved / bytes_per_ms;
+}
 
 __global__ void fw_square_sum_kernel(const uint32_t* __restrict__ xadj, int32_t V, double* sum) {
   const int stride = gridDim.x * blockDim.x;
@@ -1639,6 +1657,30 @@ static int mean_list_length(fw_graph* g, double* out) {
     g->mean_list = sum / (double)g->E;
   }
   *out = g->mean_list;
+  return FW_OK;
+}
+
+// What a call of n queries takes without tables; steps: of one walk, on average.
+static int lists_estimate_ms(fw_graph* g, const fw_walk_params* p, int32_t n, double steps, double* out) {
+  double ms = steps * kStepLatencyMs;
+  if (steps * (double)n >= 1.0e6) {  // (a smaller first call costs little more than asking: 0.04 ms)
+    double mean = 0.0;
+    const int rc = mean_list_length(g, &mean);
+    if (rc != FW_OK) return rc;
+    double lists_ms = steps * (double)n * mean * 4.0 / kStreamBytesPerMs;
+    if (resolve_park_threshold(g, p, n) != INT_MAX) {
+      double rounds = (double)(p->max_depth - 1);
+      if (p->app == FW_APP_PPR && p->tp > 0.0f && p->tp < 1.0f) {  // until the last of n walks stops
+        const double longest = -log((double)n) / log1p(-(double)p->tp);
+        if (longest < rounds) rounds = longest;
+      }
+      const double parked_ms = rounds * kParkedRoundMs + steps * (double)n * kParkedStepMs;
+      if (parked_ms < lists_ms) lists_ms = parked_ms;
+      if (g->hub_index == nullptr) lists_ms += kParkIndexEdgeMs * (double)g->E;
+    }
+    if (ms < lists_ms) ms = lists_ms;
+  }
+  *out = ms;
   return FW_OK;
 }
 
@@ -1753,15 +1795,7 @@ static bool sets_for_call(const fw_graph* g, const fw_walk_params* p, fw_tables*
   return t->sets != nullptr;  // (without weights the return edge is searched for)
 }
 
-// MetaPath's tables, for the labels of the call's schema; otherwise as tables_for_call below.  Making them takes
-// 15 ps per edge (16 ms on R-MAT 26, 1.07 G edges).  A walk without them shares its lists through parking, which on R-MAT 26 took 7.1 ms
-// for 10^7 queries of 5 steps, most of which end before: 0.13 ns per step asked for; less where all lists together are short.  The first
-// one that parks makes the parking index as well (10 to 16 ps per edge), so a large first call is better off with the tables: 20 ms
-// on R-MAT 26 against 27.
-constexpr double kParkedStepMs = 0.13e-6;
-constexpr double kParkIndexEdgeMs = 10e-9;
-constexpr double kLabelMakeEdgeMs = 15e-9;
-
+// MetaPath's tables, for the labels of the call's schema; otherwise as tables_for_call below.
 static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipStream_t stream, const fw_tables** out,
                                  int* launches, hipEvent_t ev_start, hipEvent_t ev0, hipEvent_t ev1) {
   if (p->park_threshold != 0 || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) || g->host_edges || g->table_limit == 0u ||
@@ -1788,20 +1822,13 @@ static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n
     *out = t;
     return FW_OK;
   }
-  int rc = FW_OK;
   const double steps = (double)(p->max_depth - 1);
-  double ms = steps * kStepLatencyMs;
-  if (steps * (double)n >= 1.0e6) {
-    double mean = 0.0;
-    rc = mean_list_length(g, &mean);
-    if (rc != FW_OK) return rc;
-    const double stream_ms = steps * (double)n * mean * 4.0 / kStreamBytesPerMs, parked_ms = steps * (double)n * kParkedStepMs;
-    const double lists_ms = stream_ms < parked_ms ? stream_ms : parked_ms;
-    if (ms < lists_ms) ms = lists_ms;
-  }
-  const double make_ms = kLabelMakeEdgeMs * (double)g->E + kMakeFixedMs;
-  if (g->hub_index == nullptr && resolve_park_threshold(g, p, n) != INT_MAX) ms += kParkIndexEdgeMs * (double)g->E;
-  if ((g->borrowed ? 0.0 : g->label_ms) + ms < make_ms) return FW_OK;
+  double ms = 0.0;
+  int rc;
+  if ((rc = lists_estimate_ms(g, p, n, steps, &ms)) != FW_OK) return rc;
+  const double held = 4.0 * (double)g->E + 36.0 * (double)g->V;
+  const double make_ms = make_estimate_ms(t ? 0.0 : held, held + 8.0 * (double)g->E, kLabelMakeBytesPerMs);
+  if ((g->borrowed ? 0.0 : g->label_ms) + ms < kMakeMargin * make_ms) return FW_OK;
   if (!t) {
     g->label_tables.reset(new (std::nothrow) fw_tables);
     t = g->label_tables.get();
@@ -1859,16 +1886,13 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
   double steps = (double)(p->max_depth - 1);
   if (make_tables) {
     if (p->app == FW_APP_PPR && p->tp > 0.0f && 1.0 / (double)p->tp < steps) steps = 1.0 / (double)p->tp;
-    double ms = steps * kStepLatencyMs;
-    if (steps * (double)n >= 1.0e6) {  // (a smaller first call costs little more than asking: 0.04 ms)
-      double mean = 0.0;
-      const int rc = mean_list_length(g, &mean);
-      if (rc != FW_OK) return rc;
-      const double stream_ms = steps * (double)n * mean * 4.0 / kStreamBytesPerMs;
-      if (ms < stream_ms) ms = stream_ms;
-    }
+    double ms = 0.0;
+    const int rc = lists_estimate_ms(g, p, n, steps, &ms);
+    if (rc != FW_OK) return rc;
+    const double held = 8.0 * (double)g->E + 84.0 * (double)g->V;
+    const double make_ms = make_estimate_ms(t ? 0.0 : held, held + 8.0 * (double)g->E, kListMakeBytesPerMs);
     // (an adopted graph's tables last one call: only its own work can pay for them)
-    if ((g->borrowed ? 0.0 : g->streamed_ms) + ms < kMakeMargin * (17.0 * (double)g->E / kMakeBytesPerMs + kMakeFixedMs)) return FW_OK;
+    if ((g->borrowed ? 0.0 : g->streamed_ms) + ms < kMakeMargin * make_ms) return FW_OK;
   }
   if (make_tables) {
     if (!t) {

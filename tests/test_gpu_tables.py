@@ -306,6 +306,30 @@ def test_small_calls_on_adopted_arrays(gpu):
         g.destroy()
 
 
+@pytest.mark.parametrize("vertices,hub,n,length,engine", [(300000, 23000, 50000, 20, "STREAM"), (1000000, 100000, 70000, 15, "PARK"),
+                                                          (1000000, 100000, 300000, 40, "TABLES")])
+def test_first_call_makes_tables_only_for_itself(gpu, vertices, hub, n, length, engine):
+    """A first call that takes less without tables than making them takes (0.7 ms of its 0.9, 0.9 ms of its 1.0 in rounds of the
+    parking pipeline) goes without; one that takes several times as much makes them."""
+    rng = np.random.RandomState(vertices)
+    deg = np.full(vertices, 3, dtype=np.int64)
+    deg[rng.permutation(vertices)[:2]] = hub
+    xadj = np.zeros(vertices + 1, dtype=np.uint32)
+    np.cumsum(deg, out=xadj[1:])
+    adj = rng.randint(0, vertices, size=int(xadj[-1])).astype(np.int32)
+    w = (1.0 + 99.0 * rng.random_sample(len(adj))).astype(np.float32)
+    g = gpu.Graph.from_csr(xadj, adj, w)
+    try:
+        par = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=length + 1, seed=4)
+        starts = rng.randint(0, vertices, size=n).astype(np.int32)
+        paths, _ = g.walk(par, starts)
+        assert g.engine()[0] == getattr(gpu, "ENGINE_" + engine)
+        ref, _, _ = _oracle.walk(_oracle.Graph(xadj, adj, w), _oracle.from_walk_params(par), starts[:2000])
+        assert (paths[:2000] == ref).all()
+    finally:
+        g.destroy()
+
+
 def test_two_granularities_in_turn(gpu):
     """One set of tables per graph: calls of two granularities in turn replace it only after lists have been streamed for as long as
     making it takes, not in every call."""
