@@ -1768,20 +1768,33 @@ static int plan_tables(const fw_graph* g, fw_tables* t, hipStream_t stream) {
 }
 
 // Whether this call makes the hash sets of node2vec's adjacency tests, and for the return edge their weights (the memory is there
-// then).  They are made once the calls' searches
-// have cost, or are about to cost, half as much again as making them: a search that finds the chip busy costs 0.05 ns (five
-// scattered reads at 51 G/s, half of the tests undecided; R-MAT 24: 41 ms of 709 M steps), one in a chain of a few walkers 4 us, and the sets take
-// 0.2 ms and 20 bytes per edge at 2.5 TB/s.
-static bool sets_for_call(const fw_graph* g, const fw_walk_params* p, fw_tables* t, double all_steps, double steps) {
+// then).  They are made once the calls' searches have cost, or are about to cost, a quarter more than making them.
+// A search that finds the chip busy costs 0.03 ns (R-MAT 24: 41 ms of 1.34 G steps asked for, R-MAT 23 0.5 of 20 M), a step of a few
+// walkers 4 us, and a q above 1 takes about q trials.  Making takes 0.2 ms per new array and moves 12 bytes per edge and 64 per vertex, with weights
+// as much again, at 0.75 TB/s, and reads a long list once per 8192 entries: R-MAT 24 symmetrised 10.9 ms (estimated 10.6), R-MAT
+// 23 with 268 M edges 4.8 (5.3), R-MAT 20 with 33 M 0.73 (0.83), with 4 M 0.25 (0.36).
+constexpr double kSearchMs = 0.03e-6;
+constexpr double kSearchStepMs = 0.004;
+constexpr double kSetMakeBytesPerMs = 0.75e9;
+constexpr double kSetMakeFixedMs = 0.2;
+constexpr double kSetRereadBytesPerMs = 3.0e9;
+
+static bool sets_for_call(fw_graph* g, const fw_walk_params* p, fw_tables* t, double all_steps, double steps) {
   const bool back = p->p < 1.0f && p->p < p->q;  // the return edge is a component of its own
   if (p->app != FW_APP_NODE2VEC || (p->q == 1.0f && !back)) return false;
   const bool want_weights = back && !t->have_weights;
   if (t->have_sets && !want_weights) return false;
-  if (!t->have_sets) {
-    const double ms = all_steps * 0.05e-6 > steps * 0.004 ? all_steps * 0.05e-6 : steps * 0.004;
-    t->search_ms = (g->borrowed ? 0.0 : t->search_ms) + ms;  // (an adopted graph's sets last one call)
-    if (t->search_ms < kMakeMargin * (20.0 * (double)g->E / 2.5e9 + 0.2)) return false;
-  }
+  // (sets that are there have to be made again with their weights; then it is the searches for the return edge that pay)
+  const double trials = !t->have_sets && p->q > 1.0f ? (double)p->q : 1.0;
+  const double busy_ms = all_steps * trials * kSearchMs, chain_ms = steps * kSearchStepMs;
+  t->search_ms = (g->borrowed ? 0.0 : t->search_ms) + (busy_ms > chain_ms ? busy_ms : chain_ms);  // (an adopted graph's sets last one call)
+  const double arrays = (t->sets == nullptr ? 1.0 : 0.0) + (want_weights && t->set_weights == nullptr ? 1.0 : 0.0);
+  double make_ms = arrays * kSetMakeFixedMs + (want_weights ? 2.0 : 1.0) * (12.0 * (double)g->E + 64.0 * (double)g->V) / kSetMakeBytesPerMs;
+  if (t->search_ms < kMakeMargin * make_ms) return false;
+  double mean = 0.0;
+  if (mean_list_length(g, &mean) != FW_OK) return false;
+  make_ms += 4.0 * (double)g->E * mean / 8192.0 / kSetRereadBytesPerMs;
+  if (t->search_ms < kMakeMargin * make_ms) return false;
   if (t->skip_sets > 0) {
     --t->skip_sets;
     return false;
@@ -1929,6 +1942,7 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
       if ((rc = fw_sets_make(g, t, stream, launches)) != FW_OK) return rc;
       t->have_sets = true;
       t->have_weights = t->set_weights != nullptr;
+      t->search_ms = 0.0;
     }
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
     if (!make_tables) return FW_OK;

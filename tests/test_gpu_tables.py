@@ -189,6 +189,29 @@ def test_node2vec_on_hash_sets(gpu, kind):
         g.destroy()
 
 
+def test_weights_of_sets_have_to_be_earned(gpu):
+    """Sets that are there are made again with their entries' weights only once the searches for the return edge have cost that: a small
+    call with p < 1 searches the lists, a loop of them gets the weights."""
+    csr, at = _lists("even")
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    starts = at[np.random.RandomState(3).randint(0, len(at), size=70000)].astype(np.int32)
+    try:
+        for _ in range(8):
+            g.walk(gpu.default_params(app=gpu.APP_NODE2VEC, max_depth=21, seed=6, p=2.0, q=0.5), starts)
+        sets = g.engine()
+        par = gpu.default_params(app=gpu.APP_NODE2VEC, max_depth=21, seed=7, p=0.25, q=4.0)
+        ref, _, _ = _oracle.walk(og, _oracle.from_walk_params(par), starts[:20])
+        for i in range(20):
+            paths, _ = g.walk(par, starts[:20])
+            assert (paths == ref).all()
+            if i == 0:
+                assert g.engine() == sets
+        assert g.engine()[2] > sets[2]
+    finally:
+        g.destroy()
+
+
 def test_memory_of_tables(gpu):
     """fw_graph_limit_tables: what is above the bound is given back at once and not taken again, tables without room for sets, sets without
     room for their weights; the walks are the same."""
