@@ -1579,18 +1579,17 @@ static TrafficModel traffic_model(const fw_walk_params* p, int32_t n, bool parke
 }
 
 
-// The same for a walk on list tables: a step reads its vertex's record, a row and a lane of the list's table; path entries leave in
-// lines.  made: the tables were made in this call.
-static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params* p, int32_t n, bool made, bool sets, uint64_t steps) {
+// The same for a walk on list tables; path entries leave in lines.  A step reads its vertex's record, a row and a lane of the
+// list's table, for MetaPath the record and one neighbour; node2vec tests the accepted neighbour of all but a walk's first step in N(prev).  node2vec's
+// turned-down trials are not counted (a row, a lane and a test each), nor the sums of lists of several groups, so the model is a lower bound.
+static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params* p, int32_t n, bool sets, uint64_t steps) {
   TrafficModel m;
-  m.scattered_reads = 3 * steps + (uint64_t)n;
-  if (p->app == FW_APP_NODE2VEC) m.scattered_reads += (sets ? 1 : 4) * steps;  // the tests in N(prev): a hash set, or searches
+  m.scattered_reads = (p->app == FW_APP_METAPATH ? 2 : 3) * steps + (uint64_t)n;
+  if (p->app == FW_APP_NODE2VEC && steps > (uint64_t)n) m.scattered_reads += (sets ? 1 : 4) * (steps - (uint64_t)n);  // a hash set, or a search
   m.scattered_writes = steps / 16u + 2u * (uint64_t)n;            // whole lines, the row's first and last entries
   m.record_bytes = 4 * (uint64_t)n + 4 * (uint64_t)n * (uint64_t)p->max_depth;
-  if (made) {
-    m.list_bytes = 8 * g->E;
-    m.record_bytes += 9 * g->E + 24 * (uint64_t)g->V;
-  }
+  m.list_bytes = g->made_read;
+  m.record_bytes += g->made_written;
   return m;
 }
 
@@ -1862,6 +1861,8 @@ static int label_tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev0, stream));
     const int made = fw_label_tables_make(g, t, stream, launches);
     if (made != FW_OK) return made;
+    g->made_read += 8 * g->E + 4 * (uint64_t)g->V;
+    g->made_written += 4 * g->E + 32 * (uint64_t)g->V + t->data_bytes;
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
     FW_HIP(hipStreamSynchronize(stream));  // (the batch entry walks on other streams)
     return FW_OK;
@@ -1882,6 +1883,7 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
                            int* launches, hipEvent_t ev_start, hipEvent_t ev0, hipEvent_t ev1) {
   *out = nullptr;
   *launches = 0;
+  g->made_read = g->made_written = 0u;
   // an explicit parking degree asks for the parking pipeline, a negative one for walkers that stream their lists
   if (p->app == FW_APP_METAPATH) return label_tables_for_call(g, p, n, stream, out, launches, ev_start, ev0, ev1);
   if (p->park_threshold != 0 || (p->sampler != FW_SAMPLER_ZPRS && p->sampler != FW_SAMPLER_DPRS) ||
@@ -1937,12 +1939,17 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     if (make_tables) {
       FW_HIP(hipMemsetAsync(t->flag, 0, sizeof(uint32_t), stream));
       if ((rc = fw_table_make(g, t, stream, launches)) != FW_OK) return rc;
+      g->made_read += 8 * g->E + 4 * (uint64_t)g->V;
+      g->made_written += 16 * (uint64_t)g->V + t->data_bytes;
     }
     if (make_sets) {
       if ((rc = fw_sets_make(g, t, stream, launches)) != FW_OK) return rc;
       t->have_sets = true;
       t->have_weights = t->set_weights != nullptr;
       t->search_ms = 0.0;
+      const uint64_t arrays = t->have_weights ? 2u : 1u;
+      g->made_read += arrays * 4 * g->E + 16 * (uint64_t)g->V;
+      g->made_written += arrays * 64u * (fw_set_first((uint32_t)g->E, (uint32_t)g->V) + 1u);
     }
     if (p->time_kernels != 0) FW_HIP(hipEventRecord(ev1, stream));
     if (!make_tables) return FW_OK;
@@ -2129,7 +2136,7 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
     stats->hub_kernel_ms = times.hub_ms;
     stats->hub_steps = h.counters[2];
     stats->hub_sampled_edges = h.counters[3];
-    const TrafficModel tm = tables ? table_traffic_model(g, p, n, launches > 3, tables->have_sets, stats->steps)
+    const TrafficModel tm = tables ? table_traffic_model(g, p, n, tables->have_sets, stats->steps)
                                    : traffic_model(p, n, launches > 1, park_threshold, g->adj_hub != nullptr, h.counters[0],
                                                    h.counters[1], h.counters[2], times);
     stats->requested_bytes = tm.total();
@@ -2479,7 +2486,7 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     stats->grid = grid_used;
     stats->walk_kernel_ms = stats->hub_steps == 0 && make_launches == 0 ? kernel_ms : times.walk_ms;  // the split: with time_kernels only
     stats->hub_kernel_ms = times.hub_ms;
-    const TrafficModel tm = tables ? table_traffic_model(g, p, n, make_launches != 0, tables->have_sets, stats->steps)
+    const TrafficModel tm = tables ? table_traffic_model(g, p, n, tables->have_sets, stats->steps)
                                    : traffic_model(p, n, times.sorted_records != 0, park_threshold, g->adj_hub != nullptr,
                                                    stats->steps - stats->hub_steps,
                                                    stats->sampled_edges - stats->hub_sampled_edges, stats->hub_steps, times);

@@ -97,6 +97,7 @@ struct fw_graph {
   double label_ms = 0.0;              // device time of the MetaPath calls without them, since they were last made
   uint64_t table_limit = UINT64_MAX;  // bytes that all tables of the graph together may take (fw_graph_limit_tables)
   int last_engine = FW_ENGINE_NONE, last_made = 0;  // fw_graph_engine
+  uint64_t made_read = 0, made_written = 0;         // bytes that making tables read and wrote in the last call
   std::atomic<int> busy{0};           // a walk call is running on this graph (the caches above are per graph)
 };
 
