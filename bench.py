@@ -9,11 +9,12 @@ Prints ONE JSON line with the walk-steps/s of the whole job, the HBM roofline of
 stated bases (what the kernels of one pass ask of the memory, modelled from the run's counters; the
 useful part of it; the algorithmic bytes every walker would read alone -- all over the device time of
 that pass, measured with HIP events on the launch stream), the profiler's measured traffic for the same
-workload when the summary under profiles/ was taken on these sources, one line per benchmark
+workload and, when the summary under profiles/ was taken on these sources, its share of the peak, one line per benchmark
 configuration measured after the timed region (`configs`) and the CPU oracle timed on the host cores
-of the same box over a bounded prefix of the same queries.  With hub parking (the default for large batches) one pass is a short pipeline of launches --
-fw_walk_zprs, then per round fw_hub_scan + fw_hub_batch + fw_walk_zprs -- and the HIP events bracket the whole
-pipeline, host-side round trips included.
+of the same box over a bounded prefix of the same queries.  A pass of the default workload is one walk on list tables
+(fw_table_walk), which the first call on the graph makes: in the warm-up, or with --warmup 0 in the first timed pass.  With
+--park-threshold N it is a pipeline of launches -- fw_walk_zprs, then per round fw_hub_scan + fw_hub_batch + fw_walk_zprs -- and
+the HIP events bracket the whole pipeline, host-side round trips included.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME] [--no-cpu] [--no-configs]
 """
@@ -289,8 +290,9 @@ def main():
         kernel_ms.append(last.kernel_ms)
     fw.check(fw.lib().fw_dev_sync())
     wall = time.perf_counter() - t0
+    engine = g.engine()[0]
     split = None
-    if last.launches > 1 and not args.no_configs:
+    if engine == fw.ENGINE_PARK and not args.no_configs:
         # per-kernel view: one more pass, outside the timed region, with an event pair around every launch (the timed
         # passes do without: an event costs the stream about 5 us, and a pass is some 150 launches)
         params.time_kernels = 1
@@ -305,14 +307,16 @@ def main():
     avg_kernel_ms = float(np.mean(kernel_ms))
     roofline = roofline_of(wl["app"], last, n, avg_kernel_ms)
     roofline["kernel"] = ("fw_walk_ref" if args.sampler != "native" else
-                          "fw_walk_zprs" if last.launches == 1 else "fw_walk_zprs + fw_hub_scan + fw_hub_batch + fw_hub_quad pipeline")
+                          "fw_table_walk" if engine == fw.ENGINE_TABLES else
+                          "fw_walk_zprs" if engine == fw.ENGINE_STREAM else "fw_walk_zprs + fw_hub_scan + fw_hub_batch + fw_hub_quad pipeline")
     # the profiler's view of the same workload (library defaults only: any override makes it another run)
     sources_sha = fw.sources_sha()
-    prof = profiled_traffic(args.workload, sources_sha) if defaults and last.launches > 1 else None
+    prof = profiled_traffic(args.workload, sources_sha) if defaults and engine == fw.ENGINE_TABLES else None
     roofline["traffic"] = None
     if prof:
         roofline.update(prof)
-        roofline["traffic_frac"] = prof["traffic"] / (avg_kernel_ms * 1e-3) / 1e9 / HBM_PEAK_GBS
+        if prof["traffic_taken_on_these_sources"]:
+            roofline["traffic_frac"] = prof["traffic"] / (avg_kernel_ms * 1e-3) / 1e9 / HBM_PEAK_GBS
     if split is not None:
         roofline["kernels"] = [
             {"kernel": "fw_walk_zprs", "total_ms": split.walk_kernel_ms, "steps": int(split.steps - split.hub_steps)},

@@ -301,3 +301,17 @@ def test_bench_line_contract(gpu):
     assert rf["bound"] == "hbm" and rf["peak"] == 8000.0 and 0.0 < rf["frac"] <= 1.0
     assert abs(rf["frac"] - rf["achieved"] / rf["peak"]) < 1e-9
     assert d["value"] > 0 and abs(d["value"] - d["config"]["walk_steps_per_pass"] / (d["ms_per_step"] * 1e-3)) < 1e-6 * d["value"]
+
+
+@pytest.mark.parametrize("extra,kernel", [([], "fw_table_walk"), (["--park-threshold", "64"], "fw_walk_zprs + fw_hub_scan + fw_hub_batch + fw_hub_quad pipeline"),
+                                          (["--park-threshold", "-1"], "fw_walk_zprs")])
+def test_bench_names_what_ran(gpu, extra, kernel):
+    """roofline.kernel and its per-kernel split are those of the engine that the timed passes ran on."""
+    import json
+    import sys
+    r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--scale", "17", "--steps", "1", "--warmup", "1", "--no-cpu"] + extra,
+                       stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr
+    rf = json.loads(r.stdout)["roofline"]
+    assert rf["kernel"] == kernel
+    assert ("kernels" in rf) == ("pipeline" in kernel)
