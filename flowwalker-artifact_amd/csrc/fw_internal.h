@@ -216,7 +216,7 @@ struct fw_hub_args {
 };
 
 // Workload counters of a table walk: FW_TABLE_STRIPES lines of {steps, source degrees, the same two for vertices above
-// the parking degree}, added up by the host.
+// the parking degree}, added up by fw_table_end.
 constexpr uint32_t FW_TABLE_STRIPES = 64;
 constexpr size_t FW_TABLE_COUNTER_BYTES = FW_TABLE_STRIPES * 64u;
 

@@ -419,7 +419,9 @@ constexpr uint32_t kSetPart = 1040u;    // buckets a workgroup makes at a time, 
 constexpr uint32_t kSetSmall = 1024u / 8u + 1u;  // buckets of a list of one group
 
 __device__ __forceinline__ uint32_t set_bucket(int32_t neighbour, uint32_t buckets) {
-  uint32_t h = (uint32_t)neighbour * 0x9E3779B1u;  // Knuth's multiplicative hash, folded and repeated: R-MAT ids differ in few bits
+  // xxHash32's first two primes (Y. Collet) with the first fold of its finish between them: R-MAT ids differ in few bits, and the
+  // high bits, which pick the bucket, take all of them in
+  uint32_t h = (uint32_t)neighbour * 0x9E3779B1u;
   h = (h ^ (h >> 15)) * 0x85EBCA77u;
   return __umulhi(h, buckets);
 }
@@ -482,8 +484,8 @@ __global__ __launch_bounds__(256) void fw_sets_small_kernel(const uint4* __restr
   }
 }
 
-// Long lists: one workgroup per eight groups of a list makes kSetPart buckets and reads the whole list for them (a list of
-// 100,000 entries is read 13 times, from the cache).
+// Long lists: one workgroup per eight groups of a list makes kSetPart buckets and reads the whole list for them: a list of 100,000
+// entries is read 13 times, from the cache, and the reads grow with the square of the length, which the rule that decides on sets prices.
 __global__ __launch_bounds__(512) void fw_sets_long_kernel(const uint4* __restrict__ vrec, const int32_t* __restrict__ adjncy,
                                                            const float* __restrict__ weight, const uint2* __restrict__ items,
                                                            uint32_t n_items, int32_t* sets, float* set_weights) {
@@ -538,9 +540,10 @@ __device__ __forceinline__ int64_t set_find(const int32_t* __restrict__ sets, ui
 // whichever order it is added up, and "the first element whose running sum is above t" is the element of rank floor(t)
 // among those of the label (the last one if t reaches the count).  So the neighbours of a group are stored sorted by label, in the order
 // the sampler's lanes hold them, at the group's own places of the edge array (4 bytes written per edge), and a step reads
-// its vertex's record and one neighbour: 10^7 walks of 5 steps on R-MAT 26 take 2.01 ms, 6.85 through parking.  vrec[2v] = {region, degree, 0, CSR offset}, vrec[2v + 1] = where each label's
-// neighbours end in a list of one group (8 x 16 bits).  A longer list has a region, in blocks of 128 bytes: the labels' totals (floats), per
-// label the sums of its groups as above, per group the ends of its labels.
+// its vertex's record and one neighbour: 10^7 walks of 5 steps on R-MAT 26 take 1.36 ms, 6.85 through parking.
+// vrec[2v] = {region, degree, 0, CSR offset}, vrec[2v + 1] = where each label's neighbours end in a list of one group (8 x 16 bits).
+// A longer list has a region, in blocks of 128 bytes: the labels' totals (floats), per label the sums of its groups as
+// above, per group the ends of its labels.
 
 // The ends of up to 8 labels in a group of at most 1024 elements, two in a word.
 struct LabelCounts {

@@ -123,7 +123,8 @@ typedef struct {
                              tables: begin, walk, end, and the launches that made the tables when it made them) */
   int32_t grid;           /* workgroups per launch actually used */
   /* per-kernel breakdown of kernel_ms / steps / sampled_edges (hub parking splits a pass over two kernels) */
-  double walk_kernel_ms;      /* sum over fw_walk_zprs launches (with fw_walk_params.time_kernels, else 0) */
+  double walk_kernel_ms;      /* sum over fw_walk_zprs launches, or the walk on list tables (with
+                                 fw_walk_params.time_kernels, else 0) */
   double hub_kernel_ms;       /* sum over the hub launches of every round: fw_hub_scan, fw_hub_batch, fw_hub_quad
                                  (with fw_walk_params.time_kernels, else 0); a walk on list tables: the making of
                                  the tables, 0 in a call that found them made */
