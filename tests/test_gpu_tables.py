@@ -309,6 +309,50 @@ def test_kernel_times_leave_the_tables(gpu):
         g.destroy()
 
 
+def test_calls_on_other_streams_and_threads(gpu):
+    """Tables made in a call on one stream, sets on another, walked on from a third and from another thread."""
+    import threading
+    (xadj, adj, w), at = _lists("even")
+    lab = np.random.RandomState(1).randint(0, 3, size=len(adj)).astype(np.int32)
+    g = gpu.Graph.from_csr(xadj, adj, w, lab)
+    og = _oracle.Graph(xadj, adj, w, lab)
+    starts = at[np.random.RandomState(9).randint(0, len(at), size=70000)].astype(np.int32)
+    d_starts = torch.from_numpy(starts).cuda()
+    d_paths = torch.empty((70000, 21), dtype=torch.int32, device="cuda")
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    apps = [dict(app=gpu.APP_DEEPWALK), dict(app=gpu.APP_NODE2VEC, p=0.25, q=4.0), dict(app=gpu.APP_METAPATH, schema=[0, 1, 2])]
+    refs = []
+    for kw in apps:
+        par = gpu.default_params(max_depth=21, seed=8, **kw)
+        refs.append((par, _oracle.walk(og, _oracle.from_walk_params(par), starts[:5000])[0]))
+    errors = []
+
+    def walk(stream, par, ref):
+        try:
+            st = gpu.WalkStats()
+            gpu.check(gpu.lib().fw_walk_device(g.handle, C.byref(par), C.c_void_p(d_starts.data_ptr()), 70000,
+                                               C.c_void_p(d_paths.data_ptr()), C.c_void_p(stream.cuda_stream), C.byref(st)))
+            assert (d_paths[:5000].cpu().numpy() == ref).all()
+        except BaseException as e:  # noqa: B902
+            errors.append(e)
+
+    try:
+        for i in range(24):
+            par, ref = refs[i % 3]
+            args = (streams[(i // 2) % 3], par, ref)
+            if i % 4 == 3:
+                t = threading.Thread(target=walk, args=args)
+                t.start()
+                t.join()
+            else:
+                walk(*args)
+            assert not errors, (i, errors)
+        assert g.engine()[:2] == (gpu.ENGINE_TABLES, 0)
+    finally:
+        g.destroy()
+
+
 def test_changed_biases_on_adopted_arrays(gpu):
     """An adopted graph's owner may change the biases between calls: tables and the sets' weights are made anew."""
     csr, at = _lists("even")
