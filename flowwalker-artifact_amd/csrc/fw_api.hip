@@ -1600,11 +1600,15 @@ static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params*
 // them (measured) or are about to spend (estimated) a quarter more than making them takes: a first call makes them only if it gains by
 // that itself, and a loop of small calls gets them after a few and never pays more than about twice what it would have.
 //
-// What a call takes without tables: lists stream at 6.5 TB/s; a step of a walk that finds the chip idle takes 2 us; a call that
-// parks takes 0.05 ms a round (one per step of its longest walks) and 0.1 ns per step asked for (R-MAT 14 to 26, 100,000 to 16.8 M
-// queries: 0.07 to 0.3; DeepWalk R-MAT 24 0.09, MetaPath R-MAT 26 0.14), and the first one makes the parking index, 17 ps
-// per edge (R-MAT 22 28, R-MAT 24 15.5, R-MAT 26 19).
+// What a call takes without tables: lists stream at 6.5 TB/s, but a step takes at least 0.06 ns, however short its list
+// (uniform graphs of mean degree 4 to 24, 60,000 to 4,000,000 walks of 80 steps: 0.06 to 0.2 per step asked for; MetaPath, most
+// of whose walks end early, 0.006 to 0.1); a step of a walk that finds the chip idle takes 2 us; a call that parks takes 0.05 ms a
+// round (one per step of its longest walks) and 0.1 ns per step asked for (R-MAT 14 to 26, 100,000 to 16.8 M queries: 0.07 to
+// 0.3; DeepWalk R-MAT 24 0.09, MetaPath R-MAT 26 0.14), and the first one makes the parking index, 17 ps per edge (R-MAT 22 28,
+// R-MAT 24 15.5, R-MAT 26 19).
 constexpr double kStreamBytesPerMs = 6.5e9;
+constexpr double kShortStepMs = 0.06e-6;
+constexpr double kShortMetaPathStepMs = 0.015e-6;
 constexpr double kStepLatencyMs = 0.002;
 constexpr double kParkedRoundMs = 0.05;
 constexpr double kParkedStepMs = 0.1e-6;
@@ -1666,7 +1670,8 @@ static int lists_estimate_ms(fw_graph* g, const fw_walk_params* p, int32_t n, do
     double mean = 0.0;
     const int rc = mean_list_length(g, &mean);
     if (rc != FW_OK) return rc;
-    double lists_ms = steps * (double)n * mean * 4.0 / kStreamBytesPerMs;
+    const double short_ms = p->app == FW_APP_METAPATH ? kShortMetaPathStepMs : kShortStepMs, list_ms = mean * 4.0 / kStreamBytesPerMs;
+    double lists_ms = steps * (double)n * (list_ms > short_ms ? list_ms : short_ms);
     if (resolve_park_threshold(g, p, n) != INT_MAX) {
       double rounds = (double)(p->max_depth - 1);
       if (p->app == FW_APP_PPR && p->tp > 0.0f && p->tp < 1.0f) {  // until the last of n walks stops

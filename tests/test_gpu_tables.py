@@ -403,10 +403,10 @@ def test_small_calls_on_adopted_arrays(gpu):
 
 
 @pytest.mark.parametrize("vertices,hub,n,length,engine", [(300000, 23000, 50000, 20, "STREAM"), (1000000, 100000, 70000, 15, "PARK"),
-                                                          (1000000, 100000, 300000, 40, "TABLES")])
+                                                          (1000000, 100000, 300000, 40, "TABLES"), (40000, 30, 500000, 80, "TABLES")])
 def test_first_call_makes_tables_only_for_itself(gpu, vertices, hub, n, length, engine):
     """A first call that takes less without tables than making them takes (0.7 ms of its 0.9, 0.9 ms of its 1.0 in rounds of the
-    parking pipeline) goes without; one that takes several times as much makes them."""
+    parking pipeline) goes without; one that takes several times as much makes them, also where all lists are short (3 ms of walks, 0.3 of making)."""
     rng = np.random.RandomState(vertices)
     deg = np.full(vertices, 3, dtype=np.int64)
     deg[rng.permutation(vertices)[:2]] = hub
