@@ -82,7 +82,8 @@ def test_batches_come_before_tables(gpu):
                     g.walk(big, starts[:70000])
                 assert g.engine()[0] == gpu.ENGINE_TABLES
             assert (g.engine()[2] > 300 << 20) == tables
-            held = _fill_memory(gpu, 900 << 20 if not tables else 700 << 20)
+            # 820 MB fit beside 900, but not beside 500 and what the runtime holds of freed memory without counting it as free (130 MB seen)
+            held = _fill_memory(gpu, 900 << 20 if not tables else 500 << 20)
             paths, st2 = g.walk_batch(big, starts, batch_size=n)
             assert g.engine()[0] == gpu.ENGINE_STREAM and g.engine()[2] == 0
             assert (paths == ref).all() and st2.steps == st.steps
