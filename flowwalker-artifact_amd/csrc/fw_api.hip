@@ -1784,14 +1784,14 @@ static int plan_tables(const fw_graph* g, fw_tables* t, hipStream_t stream) {
 // Whether this call makes the hash sets of node2vec's adjacency tests, and for the return edge their weights (the memory is there
 // then).  They are made once the calls' searches have cost, or are about to cost, a quarter more than making them.
 // A search that finds the chip busy costs 0.03 ns (R-MAT 24: 41 ms of 1.34 G steps asked for, R-MAT 23 0.5 of 20 M), a step of a few
-// walkers 4 us, and a q above 1 takes about q trials.  Making takes 0.2 ms per new array and moves 12 bytes per edge and 64 per vertex, with weights
-// as much again, at 0.75 TB/s, and reads a long list once per 8192 entries: R-MAT 24 symmetrised 10.9 ms (estimated 10.6), R-MAT
-// 23 with 268 M edges 4.8 (5.3), R-MAT 20 with 33 M 0.73 (0.83), with 4 M 0.25 (0.36).
+// walkers 4 us, and a q above 1 takes about q trials.  Making takes 0.2 ms per new array and moves 12 bytes per edge and 64 per
+// vertex, with weights as much again, at 0.85 TB/s: R-MAT 23 with 268 M edges 4.8 ms, R-MAT 20 with 33 M 0.73, with 4 M 0.25.  A long list is read
+// once per 8192 entries, at 0.35 TB/s: one of 4 M entries takes 23 ms (estimated 22), one of 16 M 352 (358); R-MAT 24 symmetrised 10.9 in all.
 constexpr double kSearchMs = 0.03e-6;
 constexpr double kSearchStepMs = 0.004;
-constexpr double kSetMakeBytesPerMs = 0.75e9;
+constexpr double kSetMakeBytesPerMs = 0.85e9;
 constexpr double kSetMakeFixedMs = 0.2;
-constexpr double kSetRereadBytesPerMs = 3.0e9;
+constexpr double kSetRereadBytesPerMs = 0.35e9;
 
 static bool sets_for_call(fw_graph* g, const fw_walk_params* p, fw_tables* t, double all_steps, double steps) {
   const bool back = p->p < 1.0f && p->p < p->q;  // the return edge is a component of its own

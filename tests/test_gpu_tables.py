@@ -213,6 +213,29 @@ def test_weights_of_sets_have_to_be_earned(gpu):
         g.destroy()
 
 
+def test_sets_of_a_long_list_have_to_be_earned(gpu):
+    """A list of 3,000,000 entries takes its sets some 13 ms (it is read once per 8192 entries): a call whose searches cost 3 ms goes without
+    them."""
+    rng = np.random.RandomState(5)
+    hub, vertices = 3000000, 20000
+    xadj = np.full(vertices + 1, hub, dtype=np.uint32) + np.arange(-1, vertices, dtype=np.int64).astype(np.uint32)
+    xadj[0] = 0
+    adj = np.zeros(int(xadj[-1]), dtype=np.int32)
+    adj[:hub] = np.sort(rng.randint(0, vertices, size=hub))
+    w = (1.0 + 9.0 * rng.random_sample(len(adj))).astype(np.float32)
+    g = gpu.Graph.from_csr(xadj, adj, w)
+    try:
+        starts = rng.randint(0, vertices, size=1000000).astype(np.int32)
+        par = gpu.default_params(app=gpu.APP_NODE2VEC, max_depth=101, p=2.0, q=0.5, seed=3)
+        paths, st = g.walk(par, starts)
+        engine, made, _ = g.engine()
+        assert engine == gpu.ENGINE_TABLES and made == 3  # the lists, without sets
+        ref, _, _ = _oracle.walk(_oracle.Graph(xadj, adj, w), _oracle.from_walk_params(par), starts[:5])
+        assert (paths[:5] == ref).all()
+    finally:
+        g.destroy()
+
+
 def test_memory_of_tables(gpu):
     """fw_graph_limit_tables: what is above the bound is given back at once and not taken again, tables without room for sets, sets without
     room for their weights; the walks are the same."""
