@@ -67,15 +67,17 @@ struct N2vTest {
   bool take_prev;    // the step goes back to the previous vertex whatever was proposed
 };
 
-__device__ __forceinline__ N2vTest n2v_test(const fw_kargs& a, int32_t post, int32_t prev, uint32_t walker, uint32_t step,
-                                            uint32_t trial, float T, float w_ret) {
+// draw: gives block 0 of the trial's acceptance stream
+template <typename Draw>
+__device__ __forceinline__ N2vTest n2v_test(const fw_kargs& a, int32_t post, int32_t prev, uint32_t trial, float T, float w_ret,
+                                            Draw draw) {
   N2vTest t;
   t.uF = 0.0f;
   t.decided = true;
   t.accept = true;
   t.take_prev = false;
   if (prev == -1 || trial == kMaxTrials - 1u) return t;
-  const uint4 bits = philox4x32_10(walker, step, kStreamAccept | (trial << 8), 0u, a.seed_lo, a.seed_hi);
+  const uint4 bits = draw();
   t.uF = u24(bits.x) * a.n2v_fmax;
   if (a.n2v_extra > 0.0f) {
     const float gx = a.n2v_extra * w_ret;
@@ -94,6 +96,11 @@ __device__ __forceinline__ N2vTest n2v_test(const fw_kargs& a, int32_t post, int
   if (!(t.uF < f_hi)) return t;         // rejected as either
   t.decided = false;
   return t;
+}
+
+__device__ __forceinline__ N2vTest n2v_test(const fw_kargs& a, int32_t post, int32_t prev, uint32_t walker, uint32_t step,
+                                            uint32_t trial, float T, float w_ret) {
+  return n2v_test(a, post, prev, trial, T, w_ret, [&] { return philox4x32_10(walker, step, kStreamAccept | (trial << 8), 0u, a.seed_lo, a.seed_hi); });
 }
 
 // the other half: `common` = the proposal is a neighbour of prev

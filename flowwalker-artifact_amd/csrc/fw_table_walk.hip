@@ -1193,6 +1193,244 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
     atomicAdd(&tb.counters[(blockIdx.x & (FW_TABLE_STRIPES - 1u)) * 8u + threadIdx.x], s_acc[threadIdx.x]);
 }
 
+// ---- the walk of few walkers ------------------------------------------------------------------------------
+//
+// A call of few walkers is a chain of dependent reads per step, and nothing else fills the time: the chip has lanes and memory to
+// spare.  So a whole wave walks one walker.  A step takes its record; the row of the group and the pairs around the proportional
+// guess together (1 KB of pairs, eight lanes' worth of a full group, so the guess is nearly always good enough); for a long list
+// the sums of 64 groups before that.  Every search is a comparison in all lanes and a ballot, and the draws a step may take are
+// made by the lanes side by side while the record is on its way.
+// Results are fw_table_walk's: the same sums, the same draws, the same comparisons.
+
+__device__ __forceinline__ uint32_t uniform_u32(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+__device__ __forceinline__ uint32_t readlane_u32(uint32_t x, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)l); }
+
+constexpr int kWalkerWaves = 8;  // waves per SIMD
+
+// The draws of a trial, lane by lane: lanes 0 .. 47 hold blocks 0, 1, 2 of the sequences' streams (lane = block * 16 + sequence), the
+// next three one block each of the streams below.
+constexpr uint32_t kWaveLane = 48u, kStopLane = 49u, kAcceptLane = 50u;
+
+__device__ __forceinline__ uint4 wave_draws(const fw_kargs& a, uint32_t walker, uint32_t step, uint32_t trial, uint32_t lane) {
+  const uint32_t sbase = trial << 8;
+  uint32_t stream = sbase | (lane & 15u);
+  stream = lane == kWaveLane ? kStreamWave | sbase : stream;
+  stream = lane == kStopLane ? kStreamStop : stream;
+  stream = lane == kAcceptLane ? kStreamAccept | sbase : stream;
+  return philox4x32_10(walker, step, stream, lane < kWaveLane ? lane >> 4 : 0u, a.seed_lo, a.seed_hi);
+}
+
+// sums_reservoir by a wave.  S_last: the sequence's last sum.  total: of the group it ends with.
+__device__ __forceinline__ uint32_t wave_reservoir(const fw_kargs& a, const float* sums, const uint32_t nb, const float S_last,
+                                                   const uint4 d, const uint32_t walker, const uint32_t step, const uint32_t seq,
+                                                   const uint32_t sbase, const uint32_t lane, float& tu_out, float& total) {
+  const uint32_t at = 32u * (lane >> 4) + (lane & 15u);  // of the lane's sum in four blocks of sums
+  uint32_t c0 = 0u;  // first of the four blocks in registers
+  float s = 0.0f, T = 0.0f;
+  if ((lane >> 4) < nb) {
+    s = sums[at];
+    T = sums[at + 16u];
+  }
+  uint4 e = d;
+  float Sj = 0.0f, u = 1.0f, tu = 0.0f;
+  uint32_t k = 0u;
+  float Tk = 0.0f;
+  for (uint32_t i = 0u; S_last * u > Sj; ++i) {
+    uint64_t m = __ballot(s * u > Sj);
+    if (m == 0ull) {  // behind the blocks in registers: 64 blocks' last sums at a time, then the four blocks from the first that passes
+      uint32_t lo = c0 + 4u, hi = nb - 1u;
+      while (hi - lo >= 4u) {
+        const uint32_t stride = (hi - lo + 64u) >> 6;
+        uint32_t b = lo + (lane + 1u) * stride - 1u;
+        b = b < hi ? b : hi;
+        const uint32_t f = (uint32_t)__builtin_ctzll(__ballot(sums[32u * b + 15u] * u > Sj || b == hi));
+        hi = readlane_u32(b, f);
+        lo = f != 0u ? readlane_u32(b, f - 1u) + 1u : lo;
+      }
+      c0 = lo;
+      s = T = 0.0f;
+      if (c0 + (lane >> 4) < nb) {
+        s = sums[32u * c0 + at];
+        T = sums[32u * c0 + at + 16u];
+      }
+      m = __ballot(s * u > Sj);
+    }
+    const uint32_t l = (uint32_t)__builtin_ctzll(m | (1ull << 63));
+    k = 16u * c0 + l;
+    Sj = readlane_f(s, (int)l);
+    Tk = readlane_f(T, (int)l);
+    uint32_t from = seq + 16u * (i >> 1);
+    if (i >= 6u) {  // past the blocks made beforehand
+      if (i == 6u || (i & 127u) == 0u) e = philox4x32_10(walker, step, seq | sbase, 64u * (i >> 7) + lane, a.seed_lo, a.seed_hi);
+      from = (i >> 1) & 63u;
+    }
+    tu = u24(readlane_u32((i & 1u) ? e.z : e.x, from));
+    u = u24(readlane_u32((i & 1u) ? e.w : e.y, from));
+  }
+  tu_out = tu;
+  total = Tk;
+  return k;
+}
+
+// table_pick by a wave: everything but the lanes' own pieces is the same in all lanes.
+__device__ __forceinline__ int32_t wave_pick(const fw_kargs& a, const fw_table_args& tb, const uint4 rec, const uint4 d,
+                                             const uint32_t walker, const uint32_t step, const uint32_t sbase, const uint32_t lane) {
+  const uint32_t nq = list_quartets(rec.w, rec.y);
+  const unsigned char* row = tb.data + (uint64_t)rec.x * 128u;
+  uint32_t nqg = nq, row_units = 8u;
+  float T = __uint_as_float(rec.z), tu;
+  if (nq <= kGq) {
+    tu = u24(readlane_u32(d.x, 0u));
+    if (nq < 64u) row_units = (nq + 7u) >> 3;
+  } else {
+    const uint32_t ngroups = (nq + kGq - 1u) / kGq;
+    const bool wg = (int32_t)rec.y > a.hub_threshold;
+    const uint32_t nb = seq_blocks(ngroups, wg, tb.nw_shift);
+    const float* sums = reinterpret_cast<const float*>(row);
+    uint32_t seq = 0u;
+    float S_last = T;
+    if (wg) {  // which sequence, then the reservoir over it with draws of its own stream
+      const float target = u24(readlane_u32(d.x, kWaveLane)) * T;
+      seq = (uint32_t)__builtin_popcountll(__ballot(lane < 16u && sums[lane & 15u] <= target));
+      sums += 32u + 32u * nb * seq;
+      S_last = sums[32u * (nb - 1u) + 15u];
+    }
+    const uint32_t k = wave_reservoir(a, sums, nb, S_last, d, walker, step, seq, sbase, lane, tu, T);
+    const uint32_t g = wg ? seq + (k << tb.nw_shift) : k;
+    row += (uint64_t)32u * (header_units(ngroups, wg, tb.nw_shift) + kGroupUnits * g);
+    nqg = nq - g * kGq < kGq ? nq - g * kGq : kGq;
+  }
+  const float t = tu * T;
+  const uint32_t nl = nqg < 64u ? nqg : 64u;
+  const uint32_t J = (nqg + 63u) >> 6;
+  // two pairs a lane, from some lanes before the guess on
+  const uint4* pairs = reinterpret_cast<const uint4*>(row + 32u * row_units);
+  const uint32_t n2 = 2u * J * nl;
+  const uint32_t guess = (uint32_t)(tu * (float)n2);
+  uint32_t w = guess > 32u ? guess - 32u : 0u;
+  const uint32_t wmax = n2 > 64u ? n2 - 64u : 0u;
+  w = w < wmax ? w : wmax;
+  uint4 p = make_uint4(0u, 0u, 0u, 0u);
+  if (w + lane < n2) p = pairs[w + lane];
+  const float m = lane < nl ? reinterpret_cast<const float*>(row)[lane] : kInf;
+  const uint32_t l = (uint32_t)__builtin_ctzll(__ballot(!(m <= t)) | (1ull << 63));
+  const uint32_t first = 2u * J * l;  // of the lane's pieces
+  if (first < w || first + 2u * J > w + 64u) {
+    w = first;
+    if (w + lane < n2) p = pairs[w + lane];
+  }
+  const uint64_t mine = ((1ull << (2u * J)) - 1ull) << (first - w);
+  const uint64_t m0 = __ballot(!(__uint_as_float(p.x) <= t)) & mine, m1 = __ballot(!(__uint_as_float(p.z) <= t)) & mine;
+  const uint32_t f = (uint32_t)__builtin_ctzll(m0 | m1 | (1ull << (first - w + 2u * J - 1u)));  // (the last piece has a key above)
+  return (int32_t)(((m0 >> f) & 1ull) != 0ull ? readlane_u32(p.y, f) : readlane_u32(p.w, f));
+}
+
+// set_find by a wave, from the lane's place of the bucket (lanes 0 .. 15)
+__device__ __forceinline__ int64_t wave_set_find(const int32_t* __restrict__ sets, uint32_t v, uint32_t off, uint32_t deg, int32_t target,
+                                                 uint32_t lane) {
+  const uint64_t first = 16u * (fw_set_first(off, v) + set_bucket(target, fw_set_buckets(deg)));
+  const int32_t x = sets[first + (lane & 15u)];
+  const uint32_t hit = (uint32_t)__ballot(x == target) & 0xFFFFu;
+  if (hit != 0u) return (int64_t)first + __builtin_ctz(hit);
+  return __builtin_amdgcn_readlane(x, 15) == kSetOverflow ? -2 : -1;
+}
+
+// One wave, one walker.  Bound: latency, three dependent reads a step (four and five on long lists; node2vec one more a trial): 1.3 us a step of
+// 1,000 walkers on R-MAT 20, 2.0 where a lane walked each.
+template <int kApp>
+__global__ __launch_bounds__(256, kWalkerWaves) void fw_table_walk_wave(const fw_kargs a, const fw_table_args tb) {
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t md = (uint32_t)a.max_depth;
+  const uint32_t q = blockIdx.x * 4u + uniform_u32(threadIdx.x >> 6);
+  if (q >= (uint32_t)a.n) return;
+  uint32_t n_steps = 0u, n_hub = 0u;
+  unsigned long long n_edges = 0ull, hub_edges = 0ull;
+  const uint32_t walker = a.walker_base + q;
+  int32_t* const path = a.paths + (uint64_t)q * md;
+  uint32_t v = uniform_u32((uint32_t)a.starts[q]);
+  int32_t mine = lane == 0u ? (int32_t)v : -1;  // the path's entry of the lane's place among the 64 that are not stored yet
+  uint32_t len = 1u, kept = 0u;  // entries, and those that are stored
+  if (v < (uint32_t)a.V && md > 1u) {
+    uint32_t prev_off = 0u, prev_deg = 0u;
+    int32_t prev = -1;
+    uint4 r = tb.vrec[v];
+    for (bool ended = false; !ended;) {
+      const uint32_t step = len - 1u;
+      uint4 d = wave_draws(a, walker, step, 0u, lane);
+      const uint4 rec = make_uint4(uniform_u32(r.x), uniform_u32(r.y), uniform_u32(r.z), uniform_u32(r.w));
+      if (!(__uint_as_float(rec.z) > 0.0f)) break;  // no neighbour with a positive bias (include/walker.cuh:1373-1374)
+      int32_t nv = wave_pick(a, tb, rec, d, walker, step, 0u, lane);
+      if (kApp == FW_APP_NODE2VEC && prev >= 0) {
+        float w_ret = 0.0f;
+        if (a.n2v_extra > 0.0f) {
+          const int64_t at = tb.set_weights != nullptr ? wave_set_find(tb.sets, v, rec.w, rec.y, prev, lane) : -2;
+          if (at >= 0) w_ret = tb.set_weights[at];
+          if (at == -2) w_ret = return_weight(a.adjncy + rec.w, a.weight + rec.w, rec.y, prev);
+        }
+        for (uint32_t trial = 0u;;) {
+          r = tb.vrec[(uint32_t)nv < (uint32_t)a.V ? (uint32_t)nv : v];  // mostly the next vertex: on its way during the test
+          const uint4 bits = make_uint4(readlane_u32(d.x, kAcceptLane), readlane_u32(d.y, kAcceptLane), 0u, 0u);
+          const N2vTest t = n2v_test(a, nv, prev, trial, __uint_as_float(rec.z), w_ret, [&] { return bits; });
+          if (t.take_prev) {
+            nv = prev;
+            r = tb.vrec[(uint32_t)prev];
+            break;
+          }
+          bool common = false;
+          if (!t.decided) {
+            const int64_t at = tb.sets != nullptr ? wave_set_find(tb.sets, (uint32_t)prev, prev_off, prev_deg, nv, lane) : -2;
+            common = at >= 0;
+            if (at == -2) common = sorted_contains(a.adjncy + prev_off, (int32_t)prev_deg, nv);
+          }
+          if (n2v_finish(a, t, common)) break;
+          trial += 1u;
+          d = wave_draws(a, walker, step, trial, lane);
+          nv = wave_pick(a, tb, rec, d, walker, step, trial << 8, lane);
+        }
+      }
+      if ((int32_t)rec.y > a.park_threshold) {
+        n_hub += 1u;
+        hub_edges += rec.y;
+      } else {
+        n_steps += 1u;
+        n_edges += rec.y;
+      }
+      const bool loaded = kApp == FW_APP_NODE2VEC && prev >= 0;  // r is the new vertex's already
+      if (kApp == FW_APP_NODE2VEC) {
+        prev = (int32_t)v;
+        prev_off = rec.w;
+        prev_deg = rec.y;
+      }
+      v = (uint32_t)nv;
+      len += 1u;
+      ended = len >= md;
+      if (kApp == FW_APP_PPR && !ended) ended = u24(readlane_u32(d.x, kStopLane)) < a.tp;  // include/app.cuh:88-94
+      if (!ended && !loaded) r = tb.vrec[v];
+      mine = lane == len - 1u - kept ? nv : mine;
+      if (len - kept == 64u) {
+        path[kept + lane] = mine;
+        mine = -1;
+        kept = len;
+      }
+    }
+  }
+  for (uint32_t p = kept + lane; p < md; p += 64u) {
+    path[p] = mine;
+    mine = -1;
+  }
+  if (lane == 0u) {
+    unsigned long long* const c = &tb.counters[(blockIdx.x & (FW_TABLE_STRIPES - 1u)) * 8u];
+    if (n_steps != 0u) {
+      atomicAdd(&c[0], (unsigned long long)n_steps);
+      atomicAdd(&c[1], n_edges);
+    }
+    if (n_hub != 0u) {
+      atomicAdd(&c[2], (unsigned long long)n_hub);
+      atomicAdd(&c[3], hub_edges);
+    }
+  }
+}
+
 // Around the walk: the counters start at zero, and their sums go to the host (pinned memory: the call waits for the stream
 // anyway, and a copy of its own would cost a small call as much as its launch).
 __global__ void fw_table_begin_kernel(unsigned long long* counters, uint32_t* scratch, uint32_t words) {
@@ -1220,12 +1458,24 @@ int launch_table_walk(const fw_kargs& a, fw_table_args tb, int grid, hipStream_t
   FW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   const uint32_t n = (uint32_t)a.n;
   uint64_t waves;
+  if constexpr (kApp != FW_APP_METAPATH) {  // (whose step is two reads, and no search)
+    // As many walkers as there are waves resident: a wave each.  Measured, wave per walker / lane per walker, us of a call of 40 steps on R-MAT 20,
+    // symmetrised: 1,000 walkers DeepWalk 73 / 92, PPR 52 / 76, node2vec 164 / 245; 8,000: 121 / 172, 72 / 94, 227 / 345 (q = 4: 555 / 760);
+    // with two walks a wave (16,000): 261 / 191, 238 / 99, 367 / 422.
+    if (grid <= 0 && n <= (uint32_t)cus * 4u * kWalkerWaves) {
+      const unsigned blocks = (n + 3u) / 4u;
+      hipLaunchKernelGGL((fw_table_walk_wave<kApp>), dim3(blocks), dim3(256), 0, stream, a, tb);
+      FW_HIP(hipGetLastError());
+      if (grid_used) *grid_used = (int)blocks;
+      return FW_OK;
+    }
+  }
   if (grid > 0) {
     waves = (uint64_t)grid * 4u;
     tb.lanes = 64u;
   } else {
-    // few queries are spread over the chip, down to one lane per wave: their walks are chains of dependent look-ups, and a
-    // wave waits for the slowest of its lanes
+    // few queries are spread over the chip, down to a few lanes per wave: their walks are chains of dependent look-ups, and a
+    // wave waits for the slowest of its lanes (16 waves per CU instead of 8: 16,000 to 200,000 walkers within 5 % either way)
     const uint32_t spread = (uint32_t)cus * 8u;
     tb.lanes = n / spread < 64u ? n / spread + 1u : 64u;
     if (tb.lanes > 64u) tb.lanes = 64u;

@@ -166,6 +166,57 @@ def test_walks_on_tables(gpu, kind, wg, thr):
         g.destroy()
 
 
+@pytest.mark.parametrize("wg,thr", [(512, 16384), (256, 1024)])
+@pytest.mark.parametrize("n", [8192, 8193])
+def test_wave_or_lane_per_walker(gpu, n, wg, thr):
+    """Either side of the number of walkers up to which a wave walks each."""
+    csr, at = _lists("uneven")
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    rng = np.random.RandomState(n)
+    try:
+        g.walk(gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21, wg_threads=wg, hub_threshold=thr), at[rng.randint(0, len(at), size=70000)].astype(np.int32))
+        for kw in (dict(app=gpu.APP_DEEPWALK, max_depth=66), dict(app=gpu.APP_PPR, max_depth=20, tp=0.1), dict(app=gpu.APP_NODE2VEC, max_depth=9, p=0.25, q=4.0),
+                   dict(app=gpu.APP_NODE2VEC, max_depth=9, p=2.0, q=0.5)):
+            p = gpu.default_params(wg_threads=wg, hub_threshold=thr, seed=n, **kw)
+            starts = at[rng.randint(0, len(at), size=n)].astype(np.int32)
+            ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(p), starts)
+            paths, st = g.walk(p, starts)
+            assert g.engine()[0] == gpu.ENGINE_TABLES
+            assert (paths == ref).all() and (st.steps, st.sampled_edges) == (steps, edges), kw
+    finally:
+        g.destroy()
+
+
+@pytest.mark.parametrize("wg,thr", [(256, 16384), (512, 1 << 30)])
+def test_sums_beyond_four_blocks(gpu, wg, thr):
+    """Lists of 69 and 4297 groups: the sums of 64 groups are in registers, and behind them 64 blocks are looked at together."""
+    V, hubs = 2000, (70001, 4400001)
+    rng = np.random.RandomState(5)
+    deg = np.full(V, 2, dtype=np.int64)
+    deg[:2] = hubs
+    xadj = np.zeros(V + 1, dtype=np.uint32)
+    np.cumsum(deg, out=xadj[1:])
+    adj = np.tile(np.array([0, 1], dtype=np.int32), int(xadj[-1]) // 2 + 1)[:int(xadj[-1])]  # every other vertex leads to the two
+    for v in (0, 1):
+        adj[xadj[v]:xadj[v + 1]] = np.sort(rng.randint(2, V, size=deg[v]))
+    w = np.exp(rng.normal(0.0, 3.0, size=len(adj))).astype(np.float32)
+    g = gpu.Graph.from_csr(xadj, adj, w)
+    og = _oracle.Graph(xadj, adj, w)
+    try:
+        kw = dict(app=gpu.APP_DEEPWALK, wg_threads=wg, hub_threshold=thr)
+        g.walk(gpu.default_params(max_depth=11, **kw), rng.randint(0, V, size=70000).astype(np.int32))
+        starts = rng.randint(0, V, size=100).astype(np.int32)
+        starts[:40] = np.arange(40) % 2
+        p = gpu.default_params(max_depth=4, seed=9, **kw)
+        ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(p), starts)
+        paths, st = g.walk(p, starts)
+        assert g.engine()[0] == gpu.ENGINE_TABLES
+        assert (paths == ref).all() and (st.steps, st.sampled_edges) == (steps, edges)
+    finally:
+        g.destroy()
+
+
 @pytest.mark.parametrize("kind", ["even", "uneven"])
 def test_node2vec_on_hash_sets(gpu, kind):
     """The first call is long enough to pay for the sets (one walk of 100 steps counts as 0.4 ms of searches, 1.5 times 0.2 ms are asked
