@@ -543,6 +543,7 @@ static void fill_kargs(fw_kargs* a, const fw_graph* g, const fw_walk_params* p) 
   a->adjncy = g->adjncy;
   a->weight = g->weight;
   a->label = g->label;
+  a->host_edges = g->host_edges;
   a->V = g->V;
   a->max_depth = p->max_depth;
   a->hub_threshold = p->hub_threshold;

@@ -143,6 +143,7 @@ struct fw_kargs {
   uint32_t* parked_count;            // += walkers parked (one update per workgroup)
   uint32_t* bucket_count;            // [n_hubs * n_labels_per_hub]
   const fw_walker_rec* resume;       // in: walkers to continue instead of fresh queries (NULL: use starts)
+  int32_t host_edges;                // the edge arrays are read over the bus
   const uint32_t* n_dev;             // in: when not NULL, the number of entries is read here (n is an upper bound
                                      // the grid was sized for) and slot_limit follows from it
 };

@@ -129,4 +129,41 @@ __device__ __forceinline__ float next_uniform_lane(LaneDraw& d, const fw_kargs& 
   return u;
 }
 
+// ---- draws of a wave that works on one walker -------------------------------------------------------------
+
+__device__ __forceinline__ uint32_t uniform_u32(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+__device__ __forceinline__ uint32_t readlane_u32(uint32_t x, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)l); }
+
+// The draws of a trial, lane by lane: lanes 0 .. 47 hold blocks 0, 1, 2 of the sequences' streams (lane = block * 16 + sequence), the
+// next three one block each of the streams below.
+constexpr uint32_t kWaveLane = 48u, kStopLane = 49u, kAcceptLane = 50u;
+
+__device__ __forceinline__ uint4 wave_draws(const fw_kargs& a, uint32_t walker, uint32_t step, uint32_t trial, uint32_t lane) {
+  const uint32_t sbase = trial << 8;
+  uint32_t stream = sbase | (lane & 15u);
+  stream = lane == kWaveLane ? kStreamWave | sbase : stream;
+  stream = lane == kStopLane ? kStreamStop : stream;
+  stream = lane == kAcceptLane ? kStreamAccept | sbase : stream;
+  return philox4x32_10(walker, step, stream, lane < kWaveLane ? lane >> 4 : 0u, a.seed_lo, a.seed_hi);
+}
+
+// The uniforms of a sequence's reservoir, two per accepted group: the words of its stream in order.
+struct WavePairs {
+  uint4 e;       // wave_draws, later blocks of the sequence's own stream
+  uint32_t seq;
+  uint32_t i;    // pairs taken
+};
+
+__device__ __forceinline__ void next_pair(WavePairs& p, const fw_kargs& a, uint32_t walker, uint32_t step, uint32_t sbase,
+                                          uint32_t lane, float& first, float& second) {
+  uint32_t from = p.seq + 16u * (p.i >> 1);
+  if (p.i >= 6u) {  // past the blocks made beforehand
+    if (p.i == 6u || (p.i & 127u) == 0u) p.e = philox4x32_10(walker, step, p.seq | sbase, 64u * (p.i >> 7) + lane, a.seed_lo, a.seed_hi);
+    from = (p.i >> 1) & 63u;
+  }
+  first = u24(readlane_u32((p.i & 1u) ? p.e.z : p.e.x, from));
+  second = u24(readlane_u32((p.i & 1u) ? p.e.w : p.e.y, from));
+  ++p.i;
+}
+
 }  // namespace

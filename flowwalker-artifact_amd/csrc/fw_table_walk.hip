@@ -1202,23 +1202,7 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
 // made by the lanes side by side while the record is on its way.
 // Results are fw_table_walk's: the same sums, the same draws, the same comparisons.
 
-__device__ __forceinline__ uint32_t uniform_u32(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
-__device__ __forceinline__ uint32_t readlane_u32(uint32_t x, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)l); }
-
 constexpr int kWalkerWaves = 8;  // waves per SIMD
-
-// The draws of a trial, lane by lane: lanes 0 .. 47 hold blocks 0, 1, 2 of the sequences' streams (lane = block * 16 + sequence), the
-// next three one block each of the streams below.
-constexpr uint32_t kWaveLane = 48u, kStopLane = 49u, kAcceptLane = 50u;
-
-__device__ __forceinline__ uint4 wave_draws(const fw_kargs& a, uint32_t walker, uint32_t step, uint32_t trial, uint32_t lane) {
-  const uint32_t sbase = trial << 8;
-  uint32_t stream = sbase | (lane & 15u);
-  stream = lane == kWaveLane ? kStreamWave | sbase : stream;
-  stream = lane == kStopLane ? kStreamStop : stream;
-  stream = lane == kAcceptLane ? kStreamAccept | sbase : stream;
-  return philox4x32_10(walker, step, stream, lane < kWaveLane ? lane >> 4 : 0u, a.seed_lo, a.seed_hi);
-}
 
 // sums_reservoir by a wave.  S_last: the sequence's last sum.  total: of the group it ends with.
 __device__ __forceinline__ uint32_t wave_reservoir(const fw_kargs& a, const float* sums, const uint32_t nb, const float S_last,
@@ -1231,11 +1215,11 @@ __device__ __forceinline__ uint32_t wave_reservoir(const fw_kargs& a, const floa
     s = sums[at];
     T = sums[at + 16u];
   }
-  uint4 e = d;
+  WavePairs pairs{d, seq, 0u};
   float Sj = 0.0f, u = 1.0f, tu = 0.0f;
   uint32_t k = 0u;
   float Tk = 0.0f;
-  for (uint32_t i = 0u; S_last * u > Sj; ++i) {
+  while (S_last * u > Sj) {
     uint64_t m = __ballot(s * u > Sj);
     if (m == 0ull) {  // behind the blocks in registers: 64 blocks' last sums at a time, then the four blocks from the first that passes
       uint32_t lo = c0 + 4u, hi = nb - 1u;
@@ -1259,13 +1243,7 @@ __device__ __forceinline__ uint32_t wave_reservoir(const fw_kargs& a, const floa
     k = 16u * c0 + l;
     Sj = readlane_f(s, (int)l);
     Tk = readlane_f(T, (int)l);
-    uint32_t from = seq + 16u * (i >> 1);
-    if (i >= 6u) {  // past the blocks made beforehand
-      if (i == 6u || (i & 127u) == 0u) e = philox4x32_10(walker, step, seq | sbase, 64u * (i >> 7) + lane, a.seed_lo, a.seed_hi);
-      from = (i >> 1) & 63u;
-    }
-    tu = u24(readlane_u32((i & 1u) ? e.z : e.x, from));
-    u = u24(readlane_u32((i & 1u) ? e.w : e.y, from));
+    next_pair(pairs, a, walker, step, sbase, lane, tu, u);
   }
   tu_out = tu;
   total = Tk;

@@ -1948,10 +1948,297 @@ int launch_hub_app(const fw_kargs& a, const fw_hub_args& h, int wg_threads, uint
 // the smaller batches) take as many workgroups as give each about a refill and a half of its task table.
 constexpr int kEntriesPerWorkgroup = 700;
 
+// ---- few walkers ---------------------------------------------------------------------------------------
+//
+// With at most a walker per resident wave the rounds above wait, between two barriers, for the longest list that any walker of a workgroup
+// stands on, and a long list is a chain of one read per group.  Here a wave walks one walker from its start to its end, at its own
+// pace, with the reads of kFewGroups groups in flight.  The sequences of a hub's list are offered to the other waves of the workgroup: every wave looks
+// for such work before each of its steps, and once its own walk is over, until the workgroup has no walker left.  A wave that waits for the helpers of its
+// list has no sequence left to take, and a helper waits for nothing, so every wait ends.
+// Bound: latency, two dependent reads a step on a list of one group (the vertex's range, the list with its neighbours) and one more on a longer one:
+// 3,001 DeepWalk walkers of 40 steps on R-MAT 18 258 -> 152 us.
+
+constexpr int kFewGroups = 4;
+constexpr int kFewWaves = 4;  // waves per SIMD
+
+// wave_stream without the vertex, kFewGroups groups at a time.
+template <int kApp>
+__device__ __forceinline__ void wave_stream_ahead(const fw_kargs& a, const StepCtx& c, const int lane, const uint32_t w, const uint32_t nw,
+                                                  const uint4 draws, float& S_out, int32_t& sel_out) {
+  constexpr uint32_t kG = 64u * kGroupQuartets;
+  constexpr int kEl = 4 * kGroupQuartets;
+  const uint32_t a0 = c.off & ~3u;
+  const uint32_t nq = (c.off + (uint32_t)c.deg - a0 + 3u) >> 2;
+  const uint32_t ngroups = (nq + kG - 1u) / kG;
+  const uint32_t* __restrict__ bias =
+      reinterpret_cast<const uint32_t*>(kApp == FW_APP_METAPATH ? (const void*)a.label : (const void*)a.weight);
+  float S = 0.0f, Sj = 0.0f, u = 1.0f;
+  int32_t sel = -1;
+  WavePairs pairs{draws, w, 0u};
+  for (uint32_t g0 = w; g0 < ngroups; g0 += (uint32_t)kFewGroups * nw) {
+    uint4 raw[kFewGroups][kGroupQuartets];
+#pragma unroll
+    for (int b = 0; b < kFewGroups; ++b)
+#pragma unroll
+      for (int j = 0; j < kGroupQuartets; ++j) {
+        const uint32_t k = (g0 + (uint32_t)b * nw) * kG + (uint32_t)lane + 64u * (uint32_t)j;
+        raw[b][j] = make_uint4(0u, 0u, 0u, 0u);
+        if (k < nq) raw[b][j] = *reinterpret_cast<const uint4*>(bias + a0 + 4u * k);
+      }
+#pragma unroll
+    for (int b = 0; b < kFewGroups; ++b) {
+      const uint32_t g = g0 + (uint32_t)b * nw;
+      if (g >= ngroups) break;  // wave-uniform
+      const uint32_t kb = g * kG + (uint32_t)lane;
+      float x[kEl];
+#pragma unroll
+      for (int j = 0; j < kGroupQuartets; ++j) {
+        const uint32_t li = a0 + 4u * (kb + 64u * (uint32_t)j) - c.off;  // as in wave_stream
+        const uint32_t r[4] = {raw[b][j].x, raw[b][j].y, raw[b][j].z, raw[b][j].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float y = kApp == FW_APP_METAPATH ? ((int32_t)r[i] == c.want ? 1.0f : 0.0f) : __uint_as_float(r[i]);
+          x[4 * j + i] = li + (uint32_t)i < (uint32_t)c.deg ? y : 0.0f;
+        }
+      }
+      float q = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kEl; ++i) q = q + x[i];
+      const float I = wave_scan(q);
+      const float T = readlane_f(I, 63);
+      const float Snew = S + T;
+      if (Snew * u > Sj) {
+        float tu, u2;
+        next_pair(pairs, a, c.walker, c.step, c.sbase, (uint32_t)lane, tu, u2);
+        const float target = tu * T;
+        const bool pos = q > 0.0f;
+        const uint64_t m = __ballot(pos && I > target);
+        const int l = m != 0ull ? __builtin_ctzll(m) : 63 - __builtin_clzll(__ballot(pos));
+        float e = I - q;
+        uint32_t cnt = 0u, pm = 0u;
+#pragma unroll
+        for (int i = 0; i < kEl; ++i) {
+          e = e + x[i];
+          cnt += e <= target ? 1u : 0u;
+          pm |= (x[i] > 0.0f ? 1u : 0u) << i;
+        }
+        const uint32_t cand = pm >> cnt;
+        const int pick = cand != 0u ? (int)cnt + __builtin_ctz(cand) : 31 - __builtin_clz(pm | 1u);
+        sel = __builtin_amdgcn_readlane((int32_t)(a0 + 4u * kb + 256u * (uint32_t)(pick >> 2) + (uint32_t)(pick & 3) - c.off), l);
+        Sj = Snew;
+        u = u2;
+      }
+      S = Snew;
+    }
+  }
+  S_out = S;
+  sel_out = sel;
+}
+
+// A hub's list whose sequences the waves of a workgroup share out.
+struct HubOffer {
+  StepCtx c;
+  uint32_t claim;  // sequences handed out; at least the number of waves: nothing is on offer
+  uint32_t done;   // sequences whose total and selection are there
+  float w[16];
+  int32_t sel[16];
+};
+
+// One sequence of the list on offer, if any is left.  The wave barriers hold the lanes together: without them the compiler joins the two blocks of
+// lane 0 across the iterations of a caller's loop, lane 0 leaves the others, and these take the value of a lane that has claimed nothing.
+template <int kApp, int kNW>
+__device__ __forceinline__ bool take_sequence(const fw_kargs& a, HubOffer& o, const int lane) {
+  uint32_t seq = 0u;
+  __builtin_amdgcn_wave_barrier();
+  if (lane == 0) seq = __hip_atomic_fetch_add(&o.claim, 1u, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  __builtin_amdgcn_wave_barrier();
+  seq = uniform_u32(seq);
+  if (seq >= (uint32_t)kNW) return false;
+  StepCtx c;
+  c.off = uniform_u32(o.c.off);
+  c.deg = (int32_t)uniform_u32((uint32_t)o.c.deg);
+  c.prev = -1;
+  c.prev_off = 0u;
+  c.prev_deg = 0;
+  c.want = (int32_t)uniform_u32((uint32_t)o.c.want);
+  c.walker = uniform_u32(o.c.walker);
+  c.step = uniform_u32(o.c.step);
+  c.sbase = uniform_u32(o.c.sbase);
+  const uint4 d = wave_draws(a, c.walker, c.step, c.sbase >> 8, (uint32_t)lane);
+  float W;
+  int32_t sel;
+  wave_stream_ahead<kApp>(a, c, lane, seq, (uint32_t)kNW, d, W, sel);
+  if (lane == 0) {
+    o.w[seq] = W;
+    o.sel[seq] = sel;
+    __hip_atomic_fetch_add(&o.done, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __builtin_amdgcn_wave_barrier();
+  return true;
+}
+
+template <int kApp, int kWGT>
+__global__ __launch_bounds__(kWGT, kFewWaves) void fw_walk_few(const fw_kargs a) {
+  constexpr int kNW = kWGT / 64;
+  __shared__ HubOffer s_offer[kNW];
+  __shared__ uint32_t s_open, s_live;  // waves with a list on offer (bits), waves that walk
+  __shared__ unsigned long long s_acc[2];
+  __shared__ int32_t s_schema[kApp == FW_APP_METAPATH ? FW_MAX_SCHEMA : 1];
+  const int lane = lane_id();
+  const uint32_t wave = uniform_u32(threadIdx.x >> 6);
+  if (threadIdx.x < (uint32_t)kNW) s_offer[threadIdx.x].claim = (uint32_t)kNW;
+  if (threadIdx.x == 0u) {
+    s_open = s_live = 0u;
+    s_acc[0] = s_acc[1] = 0ull;
+    if (kApp == FW_APP_METAPATH) {
+#pragma unroll
+      for (int i = 0; i < FW_MAX_SCHEMA; ++i) s_schema[i] = a.schema[i];
+    }
+  }
+  __syncthreads();
+  const uint32_t q = blockIdx.x * (uint32_t)a.slot_limit + wave;
+  uint32_t v = 0xFFFFFFFFu;
+  StepCtx c;
+  c.off = 0u; c.deg = 0; c.prev = -1; c.prev_off = 0u; c.prev_deg = 0; c.want = 0; c.sbase = 0u; c.step = 0u;
+  c.walker = a.walker_base + q;
+  int32_t* const path = a.paths + (uint64_t)q * (uint64_t)a.max_depth;
+  if (wave < (uint32_t)a.slot_limit && q < (uint32_t)a.n) {
+    v = uniform_u32((uint32_t)a.starts[q]);
+    if (lane == 0) path[0] = (int32_t)v;
+    if (v < (uint32_t)a.V && a.max_depth > 1) {
+      c.off = uniform_u32(a.xadj[v]);
+      c.deg = (int32_t)(uniform_u32(a.xadj[v + 1u]) - c.off);
+    }
+  }
+  bool alive = c.deg > 0;
+  if (alive && lane == 0) __hip_atomic_fetch_add(&s_live, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  __syncthreads();
+
+  auto offers = [&] { return uniform_u32(__hip_atomic_load(&s_open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)); };
+  unsigned long long n_edges = 0ull;
+  uint32_t n_steps = 0u;
+  uint32_t kept = 1u;  // entries of the path that are stored
+  int32_t mine = -1;   // the path's entry of the lane's place behind them
+  bool walking = alive;
+  while (walking) {
+    const uint32_t open = offers();
+    if (open != 0u) take_sequence<kApp, kNW>(a, s_offer[__builtin_ctz(open)], lane);
+    if (kApp == FW_APP_METAPATH) c.want = s_schema[c.step % (uint32_t)a.schema_len];
+    const uint4 d = wave_draws(a, c.walker, c.step, c.sbase >> 8, (uint32_t)lane);
+    float W;
+    int32_t sel, nv = -1;
+    if (c.deg > a.hub_threshold) {
+      HubOffer& o = s_offer[wave];
+      if (lane == 0) {
+        o.c = c;
+        o.done = 0u;
+        __hip_atomic_store(&o.claim, 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_or(&s_open, 1u << wave, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      __builtin_amdgcn_wave_barrier();
+      while (take_sequence<kApp, kNW>(a, o, lane)) {}
+      if (lane == 0) __hip_atomic_fetch_and(&s_open, ~(1u << wave), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __builtin_amdgcn_wave_barrier();
+      while (uniform_u32(__hip_atomic_load(&o.done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)) < (uint32_t)kNW) __builtin_amdgcn_s_sleep(1);
+      // inverse transform over the sequences' totals, as in phase B of fw_walk_zprs
+      float Wl = 0.0f;
+      int32_t s = -1;
+      if (lane < kNW) {
+        Wl = o.w[lane];
+        s = o.sel[lane];
+      }
+      const float J = row_scan(Wl);
+      W = readlane_f(J, kNW - 1);
+      const float target = u24(readlane_u32(d.x, kWaveLane)) * W;
+      const bool pos = Wl > 0.0f;
+      const uint64_t m = __ballot(pos && J > target), any = __ballot(pos);
+      sel = -1;
+      if (any != 0ull) sel = __builtin_amdgcn_readlane(s, m != 0ull ? __builtin_ctzll(m) : 63 - __builtin_clzll(any));
+      if (sel >= 0) nv = a.adjncy[c.off + (uint32_t)sel];
+    } else {
+      const uint32_t nq = (c.off + (uint32_t)c.deg - (c.off & ~3u) + 3u) >> 2;
+      if (nq <= 64u * kGroupQuartets) {  // one group: the adjacency with the biases, no dependent load
+        DrawQueue dq;
+        dq.q0 = readlane_u32(d.x, 0u);
+        dq.q1 = readlane_u32(d.y, 0u);
+        dq.q2 = readlane_u32(d.z, 0u);
+        dq.q3 = readlane_u32(d.w, 0u);
+        dq.avail = 4u;
+        dq.blk = 1u;
+        if (nq <= 64u) wave_stream<kApp, 1, true>(a, c, lane, 0u, 1u, dq, W, sel, nv);
+        else wave_stream<kApp, kGroupQuartets, true>(a, c, lane, 0u, 1u, dq, W, sel, nv);
+      } else {
+        wave_stream_ahead<kApp>(a, c, lane, 0u, 1u, d, W, sel);
+        if (sel >= 0) nv = a.adjncy[c.off + (uint32_t)sel];
+      }
+    }
+    if (sel < 0) break;  // no neighbour with a positive bias
+    nv = (int32_t)uniform_u32((uint32_t)nv);
+    if (!n2v_wave_accept<kApp>(a, c, nv, true, lane, W)) {
+      c.sbase += 1u << 8;
+      continue;
+    }
+    n_steps += 1u;
+    n_edges += (unsigned long long)(uint32_t)c.deg;
+    c.prev = (int32_t)v;
+    c.prev_off = c.off;
+    c.prev_deg = c.deg;
+    c.sbase = 0u;
+    c.step += 1u;
+    v = (uint32_t)nv;
+    mine = (uint32_t)lane == c.step - kept ? nv : mine;
+    if (c.step + 1u - kept == 64u) {
+      path[kept + (uint32_t)lane] = mine;
+      kept += 64u;
+    }
+    walking = c.step + 1u < (uint32_t)a.max_depth;
+    if (kApp == FW_APP_PPR && walking) walking = !(u24(readlane_u32(d.x, kStopLane)) < a.tp);  // include/app.cuh:88-94
+    if (walking) {
+      c.off = uniform_u32(a.xadj[v]);
+      c.deg = (int32_t)(uniform_u32(a.xadj[v + 1u]) - c.off);
+      walking = c.deg > 0;
+    }
+  }
+  if (alive && kept + (uint32_t)lane <= c.step) path[kept + (uint32_t)lane] = mine;
+  if (alive && lane == 0) {
+    atomicAdd(&s_acc[0], (unsigned long long)n_steps);
+    atomicAdd(&s_acc[1], n_edges);
+    __hip_atomic_fetch_sub(&s_live, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __builtin_amdgcn_wave_barrier();
+  while (uniform_u32(__hip_atomic_load(&s_live, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != 0u) {
+    const uint32_t open = offers();
+    if (open == 0u || !take_sequence<kApp, kNW>(a, s_offer[__builtin_ctz(open)], lane)) __builtin_amdgcn_s_sleep(8);
+  }
+  __syncthreads();
+  if (threadIdx.x < 2u && s_acc[threadIdx.x] != 0ull) atomicAdd(&a.counters[threadIdx.x], s_acc[threadIdx.x]);
+}
+
 template <int kApp, int kWGT>
 int launch_one(fw_kargs a, int grid, uint32_t entries_hint, hipStream_t stream, int* grid_used) {
   // launches of the parking pipeline (they park, or they continue parked walkers) take the variant with several
   // bundles in flight
+  // Walkers of whole walks, at most as many as waves are resident: a wave each.  Edges that come over the bus stay with the task table, which reads
+  // no neighbours of lists longer than 256.  Measured, wave per walker / task table, us of a call of 40 steps on R-MAT 18, symmetrised: 100 walkers
+  // DeepWalk 118 / 165, PPR 82 / 113, node2vec 144 / 215; 4,096: 179 / 291, 119 / 180, 247 / 566; MetaPath on R-MAT 22 185 / 326.  4,096 walkers of 20
+  // steps from the hubs of R-MAT 22, symmetrised, at a hub threshold of 1024: 314 / 318, 166 / 204, 620 / 824; twice as many there 547 / 486.
+  if (grid <= 0 && a.host_edges == 0 && a.park_threshold == 0x7FFFFFFF && a.resume == nullptr && a.n_dev == nullptr) {
+    int dev = 0, cus = 0;
+    FW_HIP(hipGetDevice(&dev));
+    FW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    if (a.n <= cus * 4 * kFewWaves) {
+      // spread over the workgroups that are resident; the waves without a walker help those that stand on hubs
+      constexpr int kNW = kWGT / 64;
+      const int resident = cus * (4 * kFewWaves / kNW);
+      a.slot_limit = (a.n + resident - 1) / resident;
+      if (a.slot_limit > kNW) a.slot_limit = kNW;
+      const int blocks = (a.n + a.slot_limit - 1) / a.slot_limit;
+      hipLaunchKernelGGL((fw_walk_few<kApp, kWGT>), dim3(blocks), dim3(kWGT), 0, stream, a);
+      FW_HIP(hipGetLastError());
+      if (grid_used) *grid_used = blocks;
+      return FW_OK;
+    }
+  }
   constexpr int kFlight = kPipelineInFlight;
   const bool pipeline = kFlight != 1 && (a.park_threshold != 0x7FFFFFFF || a.resume != nullptr);
   if (grid <= 0) {

@@ -599,3 +599,45 @@ def test_random_access_calibration(gpu):
             assert 1e9 < rate.value < 1e13
     finally:
         buf.free()
+
+
+@pytest.mark.parametrize("wg,thr", [(256, 1024), (512, 16384), (1024, 1024), (512, 1 << 30)])
+def test_few_walkers(gpu, wg, thr):
+    """Either side of the number of walkers up to which a wave walks each, streaming lists and on list tables: lists of one group, of four and five
+    groups at a time, hubs, and biases that grow so fast that a reservoir takes more groups than its draws are made ahead for."""
+    V = 9000
+    rng = np.random.RandomState(wg)
+    deg = rng.randint(0, 9, size=V).astype(np.int64)
+    lengths = [255, 256, 257, 1020, 1024, 1025, 4093, 4096, 4097, 5121, 16385, 40000, 41000, 60000]
+    deg[:len(lengths)] = lengths
+    xadj = np.zeros(V + 1, dtype=np.uint32)
+    np.cumsum(deg, out=xadj[1:])
+    E = int(xadj[-1])
+    adj = np.where(rng.random_sample(E) < 0.3, rng.randint(0, len(lengths), size=E), rng.randint(0, V, size=E)).astype(np.int32)
+    w = (1.0 + rng.random_sample(E)).astype(np.float32)
+    for v in range(V):
+        adj[xadj[v]:xadj[v + 1]].sort()
+        if deg[v] >= 40000:
+            w[xadj[v]:xadj[v + 1]] = np.exp(np.arange(deg[v]) * 0.0005)
+    lab = rng.randint(0, 5, size=E).astype(np.int32)
+    g = gpu.Graph.from_csr(xadj, adj, w, lab)
+    og = _oracle.Graph(xadj, adj, w, lab)
+    try:
+        for i, (kw, n) in enumerate(((dict(app=gpu.APP_DEEPWALK, max_depth=66), 301), (dict(app=gpu.APP_DEEPWALK, max_depth=4), 4096),
+                                     (dict(app=gpu.APP_DEEPWALK, max_depth=4), 4097), (dict(app=gpu.APP_PPR, max_depth=130, tp=0.05), 303),
+                                     (dict(app=gpu.APP_NODE2VEC, max_depth=9, p=0.25, q=4.0), 305), (dict(app=gpu.APP_NODE2VEC, max_depth=9, p=2.0, q=0.5), 307),
+                                     (dict(app=gpu.APP_METAPATH, max_depth=8), 309), (dict(app=gpu.APP_DEEPWALK, max_depth=1), 5))):
+            p = gpu.default_params(wg_threads=wg, hub_threshold=thr, seed=i, park_threshold=-1, **kw)
+            starts = np.where(rng.random_sample(n) < 0.5, rng.randint(0, len(lengths), size=n), rng.randint(-1, V + 1, size=n)).astype(np.int32)
+            ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(p), starts)
+            paths, st = g.walk(p, starts)
+            assert g.engine()[0] == gpu.ENGINE_STREAM
+            assert (paths == ref).all() and (st.steps, st.sampled_edges) == (steps, edges), (kw, n)
+            if kw["app"] != gpu.APP_METAPATH:
+                p.park_threshold = 0
+                g.walk(gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21, wg_threads=wg, hub_threshold=thr), np.resize(starts, 70000))
+                paths, st = g.walk(p, starts)
+                assert g.engine()[0] == gpu.ENGINE_TABLES
+                assert (paths == ref).all() and (st.steps, st.sampled_edges) == (steps, edges), (kw, n)
+    finally:
+        g.destroy()
