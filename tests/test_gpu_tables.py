@@ -625,3 +625,35 @@ def test_short_rows_of_many_queries(gpu, grid, n, depth):
             assert (st.steps, st.sampled_edges) == (steps, edges)
     finally:
         g.destroy()
+
+
+@pytest.mark.parametrize("depth", [17, 31, 32, 33, 65, 100])
+def test_rows_end_anywhere_in_a_line(gpu, depth):
+    """Rows that begin and end at every place of a 64-byte line, walks of one entry to all of them, many that end together; nothing is
+    stored before the matrix or behind it."""
+    csr, at = _lists("uneven")
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    rng = np.random.RandomState(depth)
+    n = 3001
+    try:
+        g.walk(gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21), at[rng.randint(0, len(at), size=70000)].astype(np.int32))
+        starts = np.where(rng.random_sample(n) < 0.5, at[rng.randint(0, len(at), size=n)], rng.randint(0, V, size=n)).astype(np.int32)
+        starts_dev = torch.from_numpy(starts).cuda()
+        for app, tp, before in ((gpu.APP_PPR, 0.3, 0), (gpu.APP_PPR, 0.03, 7), (gpu.APP_DEEPWALK, 0.0, 5)):
+            p = gpu.default_params(app=app, max_depth=depth, tp=tp, seed=depth, grid=2)
+            ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(p), starts)
+            room = torch.full((before + n * depth + 32,), 12345, dtype=torch.int32, device="cuda")
+            torch.cuda.synchronize()
+            st = gpu.WalkStats()
+            gpu.check(gpu.lib().fw_walk_device(g.handle, C.byref(p), C.c_void_p(starts_dev.data_ptr()), n,
+                                               C.c_void_p(room.data_ptr() + 4 * before), None, C.byref(st)))
+            assert g.engine()[0] == gpu.ENGINE_TABLES
+            out = room.cpu().numpy()
+            paths = out[before:before + n * depth].reshape(n, depth)
+            bad = np.nonzero((paths != ref).any(axis=1))[0]
+            assert len(bad) == 0, (app, before, bad[0], paths[bad[0]], ref[bad[0]])
+            assert (out[:before] == 12345).all() and (out[before + n * depth:] == 12345).all()
+            assert (st.steps, st.sampled_edges) == (steps, edges)
+    finally:
+        g.destroy()
