@@ -9,21 +9,25 @@ namespace {
 
 // ---- Philox4x32-10 ---------------------------------------------------------------------------
 
-// x ^ y ^ z in one instruction (the compiler makes two of it, 20 more in a block of draws, and a step begins with one: 3,001 streaming
-// walkers 153.6 -> 150.4 us, 50,021 node2vec walkers on tables 489 -> 477, large calls unchanged).
+// x ^ y ^ z.  kLanes: in one vector instruction (the compiler makes two of it, 20 more in a block of draws: 3,001 streaming walkers
+// 153.6 -> 150.4 us, 50,021 node2vec walkers on tables 489 -> 477).
+template <bool kLanes>
 __device__ __forceinline__ uint32_t xor3(uint32_t x, uint32_t y, uint32_t z) {
-  return (uint32_t)__builtin_amdgcn_bitop3_b32((int)x, (int)y, (int)z, 0x96);
+  return kLanes ? (uint32_t)__builtin_amdgcn_bitop3_b32((int)x, (int)y, (int)z, 0x96) : x ^ y ^ z;
 }
 
+// kLanes: the lanes ask for blocks of their own.  Off where all of them ask for the same one: the whole block is then made on the scalar unit, which
+// has no three-way exclusive or, and one vector instruction would take all of it from there.
+template <bool kLanes = false>
 __device__ __forceinline__ uint4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
                                                uint32_t k1) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
     const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
     const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
-    const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c1, k0);
+    const uint32_t n0 = xor3<kLanes>((uint32_t)(p1 >> 32), c1, k0);
     const uint32_t n1 = (uint32_t)p1;
-    const uint32_t n2 = xor3((uint32_t)(p0 >> 32), c3, k1);
+    const uint32_t n2 = xor3<kLanes>((uint32_t)(p0 >> 32), c3, k1);
     const uint32_t n3 = (uint32_t)p0;
     c0 = n0; c1 = n1; c2 = n2; c3 = n3;
     k0 += 0x9E3779B9u;

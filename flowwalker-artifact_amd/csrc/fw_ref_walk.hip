@@ -126,7 +126,7 @@ struct RefDraws {
   __device__ __forceinline__ float next(const fw_kargs& a, const RefStep& s, const RefRng& r, uint32_t W, uint32_t t,
                                         uint32_t j) {
     if (kRng == 0) {
-      if ((j & 3u) == 0u) blk = philox4x32_10(s.walker, s.step, kStreamRef, (j >> 2) * W + t, a.seed_lo, a.seed_hi);
+      if ((j & 3u) == 0u) blk = philox4x32_10<true>(s.walker, s.step, kStreamRef, (j >> 2) * W + t, a.seed_lo, a.seed_hi);
       const uint32_t k = j & 3u;
       const uint32_t bits = k == 0u ? blk.x : (k == 1u ? blk.y : (k == 2u ? blk.z : blk.w));
       return ref_u(bits);
@@ -135,7 +135,7 @@ struct RefDraws {
     if (kRng == 1) {
       const uint32_t n = r.lds_n[r.tid];
       if ((n & 3u) == 0u) {
-        const uint4 b = philox4x32_10(r.gid, n >> 2, kStreamThread, 0u, a.seed_lo, a.seed_hi);
+        const uint4 b = philox4x32_10<true>(r.gid, n >> 2, kStreamThread, 0u, a.seed_lo, a.seed_hi);
         r.lds_w[0u * r.threads + r.tid] = b.x;
         r.lds_w[1u * r.threads + r.tid] = b.y;
         r.lds_w[2u * r.threads + r.tid] = b.z;
@@ -147,7 +147,7 @@ struct RefDraws {
       volatile RefThreadState* st = r.dev;  // every draw goes to memory and back, as a cuRAND state does
       const uint32_t n = st->n;
       if ((n & 3u) == 0u) {
-        const uint4 b = philox4x32_10(r.gid, n >> 2, kStreamThread, 0u, a.seed_lo, a.seed_hi);
+        const uint4 b = philox4x32_10<true>(r.gid, n >> 2, kStreamThread, 0u, a.seed_lo, a.seed_hi);
         st->w[0] = b.x;
         st->w[1] = b.y;
         st->w[2] = b.z;
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(1024) void fw_walk_ref(const fw_kargs a, const int 
         stop = len >= a.max_depth || t_deg[tid] == 0;
         if (kApp == FW_APP_PPR && !stop && t_moved[tid]) {  // include/app.cuh:88-94: one draw per completed step
           const uint32_t w = a.walker_base + (uint32_t)t_walker[tid];
-          const uint32_t bits = philox4x32_10(w, (uint32_t)(len - 2), kStreamStopRef, 0u, a.seed_lo, a.seed_hi).x;
+          const uint32_t bits = philox4x32_10<true>(w, (uint32_t)(len - 2), kStreamStopRef, 0u, a.seed_lo, a.seed_hi).x;
           stop = u24(bits) < a.tp;
         }
         t_moved[tid] = 0;

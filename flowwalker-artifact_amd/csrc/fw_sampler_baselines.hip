@@ -142,7 +142,7 @@ __global__ __launch_bounds__(1024) void fw_bench_its_block(const BenchArgs a) {
 // Proposals of one round: lane-th (index, height) pair of round r of task position p.
 __device__ __forceinline__ bool rjs_try(const BenchArgs& a, const float* w, uint32_t p, uint32_t round, uint32_t t,
                                         float wmax, uint32_t* idx_out) {
-  const uint4 b = philox4x32_10(p, round, kStreamBench + 1u, t, a.seed_lo, a.seed_hi);
+  const uint4 b = philox4x32_10<true>(p, round, kStreamBench + 1u, t, a.seed_lo, a.seed_hi);
   const uint32_t x = (uint32_t)(((uint64_t)b.x * a.list_len) >> 32);  // uniform index
   const float y = u24(b.y) * wmax;
   *idx_out = x;

@@ -98,9 +98,11 @@ __device__ __forceinline__ N2vTest n2v_test(const fw_kargs& a, int32_t post, int
   return t;
 }
 
+template <bool kLanes>
 __device__ __forceinline__ N2vTest n2v_test(const fw_kargs& a, int32_t post, int32_t prev, uint32_t walker, uint32_t step,
                                             uint32_t trial, float T, float w_ret) {
-  return n2v_test(a, post, prev, trial, T, w_ret, [&] { return philox4x32_10(walker, step, kStreamAccept | (trial << 8), 0u, a.seed_lo, a.seed_hi); });
+  return n2v_test(a, post, prev, trial, T, w_ret,
+                  [&] { return philox4x32_10<kLanes>(walker, step, kStreamAccept | (trial << 8), 0u, a.seed_lo, a.seed_hi); });
 }
 
 // the other half: `common` = the proposal is a neighbour of prev
@@ -118,7 +120,7 @@ struct LaneDraw {
 __device__ __forceinline__ float next_uniform_lane(LaneDraw& d, const fw_kargs& a, uint32_t walker, uint32_t step,
                                                    uint32_t stream) {
   if (d.avail == 0u) {
-    const uint4 b = philox4x32_10(walker, step, stream, d.blk, a.seed_lo, a.seed_hi);
+    const uint4 b = philox4x32_10<true>(walker, step, stream, d.blk, a.seed_lo, a.seed_hi);
     d.q0 = b.x; d.q1 = b.y; d.q2 = b.z; d.q3 = b.w;
     d.avail = 4u;
     ++d.blk;
@@ -144,7 +146,7 @@ __device__ __forceinline__ uint4 wave_draws(const fw_kargs& a, uint32_t walker, 
   stream = lane == kWaveLane ? kStreamWave | sbase : stream;
   stream = lane == kStopLane ? kStreamStop : stream;
   stream = lane == kAcceptLane ? kStreamAccept | sbase : stream;
-  return philox4x32_10(walker, step, stream, lane < kWaveLane ? lane >> 4 : 0u, a.seed_lo, a.seed_hi);
+  return philox4x32_10<true>(walker, step, stream, lane < kWaveLane ? lane >> 4 : 0u, a.seed_lo, a.seed_hi);
 }
 
 // The uniforms of a sequence's reservoir, two per accepted group: the words of its stream in order.
@@ -158,7 +160,7 @@ __device__ __forceinline__ void next_pair(WavePairs& p, const fw_kargs& a, uint3
                                           uint32_t lane, float& first, float& second) {
   uint32_t from = p.seq + 16u * (p.i >> 1);
   if (p.i >= 6u) {  // past the blocks made beforehand
-    if (p.i == 6u || (p.i & 127u) == 0u) p.e = philox4x32_10(walker, step, p.seq | sbase, 64u * (p.i >> 7) + lane, a.seed_lo, a.seed_hi);
+    if (p.i == 6u || (p.i & 127u) == 0u) p.e = philox4x32_10<true>(walker, step, p.seq | sbase, 64u * (p.i >> 7) + lane, a.seed_lo, a.seed_hi);
     from = (p.i >> 1) & 63u;
   }
   first = u24(readlane_u32((p.i & 1u) ? p.e.z : p.e.x, from));

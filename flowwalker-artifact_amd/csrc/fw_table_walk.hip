@@ -885,7 +885,7 @@ __device__ __forceinline__ const float* sums_reservoir(const fw_kargs& a, const 
 // The sequence of groups a step at workgroup granularity goes to, by the scan of the sequences' totals.
 __device__ __forceinline__ uint32_t which_sequence(const fw_kargs& a, const float* scan, const float total, const uint32_t walker,
                                                    const uint32_t step, const uint32_t sbase) {
-  const float target = u24(philox4x32_10(walker, step, kStreamWave | sbase, 0u, a.seed_lo, a.seed_hi).x) * total;
+  const float target = u24(philox4x32_10<true>(walker, step, kStreamWave | sbase, 0u, a.seed_lo, a.seed_hi).x) * total;
   float keys[16];
   load16(scan, keys);
   uint32_t seq = 0u;
@@ -1073,7 +1073,7 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
         rec = tb.vrec[v];
       }
     }
-    const uint4 d = philox4x32_10(walker, step, sbase, 0u, a.seed_lo, a.seed_hi);
+    const uint4 d = philox4x32_10<true>(walker, step, sbase, 0u, a.seed_lo, a.seed_hi);
     if (active && !ended) {
       int32_t nv = -1;
       bool none;  // no neighbour with a positive bias (include/walker.cuh:1373-1374)
@@ -1094,7 +1094,7 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
             w_ret = at >= 0 ? tb.set_weights[at] : 0.0f;
             if (at == -2) w_ret = return_weight(a.adjncy + rec.w, a.weight + rec.w, rec.y, prev);
           }
-          const N2vTest t = n2v_test(a, nv, prev, walker, step, trial, __uint_as_float(rec.z), w_ret);
+          const N2vTest t = n2v_test<true>(a, nv, prev, walker, step, trial, __uint_as_float(rec.z), w_ret);
           if (t.take_prev) {
             nv = prev;
           } else {
@@ -1128,7 +1128,7 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
           len += 1u;
           ended = len >= md;
           if (kApp == FW_APP_PPR && !ended) {  // include/app.cuh:88-94
-            const uint32_t bits = philox4x32_10(walker, step, kStreamStop, 0u, a.seed_lo, a.seed_hi).x;
+            const uint32_t bits = philox4x32_10<true>(walker, step, kStreamStop, 0u, a.seed_lo, a.seed_hi).x;
             ended = u24(bits) < a.tp;
           }
           if (slot == 15u) {

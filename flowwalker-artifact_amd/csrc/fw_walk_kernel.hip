@@ -14,7 +14,7 @@
 // "S * u > Sj" uses one uniform per ACCEPTED group (the probability of no acceptance between two
 // groups telescopes to a ratio of running sums), so the common iteration has no random draw and no
 // divergent branch.  Inside an accepted group the element is found by inverse transform on the scan
-// prefix.  All draws of a step are wave-uniform, so Philox runs on the scalar unit.
+// prefix.  All draws of a step are wave-uniform, so Philox runs on the scalar unit (but see kVectorDraws).
 //
 // Round structure of one workgroup (WGT threads, WGT task slots in LDS, SoA):
 //   B  every hub slot (degree > hub_threshold) is streamed by the whole workgroup, wave w taking
@@ -112,9 +112,16 @@ struct DrawQueue {
   uint32_t blk = 0;
 };
 
+// Where the wave-uniform draws are made.  On the scalar unit they take no vector registers: in vector form the DeepWalk kernels take seven more and the one
+// of 1024 threads spills twice as much (40,000 walkers of 40 steps on R-MAT 18, symmetrised, 726 -> 754 us; PPR there 271 -> 280; with 512 threads
+// alike).  MetaPath's kernels have the registers, and the scalar unit's chain of multiplications is the longer one (uniform graph of mean degree 8, 163 -> 160).
+template <int kApp>
+constexpr bool kVectorDraws = kApp == FW_APP_METAPATH;
+
+template <int kApp>
 __device__ __forceinline__ float next_uniform(DrawQueue& d, const fw_kargs& a, const StepCtx& c, uint32_t stream) {
   if (d.avail == 0u) {
-    const uint4 b = philox4x32_10(c.walker, c.step, stream | c.sbase, d.blk, a.seed_lo, a.seed_hi);
+    const uint4 b = philox4x32_10<kVectorDraws<kApp>>(c.walker, c.step, stream | c.sbase, d.blk, a.seed_lo, a.seed_hi);
     d.q0 = b.x; d.q1 = b.y; d.q2 = b.z; d.q3 = b.w;
     d.avail = 4u;
     ++d.blk;
@@ -211,7 +218,7 @@ __device__ __forceinline__ void wave_stream(const fw_kargs& a, const StepCtx& c,
     const float T = readlane_f(I, 63);
     const float Snew = S + T;
     if (Snew * u > Sj) {  // wave-uniform: the reservoir accepts this group
-      const float target = next_uniform(dq, a, c, w) * T;
+      const float target = next_uniform<kApp>(dq, a, c, w) * T;
       const bool pos = q > 0.0f;
       const uint64_t m = __ballot(pos && I > target);
       int l;
@@ -247,7 +254,7 @@ __device__ __forceinline__ void wave_stream(const fw_kargs& a, const StepCtx& c,
         selv = __builtin_amdgcn_readlane(v, l);
       }
       Sj = Snew;
-      u = next_uniform(dq, a, c, w);
+      u = next_uniform<kApp>(dq, a, c, w);
     }
     S = Snew;
   }
@@ -322,15 +329,16 @@ __device__ __forceinline__ StepCtx load_ctx(const fw_kargs& a, const TaskTable<k
 // node2vec, all lanes of the wave: is the (wave-uniform) proposal v of the step accepted?  The lanes look it up in
 // N(prev) together when the answer matters.
 // T: the list's total as the step's sampler added it up.  v becomes the previous vertex when the trial takes the
-// return edge's own component.
-template <int kApp>
+// return edge's own component.  kLanes: the draw in vector form (in the walk of few walkers, where nothing else fills the time:
+// 3,001 of them on R-MAT 18, symmetrised, 209 -> 205 us; the task table has no registers for it, see kVectorDraws).
+template <int kApp, bool kLanes>
 __device__ __forceinline__ bool n2v_wave_accept(const fw_kargs& a, const StepCtx& c, int32_t& v, bool ok, int lane,
                                                 float T) {
   if (kApp != FW_APP_NODE2VEC || !ok) return true;
   float w_ret = 0.0f;
   if (a.n2v_extra > 0.0f && c.prev >= 0)  // wave-uniform: every lane walks the same few entries
     w_ret = return_weight(a.adjncy + c.off, a.weight + c.off, (uint32_t)c.deg, c.prev);
-  const N2vTest t = n2v_test(a, v, c.prev, c.walker, c.step, c.sbase >> 8, T, w_ret);  // wave-uniform
+  const N2vTest t = n2v_test<kLanes>(a, v, c.prev, c.walker, c.step, c.sbase >> 8, T, w_ret);  // wave-uniform
   if (t.take_prev) {
     v = c.prev;
     return true;
@@ -516,7 +524,7 @@ __device__ __forceinline__ void packed_finish(const fw_kargs& a, TaskTable<kWGT,
       }
     }
     if (active && accept) {
-      t = n2v_test(a, selv, tt.prev[slot], a.walker_base + (uint32_t)tt.walker[slot], (uint32_t)(len - 1),
+      t = n2v_test<true>(a, selv, tt.prev[slot], a.walker_base + (uint32_t)tt.walker[slot], (uint32_t)(len - 1),
                    (uint32_t)tt.trial[slot], T, w_ret);  // the same in every lane of the segment
       if (t.take_prev) selv = tt.prev[slot];
       if (!t.decided) {
@@ -651,7 +659,7 @@ __global__ __launch_bounds__(kWGT, kPackedInFlight == 1 ? 8 : 4) void fw_walk_zp
           // inverse transform over the wave totals (lanes >= kNW hold 0 and never qualify)
           const float J = row_scan(W);
           const float total = readlane_f(J, kNW - 1);
-          const uint32_t bits = philox4x32_10(c.walker, c.step, kStreamWave | c.sbase, 0u, a.seed_lo, a.seed_hi).x;
+          const uint32_t bits = philox4x32_10<kVectorDraws<kApp>>(c.walker, c.step, kStreamWave | c.sbase, 0u, a.seed_lo, a.seed_hi).x;
           const float target = u24(bits) * total;
           const bool pos = W > 0.0f;
           uint64_t m = __ballot(pos && J > target);
@@ -664,7 +672,7 @@ __global__ __launch_bounds__(kWGT, kPackedInFlight == 1 ? 8 : 4) void fw_walk_zp
           }
           int32_t v = -1;
           if (pick >= 0) v = a.adjncy[c.off + (uint32_t)pick];  // wave-uniform
-          const bool accepted = n2v_wave_accept<kApp>(a, c, v, pick >= 0, lane, total);
+          const bool accepted = n2v_wave_accept<kApp, false>(a, c, v, pick >= 0, lane, total);
           if (lane == 0) commit(a, tt, slot, c, v, pick >= 0, accepted, n_steps, n_edges);
         }
         if (hb + kHubChunk < nh) __syncthreads();  // the partial buffers are reused by the next chunk
@@ -731,7 +739,7 @@ __global__ __launch_bounds__(kWGT, kPackedInFlight == 1 ? 8 : 4) void fw_walk_zp
           wave_stream<kApp, kGroupQuartets, false>(a, c, lane, 0u, 1u, dq0, W, sel, selv);
           if (sel >= 0) v = a.adjncy[c.off + (uint32_t)sel];
         }
-        const bool accepted = n2v_wave_accept<kApp>(a, c, v, sel >= 0, lane, W);
+        const bool accepted = n2v_wave_accept<kApp, false>(a, c, v, sel >= 0, lane, W);
         if (lane == 0) commit(a, tt, slot, c, v, sel >= 0, accepted, n_steps, n_edges);
       }
       __syncthreads();
@@ -770,7 +778,7 @@ __global__ __launch_bounds__(kWGT, kPackedInFlight == 1 ? 8 : 4) void fw_walk_zp
           bool stop = len >= a.max_depth || deg == 0;
           if (kApp == FW_APP_PPR && !stop) {  // include/app.cuh:88-94: one draw per completed step
             const uint32_t w = a.walker_base + (uint32_t)tt.walker[tid];
-            const uint32_t bits = philox4x32_10(w, (uint32_t)(len - 2), kStreamStop, 0u, a.seed_lo, a.seed_hi).x;
+            const uint32_t bits = philox4x32_10<true>(w, (uint32_t)(len - 2), kStreamStop, 0u, a.seed_lo, a.seed_hi).x;
             stop = u24(bits) < a.tp;
           }
           need = stop;
@@ -905,7 +913,7 @@ __global__ __launch_bounds__(kWGT, kPackedInFlight == 1 ? 8 : 4) void fw_walk_zp
           }
           if (kApp == FW_APP_METAPATH) tt.want[tid] = tt.schema[(uint32_t)(len - 1) % (uint32_t)a.schema_len];
           const uint32_t sbase = kApp == FW_APP_NODE2VEC ? (uint32_t)tt.trial[tid] << 8 : 0u;
-          const uint4 b = philox4x32_10(a.walker_base + (uint32_t)tt.walker[tid], (uint32_t)(len - 1), sbase, 0u,
+          const uint4 b = philox4x32_10<true>(a.walker_base + (uint32_t)tt.walker[tid], (uint32_t)(len - 1), sbase, 0u,
                                         a.seed_lo, a.seed_hi);
           tt.draw[0][tid] = b.x;
           tt.draw[1][tid] = b.y;
@@ -1269,7 +1277,7 @@ __device__ __forceinline__ int32_t table_sample(const fw_kargs& a, const uint32_
     const float J = row_scan(Wl);
     const float total = readlane_f(J, kNW - 1);
     total_out = total;
-    const float target = u24(philox4x32_10(walker, step, kStreamWave | sbase, 0u, a.seed_lo, a.seed_hi).x) * total;
+    const float target = u24(philox4x32_10<true>(walker, step, kStreamWave | sbase, 0u, a.seed_lo, a.seed_hi).x) * total;
     int wlast = -1;
     wsel = -1;
 #pragma unroll
@@ -1336,7 +1344,7 @@ __device__ __forceinline__ void batch_commit(const fw_kargs& a, const fw_hub_arg
     if (kApp == FW_APP_NODE2VEC && rec.prev >= 0) {
       float w_ret = 0.0f;  // T: the list's total as the step's sampler added it up
       if (a.n2v_extra > 0.0f) w_ret = return_weight(a.adjncy + off, a.weight + off, deg, rec.prev);
-      const N2vTest t = n2v_test(a, nv, rec.prev, walker, step, trial, T, w_ret);
+      const N2vTest t = n2v_test<true>(a, nv, rec.prev, walker, step, trial, T, w_ret);
       if (t.take_prev) {  // the return edge's own component: back to the previous vertex
         nv = rec.prev;
         if (a.adj_hub != nullptr) nv_hidx = a.hub_index[nv];
@@ -1356,7 +1364,7 @@ __device__ __forceinline__ void batch_commit(const fw_kargs& a, const fw_hub_arg
   if (moved) {
     go_on = rec.len + 1 < a.max_depth;
     if (kApp == FW_APP_PPR && go_on) {
-      const uint32_t bits = philox4x32_10(walker, step, kStreamStop, 0u, a.seed_lo, a.seed_hi).x;
+      const uint32_t bits = philox4x32_10<true>(walker, step, kStreamStop, 0u, a.seed_lo, a.seed_hi).x;
       go_on = !(u24(bits) < a.tp);
     }
   }
@@ -1576,7 +1584,7 @@ __global__ __launch_bounds__(kWGT, 8) void fw_hub_batch(const fw_kargs a, const 
       const float total = readlane_f(J, kNW - 1);
       int32_t pick = -1;
       if (have) {
-        const float target = u24(philox4x32_10(walker, step, kStreamWave | (trial << 8), 0u, a.seed_lo, a.seed_hi).x) * total;
+        const float target = u24(philox4x32_10<true>(walker, step, kStreamWave | (trial << 8), 0u, a.seed_lo, a.seed_hi).x) * total;
         int wsel = -1, wlast = -1;
 #pragma unroll
         for (int w = 0; w < kNW; ++w) {
@@ -2174,7 +2182,7 @@ __global__ __launch_bounds__(kWGT, kFewWaves) void fw_walk_few(const fw_kargs a)
     }
     if (sel < 0) break;  // no neighbour with a positive bias
     nv = (int32_t)uniform_u32((uint32_t)nv);
-    if (!n2v_wave_accept<kApp>(a, c, nv, true, lane, W)) {
+    if (!n2v_wave_accept<kApp, true>(a, c, nv, true, lane, W)) {
       c.sbase += 1u << 8;
       continue;
     }

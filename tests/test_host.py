@@ -3,6 +3,7 @@ the on-disk CSR format, input validation and the command-line front end.  No GPU
 import ctypes as C
 import os
 import re
+import shutil
 import subprocess
 import sys
 
@@ -245,3 +246,29 @@ def test_bench_byte_formulas():
     assert bench.algorithmic_bytes("metapath", 10, 1000, 3) == bench.algorithmic_bytes("ppr", 10, 1000, 3)
     assert bench.algorithmic_bytes("node2vec", 10, 1000, 3) == 8 * 1000 + 24 * 10 + 16 * 3
     assert bench.HBM_PEAK_GBS == 8000.0
+
+
+def _device_code(fw, symbol, tmp_path):
+    """Instructions of one kernel of the built library."""
+    objdump = "/opt/rocm/llvm/bin/llvm-objdump"
+    lib = os.path.join(ROOT, "flowwalker-artifact_amd", "lib", "libflowwalker_hip.so")
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    shutil.copy(lib, tmp_path / "lib.so")
+    subprocess.run([objdump, "--offloading", "lib.so"], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+    for name in sorted(os.listdir(tmp_path)):
+        if name.endswith("gfx950"):
+            out = subprocess.run([objdump, "-d", "--disassemble-symbols=" + symbol, name], cwd=tmp_path, check=True,
+                                 stdout=subprocess.PIPE, text=True).stdout
+            if "<%s>:" % symbol in out:
+                return out
+    raise AssertionError("no kernel %s in the library" % symbol)
+
+
+@pytest.mark.parametrize("wg", [256, 512, 1024])
+def test_draws_of_the_streaming_kernels_are_made_on_the_scalar_unit(fw, wg, tmp_path):
+    """All lanes of a wave that streams a list ask for the same block of draws: 20 scalar multiplications, at two places of a kernel at least (the
+    reservoir's draws, the choice among a workgroup's sequences).  One vector instruction among them would take the whole block off the scalar unit."""
+    for app in (fw.APP_DEEPWALK, fw.APP_PPR, fw.APP_NODE2VEC):
+        code = _device_code(fw, "_ZN12_GLOBAL__N_112fw_walk_zprsILi%dELi%dELi1EEEv8fw_kargs" % (app, wg), tmp_path)
+        assert code.count("s_mul_hi_u32") >= 40, (app, code.count("s_mul_hi_u32"))
