@@ -1160,30 +1160,47 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
         }
         ev = 0ull;
       }
-      // Four rows at a time, 16 lanes each: one line from LDS, then pieces of 16 bytes.  (Rows one after the other, 64 entries a store, waited for LDS
-      // twice a row: 1,000,003 PPR walkers from the hub of R-MAT 21 636 -> 623 us, PPR R-MAT 22 1115 -> 1108, DeepWalk there and node2vec unchanged.)
-      while (ev != 0ull) {
-        int row_lane[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          row_lane[i] = ev != 0ull ? __builtin_ctzll(ev) : -1;
-          ev &= ev - 1ull;  // (0 stays 0)
+      if constexpr (kApp == FW_APP_NODE2VEC) {
+        // One row at a time, 64 entries a store.  Four at a time, as below, are the slower way here but for the shortest walks (one row / four, medians of five
+        // processes, all vertices of R-MAT 24, symmetrised, 80 steps 58.2 / 59.0 ms, half of them 33.7 / 34.1, 41 steps 17.14 / 17.29, 20 steps 8.37 / 8.38; R-MAT 22 80
+        // steps 7.99 / 8.01, 20 steps 2.61 / 2.60; R-MAT 20, symmetrised, p = 0.25, q = 4, 40 steps 6.28 / 6.31).
+        for (; ev != 0ull; ev &= ev - 1ull) {
+          const uint32_t l = (uint32_t)__builtin_ctzll(ev);
+          const uint32_t lq = readlane_u32(q, l), from = readlane_u32(fpos, l), to = readlane_u32(end, l);
+          const uint32_t have = readlane_u32(len, l), ls0 = readlane_u32(s0, l);
+          int32_t* const row = a.paths + (uint64_t)lq * md;
+          for (uint32_t p = from + (uint32_t)lane; p < to; p += 64u) {
+            const uint32_t slot = (ls0 + p) & 15u;
+            row[p] = p < have ? buf[l * 16u + ((((slot >> 2) ^ ((l >> 2) & 3u)) << 2) | (slot & 3u))] : -1;
+          }
         }
-        const uint32_t part = (uint32_t)lane >> 4, sub = (uint32_t)lane & 15u;
-        const int l = part < 2u ? (part == 0u ? row_lane[0] : row_lane[1]) : (part == 2u ? row_lane[2] : row_lane[3]);
-        const int src = l >= 0 ? l : 0;
-        const uint32_t lq = (uint32_t)__shfl((int)q, src), have = (uint32_t)__shfl((int)len, src);
-        const uint32_t from = (uint32_t)__shfl((int)fpos, src), ls0 = (uint32_t)__shfl((int)s0, src);
-        const uint32_t row_end = (uint32_t)__shfl((int)end, src);
-        const uint32_t to = l >= 0 ? row_end : 0u;
-        int32_t* const row = a.paths + (uint64_t)lq * md;
-        // what is not stored of the walk lies in one line: that line, then -1 in pieces of 16 bytes
-        const uint32_t line = from - ((ls0 + from) & 15u);  // (wraps where the row begins inside the line; to is below 2^31)
-        const uint32_t p = line + sub;
-        if (p >= from && p < to) row[p] = p < have ? buf[(uint32_t)src * 16u + ((((sub >> 2) ^ (((uint32_t)src >> 2) & 3u)) << 2) | (sub & 3u))] : -1;
-        uint32_t piece = line + 16u + 4u * sub;
-        for (; piece + 4u <= to; piece += 64u) *reinterpret_cast<int4*>(row + piece) = make_int4(-1, -1, -1, -1);
-        for (; piece < to; ++piece) row[piece] = -1;  // up to three, of one lane
+      } else {
+        // Four rows at a time, 16 lanes each: one line from LDS, then pieces of 16 bytes.  (Rows one after the other, 64 entries a store, waited for LDS
+        // twice a row: 1,000,003 PPR walkers from the hub of R-MAT 21 636 -> 623 us, PPR R-MAT 22 1115 -> 1108, of 20 steps 1015 -> 983, DeepWalk of 20 steps
+        // there 2175 -> 2160, of 80 unchanged.)
+        while (ev != 0ull) {
+          int row_lane[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            row_lane[i] = ev != 0ull ? __builtin_ctzll(ev) : -1;
+            ev &= ev - 1ull;  // (0 stays 0)
+          }
+          const uint32_t part = (uint32_t)lane >> 4, sub = (uint32_t)lane & 15u;
+          const int l = part < 2u ? (part == 0u ? row_lane[0] : row_lane[1]) : (part == 2u ? row_lane[2] : row_lane[3]);
+          const int src = l >= 0 ? l : 0;
+          const uint32_t lq = (uint32_t)__shfl((int)q, src), have = (uint32_t)__shfl((int)len, src);
+          const uint32_t from = (uint32_t)__shfl((int)fpos, src), ls0 = (uint32_t)__shfl((int)s0, src);
+          const uint32_t row_end = (uint32_t)__shfl((int)end, src);
+          const uint32_t to = l >= 0 ? row_end : 0u;
+          int32_t* const row = a.paths + (uint64_t)lq * md;
+          // what is not stored of the walk lies in one line: that line, then -1 in pieces of 16 bytes
+          const uint32_t line = from - ((ls0 + from) & 15u);  // (wraps where the row begins inside the line; to is below 2^31)
+          const uint32_t p = line + sub;
+          if (p >= from && p < to) row[p] = p < have ? buf[(uint32_t)src * 16u + ((((sub >> 2) ^ (((uint32_t)src >> 2) & 3u)) << 2) | (sub & 3u))] : -1;
+          uint32_t piece = line + 16u + 4u * sub;
+          for (; piece + 4u <= to; piece += 64u) *reinterpret_cast<int4*>(row + piece) = make_int4(-1, -1, -1, -1);
+          for (; piece < to; ++piece) row[piece] = -1;  // up to three, of one lane
+        }
       }
       __builtin_amdgcn_wave_barrier();
       if (partial) fpos = len;

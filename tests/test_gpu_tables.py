@@ -657,3 +657,34 @@ def test_rows_end_anywhere_in_a_line(gpu, depth):
             assert (st.steps, st.sampled_edges) == (steps, edges)
     finally:
         g.destroy()
+
+
+@pytest.mark.parametrize("depth", [17, 32, 33, 65])
+def test_node2vec_rows_end_anywhere_in_a_line(gpu, depth):
+    """As above for node2vec, whose walkers turn down proposals and come to the ends of their lines and rows at different times."""
+    csr, at = _lists("uneven")
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    rng = np.random.RandomState(depth)
+    n = 1501
+    try:
+        g.walk(gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21), at[rng.randint(0, len(at), size=70000)].astype(np.int32))
+        starts = np.where(rng.random_sample(n) < 0.5, at[rng.randint(0, len(at), size=n)], rng.randint(0, V, size=n)).astype(np.int32)
+        starts_dev = torch.from_numpy(starts).cuda()
+        p = gpu.default_params(app=gpu.APP_NODE2VEC, max_depth=depth, p=2.0, q=0.5, seed=depth, grid=2)
+        ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(p), starts)
+        for before in (0, 7):
+            room = torch.full((before + n * depth + 32,), 12345, dtype=torch.int32, device="cuda")
+            torch.cuda.synchronize()
+            st = gpu.WalkStats()
+            gpu.check(gpu.lib().fw_walk_device(g.handle, C.byref(p), C.c_void_p(starts_dev.data_ptr()), n,
+                                               C.c_void_p(room.data_ptr() + 4 * before), None, C.byref(st)))
+            assert g.engine()[0] == gpu.ENGINE_TABLES and st.grid == 2
+            out = room.cpu().numpy()
+            paths = out[before:before + n * depth].reshape(n, depth)
+            bad = np.nonzero((paths != ref).any(axis=1))[0]
+            assert len(bad) == 0, (before, bad[0], paths[bad[0]], ref[bad[0]])
+            assert (out[:before] == 12345).all() and (out[before + n * depth:] == 12345).all()
+            assert (st.steps, st.sampled_edges) == (steps, edges)
+    finally:
+        g.destroy()
