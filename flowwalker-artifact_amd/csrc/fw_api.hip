@@ -1935,6 +1935,8 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
     }
     t->have_sets = t->have_weights = false;
     const int rc = plan_tables(g, t, stream);
+    double mean = 0.0;
+    if (rc == FW_OK && mean_list_length(g, &mean) != FW_OK) (void)hipGetLastError();  // (the launches only choose by it)
     if (rc != FW_OK) g->tables.reset();  // nothing half made stays
     if (rc == FW_ERR_NOMEM) {
       g->skip_tables = kSkipTables;
@@ -1993,7 +1995,7 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
   return FW_OK;
 }
 
-static fw_table_args table_args(const fw_tables& t, unsigned long long* d_counters) {
+static fw_table_args table_args(const fw_graph* g, const fw_tables& t, unsigned long long* d_counters) {
   fw_table_args tb;
   tb.vrec = t.vrec;
   tb.data = t.data;
@@ -2002,6 +2004,8 @@ static fw_table_args table_args(const fw_tables& t, unsigned long long* d_counte
   tb.by_label = t.by_label;
   tb.labels = t.labels;
   tb.nw_shift = t.nw_shift;
+  tb.long_lists = t.n_longs;
+  tb.mean_list = (float)g->mean_list;
   tb.lanes = 0u;
   tb.counters = d_counters;
   return tb;
@@ -2094,7 +2098,7 @@ extern "C" int fw_walk_device(const fw_graph* g, const fw_walk_params* p, const 
     if (launches == 0) FW_TRY(hipEventRecord(ev0, stream));  // (tables made in this call: recorded before that)
     if (!mg->call_result) FW_TRY(hipHostMalloc(reinterpret_cast<void**>(&mg->call_result), 64, hipHostMallocDefault));
     if ((rc = fw_table_begin(d_counters, &d_scr->dispenser, sizeof(Scratch) / 4u, stream)) != FW_OK) return rc;
-    rc = fw_launch_table_walk(a, table_args(*tables, d_counters), p->app, p->grid, stream, &grid_used);
+    rc = fw_launch_table_walk(a, table_args(g, *tables, d_counters), p->app, p->grid, stream, &grid_used);
     if (rc != FW_OK) return rc;
     if ((rc = fw_table_end(d_counters, mg->call_result, stream)) != FW_OK) return rc;
     launches += 3;
@@ -2449,7 +2453,7 @@ extern "C" int fw_walk_batch(const fw_graph* g, const fw_walk_params* p, const i
     int launches = 0;
     if (tables) {
       a.park_threshold = park_threshold;
-      rc = fw_launch_table_walk(a, table_args(*tables, bc->d_stripes), p->app, p->grid, streams[s], &grid_used);
+      rc = fw_launch_table_walk(a, table_args(g, *tables, bc->d_stripes), p->app, p->grid, streams[s], &grid_used);
     } else {
       rc = run_walk_launches(g, p, a, park_threshold, use_pb ? &pbs[s] : nullptr, streams[s], &grid_used, &launches,
                              &times);

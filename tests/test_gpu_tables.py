@@ -688,3 +688,34 @@ def test_node2vec_rows_end_anywhere_in_a_line(gpu, depth):
             assert (st.steps, st.sampled_edges) == (steps, edges)
     finally:
         g.destroy()
+
+
+@pytest.mark.parametrize("two_groups", [False, True])
+def test_node2vec_of_few_walkers_on_short_lists(gpu, two_groups):
+    """Lists of one group: up to where a wave walks each follows from how many proposals are turned down (waves per SIMD: 4 without adjacency tests, 5 where
+    some list has two groups, 6 for q < 1, 8 for q > 1); either side of it the oracle's walks."""
+    simds = 4 * torch.cuda.get_device_properties(0).multi_processor_count
+    rng = np.random.RandomState(8)
+    deg = rng.randint(1, 100, size=4000)
+    if two_groups:
+        deg[17] = 1500
+    xadj = np.zeros(len(deg) + 1, dtype=np.uint32)
+    np.cumsum(deg, out=xadj[1:])
+    adj = np.concatenate([np.sort(rng.randint(0, len(deg), size=d)) for d in deg]).astype(np.int32)
+    w = (1.0 + 9.0 * rng.random_sample(len(adj))).astype(np.float32)
+    g = gpu.Graph.from_csr(xadj, adj, w)
+    og = _oracle.Graph(xadj, adj, w)
+    try:
+        for _ in range(30):
+            g.walk(gpu.default_params(app=gpu.APP_NODE2VEC, max_depth=41), rng.randint(0, len(deg), size=70000).astype(np.int32))
+        for p, q, waves in ((1.0, 1.0, 4 + two_groups), (0.25, 1.0, 4 + two_groups), (2.0, 0.5, 8 if two_groups else 6), (0.25, 4.0, 8)):
+            for n in (waves * simds, waves * simds + 1):
+                par = gpu.default_params(app=gpu.APP_NODE2VEC, max_depth=9, p=p, q=q, seed=n)
+                starts = rng.randint(0, len(deg), size=n).astype(np.int32)
+                ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(par), starts)
+                paths, st = g.walk(par, starts)
+                assert g.engine()[0] == gpu.ENGINE_TABLES
+                assert (paths == ref).all() and (st.steps, st.sampled_edges) == (steps, edges), (p, q, n)
+                assert (st.grid == (n + 3) // 4) == (n == waves * simds), (p, q, n, st.grid)
+    finally:
+        g.destroy()
