@@ -641,3 +641,54 @@ def test_few_walkers(gpu, wg, thr):
                 assert (paths == ref).all() and (st.steps, st.sampled_edges) == (steps, edges), (kw, n)
     finally:
         g.destroy()
+
+# Streaming calls of at most 4,096 walkers take a wave for each (fw_walk_few), unless they give a grid: then the task table (fw_walk_zprs) walks them.
+@pytest.mark.parametrize("wg", [256, 512, 1024])
+@pytest.mark.parametrize("thr", [64, 1000, 16384])
+def test_task_table_with_few_walkers(gpu, hub, wg, thr):
+    """Calls that a wave per walker takes where the grid is left to the library (test_deepwalk_wave_and_workgroup, test_ppr, test_node2vec, test_metapath), by the
+    task table."""
+    rng = np.random.RandomState(2)
+    starts = rng.randint(0, 12000, size=3000).astype(np.int32)
+    starts[:64] = 0  # the 9000-degree hub
+    for i, kw in enumerate((dict(app=gpu.APP_DEEPWALK, max_depth=21), dict(app=gpu.APP_PPR, max_depth=81, tp=0.2), dict(app=gpu.APP_NODE2VEC, max_depth=16, p=2.0, q=0.5),
+                            dict(app=gpu.APP_NODE2VEC, max_depth=12, p=0.25, q=4.0), dict(app=gpu.APP_METAPATH, max_depth=9, schema=[3, 1, 0]))):
+        _, st = _check(gpu, hub, starts, wg_threads=wg, hub_threshold=thr, seed=99 + i, park_threshold=-1, grid=9, **kw)
+        assert st.grid == 9
+
+
+def test_task_table_with_few_node2vec_walkers_on_long_lists(gpu):
+    """The lists of test_node2vec_on_lists_of_every_length, a multigraph's equal neighbours among them."""
+    csr = _graphs.hub_graph(V=40000, hub_degrees=(30000, 20000, 5000, 600, 70), base_degree=4, seed=23)
+    starts = np.random.RandomState(6).randint(0, 40000, size=4000).astype(np.int32)
+    starts[:300] = 0
+    starts[300:500] = 1
+    for thr, p, q in ((64, 0.5, 2.0), (4096, 0.25, 4.0), (1 << 30, 4.0, 0.25)):
+        _check(gpu, csr, starts, app=gpu.APP_NODE2VEC, max_depth=9, p=p, q=q, hub_threshold=thr, seed=31, park_threshold=-1, grid=20)
+    xadj, adj, w, lab = csr
+    adj = adj.copy()
+    for v in range(5):  # every other neighbour twice
+        row = adj[xadj[v]:xadj[v + 1]]
+        row[1::2] = row[0::2][:len(row[1::2])]
+    for p, q in ((2.0, 0.5), (0.25, 4.0)):
+        _check(gpu, (xadj, adj, w, lab), starts, app=gpu.APP_NODE2VEC, max_depth=12, p=p, q=q, hub_threshold=1000, seed=32, park_threshold=-1, grid=20)
+
+
+@pytest.mark.parametrize("wg", [256, 512, 1024])
+def test_which_kernel_streams(gpu, hub, wg):
+    """A wave per walker up to as many walkers as there are waves resident (16 per compute unit), spread over the workgroups that are; the task table beyond, on
+    the grid it takes for any number of walkers.  Either side of that the oracle's walks."""
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    most, resident = 16 * cus, 16 * cus * 64 // wg
+    starts = np.random.RandomState(5).randint(0, 12000, size=5 * most).astype(np.int32)
+    for kw in (dict(app=gpu.APP_DEEPWALK, max_depth=12), dict(app=gpu.APP_PPR, max_depth=40, tp=0.1), dict(app=gpu.APP_NODE2VEC, max_depth=8, p=0.25, q=4.0),
+               dict(app=gpu.APP_METAPATH, max_depth=7, schema=[0, 1, 2, 3, 4])):
+        grids = {}
+        for n in (most // 2 + 1, most, most + 1, 5 * most):
+            _, st = _check(gpu, hub, starts[:n], wg_threads=wg, hub_threshold=1000, seed=3, park_threshold=-1, **kw)
+            grids[n] = st.grid
+        for n in (most // 2 + 1, most):
+            each = -(-n // resident)
+            assert grids[n] == -(-n // each), (kw, grids)
+        assert grids[most + 1] == grids[5 * most] and grids[most // 2 + 1] != grids[5 * most], (kw, grids)

@@ -719,3 +719,81 @@ def test_node2vec_of_few_walkers_on_short_lists(gpu, two_groups):
                 assert (st.grid == (n + 3) // 4) == (n == waves * simds), (p, q, n, st.grid)
     finally:
         g.destroy()
+
+# Calls of at most 8,192 walkers take a wave for each (fw_table_walk_wave), unless they give a grid: then a lane walks each.
+def _compare(gpu, g, og, starts, p, what):
+    ref, steps, edges = _oracle.walk(og, _oracle.from_walk_params(p), starts)
+    paths, st = g.walk(p, starts)
+    assert g.engine()[0] == gpu.ENGINE_TABLES, what
+    bad = np.nonzero((paths != ref).any(axis=1))[0]
+    assert len(bad) == 0, (what, bad[0], paths[bad[0]], ref[bad[0]])
+    assert (st.steps, st.sampled_edges) == (steps, edges), what
+    return st
+
+
+@pytest.mark.parametrize("kind", ["even", "uneven"])
+@pytest.mark.parametrize("wg,thr", [(512, 16384), (256, 1024), (1024, 2000), (512, 1 << 30)])
+def test_lane_per_walker_with_few_walkers(gpu, kind, wg, thr):
+    """The shapes of test_walks_on_tables that a wave per walker takes there, by the kernel of a lane per walker; with the grid left to the library, the other."""
+    csr, at = _lists(kind)
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    rng = np.random.RandomState(wg)
+    try:
+        g.walk(gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21, wg_threads=wg, hub_threshold=thr), at[rng.randint(0, len(at), size=70000)].astype(np.int32))
+        cases = [(dict(app=gpu.APP_DEEPWALK, max_depth=depth), n)
+                 for n, depth in ((1, 81), (63, 2), (65, 15), (1000, 16), (777, 17), (4001, 33), (3, 1), (129, 100))]
+        cases.append((dict(app=gpu.APP_PPR, max_depth=50, tp=0.1), 3000))
+        for p, q in ((2.0, 0.5), (0.25, 4.0), (4.0, 0.25), (1.0, 1.0), (0.1, 1.0)):
+            cases.append((dict(app=gpu.APP_NODE2VEC, max_depth=18, p=p, q=q), 2000))
+        for i, (kw, n) in enumerate(cases):
+            starts = np.where(rng.random_sample(n) < 0.8, at[rng.randint(0, len(at), size=n)], rng.randint(0, V, size=n)).astype(np.int32)
+            if n > 100:
+                starts[5] = -1
+                starts[7] = V
+            for grid in (2, 0):
+                st = _compare(gpu, g, og, starts, gpu.default_params(wg_threads=wg, hub_threshold=thr, seed=100 + i, walker_base=i, grid=grid, **kw), (kw, n, grid))
+                assert st.grid == (grid if grid else (n + 3) // 4)
+    finally:
+        g.destroy()
+
+
+@pytest.mark.parametrize("kind", ["even", "uneven"])
+@pytest.mark.parametrize("wg,thr", [(512, 16384), (1024, 2000)])
+def test_node2vec_on_hash_sets_a_lane_per_walker(gpu, kind, wg, thr):
+    """test_node2vec_on_hash_sets by the kernel of a lane per walker: buckets that overflow, sets with and without weights."""
+    csr, at = _lists(kind)
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    rng = np.random.RandomState(7)
+    try:
+        g.walk(gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21, wg_threads=wg, hub_threshold=thr), at[rng.randint(0, len(at), size=70000)].astype(np.int32))
+        for i, (p, q) in enumerate(((2.0, 0.5), (0.25, 4.0), (4.0, 0.25), (1.0, 1.0), (0.1, 1.0), (1.0, 3.0), (0.5, 0.25))):
+            starts = at[rng.randint(0, len(at), size=400)].astype(np.int32)
+            par = gpu.default_params(app=gpu.APP_NODE2VEC, max_depth=101, p=p, q=q, seed=50 + i, wg_threads=wg, hub_threshold=thr, grid=2)
+            st = _compare(gpu, g, og, starts, par, (p, q))
+            assert st.grid == 2
+            assert st.launches == (5 if i < 2 else 3)  # as there
+    finally:
+        g.destroy()
+
+
+def test_which_kernel_walks_on_tables(gpu):
+    """A wave per walker up to as many walkers as there are waves resident (32 per compute unit), a lane for each beyond; MetaPath always the latter."""
+    most = 32 * torch.cuda.get_device_properties(0).multi_processor_count
+    csr, at = _lists("even")
+    xadj, adj, w = csr
+    g = gpu.Graph.from_csr(xadj, adj, w, np.random.RandomState(1).randint(0, 5, size=len(adj)).astype(np.int32))
+    rng = np.random.RandomState(2)
+    try:
+        for kw in (dict(app=gpu.APP_DEEPWALK, max_depth=21), dict(app=gpu.APP_PPR, max_depth=21, tp=0.1), dict(app=gpu.APP_NODE2VEC, max_depth=21, p=2.0, q=0.5),
+                   dict(app=gpu.APP_METAPATH, max_depth=21)):
+            p = gpu.default_params(**kw)
+            for _ in range(20):
+                g.walk(p, at[rng.randint(0, len(at), size=70000)].astype(np.int32))
+            for n in (most, most + 1):
+                _, st = g.walk(p, at[rng.randint(0, len(at), size=n)].astype(np.int32))
+                assert g.engine()[0] == gpu.ENGINE_TABLES
+                assert (st.grid == (n + 3) // 4) == (n == most and kw["app"] != gpu.APP_METAPATH), (kw, n, st.grid)
+    finally:
+        g.destroy()
