@@ -4,7 +4,8 @@
 // group of 1024 biases, the group totals, their running sums -- is the same for every walker that ever stands there; a
 // walker contributes two uniforms per accepted group.  When the walkers of a call would read the lists many times over,
 // the walker-independent part is made once (one pass over the edges: 8 bytes read and 8 written per edge) and a step
-// becomes a few look-ups, so one lane walks one walker from its start to its end: no task table, no parking, no sorting.
+// becomes a few look-ups, so one lane walks one walker from its start to its end: no task table, no parking, no sorting
+// (fw_table_walk; calls of few walkers, but for MetaPath, take a wave for each: fw_table_walk_wave).
 // The sampler's definition (fw_walk_kernel.hip) is untouched: the tables hold the very sums, prefixes and totals the streaming
 // kernels compute, in their order of additions, and the walk takes the same draws, so every walker gets the same vertex.
 //
@@ -1487,8 +1488,8 @@ int launch_table_walk(const fw_kargs& a, fw_table_args tb, int grid, hipStream_t
     waves = (uint64_t)grid * 4u;
     tb.lanes = 64u;
   } else {
-    // few queries are spread over the chip, down to a few lanes per wave: their walks are chains of dependent look-ups, and a
-    // wave waits for the slowest of its lanes (16 waves per CU instead of 8: 16,000 to 200,000 walkers within 5 % either way)
+    // few queries are spread over the chip, down to one lane per wave for MetaPath and a few for the others: their walks are chains of dependent
+    // look-ups, and a wave waits for the slowest of its lanes (16 waves per CU instead of 8: 16,000 to 200,000 walkers within 5 % either way)
     const uint32_t spread = (uint32_t)cus * 8u;
     tb.lanes = n / spread < 64u ? n / spread + 1u : 64u;
     if (tb.lanes > 64u) tb.lanes = 64u;

@@ -2052,8 +2052,10 @@ struct HubOffer {
   int32_t sel[16];
 };
 
-// One sequence of the list on offer, if any is left.  The wave barriers hold the lanes together: without them the compiler joins the two blocks of
-// lane 0 across the iterations of a caller's loop, lane 0 leaves the others, and these take the value of a lane that has claimed nothing.
+// One sequence of the list on offer, if any is left.  The wave barriers hold the lanes together: they are convergent operations, which the compiler may
+// neither duplicate nor put under another condition, so it cannot join the two blocks of lane 0 across the iterations of a caller's loop.  (Without them it
+// does, lane 0 leaves the others, and these take the value of a lane that has claimed nothing.)  A claim by all lanes, which clear a sequence's bit and
+// look by ballot for one that found it set, needs none but takes 0.5 to 3.5 % longer (3,001 node2vec walkers on R-MAT 18, symmetrised, 206 -> 213 us).
 template <int kApp, int kNW>
 __device__ __forceinline__ bool take_sequence(const fw_kargs& a, HubOffer& o, const int lane) {
   uint32_t seq = 0u;

@@ -123,8 +123,8 @@ typedef struct {
                              tables: begin, walk, end, and the launches that made the tables when it made them) */
   int32_t grid;           /* workgroups per launch actually used */
   /* per-kernel breakdown of kernel_ms / steps / sampled_edges (hub parking splits a pass over two kernels) */
-  double walk_kernel_ms;      /* sum over fw_walk_zprs launches, or the walk on list tables (with
-                                 fw_walk_params.time_kernels, else 0) */
+  double walk_kernel_ms;      /* sum over the launches that stream lists (fw_walk_zprs, fw_walk_few), or the walk on
+                                 list tables (with fw_walk_params.time_kernels, else 0) */
   double hub_kernel_ms;       /* sum over the hub launches of every round: fw_hub_scan, fw_hub_batch, fw_hub_quad
                                  (with fw_walk_params.time_kernels, else 0); a walk on list tables: the making of
                                  the tables, 0 in a call that found them made */
@@ -139,7 +139,8 @@ typedef struct {
    * scattered_writes: stores of one 32-byte write request each (path entry, scattered record); record_bytes: walker
    * records, tasks and bucket tables that are streamed.  Tables that stay in the L2 are not priced.  This sits
    * between the algorithmic bytes of src/main.cu:93-111 (4 * sampled_edges + ...) and what a profiler's HBM counters
-   * see; it is an estimate, the counters are the measurement. */
+   * see; it is an estimate, the counters are the measurement.  For calls without parking it is a lower bound: the
+   * neighbours that short lists bring along with their biases are priced as one block per step. */
   uint64_t requested_bytes;
   uint64_t list_bytes;
   uint64_t scattered_reads;
