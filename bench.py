@@ -112,6 +112,19 @@ def roofline_of(app, st, n, kernel_ms):
     }
 
 
+def kernel_of(fw, engine, sampler, st, n):
+    """The kernels of a call on the library's own grid.  On tables the wave per walker of few walkers has four of them in a workgroup; walkers that
+    stream take a wave each where sixteen per compute unit are enough."""
+    if sampler != "native":
+        return "fw_walk_ref"
+    if engine == fw.ENGINE_TABLES:
+        return "fw_table_walk_wave" if st.grid == (n + 3) // 4 else "fw_table_walk"
+    if engine == fw.ENGINE_STREAM:
+        import torch
+        return "fw_walk_few" if n <= 16 * torch.cuda.get_device_properties(0).multi_processor_count else "fw_walk_zprs"
+    return "fw_walk_zprs + fw_hub_scan + fw_hub_batch + fw_hub_quad pipeline"
+
+
 def make_graph(fw, wl):
     return fw.Graph.rmat(wl["scale"], 16, 0.57, 0.19, 0.19, symmetrise=wl["sym"], w_lo=1.0, w_hi=100.0,
                          n_labels=wl["labels"], make_weights=wl["app"] != "metapath", seed=1)
@@ -306,9 +319,7 @@ def main():
     value = steps_per_pass * args.steps / wall
     avg_kernel_ms = float(np.mean(kernel_ms))
     roofline = roofline_of(wl["app"], last, n, avg_kernel_ms)
-    roofline["kernel"] = ("fw_walk_ref" if args.sampler != "native" else
-                          "fw_table_walk" if engine == fw.ENGINE_TABLES else
-                          "fw_walk_zprs" if engine == fw.ENGINE_STREAM else "fw_walk_zprs + fw_hub_scan + fw_hub_batch + fw_hub_quad pipeline")
+    roofline["kernel"] = kernel_of(fw, engine, args.sampler, last, n)
     # the profiler's view of the same workload (library defaults only: any override makes it another run)
     sources_sha = fw.sources_sha()
     prof = profiled_traffic(args.workload, sources_sha) if defaults and engine == fw.ENGINE_TABLES else None
