@@ -1468,7 +1468,7 @@ int launch_table_walk(const fw_kargs& a, fw_table_args tb, int grid, hipStream_t
   if constexpr (kApp != FW_APP_METAPATH) {  // (whose step is two reads, and no search)
     // As many walkers as there are waves resident: a wave each.  Measured, wave per walker / lane per walker, us of a call of 40 steps on R-MAT 20,
     // symmetrised: 1,000 walkers DeepWalk 73 / 92, PPR 52 / 76, node2vec 164 / 245; 8,000: 121 / 172, 72 / 94, 227 / 345 (q = 4: 555 / 760);
-    // with two walks a wave (16,000): 261 / 191, 238 / 99, 367 / 422.
+    // with two walks a wave (16,000): 261 / 191, 238 / 99, 367 / 422; a uniform graph of mean degree 4: 1,000 47 / 66, 42 / 61, 71 / 99; 8,192 DeepWalk 87 / 94, PPR 51 / 71.
     // Lists of one group leave a wave little to search, and node2vec's tests are made for one walker at a time, so where few proposals are turned down fewer waves
     // per SIMD already cost more than lanes do.  Uniform graphs of mean degree 4 to 200, q = 0.5: 7,000 walkers 146 / 132, 8,192 157 / 135; without adjacency tests,
     // p = 1: 5,120 110 / 92, 5,500 121 / 94, 8,192 144 / 102.  Some lists of two groups, q = 1: mean list 144 (R-MAT 14) 5,500 105 / 94, 6,144 111 / 96; mean list 192

@@ -2230,8 +2230,10 @@ int launch_one(fw_kargs a, int grid, uint32_t entries_hint, hipStream_t stream, 
   // bundles in flight
   // Walkers of whole walks, at most as many as waves are resident: a wave each.  Edges that come over the bus stay with the task table, which reads
   // no neighbours of lists longer than 256.  Measured, wave per walker / task table, us of a call of 40 steps on R-MAT 18, symmetrised: 100 walkers
-  // DeepWalk 118 / 165, PPR 82 / 113, node2vec 144 / 215; 4,096: 179 / 291, 119 / 180, 247 / 566; MetaPath on R-MAT 22 185 / 326.  4,096 walkers of 20
-  // steps from the hubs of R-MAT 22, symmetrised, at a hub threshold of 1024: 314 / 318, 166 / 204, 620 / 824; twice as many there 547 / 486.
+  // DeepWalk 104 / 159, PPR 65 / 87, node2vec 121 / 202, MetaPath 111 / 156; 4,096: 156 / 278, 111 / 172, 205 / 507, 159 / 269.  4,096 walkers of 20
+  // steps from the hubs of R-MAT 22, symmetrised, at a hub threshold of 1024: 275 / 312, 144 / 196, 287 / 377; twice as many there 547 / 486.  Short lists, a uniform
+  // graph of mean degree 4: 100 walkers 64 / 123, 52 / 86, 78 / 146, MetaPath 41 / 54; 4,096: 87 / 145, 67 / 127, 114 / 175, 49 / 76.  Slower by this are calls of nearly
+  // that many walkers that all start on the longest list, with 1024 threads and a low hub threshold (R-MAT 22, 1024: DeepWalk 386 / 365, PPR 252 / 248).
   if (grid <= 0 && a.host_edges == 0 && a.park_threshold == 0x7FFFFFFF && a.resume == nullptr && a.n_dev == nullptr) {
     int dev = 0, cus = 0;
     FW_HIP(hipGetDevice(&dev));
