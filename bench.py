@@ -114,14 +114,13 @@ def roofline_of(app, st, n, kernel_ms):
 
 def kernel_of(fw, engine, sampler, st, n):
     """The kernels of a call on the library's own grid.  On tables the wave per walker of few walkers has four of them in a workgroup; walkers that
-    stream take a wave each where sixteen per compute unit are enough."""
+    stream take a wave each where sixteen on each of the 256 compute units are enough."""
     if sampler != "native":
         return "fw_walk_ref"
     if engine == fw.ENGINE_TABLES:
         return "fw_table_walk_wave" if st.grid == (n + 3) // 4 else "fw_table_walk"
     if engine == fw.ENGINE_STREAM:
-        import torch
-        return "fw_walk_few" if n <= 16 * torch.cuda.get_device_properties(0).multi_processor_count else "fw_walk_zprs"
+        return "fw_walk_few" if n <= 4096 else "fw_walk_zprs"
     return "fw_walk_zprs + fw_hub_scan + fw_hub_batch + fw_hub_quad pipeline"
 
 
