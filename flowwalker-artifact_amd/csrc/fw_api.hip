@@ -1582,9 +1582,10 @@ static TrafficModel traffic_model(const fw_walk_params* p, int32_t n, bool parke
 }
 
 
-// The same for a walk on list tables; path entries leave in lines.  A step reads its vertex's record, a row and a lane of the
-// list's table, for MetaPath the record and one neighbour; node2vec tests the accepted neighbour of all but a walk's first step in N(prev).  node2vec's
-// turned-down trials are not counted (a row, a lane and a test each), nor the sums of lists of several groups, so the model is a lower bound.
+// The same for a walk on list tables; path entries leave in lines.  A step reads its vertex's record, one or two blocks of the list's pairs and for lists of
+// several groups a block of sums, three in all, for MetaPath the record and one neighbour; node2vec tests the accepted neighbour of all but a walk's first step in
+// N(prev).  Blocks that are found in the caches are charged too, node2vec's turned-down trials are not (the counters, past the L2: DeepWalk R-MAT 24 2.6 blocks a step, node2vec
+// 3.2 with its trials).
 static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params* p, int32_t n, bool sets, uint64_t steps) {
   TrafficModel m;
   m.scattered_reads = (p->app == FW_APP_METAPATH ? 2 : 3) * steps + (uint64_t)n;
@@ -1598,7 +1599,7 @@ static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params*
 
 // ---- list tables: when, and making them ---------------------------------------------------------------------
 //
-// A walk on list tables reads three or four blocks of memory per step, whatever the lists' lengths; without them a step
+// A walk on list tables reads some three blocks of memory per step, whatever the lists' lengths; without them a step
 // reads its list, or shares it with the others that are parked there.  The tables are made once the calls on a graph have spent without
 // them (measured) or are about to spend (estimated) a quarter more than making them takes: a first call makes them only if it gains by
 // that itself, and a loop of small calls gets them after a few and never pays more than about twice what it would have.

@@ -13,19 +13,24 @@
 //
 // Layout.  vrec[v] = {region, degree, total, CSR offset}: `region` in blocks of 128 bytes (the memory's request size) into
 // `data`, `total` = the list's total as the step's sampler adds it up.  A region, in units of 32 bytes:
-//   list of one group (at most 256 aligned quartets):  row M, then the entries
-//   longer list:  header (sums), then per group {row M (8 units), entries}
-//   row M: for every lane of the group (a lane holds J quartets, J = 1 .. 4) the running maximum of the positive lanes' prefixes;
-//     from the last positive lane on +inf.  "First lane whose prefix exceeds the target, else the last positive lane" is then
-//     "first entry above the target".
-//   entries: lane after lane, 4 J pairs {key, neighbour}; key = the lane's running sum up to the element, for an element
-//     without bias the key before it, from the lane's last positive element on +inf: the element is the first key
-//     above the target.  A lane of a full group is 16 pairs = one block, so the pick and the neighbour come in one request.
+//   list of one group (at most 256 aligned quartets):  the entries, then, but for lists of at most 16 quartets, row M
+//   longer list:  header (sums), then per group {entries, row M (8 units)}
+//   row M: for every lane of the group (a lane holds up to four quartets) the running maximum of the positive lanes' prefixes;
+//     from the last positive lane on +inf.  The sampler picks the first lane whose prefix exceeds the target, or else the last positive lane:
+//     the first entry above the target.
+//   entries: lane after lane, for each of its elements a pair {key, neighbour}, 16 pairs a block.  Inside its lane the sampler picks the first element whose
+//     running sum exceeds the target, or else the last positive one; key = that running sum, for an element without bias the one before it, from the
+//     lane's last positive element on +inf, and all of it not below row M's entry of the lane before nor above the lane's own.  So the keys of
+//     a whole group never decrease, and the element is the first one whose key is above the target.
+//   Where the weights are close to evenly spread over a group the walk looks for that element from the proportional guess on and row M is not read: the
+//   block of the guess holds it for 65 % (1024 weights from 1 to 100) to 95 % of the targets, one next to it nearly always.  So a step reads some 1.4 blocks of
+//   a group, with row M it read 2.2 (DeepWalk R-MAT 24, symmetrised: 2.50e9 -> 1.84e9 blocks in all, 47.4 -> 35.5 ms).  A group a quarter of whose lanes end more
+//   than a block elsewhere has the sign of its total set, or in a list of one group the top bit of `region`, and is entered through row M (three blocks at most;
+//   from the guess on it would be five or six).
 //   sums: blocks of 16 running sums of a sequence's groups and their 16 totals, every sequence from a block of its own, filled up
 //     with the last sum; with more than one sequence (workgroup granularity) a block in front: the inclusive scan of the
 //     sequences' totals, as keys like the above (16 floats).
-// All keys of a row or a lane never decrease, so any search finds the same entry; weights are close to evenly spread
-// over a list, so the searches start from the proportional guess and mostly end there.
+// All keys of a row or a group never decrease, so any search finds the same entry.
 
 #include <hip/hip_runtime.h>
 
@@ -37,7 +42,9 @@
 namespace {
 
 constexpr uint32_t kGq = 64u * kGroupQuartets;  // quartets of a full group
-constexpr uint32_t kGroupUnits = 8u + kGq;      // units of a group in a list of several: row M and the entries of 64 lanes
+constexpr uint32_t kGroupUnits = kGq + 8u;      // units of a group in a list of several: the entries of 64 lanes and row M
+constexpr uint32_t kNoRow = 16u;                // quartets of a list without row M: its entries are at most four blocks
+constexpr uint32_t kUneven = 0x80000000u;       // in vrec's region: row M first
 constexpr float kInf = __builtin_inff();
 // Waves per SIMD of the walk: 4, 5, 6 and 8 were measured (DeepWalk R-MAT 24 47.9 / 49.1 / 50.0 / 72.1 ms, the last one with
 // spilled registers; R-MAT 22 6.8 / 6.8 / 7.0 / 11.3): more walkers in flight only compete for the caches.
@@ -64,13 +71,10 @@ __device__ __forceinline__ uint32_t region_blocks(uint32_t off, uint32_t deg, bo
   const uint32_t nq = list_quartets(off, deg);
   uint32_t units;
   if (nq <= kGq) {
-    const uint32_t nl = nq < 64u ? nq : 64u;
-    units = ((nl + 7u) >> 3) + nl * ((nq + 63u) >> 6);
+    units = nq + (nq <= kNoRow ? 0u : (nq < 64u ? (nq + 7u) >> 3 : 8u));
   } else {
     const uint32_t ngroups = (nq + kGq - 1u) / kGq;
-    const uint32_t last = nq - (ngroups - 1u) * kGq;
-    const uint32_t nl = last < 64u ? last : 64u;
-    units = header_units(ngroups, wg, nw_shift) + kGroupUnits * (ngroups - 1u) + 8u + nl * ((last + 63u) >> 6);
+    units = header_units(ngroups, wg, nw_shift) + nq + 8u * ngroups;
   }
   return (units + 3u) >> 2;
 }
@@ -161,9 +165,17 @@ __device__ __forceinline__ void load_lane(const float* __restrict__ weight, cons
   for (int i = 0; i < 4 * kJ; ++i) bad = bad || !(x[i] >= 0.0f);
 }
 
-// The lane's pairs: e0 = its prefix before its own elements.  The first 4 J of the 4 kJ elements are stored.
+// The first quartet of lane `lane` among the entries of a group of nqg quartets: the quartets lane, lane + 64, ... of the group, for lane after lane.
+__device__ __forceinline__ uint32_t lane_start(const uint32_t lane, const uint32_t nqg) {
+  const uint32_t J = (nqg + 63u) >> 6, full = nqg - 64u * (J - 1u);  // lanes with J quartets, the others have one less
+  return J * lane - (lane > full ? lane - full : 0u);
+}
+
+// The lane's pairs: e0 = its prefix before its own elements, below and above = row M's entries of the lane before and of its own.  The first n of its
+// kJ quartets are stored.
 template <int kJ>
-__device__ __forceinline__ void store_lane(uint2* out, uint32_t J, float e0, const float (&x)[4 * kJ], const int32_t (&nb)[4 * kJ]) {
+__device__ __forceinline__ void store_lane(uint2* out, uint32_t n, float e0, float below, float above, const float (&x)[4 * kJ],
+                                           const int32_t (&nb)[4 * kJ]) {
   uint32_t pm = 0u;
 #pragma unroll
   for (int i = 0; i < 4 * kJ; ++i) pm |= (x[i] > 0.0f ? 1u : 0u) << i;
@@ -177,14 +189,23 @@ __device__ __forceinline__ void store_lane(uint2* out, uint32_t J, float e0, con
     for (int b = 0; b < 2; ++b) {
       e = e + x[i + b];
       key = x[i + b] > 0.0f ? e : key;
-      k[b] = __float_as_uint(pm != 0u && i + b >= last ? kInf : key);
+      float g = pm != 0u && i + b >= last ? kInf : key;
+      g = g < below ? below : g;
+      k[b] = __float_as_uint(g > above ? above : g);
     }
-    if ((uint32_t)i < 4u * J) o[i >> 1] = make_uint4(k[0], (uint32_t)nb[i], k[1], (uint32_t)nb[i + 1]);
+    if ((uint32_t)i < 4u * n) o[i >> 1] = make_uint4(k[0], (uint32_t)nb[i], k[1], (uint32_t)nb[i + 1]);
   }
 }
 
+// Whether a quarter of a group's lanes end more than a block of 16 pairs from where even weights would have them.  M: the running maximum of the positive
+// lanes' prefixes; lanes: the nl lanes of the group's segment.
+__device__ __forceinline__ bool uneven_group(const float M, const float T, const uint32_t c, const uint32_t nqg, const uint64_t lanes, const uint32_t nl) {
+  const float d = M * (float)(4u * nqg) - T * (float)(4u * lane_start(c + 1u, nqg));
+  return 4u * (uint32_t)__builtin_popcountll(__ballot(!(__builtin_fabsf(d) <= 16.0f * T)) & lanes) > nl;
+}
+
 // One list of at most kSeg quartets per segment of kSeg lanes (one or two DPP rows, or the wave); off, deg, region are the
-// segment's.  Returns the list's total in every lane of the segment.  The scan network is the packed step's.
+// segment's.  Returns the list's total in every lane of the segment, with its sign set for an uneven list.  The scan network is the packed step's.
 template <int kSeg>
 __device__ __forceinline__ float table_segment(const float* __restrict__ weight, const int32_t* __restrict__ adjncy, uint32_t off,
                                                uint32_t deg, unsigned char* region, int lane, bool& bad) {
@@ -211,16 +232,20 @@ __device__ __forceinline__ float table_segment(const float* __restrict__ weight,
   const uint64_t mpos = __ballot(pos) >> (lane & ~(kSeg - 1));
   const uint64_t mine = kSeg == 64 ? mpos : (mpos & ((1ull << (kSeg & 63)) - 1ull));
   const uint32_t lastpos = 63u - (uint32_t)__builtin_clzll(mine | 1ull);
-  const uint32_t mu = (nq + 7u) >> 3;
-  if (c < 8u * mu) reinterpret_cast<float*>(region)[c] = c >= lastpos ? kInf : M;
-  if (c < nq) store_lane<1>(reinterpret_cast<uint2*>(region + 32u * (mu + c)), 1u, I - q, x, nb);
-  return T;
+  const int seg = lane & ~(kSeg - 1);
+  bool uneven = false;
+  if (kSeg > 16) uneven = uneven_group(M, T, c, nq, (nq < 64u ? (1ull << nq) - 1ull : ~0ull) << seg, nq);
+  M = c >= lastpos ? kInf : M;
+  const float prev = bperm_f((lane - 1) << 2, M);
+  if (nq > kNoRow && c < ((nq + 7u) & ~7u)) reinterpret_cast<float*>(region + 32u * nq)[c] = M;
+  if (c < nq) store_lane<1>(reinterpret_cast<uint2*>(region + 32u * c), 1u, I - q, c != 0u ? prev : 0.0f, M, x, nb);
+  return uneven ? -T : T;
 }
 
-// One group of more than 64 quartets or of a long list, by a whole wave.  Returns its total.
+// One group of more than 64 quartets or of a long list, by a whole wave.  Returns its total, with its sign set for an uneven group.
 __device__ __forceinline__ float table_group(const float* __restrict__ weight, const int32_t* __restrict__ adjncy, uint32_t off,
-                                             uint32_t deg, uint32_t kb, uint32_t nqg, unsigned char* row, uint32_t row_units,
-                                             int lane, bool& bad) {
+                                             uint32_t deg, uint32_t kb, uint32_t nqg, unsigned char* entries, int lane,
+                                             bool& bad) {
   constexpr int kEl = 4 * kGroupQuartets;
   float x[kEl];
   int32_t nb[kEl];
@@ -230,13 +255,20 @@ __device__ __forceinline__ float table_group(const float* __restrict__ weight, c
   for (int i = 0; i < kEl; ++i) q = q + x[i];
   const float I = wave_scan(q);
   const bool pos = q > 0.0f;
-  const float M = wave_prefix_max(pos ? I : 0.0f);
+  float M = wave_prefix_max(pos ? I : 0.0f);
   const uint32_t lastpos = 63u - (uint32_t)__builtin_clzll(__ballot(pos) | 1ull);
-  const uint32_t nl = nqg < 64u ? nqg : 64u, J = (nqg + 63u) >> 6;
-  reinterpret_cast<float*>(row)[lane] = (uint32_t)lane >= lastpos ? kInf : M;
-  if ((uint32_t)lane < nl)
-    store_lane<kGroupQuartets>(reinterpret_cast<uint2*>(row + 32u * (row_units + (uint32_t)lane * J)), J, I - q, x, nb);
-  return readlane_f(I, 63);
+  const uint32_t nl = nqg < 64u ? nqg : 64u;
+  const float T = readlane_f(I, 63);
+  const bool uneven = uneven_group(M, T, (uint32_t)lane, nqg, nl < 64u ? (1ull << nl) - 1ull : ~0ull, nl);
+  M = (uint32_t)lane >= lastpos ? kInf : M;
+  const float prev = bperm_f((lane - 1) << 2, M);
+  reinterpret_cast<float*>(entries + 32u * nqg)[lane] = M;
+  if ((uint32_t)lane < nl) {
+    const uint32_t at = lane_start((uint32_t)lane, nqg);
+    store_lane<kGroupQuartets>(reinterpret_cast<uint2*>(entries + 32u * at), lane_start((uint32_t)lane + 1u, nqg) - at, I - q,
+                               lane != 0 ? prev : 0.0f, M, x, nb);
+  }
+  return uneven ? -T : T;
 }
 
 // Lists of one group: a wave takes 64 consecutive vertices; lists of at most 16 (32) quartets four (two) at a time, the others
@@ -304,15 +336,15 @@ __global__ __launch_bounds__(256) void fw_table_lists_kernel(const uint32_t* __r
       const int l = __builtin_ctzll(m);
       const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)off, l), d = (uint32_t)__builtin_amdgcn_readlane((int)deg, l);
       const uint32_t g = (uint32_t)__builtin_amdgcn_readlane((int)reg, l);
-      const float T = table_group(weight, adjncy, o, d, 0u, list_quartets(o, d), data + (uint64_t)g * 128u, 8u, lane, bad);
+      const float T = table_group(weight, adjncy, o, d, 0u, list_quartets(o, d), data + (uint64_t)g * 128u, lane, bad);
       if (lane == 0) s_total[wave][l] = T;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const float total = s_total[wave][lane];
-    bad = bad || !(total < kInf);
-    if (have) vrec[v] = make_uint4(reg, deg, __float_as_uint(total), off);
+    bad = bad || !(__builtin_fabsf(total) < kInf);
+    if (have) vrec[v] = make_uint4(reg | (total < 0.0f ? kUneven : 0u), deg, __float_as_uint(__builtin_fabsf(total)), off);
     __builtin_amdgcn_wave_barrier();
   }
   if (__ballot(bad) != 0ull && lane == 0) *flag = 1u;
@@ -336,8 +368,8 @@ __global__ __launch_bounds__(256) void fw_table_groups_kernel(const uint4* __res
     const uint32_t ngroups = (nq + kGq - 1u) / kGq;
     const bool wg = (int32_t)deg > hub_threshold;
     const uint32_t left = nq - g * kGq;
-    unsigned char* const row = region + (uint64_t)32u * (header_units(ngroups, wg, nw_shift) + kGroupUnits * g);
-    const float T = table_group(weight, adjncy, off, deg, g * kGq, left < kGq ? left : kGq, row, 8u, lane, bad);
+    unsigned char* const entries = region + (uint64_t)32u * (header_units(ngroups, wg, nw_shift) + kGroupUnits * g);
+    const float T = table_group(weight, adjncy, off, deg, g * kGq, left < kGq ? left : kGq, entries, lane, bad);
     const uint32_t k = wg ? g >> nw_shift : g;
     const uint32_t block = wg ? 1u + (g & ((1u << nw_shift) - 1u)) * seq_blocks(ngroups, wg, nw_shift) + (k >> 4) : k >> 4;
     if (lane == 0) reinterpret_cast<float*>(region)[32u * block + 16u + (k & 15u)] = T;
@@ -358,7 +390,7 @@ __device__ __forceinline__ float list_sums(float* region, uint32_t ngroups, bool
       const uint32_t L = (ngroups >> nw_shift) + ((uint32_t)lane < (ngroups & (nw - 1u)) ? 1u : 0u);
       for (uint32_t k = 0; k < 16u * nb; ++k) {
         float* const at = sums + 32u * (k >> 4) + (k & 15u);
-        if (k < L) S = S + at[16];
+        if (k < L) S = S + __builtin_fabsf(at[16]);  // (the sign: see the layout)
         at[0] = S;
       }
     }
@@ -373,7 +405,7 @@ __device__ __forceinline__ float list_sums(float* region, uint32_t ngroups, bool
     for (uint32_t g0 = 0; g0 < 16u * nb; g0 += 64u) {
       const uint32_t g = g0 + (uint32_t)lane;
       float* const at = region + 32u * (g >> 4) + (g & 15u);
-      const float T = g < ngroups ? at[16] : 0.0f;
+      const float T = g < ngroups ? __builtin_fabsf(at[16]) : 0.0f;
       float mine = 0.0f;
 #pragma unroll 8
       for (int l = 0; l < 64; ++l) {
@@ -755,31 +787,26 @@ __global__ __launch_bounds__(256) void fw_label_sums_kernel(const uint4* __restr
 
 // First entry above t of the n entries of a row (they never decrease, the last one is above t; rows are padded to 8
 // entries with +inf), from a guess.  Eight entries per look, so that nearly every walker of a wave finds its entry with the first; when
-// the guess was off twice the rest is halved.  below: the entry before, 0 for the first.
-__device__ __forceinline__ uint32_t row_search(const float* row, uint32_t n, uint32_t guess, float t, float& below) {
+// the guess was off twice the rest is halved.
+__device__ __forceinline__ uint32_t row_search(const float* row, uint32_t n, uint32_t guess, float t) {
   const uint32_t wmax = ((n + 7u) & ~7u) - 8u;
   uint32_t lo = 0u, hi = n - 1u;
   uint32_t w = guess > 3u ? guess - 3u : 0u;
-  below = 0.0f;
   for (int looks = 0;; ++looks) {
     w = w < wmax ? w : wmax;
     const f4_at4 m0 = *reinterpret_cast<const f4_at4*>(row + w);
     const f4_at4 m1 = *reinterpret_cast<const f4_at4*>(row + w + 4u);
     uint32_t cnt = 0u;
-    float at = 0.0f;  // the largest entry that is not above t
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float m = i < 4 ? m0[i & 3] : m1[i & 3];
-      const bool le = m <= t;
-      cnt += le ? 1u : 0u;
-      at = le ? m : at;
+      cnt += m <= t ? 1u : 0u;
     }
     if (cnt == 0u) {
       if (w <= lo) return w;
       hi = w;
       w = looks == 0 || hi - lo <= 16u ? (hi > lo + 7u ? hi - 7u : lo) : (lo + hi) >> 1;
     } else {
-      below = at;
       if (cnt < 8u) return w + cnt;
       lo = w + 8u;
       if (lo >= hi) return hi;
@@ -788,32 +815,78 @@ __device__ __forceinline__ uint32_t row_search(const float* row, uint32_t n, uin
   }
 }
 
-// The neighbour of the first pair whose key is above t (n = 4 J pairs of one lane, keys as above), kW pairs per look.
-template <uint32_t kW>
-__device__ __forceinline__ int32_t pair_search(const uint2* pairs, uint32_t n, uint32_t guess, float t) {
-  const uint32_t wmax = n - kW;
-  uint32_t lo = 0u;
-  uint32_t w = guess > kW / 2u - 1u ? (guess - (kW / 2u - 1u)) & ~1u : 0u;
-  for (;;) {
-    w = w < wmax ? w : wmax;
-    uint4 p[kW / 2u];
+// A look at one block of pairs for every lane with `need` (the lanes of m): first = the neighbour of its first key above t, at_start = that is the
+// block's first, none = there is none.  All lanes take part.  Eight lanes read a walker's block together, 16 bytes each, and eight walkers are
+// served by a load: a lane that loads its block alone makes eight requests to the first-level cache, each of which may wait for the address's translation.
+// A lane for each block / eight lanes: DeepWalk R-MAT 24 (5 GB of regions) 4.9e9 / 0.95e9 translation misses, 66.4 / 35.5 ms; R-MAT 22 5.92 / 4.92 ms, node2vec
+// R-MAT 20 with q = 4 5.99 / 5.35; with row M and the pairs by each lane these were 47.4, 6.65 and 6.26.
+struct BlockLook {
+  uint32_t first;
+  bool at_start, none;
+};
+
+__device__ __forceinline__ BlockLook look_at_blocks(const unsigned char* data, const uint64_t m, const bool need, const uint32_t block, const float t,
+                                                    const uint32_t lane) {
+  const uint32_t n = (uint32_t)__builtin_popcountll(m);
+  const uint32_t rank = (uint32_t)__builtin_popcountll(m & ((1ull << lane) - 1ull));
+  const int to = (int)(need ? rank : n + lane - rank) << 2;  // the lanes that look first, in order, then the others
+  const int blocks = __builtin_amdgcn_ds_permute(to, (int)(need ? block : 0u));
+  const int targets = __builtin_amdgcn_ds_permute(to, (int)__float_as_uint(t));
+  const uint32_t of = lane >> 3, piece = lane & 7u;
+  uint4 x[8];
 #pragma unroll
-    for (uint32_t i = 0; i < kW / 2u; ++i) p[i] = *reinterpret_cast<const uint4*>(pairs + w + 2u * i);
-    const bool first = !(__uint_as_float(p[0].x) <= t);
-    if (first && w > lo) {  // (lo: nothing before it is above t)
-      w = w > lo + kW - 1u ? (w - (kW - 2u)) & ~1u : lo & ~1u;
-      continue;
+  for (uint32_t i = 0; i < 8u; ++i) {
+    if (8u * i < n) {
+      const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(8u * i + of) << 2, blocks);
+      x[i] = *reinterpret_cast<const uint4*>(data + (uint64_t)b * 128u + 16u * piece);
     }
-    uint32_t nb = p[kW / 2u - 1u].w;
-    const bool all = __uint_as_float(p[kW / 2u - 1u].z) <= t;
+  }
+  BlockLook r = {0u, false, true};
 #pragma unroll
-    for (int i = (int)kW - 2; i >= 0; --i) {
-      const uint32_t key = (i & 1) ? p[i >> 1].z : p[i >> 1].x, v = (i & 1) ? p[i >> 1].w : p[i >> 1].y;
-      nb = __uint_as_float(key) <= t ? nb : v;
+  for (uint32_t i = 0; i < 8u; ++i) {
+    if (8u * i < n) {
+      const float ti = __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)(8u * i + of) << 2, targets));
+      const bool c0 = !(__uint_as_float(x[i].x) <= ti);
+      const uint64_t m0 = __ballot(c0), any = m0 | __ballot(!(__uint_as_float(x[i].z) <= ti));
+      const uint32_t at = 8u * (rank & 7u);
+      const uint32_t above = (uint32_t)(any >> at) & 0xFFu;
+      const uint32_t f = at + (uint32_t)__builtin_ctz(above | 0x80u);
+      const uint32_t nb = (uint32_t)__builtin_amdgcn_ds_bpermute((int)f << 2, (int)(c0 ? x[i].y : x[i].w));
+      if (need && (rank >> 3) == i) r = {nb, ((m0 >> at) & 1ull) != 0ull, above == 0u};
     }
-    lo = w + kW;
-    if (!all || lo >= n) return (int32_t)nb;
-    w = lo;
+  }
+  return r;
+}
+
+// Where a step's neighbour is looked for: the first of the n pairs of a group, from block `pairs` of the tables on, whose key is above t.  It does
+// not lie before block `lo` of them and is guessed to lie in block b.
+struct PairPlace {
+  uint32_t pairs, n, b, lo;
+  float t;
+};
+
+// That neighbour, for the lanes with `need`; all lanes take part.  From the guess on block after block; after three looks what is left is halved.
+__device__ __forceinline__ uint32_t pair_search(const unsigned char* data, bool need, PairPlace p, const uint32_t lane) {
+  const uint32_t top = (p.n - 1u) >> 4;
+  uint32_t end = top + 1u;  // where the blocks end that may hold it; behind the last one it is `found`
+  uint32_t found = 0u;
+  p.b = p.b < top ? p.b : top;
+  for (uint32_t looks = 0u;; ++looks) {
+    const uint64_t m = __ballot(need);
+    if (m == 0ull) return found;
+    const BlockLook k = look_at_blocks(data, m, need, p.pairs + p.b, p.t, lane);
+    if (need) {
+      if (k.none && p.b < top) {  // (what follows the pairs in the last block comes after a key that is above t)
+        p.lo = p.b + 1u;
+        need = p.lo != end;
+        p.b = looks >= 3u ? (p.lo + end) >> 1 : p.lo;
+      } else {
+        found = k.first;
+        need = k.at_start && p.b > p.lo;
+        end = p.b;
+        p.b = looks >= 3u ? (p.lo + end) >> 1 : p.b - 1u;
+      }
+    }
   }
 }
 
@@ -933,21 +1006,20 @@ __device__ __forceinline__ int32_t label_pick(const fw_kargs& a, const fw_table_
   return tb.by_label[first + start + (r < n ? r : n - 1u)];
 }
 
-// One proposal of the step's sampler for a list with a positive total: the selected neighbour.  d: block 0 of the step's stream 0.
-__device__ __forceinline__ int32_t table_pick(const fw_kargs& a, const fw_table_args& tb, const uint4 rec, const uint4 d,
+// One proposal of the step's sampler for a list with a positive total: where the selected neighbour is looked for.  d: block 0 of the step's stream 0.
+__device__ __forceinline__ PairPlace table_pick(const fw_kargs& a, const fw_table_args& tb, const uint4 rec, const uint4 d,
                                               const uint32_t walker, const uint32_t step, const uint32_t sbase) {
   const float total = __uint_as_float(rec.z);
   const uint32_t nq = list_quartets(rec.w, rec.y);
-  const unsigned char* row = tb.data + (uint64_t)rec.x * 128u;
-  uint32_t nqg = nq, row_units = 8u;
+  uint32_t entries = rec.x & ~kUneven;  // the block they begin with
+  uint32_t nqg = nq;
   float T = total, tu = u24(d.x);
-  if (nq <= kGq) {
-    if (nq < 64u) row_units = (nq + 7u) >> 3;
-  } else {
+  bool uneven = (rec.x & kUneven) != 0u;
+  if (nq > kGq) {
     const uint32_t ngroups = (nq + kGq - 1u) / kGq;
     const bool wg = (int32_t)rec.y > a.hub_threshold;
     const uint32_t nb = seq_blocks(ngroups, wg, tb.nw_shift);
-    const float* sums = reinterpret_cast<const float*>(row);
+    const float* sums = reinterpret_cast<const float*>(tb.data + (uint64_t)entries * 128u);
     uint32_t seq = 0u;
     LaneDraw dq;
     if (wg) {  // which sequence, then the reservoir over it with draws of its own stream
@@ -961,18 +1033,18 @@ __device__ __forceinline__ int32_t table_pick(const fw_kargs& a, const fw_table_
     uint32_t k;
     T = *sums_reservoir(a, sums, nb, dq, walker, step, seq | sbase, k, tu);
     const uint32_t g = wg ? seq + (k << tb.nw_shift) : k;
-    row += (uint64_t)32u * (header_units(ngroups, wg, tb.nw_shift) + kGroupUnits * g);
+    entries += (header_units(ngroups, wg, tb.nw_shift) + kGroupUnits * g) >> 2;
     nqg = nq - g * kGq < kGq ? nq - g * kGq : kGq;
+    uneven = T < 0.0f;
+    T = __builtin_fabsf(T);
   }
-  const float t = tu * T;
-  const uint32_t nl = nqg < 64u ? nqg : 64u;
-  const uint32_t J = (nqg + 63u) >> 6;
-  float below;
-  const uint32_t l = row_search(reinterpret_cast<const float*>(row), nl, (uint32_t)(tu * (float)nl), t, below);
-  const uint2* pairs = reinterpret_cast<const uint2*>(row + 32u * (row_units + l * J));
-  if (J == 1u) return pair_search<4>(pairs, 4u, 0u, t);
-  const float guess = (t - below) * (float)(4u * J * nl) * __builtin_amdgcn_rcpf(T);
-  return pair_search<8>(pairs, 4u * J, guess > 0.0f ? (guess < 15.0f ? (uint32_t)guess : 15u) : 0u, t);
+  PairPlace p = {entries, 4u * nqg, (uint32_t)(tu * (float)(4u * nqg)) >> 4, 0u, tu * T};
+  if (uneven) {
+    const uint32_t nl = nqg < 64u ? nqg : 64u;
+    const float* const row = reinterpret_cast<const float*>(tb.data + (uint64_t)entries * 128u + 32u * nqg);
+    p.lo = p.b = lane_start(row_search(row, nl, (uint32_t)(tu * (float)nl), p.t), nqg) >> 2;
+  }
+  return p;
 }
 
 // One lane, one walker, from its start to its end; a lane whose walk is over takes the next query of its wave's range.
@@ -1075,19 +1147,21 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
       }
     }
     const uint4 d = philox4x32_10<true>(walker, step, sbase, 0u, a.seed_lo, a.seed_hi);
+    int32_t nv = -1;
+    bool go = active && !ended;  // to a neighbour with a positive bias, if there is one (include/walker.cuh:1373-1374)
+    if (kApp == FW_APP_METAPATH) {
+      if (go) nv = label_pick(a, tb, rec, ends, s_slot[step % (uint32_t)a.schema_len], d, walker, step);
+      go = go && nv >= 0;
+    } else {
+      go = go && __uint_as_float(rec.z) > 0.0f;
+      PairPlace place = {0u, 1u, 0u, 0u, 0.0f};
+      if (go) place = table_pick(a, tb, rec, d, walker, step, sbase);
+      nv = (int32_t)pair_search(tb.data, go, place, (uint32_t)lane);
+    }
     if (active && !ended) {
-      int32_t nv = -1;
-      bool none;  // no neighbour with a positive bias (include/walker.cuh:1373-1374)
-      if (kApp == FW_APP_METAPATH) {
-        nv = label_pick(a, tb, rec, ends, s_slot[step % (uint32_t)a.schema_len], d, walker, step);
-        none = nv < 0;
-      } else {
-        none = !(__uint_as_float(rec.z) > 0.0f);
-      }
-      if (none) {
+      if (!go) {
         ended = true;
       } else {
-        if (kApp != FW_APP_METAPATH) nv = table_pick(a, tb, rec, d, walker, step, sbase);
         bool moved = true;
         if (kApp == FW_APP_NODE2VEC && prev >= 0) {
           if (a.n2v_extra > 0.0f && fresh) {
@@ -1225,8 +1299,8 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
 // ---- the walk of few walkers ------------------------------------------------------------------------------
 //
 // A call of few walkers is a chain of dependent reads per step, and nothing else fills the time: the chip has lanes and memory to
-// spare.  So a whole wave walks one walker.  A step takes its record; the row of the group and the pairs around the proportional
-// guess together (1 KB of pairs, eight lanes' worth of a full group, so the guess is nearly always good enough); for a long list
+// spare.  So a whole wave walks one walker.  A step takes its record and the group's pairs around the proportional
+// guess (1 KB of them, an eighth of a full group, so the guess is nearly always good enough); for a long list
 // the sums of 64 groups before that.  Every search is a comparison in all lanes and a ballot, and the draws a step may take are
 // made by the lanes side by side while the record is on its way.
 // Results are fw_table_walk's: the same sums, the same draws, the same comparisons.
@@ -1283,17 +1357,17 @@ __device__ __forceinline__ uint32_t wave_reservoir(const fw_kargs& a, const floa
 __device__ __forceinline__ int32_t wave_pick(const fw_kargs& a, const fw_table_args& tb, const uint4 rec, const uint4 d,
                                              const uint32_t walker, const uint32_t step, const uint32_t sbase, const uint32_t lane) {
   const uint32_t nq = list_quartets(rec.w, rec.y);
-  const unsigned char* row = tb.data + (uint64_t)rec.x * 128u;
-  uint32_t nqg = nq, row_units = 8u;
+  const unsigned char* entries = tb.data + (uint64_t)(rec.x & ~kUneven) * 128u;
+  uint32_t nqg = nq;
   float T = __uint_as_float(rec.z), tu;
+  bool uneven = (rec.x & kUneven) != 0u;
   if (nq <= kGq) {
     tu = u24(readlane_u32(d.x, 0u));
-    if (nq < 64u) row_units = (nq + 7u) >> 3;
   } else {
     const uint32_t ngroups = (nq + kGq - 1u) / kGq;
     const bool wg = (int32_t)rec.y > a.hub_threshold;
     const uint32_t nb = seq_blocks(ngroups, wg, tb.nw_shift);
-    const float* sums = reinterpret_cast<const float*>(row);
+    const float* sums = reinterpret_cast<const float*>(entries);
     uint32_t seq = 0u;
     float S_last = T;
     if (wg) {  // which sequence, then the reservoir over it with draws of its own stream
@@ -1304,32 +1378,36 @@ __device__ __forceinline__ int32_t wave_pick(const fw_kargs& a, const fw_table_a
     }
     const uint32_t k = wave_reservoir(a, sums, nb, S_last, d, walker, step, seq, sbase, lane, tu, T);
     const uint32_t g = wg ? seq + (k << tb.nw_shift) : k;
-    row += (uint64_t)32u * (header_units(ngroups, wg, tb.nw_shift) + kGroupUnits * g);
+    entries += (uint64_t)32u * (header_units(ngroups, wg, tb.nw_shift) + kGroupUnits * g);
     nqg = nq - g * kGq < kGq ? nq - g * kGq : kGq;
+    uneven = T < 0.0f;
+    T = __builtin_fabsf(T);
   }
   const float t = tu * T;
-  const uint32_t nl = nqg < 64u ? nqg : 64u;
-  const uint32_t J = (nqg + 63u) >> 6;
-  // two pairs a lane, from some lanes before the guess on
-  const uint4* pairs = reinterpret_cast<const uint4*>(row + 32u * row_units);
-  const uint32_t n2 = 2u * J * nl;
+  // two pairs a lane, from some before the guess on, or from the first of the lane that row M names
+  const uint4* pairs = reinterpret_cast<const uint4*>(entries);
+  const uint32_t n2 = 2u * nqg;
   const uint32_t guess = (uint32_t)(tu * (float)n2);
-  uint32_t w = guess > 32u ? guess - 32u : 0u;
   const uint32_t wmax = n2 > 64u ? n2 - 64u : 0u;
-  w = w < wmax ? w : wmax;
-  uint4 p = make_uint4(0u, 0u, 0u, 0u);
-  if (w + lane < n2) p = pairs[w + lane];
-  const float m = lane < nl ? reinterpret_cast<const float*>(row)[lane] : kInf;
-  const uint32_t l = (uint32_t)__builtin_ctzll(__ballot(!(m <= t)) | (1ull << 63));
-  const uint32_t first = 2u * J * l;  // of the lane's pieces
-  if (first < w || first + 2u * J > w + 64u) {
-    w = first;
-    if (w + lane < n2) p = pairs[w + lane];
+  uint32_t w = guess > 32u ? guess - 32u : 0u;
+  if (uneven) {
+    const float m = lane < nqg ? reinterpret_cast<const float*>(entries + 32u * nqg)[lane] : kInf;
+    w = 2u * lane_start((uint32_t)__builtin_ctzll(__ballot(!(m <= t)) | (1ull << 63)), nqg);
   }
-  const uint64_t mine = ((1ull << (2u * J)) - 1ull) << (first - w);
-  const uint64_t m0 = __ballot(!(__uint_as_float(p.x) <= t)) & mine, m1 = __ballot(!(__uint_as_float(p.z) <= t)) & mine;
-  const uint32_t f = (uint32_t)__builtin_ctzll(m0 | m1 | (1ull << (first - w + 2u * J - 1u)));  // (the last piece has a key above)
-  return (int32_t)(((m0 >> f) & 1ull) != 0ull ? readlane_u32(p.y, f) : readlane_u32(p.w, f));
+  w = w < wmax ? w : wmax;
+  for (uint32_t lo = uneven ? w : 0u;;) {
+    uint4 p = make_uint4(0x7F800000u, 0u, 0x7F800000u, 0u);
+    if (w + lane < n2) p = pairs[w + lane];
+    const uint64_t m0 = __ballot(!(__uint_as_float(p.x) <= t)), m1 = __ballot(!(__uint_as_float(p.z) <= t));
+    if ((m0 | m1) == 0ull) {  // (the last pair's key is above: there are more)
+      lo = w = w + 64u;
+    } else if ((m0 & 1ull) != 0ull && w > lo) {
+      w = w > lo + 63u ? w - 63u : lo;
+    } else {
+      const uint32_t f = (uint32_t)__builtin_ctzll(m0 | m1);
+      return (int32_t)(((m0 >> f) & 1ull) != 0ull ? readlane_u32(p.y, f) : readlane_u32(p.w, f));
+    }
+  }
 }
 
 // set_find by a wave, from the lane's place of the bucket (lanes 0 .. 15)

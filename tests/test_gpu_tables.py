@@ -797,3 +797,36 @@ def test_which_kernel_walks_on_tables(gpu):
                 assert (st.grid == (n + 3) // 4) == (n == most and kw["app"] != gpu.APP_METAPATH), (kw, n, st.grid)
     finally:
         g.destroy()
+
+
+@pytest.mark.parametrize("side", ["front", "back"])
+@pytest.mark.parametrize("wg,thr", [(512, 16384), (256, 1024)])
+def test_groups_with_a_lump(gpu, side, wg, thr):
+    """Weights evenly spread over most lanes of a group, while the share of some fourteen lies in one of them: too few for the group to be entered through its
+    row, and far enough off for every way the search for a block goes."""
+    V = 400
+    rng = np.random.RandomState(8)
+    deg = np.r_[rng.randint(60, 70, size=100), rng.randint(120, 260, size=100), rng.randint(500, 1100, size=196), [2500, 4096, 9001, 20000]]
+    xadj = np.zeros(V + 1, dtype=np.uint32)
+    np.cumsum(deg, out=xadj[1:])
+    adj = np.concatenate([np.sort(rng.randint(0, V, size=d)) for d in deg]).astype(np.int32)
+    w = (1.0 + 4.0 * rng.random_sample(len(adj))).astype(np.float32)
+    for v in range(V):
+        i = np.arange(xadj[v], xadj[v + 1])
+        lane = ((i >> 2) - (int(xadj[v]) >> 2)) % 64  # of the group's quartets lane, lane + 64, ..
+        lanes = min(64, len(i) // 4)
+        first = 0 if side == "front" else lanes - 1
+        few = max(2, lanes * 14 // 64)
+        poor = (lane != first) & (lane < few if side == "front" else (lane >= lanes - few) & (lane < lanes))
+        w[i[poor]] = 0.001
+        w[i[lane == first]] *= few
+    g = gpu.Graph.from_csr(xadj, adj, w)
+    og = _oracle.Graph(xadj, adj, w)
+    try:
+        g.walk(gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21, wg_threads=wg, hub_threshold=thr), rng.randint(0, V, size=70000).astype(np.int32))
+        for grid, n in ((2, 3000), (0, 3000), (0, 9000)):
+            starts = rng.randint(0, V, size=n).astype(np.int32)
+            st = _compare(gpu, g, og, starts, gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=20, wg_threads=wg, hub_threshold=thr, seed=n, grid=grid), (side, grid, n))
+            assert g.engine()[0] == gpu.ENGINE_TABLES and (grid == 0 or st.grid == grid)
+    finally:
+        g.destroy()
