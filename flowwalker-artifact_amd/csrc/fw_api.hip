@@ -1998,6 +1998,12 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
   return FW_OK;
 }
 
+// Regions from which on the walk's blocks of pairs are not kept in the L2, where smaller ones meet the next walker in the memory-side cache (256 MB).
+// Kept / not kept, ms, 4,000,000 walks of 80 steps where not said: DeepWalk R-MAT 22 (4,194,304, 0.7 GB) 5.00 / 5.33, symmetrised (1.4 GB) 7.90 / 8.20, R-MAT 23
+// (1.4 GB) 5.87 / 5.90, symmetrised (2.7 GB) 9.84 / 9.29, R-MAT 24 (2.7 GB) 7.14 / 6.79, symmetrised, 16,777,216 (5.2 GB) 36.1 / 33.1; node2vec of 40 steps R-MAT 22
+// symmetrised 5.67 / 5.82, R-MAT 23 6.51 / 6.52, all of R-MAT 24, 80 steps 44.3 / 43.5.
+constexpr size_t kStreamPairsBytes = (size_t)2 << 30;
+
 static fw_table_args table_args(const fw_graph* g, const fw_tables& t, unsigned long long* d_counters) {
   fw_table_args tb;
   tb.vrec = t.vrec;
@@ -2008,6 +2014,7 @@ static fw_table_args table_args(const fw_graph* g, const fw_tables& t, unsigned 
   tb.labels = t.labels;
   tb.nw_shift = t.nw_shift;
   tb.long_lists = t.n_longs;
+  tb.stream_pairs = t.data_bytes >= kStreamPairsBytes ? 1u : 0u;
   tb.mean_list = (float)g->mean_list;
   tb.lanes = 0u;
   tb.counters = d_counters;

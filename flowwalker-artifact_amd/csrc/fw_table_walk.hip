@@ -820,11 +820,16 @@ __device__ __forceinline__ uint32_t row_search(const float* row, uint32_t n, uin
 // served by a load: a lane that loads its block alone makes eight requests to the first-level cache, each of which may wait for the address's translation.
 // A lane for each block / eight lanes: DeepWalk R-MAT 24 (5 GB of regions) 4.9e9 / 0.95e9 translation misses, 66.4 / 35.5 ms; R-MAT 22 5.92 / 4.92 ms, node2vec
 // R-MAT 20 with q = 4 5.99 / 5.35; with row M and the pairs by each lane these were 47.4, 6.65 and 6.26.
+// A block comes once, and among gigabytes of them nobody wants it again before it is gone: there (kStream) it is not kept in the L2, which holds more
+// of the records and sums instead.
+typedef uint32_t u4_vec __attribute__((ext_vector_type(4)));
+
 struct BlockLook {
   uint32_t first;
   bool at_start, none;
 };
 
+template <bool kStream>
 __device__ __forceinline__ BlockLook look_at_blocks(const unsigned char* data, const uint64_t m, const bool need, const uint32_t block, const float t,
                                                     const uint32_t lane) {
   const uint32_t n = (uint32_t)__builtin_popcountll(m);
@@ -838,7 +843,9 @@ __device__ __forceinline__ BlockLook look_at_blocks(const unsigned char* data, c
   for (uint32_t i = 0; i < 8u; ++i) {
     if (8u * i < n) {
       const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(8u * i + of) << 2, blocks);
-      x[i] = *reinterpret_cast<const uint4*>(data + (uint64_t)b * 128u + 16u * piece);
+      const u4_vec* const at = reinterpret_cast<const u4_vec*>(data + (uint64_t)b * 128u + 16u * piece);
+      const u4_vec y = kStream ? __builtin_nontemporal_load(at) : *at;
+      x[i] = make_uint4(y[0], y[1], y[2], y[3]);
     }
   }
   BlockLook r = {0u, false, true};
@@ -866,6 +873,7 @@ struct PairPlace {
 };
 
 // That neighbour, for the lanes with `need`; all lanes take part.  From the guess on block after block; after three looks what is left is halved.
+template <bool kStream>
 __device__ __forceinline__ uint32_t pair_search(const unsigned char* data, bool need, PairPlace p, const uint32_t lane) {
   const uint32_t top = (p.n - 1u) >> 4;
   uint32_t end = top + 1u;  // where the blocks end that may hold it; behind the last one it is `found`
@@ -874,7 +882,7 @@ __device__ __forceinline__ uint32_t pair_search(const unsigned char* data, bool 
   for (uint32_t looks = 0u;; ++looks) {
     const uint64_t m = __ballot(need);
     if (m == 0ull) return found;
-    const BlockLook k = look_at_blocks(data, m, need, p.pairs + p.b, p.t, lane);
+    const BlockLook k = look_at_blocks<kStream>(data, m, need, p.pairs + p.b, p.t, lane);
     if (need) {
       if (k.none && p.b < top) {  // (what follows the pairs in the last block comes after a key that is above t)
         p.lo = p.b + 1u;
@@ -1051,7 +1059,8 @@ __device__ __forceinline__ PairPlace table_pick(const fw_kargs& a, const fw_tabl
 // Path entries are collected in LDS (16 per walker, by their place in the path matrix modulo 16) and leave as whole 64-byte
 // lines; the entries of a row before its first and after its last whole line, and the -1 behind the walk, are stored by the
 // wave together, one row at a time.
-template <int kApp>
+// kStream: the blocks of pairs are not kept in the L2.
+template <int kApp, bool kStream>
 __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, const fw_table_args tb) {
   __shared__ __align__(16) int32_t s_buf[4][64 * 16];
   __shared__ unsigned long long s_acc[4];
@@ -1156,7 +1165,7 @@ __global__ __launch_bounds__(256, kWaves) void fw_table_walk(const fw_kargs a, c
       go = go && __uint_as_float(rec.z) > 0.0f;
       PairPlace place = {0u, 1u, 0u, 0u, 0.0f};
       if (go) place = table_pick(a, tb, rec, d, walker, step, sbase);
-      nv = (int32_t)pair_search(tb.data, go, place, (uint32_t)lane);
+      nv = (int32_t)pair_search<kStream>(tb.data, go, place, (uint32_t)lane);
     }
     if (active && !ended) {
       if (!go) {
@@ -1580,7 +1589,11 @@ int launch_table_walk(const fw_kargs& a, fw_table_args tb, int grid, hipStream_t
     if (waves > most) waves = most;
   }
   const unsigned blocks = (unsigned)((waves + 3u) / 4u);
-  hipLaunchKernelGGL((fw_table_walk<kApp>), dim3(blocks), dim3(256), 0, stream, a, tb);
+  if (kApp != FW_APP_METAPATH && tb.stream_pairs != 0u) {
+    hipLaunchKernelGGL((fw_table_walk<kApp, kApp != FW_APP_METAPATH>), dim3(blocks), dim3(256), 0, stream, a, tb);
+  } else {
+    hipLaunchKernelGGL((fw_table_walk<kApp, false>), dim3(blocks), dim3(256), 0, stream, a, tb);
+  }
   FW_HIP(hipGetLastError());
   if (grid_used) *grid_used = (int)blocks;
   return FW_OK;
