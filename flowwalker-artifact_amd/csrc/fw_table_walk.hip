@@ -816,10 +816,12 @@ __device__ __forceinline__ uint32_t row_search(const float* row, uint32_t n, uin
 }
 
 // A look at one block of pairs for every lane with `need` (the lanes of m): first = the neighbour of its first key above t, at_start = that is the
-// block's first, none = there is none.  All lanes take part.  Eight lanes read a walker's block together, 16 bytes each, and eight walkers are
-// served by a load: a lane that loads its block alone makes eight requests to the first-level cache, each of which may wait for the address's translation.
+// block's first, none = there is none.  All lanes take part.  Four or eight lanes read a walker's block together, 16 bytes a load each: a lane that loads its block alone makes eight requests to the first-level cache, each of which may wait for the address's translation.
 // A lane for each block / eight lanes: DeepWalk R-MAT 24 (5 GB of regions) 4.9e9 / 0.95e9 translation misses, 66.4 / 35.5 ms; R-MAT 22 5.92 / 4.92 ms, node2vec
 // R-MAT 20 with q = 4 5.99 / 5.35; with row M and the pairs by each lane these were 47.4, 6.65 and 6.26.
+// Four lanes take half the instructions of eight, which counts where the blocks are near: eight / four, 20,108 DeepWalk walkers on R-MAT 12 0.184 / 0.160 ms, 50,021
+// node2vec walkers on R-MAT 20 0.461 / 0.433, 805,111 DeepWalk walkers on a uniform graph of 40,000 vertices 0.345 / 0.320, DeepWalk R-MAT 22 4.94 / 4.86; but a block that is not
+// kept is asked for in halves then: R-MAT 24 33.2 / 35.5.
 // A block comes once, and among gigabytes of them nobody wants it again before it is gone: there (kStream) it is not kept in the L2, which holds more
 // of the records and sums instead.
 typedef uint32_t u4_vec __attribute__((ext_vector_type(4)));
@@ -837,29 +839,39 @@ __device__ __forceinline__ BlockLook look_at_blocks(const unsigned char* data, c
   const int to = (int)(need ? rank : n + lane - rank) << 2;  // the lanes that look first, in order, then the others
   const int blocks = __builtin_amdgcn_ds_permute(to, (int)(need ? block : 0u));
   const int targets = __builtin_amdgcn_ds_permute(to, (int)__float_as_uint(t));
-  const uint32_t of = lane >> 3, piece = lane & 7u;
-  uint4 x[8];
+  constexpr uint32_t kLanes = kStream ? 8u : 4u, kParts = 8u / kLanes, kLoads = kLanes, kAt = 64u / kLanes;  // lanes a block, pieces a lane, blocks a load
+  const uint32_t of = lane / kLanes, piece = lane & (kLanes - 1u);
+  uint4 x[kLoads][kParts];
 #pragma unroll
-  for (uint32_t i = 0; i < 8u; ++i) {
-    if (8u * i < n) {
-      const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(8u * i + of) << 2, blocks);
+  for (uint32_t i = 0; i < kLoads; ++i) {
+    if (kAt * i < n) {
+      const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(kAt * i + of) << 2, blocks);
       const u4_vec* const at = reinterpret_cast<const u4_vec*>(data + (uint64_t)b * 128u + 16u * piece);
-      const u4_vec y = kStream ? __builtin_nontemporal_load(at) : *at;
-      x[i] = make_uint4(y[0], y[1], y[2], y[3]);
+#pragma unroll
+      for (uint32_t j = 0; j < kParts; ++j) {
+        const u4_vec y = kStream ? __builtin_nontemporal_load(at + 4u * j) : at[4u * j];
+        x[i][j] = make_uint4(y[0], y[1], y[2], y[3]);
+      }
     }
   }
   BlockLook r = {0u, false, true};
 #pragma unroll
-  for (uint32_t i = 0; i < 8u; ++i) {
-    if (8u * i < n) {
-      const float ti = __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)(8u * i + of) << 2, targets));
-      const bool c0 = !(__uint_as_float(x[i].x) <= ti);
-      const uint64_t m0 = __ballot(c0), any = m0 | __ballot(!(__uint_as_float(x[i].z) <= ti));
-      const uint32_t at = 8u * (rank & 7u);
-      const uint32_t above = (uint32_t)(any >> at) & 0xFFu;
-      const uint32_t f = at + (uint32_t)__builtin_ctz(above | 0x80u);
-      const uint32_t nb = (uint32_t)__builtin_amdgcn_ds_bpermute((int)f << 2, (int)(c0 ? x[i].y : x[i].w));
-      if (need && (rank >> 3) == i) r = {nb, ((m0 >> at) & 1ull) != 0ull, above == 0u};
+  for (uint32_t i = 0; i < kLoads; ++i) {
+    if (kAt * i < n) {
+      const float ti = __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)(kAt * i + of) << 2, targets));
+      const uint32_t at = kLanes * (rank & (kAt - 1u));
+      uint64_t m0 = 0ull;
+      uint32_t above = 0u, mine = x[i][kParts - 1u].w;
+#pragma unroll
+      for (uint32_t j = kParts; j-- > 0u;) {  // (where no lane has a key above t in the front half, all of them offer one of the back half)
+        const bool c0 = !(__uint_as_float(x[i][j].x) <= ti), c1 = !(__uint_as_float(x[i][j].z) <= ti);
+        m0 = __ballot(c0);
+        above |= ((uint32_t)((m0 | __ballot(c1)) >> at) & ((1u << kLanes) - 1u)) << (kLanes * j);
+        mine = c0 ? x[i][j].y : c1 ? x[i][j].w : mine;
+      }
+      const uint32_t f = at + ((uint32_t)__builtin_ctz(above | 0x80u) & (kLanes - 1u));
+      const uint32_t nb = (uint32_t)__builtin_amdgcn_ds_bpermute((int)f << 2, (int)mine);
+      if (need && rank / kAt == i) r = {nb, ((m0 >> at) & 1ull) != 0ull, above == 0u};
     }
   }
   return r;
