@@ -46,8 +46,8 @@ constexpr uint32_t kGroupUnits = kGq + 8u;      // units of a group in a list of
 constexpr uint32_t kNoRow = 16u;                // quartets of a list without row M: its entries are at most four blocks
 constexpr uint32_t kUneven = 0x80000000u;       // in vrec's region: row M first
 constexpr float kInf = __builtin_inff();
-// Waves per SIMD of the walk: 4, 5, 6 and 8 were measured (DeepWalk R-MAT 24 47.9 / 49.1 / 50.0 / 72.1 ms, the last one with
-// spilled registers; R-MAT 22 6.8 / 6.8 / 7.0 / 11.3): more walkers in flight only compete for the caches.
+// Waves per SIMD of the walk: 4, 5, 6 and 8 were measured while a step read row M (DeepWalk R-MAT 24 47.9 / 49.1 / 50.0 / 72.1 ms, the last
+// one with spilled registers; R-MAT 22 6.8 / 6.8 / 7.0 / 11.3): more walkers in flight only compete for the caches.
 constexpr int kWaves = 4;
 
 typedef float f4_at4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -1441,8 +1441,8 @@ __device__ __forceinline__ int64_t wave_set_find(const int32_t* __restrict__ set
   return __builtin_amdgcn_readlane(x, 15) == kSetOverflow ? -2 : -1;
 }
 
-// One wave, one walker.  Bound: latency, three dependent reads a step (four and five on long lists; node2vec one more a trial): 1.3 us a step of
-// 1,000 walkers on R-MAT 20, 2.0 where a lane walked each.
+// One wave, one walker.  Bound: latency, two dependent reads a step (three and four on long lists; node2vec one more a trial): 1.25 us a step of
+// 1,000 walkers on R-MAT 20, where a lane walked each 2.0 (100 walkers on a small graph 70.0 -> 67.3 us a call, 1,000 from hubs 124.2 -> 119.5, since row M is not read).
 template <int kApp>
 __global__ __launch_bounds__(256, kWalkerWaves) void fw_table_walk_wave(const fw_kargs a, const fw_table_args tb) {
   const uint32_t lane = (uint32_t)lane_id();
