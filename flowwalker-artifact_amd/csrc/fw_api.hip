@@ -2004,6 +2004,9 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
 // symmetrised 5.67 / 5.82, R-MAT 23 6.51 / 6.52, all of R-MAT 24, 80 steps 44.3 / 43.5.
 constexpr size_t kStreamPairsBytes = (size_t)2 << 30;
 
+// Regions up to which the walk takes their rows M to be in the caches (the eight L2 hold as much; measured at row_eighths).
+constexpr size_t kNearRowsBytes = (size_t)32 << 20;
+
 static fw_table_args table_args(const fw_graph* g, const fw_tables& t, unsigned long long* d_counters) {
   fw_table_args tb;
   tb.vrec = t.vrec;
@@ -2015,6 +2018,7 @@ static fw_table_args table_args(const fw_graph* g, const fw_tables& t, unsigned 
   tb.nw_shift = t.nw_shift;
   tb.long_lists = t.n_longs;
   tb.stream_pairs = t.data_bytes >= kStreamPairsBytes ? 1u : 0u;
+  tb.rows_near = t.data_bytes <= kNearRowsBytes ? 1u : 0u;
   tb.mean_list = (float)g->mean_list;
   tb.lanes = 0u;
   tb.counters = d_counters;

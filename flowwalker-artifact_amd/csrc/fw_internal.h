@@ -28,7 +28,7 @@ struct fw_label_set {
 // List tables (fw_table_walk.hip): the walker-independent part of every sampling step on a graph.  They belong to the graph, and only
 // a call that holds its busy flag makes, reads or drops them.
 struct fw_tables {
-  uint4* vrec = nullptr;          // [V] {region in 128-byte blocks, degree, total, CSR offset}
+  uint4* vrec = nullptr;          // [V] {region in 128-byte blocks (top bit: a list of one group that is entered through its row M), degree, total, CSR offset}
   unsigned char* data = nullptr;  // the regions
   size_t data_bytes = 0;          // room for them
   uint32_t* longs = nullptr;      // vertices whose lists have more than one group
@@ -236,6 +236,7 @@ struct fw_table_args {
   uint32_t nw_shift;
   uint32_t long_lists;           // lists of more than one group
   uint32_t stream_pairs;         // not 0: the blocks of pairs are not kept in the L2
+  uint32_t rows_near;            // not 0: the rows M are read in two fixed looks
   float mean_list;               // the list length a step meets, on average (below 0: not known)
   uint32_t lanes;                // lanes of a wave that walk, and the queries it takes at a time (set by the launch)
   unsigned long long* counters;  // [FW_TABLE_STRIPES * 8]

@@ -24,9 +24,9 @@
 //     a whole group never decrease, and the element is the first one whose key is above the target.
 //   Where the weights are close to evenly spread over a group the walk looks for that element from the proportional guess on and row M is not read: the
 //   block of the guess holds it for 65 % (1024 weights from 1 to 100) to 95 % of the targets, one next to it nearly always.  So a step reads some 1.4 blocks of
-//   a group, with row M it read 2.2 (DeepWalk R-MAT 24, symmetrised: 2.50e9 -> 1.84e9 blocks in all, 47.4 -> 35.5 ms).  A group a quarter of whose lanes end more
-//   than a block elsewhere has the sign of its total set, or in a list of one group the top bit of `region`, and is entered through row M (three blocks at most;
-//   from the guess on it would be five or six).
+//   a group, with row M it read 2.2 (DeepWalk R-MAT 24, symmetrised: 2.50e9 -> 1.84e9 blocks in all, 47.4 -> 35.5 ms).  A group whose weights are not (uneven_group)
+//   has the sign of its total set, or in a list of one group the top bit of `region`, and is entered through row M.  Of a full group that is one or two of row M's
+//   blocks and one of pairs; otherwise row M, which begins where the entries end, may lie in three blocks and a lane's pairs in two.
 //   sums: blocks of 16 running sums of a sequence's groups and their 16 totals, every sequence from a block of its own, filled up
 //     with the last sum; with more than one sequence (workgroup granularity) a block in front: the inclusive scan of the
 //     sequences' totals, as keys like the above (16 floats).
@@ -197,11 +197,17 @@ __device__ __forceinline__ void store_lane(uint2* out, uint32_t n, float e0, flo
   }
 }
 
-// Whether a quarter of a group's lanes end more than a block of 16 pairs from where even weights would have them.  M: the running maximum of the positive
-// lanes' prefixes; lanes: the nl lanes of the group's segment.
+// Whether a group is entered through row M: a quarter of its lanes end more than 20 pairs from where even weights would have them, or one in 32 more than
+// three blocks.  M: the running maximum of the positive lanes' prefixes; lanes: the nl lanes of the group's segment.
+// A wave's walkers wait for the one that looks most often, and row M is two reads more for all of them.  16 / 20 / 24 pairs, us: 50,000 DeepWalk walkers, weights log-normal
+// with sigma 1 on R-MAT 12 204 / 186 / 183, sigma 2 on R-MAT 20 414 / 424 / 440, Pareto 1.5 on R-MAT 16 360 / 370 / 381, even (1 to 100) on R-MAT 20 379 / 369 / 365.
+// Without / with the second condition, 100,000 walkers on lists of 1000 of whose 64 lanes twelve have next to nothing and the one among them the share of all: 688 / 470; the
+// others as before.  (Even weights: 278.)
 __device__ __forceinline__ bool uneven_group(const float M, const float T, const uint32_t c, const uint32_t nqg, const uint64_t lanes, const uint32_t nl) {
   const float d = M * (float)(4u * nqg) - T * (float)(4u * lane_start(c + 1u, nqg));
-  return 4u * (uint32_t)__builtin_popcountll(__ballot(!(__builtin_fabsf(d) <= 16.0f * T)) & lanes) > nl;
+  const uint32_t off = (uint32_t)__builtin_popcountll(__ballot(!(__builtin_fabsf(d) <= 20.0f * T)) & lanes);
+  const uint32_t far = (uint32_t)__builtin_popcountll(__ballot(!(__builtin_fabsf(d) <= 48.0f * T)) & lanes);
+  return 4u * off > nl || 32u * far > nl;
 }
 
 // One list of at most kSeg quartets per segment of kSeg lanes (one or two DPP rows, or the wave); off, deg, region are the
@@ -815,6 +821,23 @@ __device__ __forceinline__ uint32_t row_search(const float* row, uint32_t n, uin
   }
 }
 
+// The same in two looks: every eighth entry, then the eight that one of them ends.
+// Where row M is in the caches, or a wave has few walkers and waits for memory anyway, row_search's looks cost more than the other block of a row; elsewhere less.
+// row_search / this one, us: 1,000,000 DeepWalk walkers, log-normal weights with sigma 2, R-MAT 12 (1 MB of regions) 1201 / 1007, Pareto R-MAT 16 (25 MB) 2107 / 1952, R-MAT 20
+// (270 MB) 2654 / 2992, R-MAT 22 6337 / 7343; 50,000 walkers, R-MAT 20, 509 / 444.
+__device__ __forceinline__ uint32_t row_eighths(const float* row, uint32_t n, float t) {
+  const uint32_t e = (n + 7u) >> 3;
+  uint32_t k = 0u;
+#pragma unroll
+  for (uint32_t i = 0; i < 7u; ++i) k += row[8u * (i < e ? i : e - 1u) + 7u] <= t ? 1u : 0u;  // (the row's last entry is +inf)
+  const f4_at4 m0 = *reinterpret_cast<const f4_at4*>(row + 8u * k);
+  const f4_at4 m1 = *reinterpret_cast<const f4_at4*>(row + 8u * k + 4u);
+  uint32_t l = 8u * k;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) l += (i < 4 ? m0[i & 3] : m1[i & 3]) <= t ? 1u : 0u;
+  return l;
+}
+
 // A look at one block of pairs for every lane with `need` (the lanes of m): first = the neighbour of its first key above t, at_start = that is the
 // block's first, none = there is none.  All lanes take part.  Four or eight lanes read a walker's block together, 16 bytes a load each: a lane that loads its block alone makes eight requests to the first-level cache, each of which may wait for the address's translation.
 // A lane for each block / eight lanes: DeepWalk R-MAT 24 (5 GB of regions) 4.9e9 / 0.95e9 translation misses, 66.4 / 35.5 ms; R-MAT 22 5.92 / 4.92 ms, node2vec
@@ -1062,7 +1085,8 @@ __device__ __forceinline__ PairPlace table_pick(const fw_kargs& a, const fw_tabl
   if (uneven) {
     const uint32_t nl = nqg < 64u ? nqg : 64u;
     const float* const row = reinterpret_cast<const float*>(tb.data + (uint64_t)entries * 128u + 32u * nqg);
-    p.lo = p.b = lane_start(row_search(row, nl, (uint32_t)(tu * (float)nl), p.t), nqg) >> 2;
+    const uint32_t l = tb.rows_near != 0u ? row_eighths(row, nl, p.t) : row_search(row, nl, (uint32_t)(tu * (float)nl), p.t);
+    p.lo = p.b = lane_start(l, nqg) >> 2;
   }
   return p;
 }
@@ -1601,6 +1625,7 @@ int launch_table_walk(const fw_kargs& a, fw_table_args tb, int grid, hipStream_t
     const uint64_t most = (uint64_t)cus * 4u * kWaves;
     if (waves > most) waves = most;
   }
+  if (tb.lanes < 64u) tb.rows_near = 1u;  // (see row_eighths)
   const unsigned blocks = (unsigned)((waves + 3u) / 4u);
   if (kApp != FW_APP_METAPATH && tb.stream_pairs != 0u) {
     hipLaunchKernelGGL((fw_table_walk<kApp, kApp != FW_APP_METAPATH>), dim3(blocks), dim3(256), 0, stream, a, tb);

@@ -799,11 +799,11 @@ def test_which_kernel_walks_on_tables(gpu):
         g.destroy()
 
 
-@pytest.mark.parametrize("side", ["front", "back"])
+@pytest.mark.parametrize("few,side", [(14, "front"), (14, "back"), (14, "middle"), (5, "front"), (5, "back"), (5, "middle")])
 @pytest.mark.parametrize("wg,thr", [(512, 16384), (256, 1024)])
-def test_groups_with_a_lump(gpu, side, wg, thr):
-    """Weights evenly spread over most lanes of a group, while the share of some fourteen lies in one of them: too few for the group to be entered through its
-    row, and far enough off for every way the search for a block goes."""
+def test_groups_with_a_lump(gpu, few, side, wg, thr):
+    """Weights evenly spread over most lanes of a group, while the share of `few` of 64 lies in one of them.  Of five, no more than two lanes of a full group end beyond three
+    blocks of where even weights would have them: it is searched from the guess on, the element up to six blocks off.  Of fourteen it is entered through its row."""
     V = 400
     rng = np.random.RandomState(8)
     deg = np.r_[rng.randint(60, 70, size=100), rng.randint(120, 260, size=100), rng.randint(500, 1100, size=196), [2500, 4096, 9001, 20000]]
@@ -815,18 +815,56 @@ def test_groups_with_a_lump(gpu, side, wg, thr):
         i = np.arange(xadj[v], xadj[v + 1])
         lane = ((i >> 2) - (int(xadj[v]) >> 2)) % 64  # of the group's quartets lane, lane + 64, ..
         lanes = min(64, len(i) // 4)
-        first = 0 if side == "front" else lanes - 1
-        few = max(2, lanes * 14 // 64)
-        poor = (lane != first) & (lane < few if side == "front" else (lane >= lanes - few) & (lane < lanes))
+        poor_lanes = max(2, lanes * few // 64)
+        lo = {"front": 0, "back": lanes - poor_lanes, "middle": (lanes - poor_lanes) // 2}[side]
+        first = {"front": 0, "back": lanes - 1, "middle": lo + v % poor_lanes}[side]
+        poor = (lane != first) & (lane >= lo) & (lane < lo + poor_lanes)
         w[i[poor]] = 0.001
-        w[i[lane == first]] *= few
+        w[i[lane == first]] *= poor_lanes
     g = gpu.Graph.from_csr(xadj, adj, w)
     og = _oracle.Graph(xadj, adj, w)
     try:
         g.walk(gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21, wg_threads=wg, hub_threshold=thr), rng.randint(0, V, size=70000).astype(np.int32))
-        for grid, n in ((2, 3000), (0, 3000), (0, 9000)):
-            starts = rng.randint(0, V, size=n).astype(np.int32)
-            st = _compare(gpu, g, og, starts, gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=20, wg_threads=wg, hub_threshold=thr, seed=n, grid=grid), (side, grid, n))
-            assert g.engine()[0] == gpu.ENGINE_TABLES and (grid == 0 or st.grid == grid)
+        for kw in (dict(app=gpu.APP_DEEPWALK, max_depth=20), dict(app=gpu.APP_PPR, max_depth=30, tp=0.1), dict(app=gpu.APP_NODE2VEC, max_depth=12, p=0.25, q=4.0)):
+            for grid, n in ((2, 3000), (0, 3000), (0, 9000)):  # full waves of walkers, a wave per walker, a few walkers in each wave
+                starts = rng.randint(0, V, size=n).astype(np.int32)
+                st = _compare(gpu, g, og, starts, gpu.default_params(wg_threads=wg, hub_threshold=thr, seed=n, grid=grid, **kw), (few, side, kw, grid, n))
+                assert st.grid == grid if grid else (st.grid == (n + 3) // 4) == (n == 3000)
+    finally:
+        g.destroy()
+
+
+def _with_vertices(csr, more):
+    """The graph and `more` vertices of one edge each into it: a block of the tables' regions each."""
+    xadj, adj, w = csr
+    rng = np.random.RandomState(5)
+    n = len(xadj) - 1
+    return (np.concatenate([xadj, (len(adj) + 1 + np.arange(more)).astype(np.uint32)]), np.concatenate([adj, rng.randint(0, n, size=more).astype(np.int32)]),
+            np.concatenate([w, (1.0 + 4.0 * rng.random_sample(more)).astype(np.float32)]))
+
+
+@pytest.mark.parametrize("kind", ["even", "uneven"])
+@pytest.mark.parametrize("more,wg,thr", [(0, 512, 16384), (300000, 512, 16384), (300000, 1024, 2000)])
+def test_lists_of_every_shape_in_regions_of_every_size(gpu, more, kind, wg, thr):
+    """Rows of groups are read in one way up to 32 MiB of regions, or by waves of few walkers, and in another beyond that (300,000 vertices more are 38 MB)."""
+    csr, at = _lists(kind)
+    csr = _with_vertices(csr, more)
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    rng = np.random.RandomState(more + wg)
+    try:
+        p = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=21, wg_threads=wg, hub_threshold=thr)
+        for _ in range(40):
+            g.walk(p, at[rng.randint(0, len(at), size=70000)].astype(np.int32))
+            if g.engine()[0] == gpu.ENGINE_TABLES:
+                break
+        assert (g.engine()[2] > 38000000) == (more != 0)
+        cases = [dict(app=gpu.APP_DEEPWALK, max_depth=40), dict(app=gpu.APP_PPR, max_depth=40, tp=0.1), dict(app=gpu.APP_NODE2VEC, max_depth=20, p=2.0, q=0.5),
+                 dict(app=gpu.APP_NODE2VEC, max_depth=20, p=0.1, q=1.0)]
+        for i, kw in enumerate(cases):
+            for grid, n in ((3, 4000), (0, 9001)):
+                starts = np.where(rng.random_sample(n) < 0.8, at[rng.randint(0, len(at), size=n)], rng.randint(0, V + more, size=n)).astype(np.int32)
+                st = _compare(gpu, g, og, starts, gpu.default_params(wg_threads=wg, hub_threshold=thr, seed=30 + i, walker_base=i, grid=grid, **kw), (kw, grid, n))
+                assert st.grid == grid or (grid == 0 and st.grid != (n + 3) // 4)
     finally:
         g.destroy()
