@@ -1430,30 +1430,48 @@ __device__ __forceinline__ int32_t wave_pick(const fw_kargs& a, const fw_table_a
     T = __builtin_fabsf(T);
   }
   const float t = tu * T;
-  // two pairs a lane, from some before the guess on, or from the first of the lane that row M names
+  // Two pairs a lane, from some before the guess on, which mostly hold the one; what else may be needed stands out of the way, since the first look is all that
+  // a step mostly pays for (walks of 80 steps, look and repeats in one loop / so: 100 walkers on a small graph 67.6 / 64.9 us, 1,000 on R-MAT 20 113.8 / 109.3).  Of an uneven
+  // group row M comes at the same time (after it, as the pairs' place was found: log-normal weights with sigma 2, 1,000 walkers on R-MAT 20 129 us, now 121).
   const uint4* pairs = reinterpret_cast<const uint4*>(entries);
   const uint32_t n2 = 2u * nqg;
   const uint32_t guess = (uint32_t)(tu * (float)n2);
   const uint32_t wmax = n2 > 64u ? n2 - 64u : 0u;
   uint32_t w = guess > 32u ? guess - 32u : 0u;
-  if (uneven) {
-    const float m = lane < nqg ? reinterpret_cast<const float*>(entries + 32u * nqg)[lane] : kInf;
-    w = 2u * lane_start((uint32_t)__builtin_ctzll(__ballot(!(m <= t)) | (1ull << 63)), nqg);
-  }
   w = w < wmax ? w : wmax;
-  for (uint32_t lo = uneven ? w : 0u;;) {
-    uint4 p = make_uint4(0x7F800000u, 0u, 0x7F800000u, 0u);
-    if (w + lane < n2) p = pairs[w + lane];
-    const uint64_t m0 = __ballot(!(__uint_as_float(p.x) <= t)), m1 = __ballot(!(__uint_as_float(p.z) <= t));
-    if ((m0 | m1) == 0ull) {  // (the last pair's key is above: there are more)
-      lo = w = w + 64u;
-    } else if ((m0 & 1ull) != 0ull && w > lo) {
-      w = w > lo + 63u ? w - 63u : lo;
-    } else {
-      const uint32_t f = (uint32_t)__builtin_ctzll(m0 | m1);
-      return (int32_t)(((m0 >> f) & 1ull) != 0ull ? readlane_u32(p.y, f) : readlane_u32(p.w, f));
+  uint4 p = make_uint4(0x7F800000u, 0u, 0x7F800000u, 0u);
+  if (w + lane < n2) p = pairs[w + lane];
+  float m = kInf;
+  if (lane < (uneven ? nqg : 0u)) m = reinterpret_cast<const float*>(entries + 32u * nqg)[lane];
+  uint64_t m0 = __ballot(!(__uint_as_float(p.x) <= t)), above = m0 | __ballot(!(__uint_as_float(p.z) <= t));
+  if (__builtin_expect(uneven || above == 0ull || ((m0 & 1ull) != 0ull && w != 0u), 0)) {
+    if (uneven) {  // it names the lane whose pairs they are
+      const uint32_t l = (uint32_t)__builtin_ctzll(__ballot(!(m <= t)) | (1ull << 63));
+      const uint32_t first = 2u * lane_start(l, nqg);
+      if (first < w || 2u * lane_start(l + 1u, nqg) > w + 64u) {
+        w = first < wmax ? first : wmax;
+        if (w + lane < n2) p = pairs[w + lane];
+        m0 = __ballot(!(__uint_as_float(p.x) <= t));
+        above = m0 | __ballot(!(__uint_as_float(p.z) <= t));
+      }
+    } else {  // the pieces next to these (those of a group that is not marked are at most 48 from the guess: one look more)
+      for (uint32_t lo = 0u;;) {
+        if (above == 0ull) {  // (the last pair's key is above: there are more)
+          lo = w = w + 64u;
+        } else if ((m0 & 1ull) != 0ull && w > lo) {
+          w = w > lo + 63u ? w - 63u : lo;
+        } else {
+          break;
+        }
+        p = make_uint4(0x7F800000u, 0u, 0x7F800000u, 0u);
+        if (w + lane < n2) p = pairs[w + lane];
+        m0 = __ballot(!(__uint_as_float(p.x) <= t));
+        above = m0 | __ballot(!(__uint_as_float(p.z) <= t));
+      }
     }
   }
+  const uint32_t f = (uint32_t)__builtin_ctzll(above);
+  return (int32_t)(((m0 >> f) & 1ull) != 0ull ? readlane_u32(p.y, f) : readlane_u32(p.w, f));
 }
 
 // set_find by a wave, from the lane's place of the bucket (lanes 0 .. 15)
@@ -1467,7 +1485,7 @@ __device__ __forceinline__ int64_t wave_set_find(const int32_t* __restrict__ set
 }
 
 // One wave, one walker.  Bound: latency, two dependent reads a step (three and four on long lists; node2vec one more a trial): 1.25 us a step of
-// 1,000 walkers on R-MAT 20, where a lane walked each 2.0 (100 walkers on a small graph 70.0 -> 67.3 us a call, 1,000 from hubs 124.2 -> 119.5, since row M is not read).
+// 1,000 walkers on R-MAT 20, where a lane walked each 2.0 (100 walkers on a small graph 70.1 -> 64.6 us a call, 1,000 from hubs 124.2 -> 113.7, since only marked groups read row M).
 template <int kApp>
 __global__ __launch_bounds__(256, kWalkerWaves) void fw_table_walk_wave(const fw_kargs a, const fw_table_args tb) {
   const uint32_t lane = (uint32_t)lane_id();
