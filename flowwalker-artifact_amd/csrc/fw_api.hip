@@ -1998,7 +1998,7 @@ static int tables_for_call(fw_graph* g, const fw_walk_params* p, int32_t n, hipS
   return FW_OK;
 }
 
-// Regions from which on the walk's blocks of pairs are not kept in the L2, where smaller ones meet the next walker in the memory-side cache (256 MB).
+// Regions from which on calls of many walkers do not keep their blocks of pairs in the L2; which calls those are, see launch_table_walk.
 // Kept / not kept, ms, 4,000,000 walks of 80 steps where not said: DeepWalk R-MAT 22 (4,194,304, 0.7 GB) 5.00 / 5.33, symmetrised (1.4 GB) 7.90 / 8.20, R-MAT 23
 // (1.4 GB) 5.87 / 5.90, symmetrised (2.7 GB) 9.84 / 9.29, R-MAT 24 (2.7 GB) 7.14 / 6.79, symmetrised, 16,777,216 (5.2 GB) 36.1 / 33.1; node2vec of 40 steps R-MAT 22
 // symmetrised 5.67 / 5.82, R-MAT 23 6.51 / 6.52, all of R-MAT 24, 80 steps 44.3 / 43.5.

@@ -235,7 +235,7 @@ struct fw_table_args {
   fw_label_set labels;
   uint32_t nw_shift;
   uint32_t long_lists;           // lists of more than one group
-  uint32_t stream_pairs;         // not 0: the blocks of pairs are not kept in the L2
+  uint32_t stream_pairs;         // not 0: so many regions that calls of many walkers do not keep their blocks of pairs in the L2
   uint32_t rows_near;            // not 0: the rows M are read in two fixed looks
   float mean_list;               // the list length a step meets, on average (below 0: not known)
   uint32_t lanes;                // lanes of a wave that walk, and the queries it takes at a time (set by the launch)

@@ -1645,11 +1645,21 @@ int launch_table_walk(const fw_kargs& a, fw_table_args tb, int grid, hipStream_t
   }
   if (tb.lanes < 64u) tb.rows_near = 1u;  // (see row_eighths)
   const unsigned blocks = (unsigned)((waves + 3u) / 4u);
-  if (kApp != FW_APP_METAPATH && tb.stream_pairs != 0u) {
-    hipLaunchKernelGGL((fw_table_walk<kApp, kApp != FW_APP_METAPATH>), dim3(blocks), dim3(256), 0, stream, a, tb);
-  } else {
-    hipLaunchKernelGGL((fw_table_walk<kApp, false>), dim3(blocks), dim3(256), 0, stream, a, tb);
+  // Blocks of pairs from gigabytes of regions are not kept in the L2 where many walkers ask for them.  Kept / not kept, us, walks of 80 steps, 40 for node2vec: R-MAT 24
+  // (2.7 GB) DeepWalk 20,000 walkers 306 / 341, 50,000 383 / 399, 200,000 561 / 572, 400,000 769 / 797, 1,000,000 1682 / 1608, from 2,048 hubs 3166 / 2964; symmetrised (5.2 GB) 200,000
+  // 672 / 688, 400,000 1409 / 1365, 1,000,000 2683 / 2524, from hubs 4214 / 3865; node2vec there 200,000 968 / 991, 400,000 1064 / 1066, 1,000,000 of 20 steps from hubs 1426 / 1404;
+  // R-MAT 23 symmetrised (2.7 GB) DeepWalk 200,000 640 / 657, 400,000 1368 / 1345, 1,000,000 2511 / 2379, node2vec 400,000 1047 / 1063.  PPR gains nowhere, its walks are short:
+  // 200,000 walkers on R-MAT 24 179 / 195, 1,000,003 from the longest list 539 / 548, 4,000,000 1067 / 1069, all 16,777,216 3632 / 3672; symmetrised 224 / 243, 614 / 621, 1172 / 1178.
+  constexpr uint32_t kStreamWalkers = 1u << 19;
+  if constexpr (kApp == FW_APP_DEEPWALK || kApp == FW_APP_NODE2VEC) {
+    if (tb.stream_pairs != 0u && n >= kStreamWalkers) {
+      hipLaunchKernelGGL((fw_table_walk<kApp, true>), dim3(blocks), dim3(256), 0, stream, a, tb);
+      FW_HIP(hipGetLastError());
+      if (grid_used) *grid_used = (int)blocks;
+      return FW_OK;
+    }
   }
+  hipLaunchKernelGGL((fw_table_walk<kApp, false>), dim3(blocks), dim3(256), 0, stream, a, tb);
   FW_HIP(hipGetLastError());
   if (grid_used) *grid_used = (int)blocks;
   return FW_OK;

@@ -868,3 +868,45 @@ def test_lists_of_every_shape_in_regions_of_every_size(gpu, more, kind, wg, thr)
                 assert st.grid == grid or (grid == 0 and st.grid != (n + 3) // 4)
     finally:
         g.destroy()
+
+
+@pytest.mark.parametrize("kind", ["even", "uneven"])
+@pytest.mark.parametrize("wg,thr", [(512, 16384), (1024, 2000)])
+def test_lists_of_every_shape_in_gigabytes_of_regions(gpu, kind, wg, thr):
+    """From 2 GiB of regions on (2^24 vertices more) and 2^19 walkers on, DeepWalk and node2vec do not keep blocks of pairs and read them by eight lanes: every row against calls of
+    half as many walkers, which keep them, some against the oracle.  PPR keeps them."""
+    csr, at = _lists(kind)
+    more = 1 << 24
+    csr = _with_vertices(csr, more)
+    g = gpu.Graph.from_csr(*csr)
+    og = _oracle.Graph(*csr)
+    rng = np.random.RandomState(wg)
+    n = (1 << 19) + 333
+    half = n // 2
+    starts = np.where(rng.random_sample(n) < 0.8, at[rng.randint(0, len(at), size=n)], rng.randint(0, V + more, size=n)).astype(np.int32)
+    try:
+        p = gpu.default_params(app=gpu.APP_DEEPWALK, max_depth=41, wg_threads=wg, hub_threshold=thr)
+        for _ in range(60):
+            g.walk(p, starts)
+            if g.engine()[0] == gpu.ENGINE_TABLES:
+                break
+        assert g.engine()[2] > 2 << 30
+        for i, kw in enumerate((dict(app=gpu.APP_DEEPWALK, max_depth=20), dict(app=gpu.APP_DEEPWALK, max_depth=7), dict(app=gpu.APP_PPR, max_depth=30, tp=0.1),
+                                dict(app=gpu.APP_NODE2VEC, max_depth=12, p=2.0, q=0.5), dict(app=gpu.APP_NODE2VEC, max_depth=12, p=0.1, q=4.0))):
+            for grid in (0, 7):
+                p = gpu.default_params(wg_threads=wg, hub_threshold=thr, seed=60 + i, grid=grid, **kw)
+                paths, st = g.walk(p, starts)
+                assert g.engine()[0] == gpu.ENGINE_TABLES and grid in (0, st.grid)
+                steps = edges = 0
+                for a, b in ((0, half), (half, n)):
+                    p.walker_base = a
+                    ref, s = g.walk(p, starts[a:b])
+                    assert (paths[a:b] == ref).all(), (kw, grid, a)
+                    steps, edges = steps + s.steps, edges + s.sampled_edges
+                assert (st.steps, st.sampled_edges) == (steps, edges)
+            for a in (0, half - 500, n - 1500):
+                p.walker_base = a
+                ref, _, _ = _oracle.walk(og, _oracle.from_walk_params(p), starts[a:a + 1500])
+                assert (paths[a:a + 1500] == ref).all(), (kw, a)
+    finally:
+        g.destroy()
