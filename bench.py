@@ -83,13 +83,13 @@ def algorithmic_bytes(app, steps, sampled_edges, queries):
     return 4 * sampled_edges + 16 * steps + 16 * queries
 
 
-def roofline_of(app, st, n, kernel_ms, tables=False):
+def roofline_of(app, st, n, kernel_ms):
     """HBM roofline of one pass on three bases, all over the same device time.
     * `achieved` / `frac`: what the kernels asked of the memory, MODELLED from the run's own counters
       (fw_walk_stats: lists as often as they were actually streamed + 128 bytes per scattered read + 32 bytes per
-      scattered store + the records streamed; `breakdown` has the parts).  For DeepWalk, PPR and node2vec on list tables the
-      library charges three blocks per step; here it is the two that every step touches, its vertex's record and one block
-      of pairs (second looks, sums and turned-down trials not counted, blocks found in the caches counted).
+      scattered store + the records streamed; `breakdown` has the parts).  On list tables those are the two blocks that
+      every step touches, its vertex's record and one block of pairs, and node2vec's test (second looks, sums and
+      turned-down trials not counted, blocks found in the caches counted).
     * `useful_frac`: the part of it an implementation cannot avoid once lists are shared: the list bytes streamed
       + 16 bytes per step + 16 bytes per query.
     * `algorithmic_rate` / `algorithmic_frac`: the bytes every walker would read on its own (4*D + 16*S + 16*Q; node2vec
@@ -97,8 +97,7 @@ def roofline_of(app, st, n, kernel_ms, tables=False):
       batch of walkers, so this exceeds the peak; `reuse_factor` = algorithmic / modelled says by how much lists were
       shared.  Without parking (roofline.no_parking) it is the fraction of the roofline the walk kernel reaches."""
     alg = algorithmic_bytes(app, st.steps, st.sampled_edges, n)
-    reads = int(st.scattered_reads) - (int(st.steps) if tables and app != "metapath" else 0)
-    req = int(st.requested_bytes) - 128 * (int(st.scattered_reads) - reads)
+    req = int(st.requested_bytes)
     sec = kernel_ms * 1e-3
     useful = int(st.list_bytes) + 16 * int(st.steps) + 16 * n
     return {
@@ -107,7 +106,7 @@ def roofline_of(app, st, n, kernel_ms, tables=False):
         "bytes_basis": "modelled from the run's counters (lists as streamed + 128 B per scattered read + 32 B per "
                        "scattered store + records)",
         "requested_bytes": req,
-        "breakdown": {"list_bytes": int(st.list_bytes), "scattered_read_bytes": 128 * reads,
+        "breakdown": {"list_bytes": int(st.list_bytes), "scattered_read_bytes": 128 * int(st.scattered_reads),
                       "scattered_write_bytes": 32 * int(st.scattered_writes), "record_bytes": int(st.record_bytes)},
         "useful_bytes": useful, "useful_frac": useful / sec / 1e9 / HBM_PEAK_GBS,
         "algorithmic_bytes": int(alg), "algorithmic_rate": alg / sec / 1e9,
@@ -161,7 +160,7 @@ def one_config(fw, g, name, wl, passes, warmup, **overrides):
         d_starts.free()
         d_paths.free()
     kernel_ms = float(np.mean(ms))
-    r = roofline_of(wl["app"], st, n, kernel_ms, g.engine()[0] == fw.ENGINE_TABLES)
+    r = roofline_of(wl["app"], st, n, kernel_ms)
     return {
         "config": CONFIG_OF.get(name, name), "workload": name, "app": wl["app"], "vertices": g.V, "csr_entries": g.E,
         "queries": n, "walk_steps_per_pass": int(st.steps), "passes": passes, "device_ms_per_pass": kernel_ms,
@@ -196,7 +195,7 @@ def config1(fw):
             _, st = g.walk(params, starts)
             ms.append(st.kernel_ms)
         kernel_ms = float(np.mean(ms))
-        r = roofline_of("deepwalk", st, 100, kernel_ms, g.engine()[0] == fw.ENGINE_TABLES)
+        r = roofline_of("deepwalk", st, 100, kernel_ms)
         return {"config": "C1", "workload": "deepwalk_uniform_7115", "app": "deepwalk", "vertices": V, "csr_entries": E,
                 "queries": 100, "walk_steps_per_pass": int(st.steps), "passes": 5, "device_ms_per_pass": kernel_ms,
                 "steps_per_s": st.steps / (kernel_ms * 1e-3), "launches_per_pass": st.launches, "frac": r["frac"],
@@ -320,7 +319,7 @@ def main():
     ms_per_step = wall * 1e3 / args.steps
     value = steps_per_pass * args.steps / wall
     avg_kernel_ms = float(np.mean(kernel_ms))
-    roofline = roofline_of(wl["app"], last, n, avg_kernel_ms, engine == fw.ENGINE_TABLES)
+    roofline = roofline_of(wl["app"], last, n, avg_kernel_ms)
     roofline["kernel"] = kernel_of(fw, engine, args.sampler, last, n)
     # the profiler's view of the same workload (library defaults only: any override makes it another run)
     sources_sha = fw.sources_sha()

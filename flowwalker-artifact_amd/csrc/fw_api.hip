@@ -1582,13 +1582,13 @@ static TrafficModel traffic_model(const fw_walk_params* p, int32_t n, bool parke
 }
 
 
-// The same for a walk on list tables; path entries leave in lines.  A step reads its vertex's record, one or two blocks of the list's pairs and for lists of
-// several groups a block of sums, three in all, for MetaPath the record and one neighbour; node2vec tests the accepted neighbour of all but a walk's first step in
-// N(prev).  Blocks that are found in the caches are charged too, node2vec's turned-down trials are not (the counters, past the L2: DeepWalk R-MAT 24 2.6 blocks a step, node2vec
-// 3.2 with its trials).
+// The same for a walk on list tables; path entries leave in lines.  A step is charged the two blocks that it cannot do without, its vertex's record and one block of the
+// list's pairs, for MetaPath one of neighbours; node2vec tests the accepted neighbour of all but a walk's first step in N(prev).  Blocks that are found in the caches are charged
+// too; second blocks of pairs, rows, sums and node2vec's turned-down trials are not.  Counted past the L2 (charged), blocks a step: DeepWalk R-MAT 24 2.4
+// (2.0), R-MAT 22 2.0 (2.0), node2vec R-MAT 24 with its trials 3.1 (3.0), PPR R-MAT 22 2.0 (2.4 with a read per start vertex).
 static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params* p, int32_t n, bool sets, uint64_t steps) {
   TrafficModel m;
-  m.scattered_reads = (p->app == FW_APP_METAPATH ? 2 : 3) * steps + (uint64_t)n;
+  m.scattered_reads = 2 * steps + (uint64_t)n;
   if (p->app == FW_APP_NODE2VEC && steps > (uint64_t)n) m.scattered_reads += (sets ? 1 : 4) * (steps - (uint64_t)n);  // a hash set, or a search
   m.scattered_writes = steps / 16u + 2u * (uint64_t)n;            // whole lines, the row's first and last entries
   m.record_bytes = 4 * (uint64_t)n + 4 * (uint64_t)n * (uint64_t)p->max_depth;

@@ -139,8 +139,10 @@ typedef struct {
    * scattered_writes: stores of one 32-byte write request each (path entry, scattered record); record_bytes: walker
    * records, tasks and bucket tables that are streamed.  Tables that stay in the L2 are not priced.  This sits
    * between the algorithmic bytes of src/main.cu:93-111 (4 * sampled_edges + ...) and what a profiler's HBM counters
-   * see; it is an estimate, the counters are the measurement.  For calls without parking it is a lower bound: the
-   * neighbours that short lists bring along with their biases are priced as one block per step. */
+   * see; it is an estimate, the counters are the measurement.  For calls that stream lists without parking it is a lower
+   * bound: the neighbours that short lists bring along with their biases are priced as one block per step.  A walk on
+   * list tables is charged two blocks per step, the vertex's record and one of the list's entries (node2vec three from a
+   * walk's second step on), whether the caches hold them or not; further blocks that a step may look at are not charged. */
   uint64_t requested_bytes;
   uint64_t list_bytes;
   uint64_t scattered_reads;
