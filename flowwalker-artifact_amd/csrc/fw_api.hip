@@ -1599,7 +1599,7 @@ static TrafficModel table_traffic_model(const fw_graph* g, const fw_walk_params*
 
 // ---- list tables: when, and making them ---------------------------------------------------------------------
 //
-// A walk on list tables reads some three blocks of memory per step, whatever the lists' lengths; without them a step
+// A walk on list tables reads two to three blocks of memory per step, whatever the lists' lengths; without them a step
 // reads its list, or shares it with the others that are parked there.  The tables are made once the calls on a graph have spent without
 // them (measured) or are about to spend (estimated) a quarter more than making them takes: a first call makes them only if it gains by
 // that itself, and a loop of small calls gets them after a few and never pays more than about twice what it would have.

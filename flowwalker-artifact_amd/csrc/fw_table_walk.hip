@@ -24,7 +24,8 @@
 //     a whole group never decrease, and the element is the first one whose key is above the target.
 //   Where the weights are close to evenly spread over a group the walk looks for that element from the proportional guess on and row M is not read: the
 //   block of the guess holds it for 65 % (1024 weights from 1 to 100) to 95 % of the targets, one next to it nearly always.  So a step reads some 1.4 blocks of
-//   a group, with row M it read 2.2 (DeepWalk R-MAT 24, symmetrised: 2.50e9 -> 1.84e9 blocks in all, 47.4 -> 35.5 ms).  A group whose weights are not (uneven_group)
+//   a group, with row M it read 2.2 (DeepWalk R-MAT 24, symmetrised: 2.50e9 -> 1.72e9 blocks in all, 47.4 -> 32.8 ms, of which
+//   1.84e9 and 35.5 while its blocks were kept in the L2).  A group whose weights are not (uneven_group)
 //   has the sign of its total set, or in a list of one group the top bit of `region`, and is entered through row M.  Of a full group that is one or two of row M's
 //   blocks and one of pairs; otherwise row M, which begins where the entries end, may lie in three blocks and a lane's pairs in two.
 //   sums: blocks of 16 running sums of a sequence's groups and their 16 totals, every sequence from a block of its own, filled up
@@ -907,7 +908,8 @@ struct PairPlace {
   float t;
 };
 
-// That neighbour, for the lanes with `need`; all lanes take part.  From the guess on block after block; after three looks what is left is halved.
+// That neighbour, for the lanes with `need`; all lanes take part.  From the guess on block after block; after four looks what is left is halved
+// (which few meet: but for one lane in 32 the pairs of a group that is not marked lie within five blocks of their guess, and a shorter list has five at most).
 template <bool kStream>
 __device__ __forceinline__ uint32_t pair_search(const unsigned char* data, bool need, PairPlace p, const uint32_t lane) {
   const uint32_t top = (p.n - 1u) >> 4;
@@ -1609,12 +1611,13 @@ int launch_table_walk(const fw_kargs& a, fw_table_args tb, int grid, hipStream_t
   uint64_t waves;
   if constexpr (kApp != FW_APP_METAPATH) {  // (whose step is two reads, and no search)
     // As many walkers as there are waves resident: a wave each.  Measured, wave per walker / lane per walker, us of a call of 40 steps on R-MAT 20,
-    // symmetrised: 1,000 walkers DeepWalk 73 / 92, PPR 52 / 76, node2vec 164 / 245; 8,000: 121 / 172, 72 / 94, 227 / 345 (q = 4: 555 / 760);
-    // with two walks a wave (16,000): 261 / 191, 238 / 99, 367 / 422; a uniform graph of mean degree 4: 1,000 47 / 66, 42 / 61, 71 / 99; 8,192 DeepWalk 87 / 94, PPR 51 / 71.
+    // symmetrised: 1,000 walkers DeepWalk 62 / 89, PPR 53 / 81, node2vec 109 / 172; 8,000: 100 / 145, 61 / 88, 174 / 280 (q = 4: 457 / 704); twice as many walkers as
+    // waves fit (16,000): 146 / 162, 67 / 94, 269 / 328, where the line does not lie yet; a uniform graph of mean degree 4: 1,000 47 / 68, 39 / 54, 74 / 91; 8,192 DeepWalk 78 / 85, PPR 50 / 71.
     // Lists of one group leave a wave little to search, and node2vec's tests are made for one walker at a time, so where few proposals are turned down fewer waves
-    // per SIMD already cost more than lanes do.  Uniform graphs of mean degree 4 to 200, q = 0.5: 7,000 walkers 146 / 132, 8,192 157 / 135; without adjacency tests,
-    // p = 1: 5,120 110 / 92, 5,500 121 / 94, 8,192 144 / 102.  Some lists of two groups, q = 1: mean list 144 (R-MAT 14) 5,500 105 / 94, 6,144 111 / 96; mean list 192
-    // (R-MAT 12) 6,144 119 / 109, but with p = 2 123 / 128.  With q = 2 on these, on lists of 300 on average, and for DeepWalk waves win throughout.
+    // per SIMD already cost more than lanes do.  Uniform graphs of mean degree 4 and 40, q = 0.5: 6,144 walkers 124 / 120 and 125 / 131, 7,000 135 / 120 and 136 / 132, 8,192 142 / 122 and 147 / 135;
+    // without adjacency tests, p = 1, q = 1: 4,096 91 / 91 and 94 / 98, 5,500 113 / 94 and 115 / 102.  Before waves and lanes searched from the guess, some lists of two groups, p = q = 1: mean list
+    // 144 (R-MAT 14) 5,500 105 / 94, 6,144 111 / 96; mean list 192 (R-MAT 12) 6,144 119 / 109, but with p = 2 123 / 128.  With q = 2 on these, on lists of 300 on average, and for
+    // DeepWalk waves win throughout.
     uint32_t per_simd = kWalkerWaves;
     if (kApp == FW_APP_NODE2VEC && a.inv_q >= 1.0f && tb.mean_list > 0.0f && tb.mean_list <= 256.0f)
       per_simd = a.inv_q == 1.0f ? (tb.long_lists == 0u ? 4u : 5u) : (tb.long_lists == 0u ? 6u : kWalkerWaves);
