@@ -1653,9 +1653,11 @@ int launch_table_walk(const fw_kargs& a, fw_table_args tb, int grid, hipStream_t
   // 672 / 688, 400,000 1409 / 1365, 1,000,000 2683 / 2524, from hubs 4214 / 3865; node2vec there 200,000 968 / 991, 400,000 1064 / 1066, 1,000,000 of 20 steps from hubs 1426 / 1404;
   // R-MAT 23 symmetrised (2.7 GB) DeepWalk 200,000 640 / 657, 400,000 1368 / 1345, 1,000,000 2511 / 2379, node2vec 400,000 1047 / 1063.  PPR gains nowhere, its walks are short:
   // 200,000 walkers on R-MAT 24 179 / 195, 1,000,003 from the longest list 539 / 548, 4,000,000 1067 / 1069, all 16,777,216 3632 / 3672; symmetrised 224 / 243, 614 / 621, 1172 / 1178.
+  // node2vec that has no hash sets yet searches lists for its tests, which the L2 then holds more of: R-MAT 24 50,021 walkers of 41 steps 502 / 470, 129,000 635 / 625, log-normal weights
+  // with sigma 1 50,021 550 / 519, R-MAT 23 symmetrised 744 / 740, 892 / 902, R-MAT 24 symmetrised 769 / 778, 912 / 930; with sets 50,021 on R-MAT 24 285 / 293.
   constexpr uint32_t kStreamWalkers = 1u << 19;
   if constexpr (kApp == FW_APP_DEEPWALK || kApp == FW_APP_NODE2VEC) {
-    if (tb.stream_pairs != 0u && n >= kStreamWalkers) {
+    if (tb.stream_pairs != 0u && (n >= kStreamWalkers || (kApp == FW_APP_NODE2VEC && tb.sets == nullptr))) {
       hipLaunchKernelGGL((fw_table_walk<kApp, true>), dim3(blocks), dim3(256), 0, stream, a, tb);
       FW_HIP(hipGetLastError());
       if (grid_used) *grid_used = (int)blocks;

@@ -875,7 +875,7 @@ def test_lists_of_every_shape_in_regions_of_every_size(gpu, more, kind, wg, thr)
 @pytest.mark.parametrize("wg,thr", [(512, 16384), (1024, 2000)])
 def test_lists_of_every_shape_in_gigabytes_of_regions(gpu, kind, wg, thr):
     """From 2 GiB of regions on (2^24 vertices more) and 2^19 walkers on, DeepWalk and node2vec do not keep blocks of pairs and read them by eight lanes: every row against calls of
-    half as many walkers, which keep them, some against the oracle.  PPR keeps them."""
+    half as many walkers, which keep them (node2vec when it has its hash sets), some against the oracle.  PPR keeps them."""
     csr, at = _lists(kind)
     more = 1 << 24
     csr = _with_vertices(csr, more)
